@@ -18,6 +18,7 @@
 // (a slot with two entries inside the band) sends the row to the full re-score.
 #pragma once
 
+#include "km_bounds.hpp"
 #include "km_common.hpp"
 
 namespace km {
@@ -45,12 +46,15 @@ struct top2 {
     }
 };
 
-// Settle one row from its slots (see the file comment).  X = ||x|| rounded up,
-// C = max_j ||c_j|| rounded up.
+// Settle one row from its slots (see the file comment).  X = ||x|| rounded up (to
+// a float: ||x|| >= X (1 - 1.2e-7)), C = max_j ||c_j|| rounded up.  With bounds kept
+// (rs.gap), a row settled here leaves its gap; a row sent to a re-score leaves
+// -inf (assigned again by the next pass).
 template <typename F>
 __device__ __forceinline__ void decide_row(int64_t row, const top2<F>* slots, int nslots,
                                            const band_consts& bc, double X, double C,
-                                           int32_t* __restrict__ labels, const refine_lists& L) {
+                                           int32_t* __restrict__ labels, const refine_lists& L,
+                                           const row_select& rs) {
     F best = fp_traits<F>::inf;
     int bi = -1;
     for (int s = 0; s < nslots; ++s) {
@@ -69,6 +73,21 @@ __device__ __forceinline__ void decide_row(int64_t row, const top2<F>* slots, in
             if (cnt < MAXC) cand[cnt] = slots[s].i1;
             cnt++;
         }
+    }
+    if (rs.gap) {
+        float g = -__builtin_inff();
+        if (cert && cnt == 1) {
+            F second = fp_traits<F>::inf;
+            for (int s = 0; s < nslots; ++s) {
+                const F v = slots[s].i1 == bi ? slots[s].m2 : slots[s].m1;
+                second = v < second ? v : second;
+            }
+            const double da = bc.a_xc * X * C + bc.a_cc * C * C;
+            const double X2 = X * X;
+            g = bound_gap(double(best) + da + X2 + (X2 + fabs(double(best))) * 1e-15,
+                          double(second) - da + X2 * (1.0 - 3e-7), rs.gam, rs.base[bi]);
+        }
+        rs.gap[row] = g;
     }
     if (cert && cnt == 1) {
         labels[row] = bi;
@@ -94,7 +113,7 @@ template <typename F>
 __global__ __launch_bounds__(256) void assign_generic_kernel(
     const F* __restrict__ X, int64_t n, int d, const F* __restrict__ C, int k,
     const F* __restrict__ cn, const float* __restrict__ xnorm_up, const double* __restrict__ cmax_p,
-    band_consts bc, int32_t* __restrict__ labels, refine_lists L) {
+    band_consts bc, int32_t* __restrict__ labels, refine_lists L, row_select rs) {
     constexpr int TN = 64, TM = 64, KC = 16, PAD = 4;
     __shared__ __align__(16) F Xs[KC][TN + PAD];
     __shared__ __align__(16) F Cs[KC][TM + PAD];
@@ -104,10 +123,14 @@ __global__ __launch_bounds__(256) void assign_generic_kernel(
     const int tx = tid & 15;   // centroid group
     const int ty = tid >> 4;   // row group
     const double cmax = *cmax_p;
-    const int64_t ntiles = (n + TN - 1) / TN;
+    const int64_t nsel = select_rows(rs, n);
+    const int64_t ntiles = (nsel + TN - 1) / TN;
+    __shared__ int64_t tile_row[TN];
 
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const int64_t n0 = tile * TN;
+        if (tid < TN) tile_row[tid] = n0 + tid < nsel ? select_row(rs, n0 + tid) : -1;
+        __syncthreads();
         top2<F> st[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) st[i].init();
@@ -125,9 +148,9 @@ __global__ __launch_bounds__(256) void assign_generic_kernel(
                 for (int r = 0; r < 4; ++r) {
                     const int e = tid + r * 256;
                     const int f = e & 15, p = e >> 4;
-                    const int64_t row = n0 + p;
+                    const int64_t row = tile_row[p];
                     const int col = k0 + f;
-                    Xs[f][p] = (row < n && col < d) ? X[row * d + col] : F(0);
+                    Xs[f][p] = (row >= 0 && col < d) ? X[row * d + col] : F(0);
                     const int cj = m0 + p;
                     Cs[f][p] = (cj < k && col < d) ? C[int64_t(cj) * d + col] : F(0);
                 }
@@ -161,9 +184,9 @@ __global__ __launch_bounds__(256) void assign_generic_kernel(
         for (int i = 0; i < 4; ++i) slots[ty * 4 + i][tx] = st[i];
         __syncthreads();
         if (tid < TN) {
-            const int64_t row = n0 + tid;
-            if (row < n) {
-                decide_row<F>(row, slots[tid], 16, bc, double(xnorm_up[row]), cmax, labels, L);
+            const int64_t row = tile_row[tid];
+            if (row >= 0) {
+                decide_row<F>(row, slots[tid], 16, bc, double(xnorm_up[row]), cmax, labels, L, rs);
             }
         }
         __syncthreads();
@@ -213,7 +236,7 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : 2) void assign_mfma_f32_kernel
     const float* __restrict__ X, int64_t ldx, int64_t n, int d, const float* __restrict__ Cpad, int k,
     const float* __restrict__ cn, const float* __restrict__ xnorm_up,
     const double* __restrict__ cmax_p, band_consts bc, int32_t* __restrict__ labels,
-    refine_lists L) {
+    refine_lists L, row_select rs) {
     constexpr int HALF = DP / 2;
     constexpr int CST = DP + 4;
     constexpr int ROWS_PER_WAVE = 32 * NB;
@@ -229,7 +252,8 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : 2) void assign_mfma_f32_kernel
     const double cmax = *cmax_p;
     const int mblocks = (k + 31) / 32;
     const int kp = mblocks * 32;
-    const int64_t ntiles = (n + ROWS_PER_WG - 1) / ROWS_PER_WG;
+    const int64_t nsel = select_rows(rs, n);
+    const int64_t ntiles = (nsel + ROWS_PER_WG - 1) / ROWS_PER_WG;
 
     float* Cs = smem;                                   // RES: kp rows; else 2 x 32 rows
     float* Cn = smem + (RES ? kp : 64) * CST;           // RES: kp; else 2 x 32
@@ -279,9 +303,9 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : 2) void assign_mfma_f32_kernel
         const int64_t wrow0 = tile * ROWS_PER_WG + int64_t(wave) * ROWS_PER_WAVE;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            const int64_t row = wrow0 + nb * 32 + r32;
-            const bool ok = tile < ntiles && row < n;
-            const float* src = X + (ok ? row : 0) * ldx;
+            const int64_t e = wrow0 + nb * 32 + r32;
+            const bool ok = tile < ntiles && e < nsel;
+            const float* src = X + (ok ? select_row(rs, e) : 0) * ldx;
 #pragma unroll
             for (int s = 0; s < HALF; s += 4) {
                 const int f = h * HALF + s;
@@ -394,9 +418,11 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : 2) void assign_mfma_f32_kernel
                 sl[2 + q].i1 = __shfl_xor(st[nb][q].i1, 32);
                 sl[2 + q].i2 = __shfl_xor(st[nb][q].i2, 32);
             }
-            const int64_t row = wrow0 + nb * 32 + r32;
-            if (h == 0 && row < n)
-                decide_row<float>(row, sl, 4, bc, double(xnorm_up[row]), cmax, labels, L);
+            const int64_t e = wrow0 + nb * 32 + r32;
+            if (h == 0 && e < nsel) {
+                const int64_t row = select_row(rs, e);
+                decide_row<float>(row, sl, 4, bc, double(xnorm_up[row]), cmax, labels, L, rs);
+            }
         }
     }
 }
@@ -428,7 +454,7 @@ __global__ __launch_bounds__(256, 2) void assign_mfma_f64_kernel(
     const double* __restrict__ X, int64_t ldx, int64_t n, int d, const double* __restrict__ Cpad, int k,
     const double* __restrict__ cn, const float* __restrict__ xnorm_up,
     const double* __restrict__ cmax_p, band_consts bc, int32_t* __restrict__ labels,
-    refine_lists L) {
+    refine_lists L, row_select rs) {
     constexpr int Q = DP / 4;           // features per lane (and MFMA steps per block)
     constexpr int CST = mfma_f64_cst(DP);
     constexpr int ROWS_PER_WAVE = 16 * NB;
@@ -442,16 +468,17 @@ __global__ __launch_bounds__(256, 2) void assign_mfma_f64_kernel(
     const int r16 = lane & 15;
     const int q = lane >> 4;
     const double cmax = *cmax_p;
-    const int64_t ntiles = (n + ROWS_PER_WG - 1) / ROWS_PER_WG;
+    const int64_t nsel = select_rows(rs, n);
+    const int64_t ntiles = (nsel + ROWS_PER_WG - 1) / ROWS_PER_WG;
     const int nchunks = (k + MFMA_F64_CB - 1) / MFMA_F64_CB;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const int64_t wrow0 = tile * ROWS_PER_WG + int64_t(wave) * ROWS_PER_WAVE;
         double xr[NB][Q];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            const int64_t row = wrow0 + nb * 16 + r16;
-            const bool ok = row < n;
-            const double* src = X + (ok ? row : 0) * ldx + q * Q;
+            const int64_t e = wrow0 + nb * 16 + r16;
+            const bool ok = e < nsel;
+            const double* src = X + (ok ? select_row(rs, e) : 0) * ldx + q * Q;
 #pragma unroll
             for (int s = 0; s < Q; s += 2) {
                 doublex2 v = {0.0, 0.0};
@@ -520,9 +547,11 @@ __global__ __launch_bounds__(256, 2) void assign_mfma_f64_kernel(
                     sl[2 * w + z].i1 = __shfl_xor(st[nb][z].i1, 16 * w);
                     sl[2 * w + z].i2 = __shfl_xor(st[nb][z].i2, 16 * w);
                 }
-            const int64_t row = wrow0 + nb * 16 + r16;
-            if (q == 0 && row < n)
-                decide_row<double>(row, sl, 8, bc, double(xnorm_up[row]), cmax, labels, L);
+            const int64_t e = wrow0 + nb * 16 + r16;
+            if (q == 0 && e < nsel) {
+                const int64_t row = select_row(rs, e);
+                decide_row<double>(row, sl, 8, bc, double(xnorm_up[row]), cmax, labels, L, rs);
+            }
         }
     }
 }

@@ -180,20 +180,21 @@ __global__ __launch_bounds__(256) void convert_rows_bf16_kernel(
 
 // ---------------------------------------------------------------------------
 // centroids -> bf16(-2 c) padded rows, ||c||^2 (F), maxima of ||c||,
-// ||bf16(c)||, ||c - bf16(c)||.  One wave per centroid.  Rows k .. kp-1
+// ||bf16(c)||, ||c - bf16(c)||, and with bounds kept how far the centroid moved.
+// One wave per centroid.  Rows k .. kp-1
 // (kp = bf16_padded_k(k)) are zero, so the last centroid blocks read defined
 // values without clamping.
 // max_bits: [0] C, [1] Ch, [2] Ec
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void centroid_prep_bf16_kernel(
     const float* __restrict__ C, int k, int kp, int d, int dpb, uint16_t* __restrict__ Cb,
-    float* __restrict__ cn, unsigned long long* __restrict__ max_bits) {
+    float* __restrict__ cn, unsigned long long* __restrict__ max_bits, drift_out dr) {
     const int lane = threadIdx.x & 63;
     const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     for (int j = k + wave; j < kp; j += nwaves)
         for (int f = lane; f < dpb; f += 64) Cb[int64_t(j) * dpb + f] = 0;
-    unsigned long long b0 = 0, b1 = 0, b2 = 0;  // lane 0: this wave's maxima
+    unsigned long long b0 = 0, b1 = 0, b2 = 0, b3 = 0;  // lane 0: this wave's maxima
     for (int j = wave; j < k; j += nwaves) {
         double s = 0.0, sh = 0.0, se = 0.0;
         for (int f = lane; f < dpb; f += 64) {
@@ -218,21 +219,28 @@ __global__ __launch_bounds__(256) void centroid_prep_bf16_kernel(
             b1 = max(b1, (unsigned long long)__double_as_longlong(sqrt(sh) * up));
             b2 = max(b2, (unsigned long long)__double_as_longlong(sqrt(se) * up + 1e-30));
         }
+        if (dr.cold) {
+            const double m = wave_drift<float>(C + int64_t(j) * d, static_cast<const float*>(dr.cold) + int64_t(j) * d,
+                                               d, lane);
+            if (lane == 0) dr.drift[j] = m;
+            b3 = max(b3, (unsigned long long)__double_as_longlong(m));
+        }
     }
     // one atomic per bound and workgroup (the maxima of non-negative doubles, or
     // NaN, taken on their bit patterns as before)
-    __shared__ unsigned long long wb[4][3];
+    __shared__ unsigned long long wb[4][4];
     const int w = threadIdx.x >> 6;
     if (lane == 0) {
         wb[w][0] = b0;
         wb[w][1] = b1;
         wb[w][2] = b2;
+        wb[w][3] = b3;
     }
     __syncthreads();
-    if (threadIdx.x < 3) {
+    if (threadIdx.x < 4) {
         const int q = threadIdx.x;
         const unsigned long long m = max(max(wb[0][q], wb[1][q]), max(wb[2][q], wb[3][q]));
-        if (m) atomicMax(&max_bits[q], m);
+        if (m) atomicMax(q < 3 ? &max_bits[q] : dr.max_drift, m);
     }
 }
 
@@ -381,7 +389,7 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
     const uint16_t* __restrict__ Xb, int64_t n, const uint16_t* __restrict__ Cb, int k,
     const float* __restrict__ cnb_g, const float* __restrict__ xnorm_up,
     const float* __restrict__ enorm_up, const bf16_params* __restrict__ params_p,
-    bf16_consts kc, int32_t* __restrict__ labels, refine_lists L, seg_lists S) {
+    bf16_consts kc, int32_t* __restrict__ labels, refine_lists L, seg_lists S, row_select rs) {
     constexpr int HALF = DPB / 2;
     constexpr int STEPS = HALF / 8;
     constexpr int ROWS_PER_WAVE = 32 * NB;
@@ -413,7 +421,7 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
     const int mblocks = bf16_padded_k(k) / 32;  // a multiple of 4
     const bf16_params P = *params_p;
     const uint32_t kmask = 0x7FFFFFFFu & ~((1u << kc.ib) - 1u);
-    const int64_t nrows = COLLECT ? int64_t(L.counters[2]) : n;
+    const int64_t nrows = COLLECT ? int64_t(L.counters[2]) : select_rows(rs, n);
     const int64_t ntiles = (nrows + ROWS_PER_WG - 1) / ROWS_PER_WG;
     // the mask lives in a VGPR so (bits & mask) | tag is one v_and_or_b32
     // (a VALU op may read only one scalar operand on this target)
@@ -487,6 +495,7 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
                 }
                 TKc[nb] = tkc;
             } else {
+                row = ok ? select_row(rs, e) : 0;
                 xn[nb] = ok ? xnorm_up[row] : 0.f;
                 xe[nb] = ok ? enorm_up[row] : 0.f;
             }
@@ -713,6 +722,26 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
                 cert = cert && (k1[q] > TK || idx_of(k1[q], q < NSL ? h : 1 - h) < k);
             }
             int outcome = 0;  // 1: candidate entry, 2: collect entry
+            if (active && rs.gap) {
+                // bounds of a settled row (km_bounds.hpp); the others are assigned
+                // again by the next pass.  Keys' values lie within da of the true ones.
+                float g = -__builtin_inff();
+                if (cert && cnt == 1) {
+                    uint32_t second = 0xFFFFFFFFu;
+#pragma unroll
+                    for (int q = 0; q < 2 * NSL; ++q) {
+                        const bool own = k1[q] == best && (q < NSL ? h : 1 - h) == hb;
+                        second = min(second, own ? k2[q] : k1[q]);
+                    }
+                    const double X = double(xnr), X2 = X * X;
+                    const double da = bf16_row_delta(kc, P, X, double(xer));
+                    const double v1 = double(__uint_as_float(best & kmask));
+                    const double v2 = double(__uint_as_float(second & kmask));
+                    g = bound_gap(v1 - P.B + da + X2 + (v1 + X2 + P.B) * 1e-15,
+                                  v2 - P.B - da + X2 * (1.0 - 3e-7), rs.gam, rs.base[idx_of(best, hb)]);
+                }
+                rs.gap[row] = g;
+            }
             if (active) {
                 if (cert && cnt == 1)
                     labels[row] = idx_of(best, hb);

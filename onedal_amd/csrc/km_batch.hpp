@@ -586,6 +586,45 @@ __global__ __launch_bounds__(256) void batch_count_kernel(const batch_inst* __re
     }
 }
 
+// Label histogram of one large instance (the single-instance engine): as
+// batch_count_kernel's per-block histograms, and the clusters whose members
+// changed since the previous call are flagged: prev holds the labels then (-1
+// before the first), and takes the new ones.
+__global__ __launch_bounds__(256) void label_hist_kernel(const int32_t* __restrict__ labels,
+                                                         int32_t* __restrict__ prev, int64_t n, int k,
+                                                         int32_t* __restrict__ bhist,
+                                                         int32_t* __restrict__ changed) {
+    __shared__ int hist[BATCH_HIST_MAX];
+    const int64_t blocks = (n + BATCH_CNT_ROWS - 1) / BATCH_CNT_ROWS;
+    for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const int64_t r0 = b * BATCH_CNT_ROWS;
+        const int nr = int(min<int64_t>(BATCH_CNT_ROWS, n - r0));
+        __syncthreads();
+        for (int j = threadIdx.x; j < k; j += 256) hist[j] = 0;
+        __syncthreads();
+        constexpr int RPT = BATCH_CNT_ROWS / 256;
+        int lv[RPT], pv[RPT];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            const int r = threadIdx.x + 256 * u;
+            lv[u] = r < nr ? labels[r0 + r] : -1;
+            pv[u] = r < nr ? prev[r0 + r] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (lv[u] < 0) continue;
+            atomicAdd(&hist[lv[u]], 1);
+            if (lv[u] != pv[u]) {
+                changed[lv[u]] = 1;
+                if (pv[u] >= 0) changed[pv[u]] = 1;
+                prev[r0 + threadIdx.x + 256 * u] = lv[u];
+            }
+        }
+        __syncthreads();
+        for (int j = threadIdx.x; j < k; j += 256) bhist[b * k + j] = hist[j];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Stable counting sort of the row ids by label within each instance (the order
 // rocPRIM's radix sort of (instance, label) keys gives: rows of a cluster in

@@ -1,0 +1,154 @@
+// km_bounds.hpp -- distance bounds that let a training pass skip settled rows.
+//
+// Hamerly's bounds (Hamerly 2010, "Making k-means even faster"; Elkan 2003): when
+// a row is settled with label a, its distance to c_a is at most `up` and its
+// distance to every other centroid at least `lo`.  Centroid j then moves by at
+// most drift_j per iteration, so after some iterations the row's label is still
+// a while  up + sum drift_a < lo - sum max_j drift_j.  One float per row is kept,
+//     gap = lo (1 - g) - up (1 + g) + base_a            (rounded down)
+// with base_a the running sum of (drift_a + max drift)(1 + g) (rounded up, in
+// double) at the time the row was settled; the row stays settled while
+//     gap > base_a + BOUND_SLACK.
+// g covers the rounding of the exact-form distances D (their relative error is
+// at most gamma_{d+2}), so a settled row's exact-form argmin is a, uniquely: the
+// labels are those of a full pass, bit for bit.  BOUND_SLACK keeps the compared
+// distances away from underflow, BOUND_MAX from overflow (such rows are always
+// assigned again).  Any NaN makes the comparison false: the row is assigned again.
+//
+// What it is for: from the fourth iteration on, clustered rows move little and
+// most labels are certain.  On the precision workload's mixture (n=2e7, d=128,
+// k=1024, 20 iterations) 29% of the row assignments remain, on the FP32 one
+// (n=1e7, d=64, k=256) 28%; where no row can be skipped a pass costs 8 bytes a
+// row more (label and gap).
+#pragma once
+
+#include "km_common.hpp"
+
+namespace km {
+
+constexpr double BOUND_SLACK = 1e-15;
+constexpr double BOUND_MAX = 1e18;
+
+// rows of one assignment pass (null rows: all n) and where their bounds go
+// (null gap: none kept)
+struct row_select {
+    const int32_t* rows;
+    const int32_t* count;
+    float* gap;
+    const double* base;
+    double gam;  // g above, with room for the float roundings of bound_gap
+};
+
+// the number of rows of the pass, and entry e's row
+__device__ __forceinline__ int64_t select_rows(const row_select& s, int64_t n) {
+    return s.rows ? int64_t(*s.count) : n;
+}
+__device__ __forceinline__ int64_t select_row(const row_select& s, int64_t e) {
+    return s.rows ? int64_t(s.rows[e]) : e;
+}
+
+// gap of a row settled with squared distances at most up2 (its centroid) and at
+// least lo2 (every other one); the float roundings here are below 1e-6
+__device__ __forceinline__ float bound_gap(double up2, double lo2, double gam, double base) {
+    const float u = sqrtf(float(fmax(up2, 0.0)));
+    const float l = sqrtf(float(fmax(lo2, 0.0)));
+    if (!(double(u) < BOUND_MAX)) return -__builtin_inff();
+    const double g = double(l) * (1.0 - gam) - double(u) * (1.0 + gam) + base;
+    return float(g - fabs(g) * 1.2e-7);
+}
+
+// Before a pass with moved centroids: base_j += (drift_j + max drift)(1 + g),
+// rounded up; the changed-cluster flags and the pass's counters (selected rows,
+// re-score lists) start at zero.
+__global__ __launch_bounds__(256) void bound_base_kernel(int k, const double* __restrict__ drift,
+                                                         const unsigned long long* __restrict__ max_drift,
+                                                         double gam, double* __restrict__ base,
+                                                         int32_t* __restrict__ changed,
+                                                         int32_t* __restrict__ sel_count,
+                                                         int32_t* __restrict__ counters) {
+    const double m = __longlong_as_double((long long)*max_drift);
+    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < k; j += gridDim.x * blockDim.x) {
+        const double b = (base[j] + (drift[j] + m) * (1.0 + gam)) * (1.0 + 1e-15);
+        base[j] = b < BOUND_MAX ? b : __builtin_inf();
+        changed[j] = 0;
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 3) counters[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 3) *sel_count = 0;
+}
+
+// The rows to assign again, as a dense list.  A workgroup takes runs of
+// SELECT_ROWS rows, counts its open rows with ballots and reserves its part of
+// the list with one atomic; rows keep their order inside a run.  8 bytes read per
+// row: bound by HBM.
+constexpr int SELECT_ROWS = 4096;
+__global__ __launch_bounds__(256) void bound_select_kernel(const int32_t* __restrict__ labels,
+                                                           const float* __restrict__ gap,
+                                                           const double* __restrict__ base, int64_t n,
+                                                           int32_t* __restrict__ rows,
+                                                           int32_t* __restrict__ count) {
+    constexpr int U = SELECT_ROWS / 256;
+    __shared__ int wtot[4];
+    __shared__ int first;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t runs = (n + SELECT_ROWS - 1) / SELECT_ROWS;
+    for (int64_t q = blockIdx.x; q < runs; q += gridDim.x) {
+        // a wave's rows are consecutive groups of 64
+        const int64_t r0 = q * SELECT_ROWS + int64_t(wave) * (SELECT_ROWS / 4) + lane;
+        int32_t lab[U];
+        float g[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t r = r0 + 64 * u;
+            lab[u] = r < n ? labels[r] : 0;
+            g[u] = r < n ? gap[r] : 0.f;
+        }
+        uint64_t open[U];
+        int mine = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool settled = double(g[u]) > base[lab[u]] + BOUND_SLACK;
+            open[u] = __ballot(r0 + 64 * u < n && !settled);
+            mine += __popcll(open[u]);
+        }
+        if (lane == 0) wtot[wave] = mine;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int t = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+            first = t ? atomicAdd(count, t) : 0;
+        }
+        __syncthreads();
+        int at = first;
+        for (int w = 0; w < wave; ++w) at += wtot[w];
+        const uint64_t below = (uint64_t(1) << lane) - 1u;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if ((open[u] >> lane) & 1u) rows[at + __popcll(open[u] & below)] = int32_t(r0 + 64 * u);
+            at += __popcll(open[u]);
+        }
+        __syncthreads();  // wtot and first are rewritten by the next run
+    }
+}
+
+// Centroid movement, taken by the preparation kernels (one wave per centroid): lane
+// partials of ||cnew - cold||^2, reduced over the wave and rounded up.  Its maximum is
+// kept as the bits of a non-negative double (a NaN wins).
+struct drift_out {
+    const void* cold;  // previous centroids (null: no bounds kept)
+    double* drift;     // k
+    unsigned long long* max_drift;
+};
+
+template <typename F>
+__device__ __forceinline__ double wave_drift(const F* __restrict__ cnew, const F* __restrict__ cold, int d,
+                                             int lane) {
+    double s = 0.0;
+    for (int f = lane; f < d; f += 64) {
+        const double v = double(cnew[f]) - double(cold[f]);
+        s = fma(v, v, s);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    return sqrt(s) * (1.0 + 1e-12);
+}
+
+}  // namespace km

@@ -36,6 +36,7 @@
 #include "km_assign.hpp"
 #include "km_assign_bf16.hpp"
 #include "km_batch.hpp"
+#include "km_bounds.hpp"
 #include "km_common.hpp"
 #include "km_csr.hpp"
 #include "km_init.hpp"
@@ -137,6 +138,10 @@ struct km_ctx {
     km::dbuf gt_d;  // empty-cluster candidates' d64
     km::dbuf stat_acc, coop_wcnt;  // device-side statistics; per-workgroup counts of ec_count_kernel
     km::dbuf cs_inst, cs_pre, cs_hist, cs_gsum;  // single-instance counting sort (label_sort)
+    km::dbuf cs_prev, cs_changed;                // its previous labels and changed-cluster flags
+    // distance bounds of a training (row_bounds): gap and open rows, per row; base
+    // and drift, per cluster
+    km::dbuf b_gap, b_rows, b_count, b_base, b_drift;
     // CSR path: values, column indices, row offsets (when uploaded), row squares,
     // transposed centroids, centroid squares, closest distances, structure flag
     km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cs, csr_closest, csr_flag;
@@ -209,7 +214,7 @@ struct work {
     refine_lists L{};
     F* cn = nullptr;
     F* cpad = nullptr;
-    unsigned long long* cmax_bits = nullptr;  // [0] max ||c|| ([1], [2]: BF16 path)
+    unsigned long long* cmax_bits = nullptr;  // [0] max ||c|| ([1], [2]: BF16 path), [3] max drift
     // BF16 path
     uint16_t* Xb = nullptr;       // n x dpad bf16 rows
     float* enorm = nullptr;       // ||x - bf16(x)|| (up)
@@ -217,6 +222,8 @@ struct work {
     uint16_t* Cb = nullptr;       // k x dpad bf16(-2 c)
     float* cnb = nullptr;         // ||c||^2 + B (rounded up), 32 * ceil(k / 32) entries
     bf16_params* params = nullptr;
+    // rows of the next assignment pass, and where their bounds go
+    row_select sel{nullptr, nullptr, nullptr, nullptr, 0.0};
     // workspace source: a fixed arena, or (null) the context's buffers
     arena* A = nullptr;
 };
@@ -266,17 +273,20 @@ static bf16_consts make_bf16_consts(int d, int k) {
     return c;
 }
 
-// per-centroid prep: ||c||^2, padded copy, max ||c||
+// per-centroid prep: ||c||^2, padded copy, max ||c||; with dr.cold (a training
+// iteration after the first, whose scan has cleared the maxima) the centroids'
+// movement too
 template <typename F>
-static void centroid_prep(km_ctx* ctx, work<F>& w, const F* C, int path) {
+static void centroid_prep(km_ctx* ctx, work<F>& w, const F* C, int path,
+                          const drift_out& dr = {nullptr, nullptr, nullptr}) {
+    if (!dr.cold) fill<unsigned long long>(ctx, w.cmax_bits, 4, 0ull);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
-            fill<unsigned long long>(ctx, w.cmax_bits, 3, 0ull);
             const int kp = bf16_padded_k(w.k);
             // four centroids per wave, so few workgroups add to the three maxima
             const int grid = grid_for(ctx, int64_t(kp) * 16, 256, 4);
             hipLaunchKernelGGL(centroid_prep_bf16_kernel, dim3(grid), dim3(256), 0, ctx->stream, C,
-                               w.k, kp, w.d, w.dpad, w.Cb, w.cn, w.cmax_bits);
+                               w.k, kp, w.d, w.dpad, w.Cb, w.cn, w.cmax_bits, dr);
             KM_LAUNCH_CHECK();
             hipLaunchKernelGGL(bf16_params_kernel, dim3(1), dim3(64), 0, ctx->stream, w.cmax_bits,
                                w.xmax_bits, make_bf16_consts(w.d, w.k), w.params);
@@ -288,10 +298,9 @@ static void centroid_prep(km_ctx* ctx, work<F>& w, const F* C, int path) {
         }
     }
     const bool need_pad = path == 2;
-    fill<unsigned long long>(ctx, w.cmax_bits, 1, 0ull);
     const int grid = grid_for(ctx, int64_t(w.k) * 64, 256, 4);
     hipLaunchKernelGGL(centroid_prep_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, C, w.k, w.d,
-                       w.dpad, w.cn, need_pad ? w.cpad : (F*)nullptr, w.cmax_bits);
+                       w.dpad, w.cn, need_pad ? w.cpad : (F*)nullptr, w.cmax_bits, dr);
     KM_LAUNCH_CHECK();
 }
 
@@ -301,7 +310,7 @@ static void launch_mfma_f32_mode(km_ctx* ctx, work<float>& w, const band_consts&
     auto kern = assign_mfma_f32_kernel<DP, NB, RES>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.Xv, w.ldx, w.n, w.d, w.cpad,
-                       w.k, w.cn, w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L);
+                       w.k, w.cn, w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -327,7 +336,7 @@ static void launch_mfma_f64(km_ctx* ctx, work<double>& w, const band_consts& bc)
     auto kern = assign_mfma_f64_kernel<DP, NB>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.Xv, w.ldx, w.n, w.d, w.cpad, w.k, w.cn,
-                       w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L);
+                       w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -355,7 +364,7 @@ static void launch_bf16(km_ctx* ctx, work<float>& w, bool collect) {
         KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    int(lds)));
         hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.Xb, w.n, w.Cb, w.k, w.cnb,
-                           w.xnorm, w.enorm, w.params, kc, w.labels, w.L, S);
+                           w.xnorm, w.enorm, w.params, kc, w.labels, w.L, S, w.sel);
         KM_LAUNCH_CHECK();
         hipLaunchKernelGGL(compact_lists_kernel, dim3((nseg + 3) / 4), dim3(256), 0, ctx->stream, S,
                            nseg, w.L);
@@ -370,7 +379,7 @@ static void launch_bf16(km_ctx* ctx, work<float>& w, bool collect) {
                                    int(clds)));
         hipLaunchKernelGGL(ckern, dim3(ctx->cu_count * 3), dim3(256), clds, ctx->stream, w.Xb, w.n,
                            w.Cb, w.k, w.cnb, w.xnorm, w.enorm, w.params, kc, w.labels, w.L,
-                           seg_lists{});
+                           seg_lists{}, row_select{nullptr, nullptr, nullptr, nullptr, 0.0});
     }
     KM_LAUNCH_CHECK();
 }
@@ -390,10 +399,11 @@ static void refine_pairs(km_ctx* ctx, work<F>& w, const F* C, const int32_t* row
     KM_LAUNCH_CHECK();
 }
 
-// assignment of every row against w.X/C (centroid_prep already done for C)
+// assignment of the selected rows against w.X/C (centroid_prep already done for C);
+// a selected pass starts with cleared counters (bound_base_kernel)
 template <typename F>
 static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
-    fill<int32_t>(ctx, w.L.counters, 3, 0);
+    if (!w.sel.rows) fill<int32_t>(ctx, w.L.counters, 3, 0);
     const band_consts bc = make_band<F>(w.d);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing) {
@@ -433,7 +443,7 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
         const int64_t tiles = (w.n + 63) / 64;
         const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * 4)));
         hipLaunchKernelGGL(assign_generic_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, w.X, w.n,
-                           w.d, C, w.k, w.cn, w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L);
+                           w.d, C, w.k, w.cn, w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L, w.sel);
         KM_LAUNCH_CHECK();
     }
     if (ctx->timing) {
@@ -556,6 +566,8 @@ struct label_sort {
     int64_t* pre = nullptr;
     int32_t* bhist = nullptr;
     int32_t* gsum = nullptr;
+    int32_t* prev = nullptr;     // labels at the previous call (counting sort)
+    int32_t* changed = nullptr;  // clusters whose members changed since then
 };
 
 // the scatter kernel's LDS limit, set to the largest use (every caller sets the
@@ -569,8 +581,12 @@ static label_sort label_sort_setup(km_ctx* ctx, int64_t n, int k) {
     label_sort ls;
     ls.n = n;
     ls.k = k;
+    ls.changed = ctx->cs_changed.get<int32_t>(k);
+    fill<int32_t>(ctx, ls.changed, k, 0);
     if (k > BATCH_HIST_MAX) return ls;
     ls.csort = true;
+    ls.prev = ctx->cs_prev.get<int32_t>(n);
+    fill<int32_t>(ctx, ls.prev, n, -1);
     ls.nb = (n + BATCH_CNT_ROWS - 1) / BATCH_CNT_ROWS;
     ls.G = int(std::min<int64_t>(ls.nb, 64));
     ls.GB = int((ls.nb + ls.G - 1) / ls.G);
@@ -590,12 +606,13 @@ static label_sort label_sort_setup(km_ctx* ctx, int64_t n, int k) {
 }
 
 // counts of the labels (with the counting sort: the block histograms, their
-// group sums, and the counts as the column sums of those)
+// group sums, and the counts as the column sums of those) and the flags of the
+// clusters whose members changed (cleared before the call)
 static void label_counts(km_ctx* ctx, const label_sort& ls, const int32_t* labels, int32_t* counts) {
     if (ls.csort) {
         const int grid = int(std::min<int64_t>(ls.nb, int64_t(ctx->cu_count) * 8));
-        hipLaunchKernelGGL(batch_count_kernel, dim3(grid), dim3(256), 0, ctx->stream, ls.I, 1, ls.pre, labels,
-                           nullptr, ls.bhist);
+        hipLaunchKernelGGL(label_hist_kernel, dim3(grid), dim3(256), 0, ctx->stream, labels, ls.prev, ls.n, ls.k,
+                           ls.bhist, ls.changed);
         KM_LAUNCH_CHECK();
         const int g2 = int((int64_t(ls.G) * ls.k + 255) / 256);
         hipLaunchKernelGGL(sort_group_sums_kernel, dim3(g2), dim3(256), 0, ctx->stream, ls.bhist, ls.nb, ls.k, ls.G,
@@ -604,6 +621,7 @@ static void label_counts(km_ctx* ctx, const label_sort& ls, const int32_t* label
         hipLaunchKernelGGL(sort_counts_kernel, dim3((ls.k + 255) / 256), dim3(256), 0, ctx->stream, ls.gsum, ls.k,
                            ls.G, counts);
     } else {
+        fill<int32_t>(ctx, ls.changed, ls.k, 1);  // not tracked: every cluster is summed again
         fill<int32_t>(ctx, counts, ls.k, 0);
         const bool lds = ls.k <= 16384;
         hipLaunchKernelGGL(count_kernel, dim3(grid_for(ctx, ls.n, 256, 4)), dim3(256),
@@ -782,6 +800,40 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
     fill<unsigned long long>(ctx, acc, 4, 0ull);
     double* d64 = ctx->d64.get<double>(n);  // per-row d64 for empty clusters
     const label_sort lsort = label_sort_setup(ctx, n, k);
+    // bounds (km_bounds.hpp): every pass after the first assigns only the rows
+    // whose label could have changed
+    double* base = nullptr;
+    drift_out drift{nullptr, nullptr, nullptr};
+    int32_t* open_rows = nullptr;
+    int32_t* open_count = nullptr;
+    if (max_iter > 0) {
+        base = ctx->b_base.get<double>(k);
+        fill<double>(ctx, base, k, 0.0);
+        drift.drift = ctx->b_drift.get<double>(k);
+        drift.max_drift = w.cmax_bits + 3;
+        open_rows = ctx->b_rows.get<int32_t>(n);
+        open_count = ctx->b_count.get<int32_t>(1);
+        w.sel.gap = ctx->b_gap.get<float>(n);
+        w.sel.base = base;
+        w.sel.gam = make_band<F>(d).g_canon + 1e-6;
+    }
+    // centroid preparation and the rows of the next pass (first: all of them)
+    auto open_pass = [&](const F* C, const F* Cold, bool first) {
+        if (first) {
+            centroid_prep<F>(ctx, w, C, path);
+            return;
+        }
+        drift.cold = Cold;
+        centroid_prep<F>(ctx, w, C, path, drift);
+        hipLaunchKernelGGL(bound_base_kernel, dim3(grid_for(ctx, k, 256, 1)), dim3(256), 0, ctx->stream, k,
+                           drift.drift, drift.max_drift, w.sel.gam, base, lsort.changed, open_count, w.L.counters);
+        KM_LAUNCH_CHECK();
+        hipLaunchKernelGGL(bound_select_kernel, dim3(grid_for(ctx, n, SELECT_ROWS, 8)), dim3(256), 0, ctx->stream,
+                           w.labels, w.sel.gap, base, n, open_rows, open_count);
+        KM_LAUNCH_CHECK();
+        w.sel.rows = open_rows;
+        w.sel.count = open_count;
+    };
 
     hipEvent_t loop0 = nullptr, loop1 = nullptr;
     ctx->ev_used = 0;
@@ -793,18 +845,18 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
     double prev = double(std::numeric_limits<F>::max());
     int64_t iter = 0;
     for (iter = 0; iter < max_iter; ++iter) {
-        centroid_prep<F>(ctx, w, Ccur, path);
+        open_pass(Ccur, Cnext, iter == 0);  // Cnext: the previous centroids
         assign<F>(ctx, w, Ccur, path);
         label_counts(ctx, lsort, w.labels, counts);
         hipLaunchKernelGGL(scan_clusters_kernel, dim3(1), dim3(1024), 0, ctx->stream, counts, k,
-                           offsets, chunk_base, empty_list, meta);
+                           offsets, chunk_base, empty_list, meta, lsort.changed, w.cmax_bits, 4);
         KM_LAUNCH_CHECK();
         label_group(ctx, lsort, w.labels, offsets, perm);
         launch_reduce<F>(ctx, w, perm, offsets, chunk_base, meta, part);
         {
             const int grid = grid_for(ctx, int64_t(k) * d, 256, 4);
             hipLaunchKernelGGL(finalize_centroids_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream,
-                               part, counts, chunk_base, k, d, Cnext);
+                               part, counts, chunk_base, lsort.changed, k, d, Ccur, Cnext);
             KM_LAUNCH_CHECK();
         }
         double* objp = nullptr;
@@ -826,7 +878,7 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
         }
     }
     // final assignment with the final centroids and the objective
-    centroid_prep<F>(ctx, w, Ccur, path);
+    open_pass(Ccur, Cnext, iter == 0);
     assign<F>(ctx, w, Ccur, path);
     double* objp = objective<F>(ctx, w, Ccur, nullptr);
     if (ctx->timing) KM_HIP(hipEventRecord(loop1, ctx->stream));
@@ -1177,9 +1229,10 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     int64_t iter = 0;
     for (iter = 0; iter < max_iter; ++iter) {
         csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest);
+        if (iter > 0) fill<int32_t>(ctx, lsort.changed, k, 0);
         label_counts(ctx, lsort, labels, counts);
         hipLaunchKernelGGL(scan_clusters_kernel, dim3(1), dim3(1024), 0, ctx->stream, counts, k,
-                           offsets, chunk_base, empty_list, meta);
+                           offsets, chunk_base, empty_list, meta, lsort.changed, (unsigned long long*)nullptr, 0);
         KM_LAUNCH_CHECK();
         label_group(ctx, lsort, labels, offsets, perm);
         const int64_t max_chunks = n / REDUCE_CHUNK + k + 1;
@@ -1188,7 +1241,7 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
                            offsets, chunk_base, meta, part);
         KM_LAUNCH_CHECK();
         hipLaunchKernelGGL(finalize_centroids_kernel<F>, dim3(grid_for(ctx, int64_t(k) * d, 256, 4)),
-                           dim3(256), 0, ctx->stream, part, counts, chunk_base, k, d, Cnext);
+                           dim3(256), 0, ctx->stream, part, counts, chunk_base, lsort.changed, k, d, Ccur, Cnext);
         KM_LAUNCH_CHECK();
         // empty clusters on the device (d64 pass gated on the empty count, the
         // selection kernels, the sparse fill): no host round trip without a
@@ -2190,7 +2243,8 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->seg_counts, &ctx->tune_x, &ctx->tune_c, &ctx->tune_l,
                         &ctx->init_d2, &ctx->init_chunks, &ctx->init_chosen, &ctx->init_ids,
                         &ctx->gt_d, &ctx->stat_acc, &ctx->coop_wcnt, &ctx->cs_inst, &ctx->cs_pre,
-                        &ctx->cs_hist, &ctx->cs_gsum, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
+                        &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
+                        &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
                         &ctx->csr_ct, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();

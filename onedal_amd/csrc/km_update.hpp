@@ -15,6 +15,7 @@
 // restatement of it.
 #pragma once
 
+#include "km_bounds.hpp"
 #include "km_common.hpp"
 
 namespace km {
@@ -68,13 +69,14 @@ __global__ __launch_bounds__(256) void row_norm_kernel(const F* __restrict__ X, 
 // ---------------------------------------------------------------------------
 // centroid preparation for one assignment pass: ||c_j||^2 in F (from a double
 // sum), max ||c_j|| (rounded up) and a zero-padded copy for the matrix-core
-// kernel.  One wave per centroid.
+// kernel, and with bounds kept how far the centroid moved.  One wave per centroid.
 // ---------------------------------------------------------------------------
 template <typename F>
 __global__ __launch_bounds__(256) void centroid_prep_kernel(const F* __restrict__ C, int k, int d,
                                                             int dpad, F* __restrict__ cn,
                                                             F* __restrict__ cpad,
-                                                            unsigned long long* __restrict__ cmax_bits) {
+                                                            unsigned long long* __restrict__ cmax_bits,
+                                                            drift_out dr) {
     const int lane = threadIdx.x & 63;
     const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
@@ -92,6 +94,13 @@ __global__ __launch_bounds__(256) void centroid_prep_kernel(const F* __restrict_
             cn[j] = F(s);
             const double r = sqrt(s) * (1.0 + 1e-12);
             atomicMax(cmax_bits, (unsigned long long)__double_as_longlong(r));
+        }
+        if (dr.cold) {
+            const double m = wave_drift<F>(C + int64_t(j) * d, static_cast<const F*>(dr.cold) + int64_t(j) * d, d, lane);
+            if (lane == 0) {
+                dr.drift[j] = m;
+                atomicMax(dr.max_drift, (unsigned long long)__double_as_longlong(m));
+            }
         }
     }
 }
@@ -124,19 +133,25 @@ __global__ __launch_bounds__(256) void count_kernel(const int32_t* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // single-workgroup scan over clusters: member offsets, chunk offsets and the
-// ascending list of empty clusters.  meta[0] = #empty, meta[1] = #chunks.
+// ascending list of empty clusters.  meta[0] = #empty, meta[1] = #chunks.  A
+// cluster whose members did not change (changed[j] = 0) has no chunks: its sums,
+// and so its centroid, are those of the previous iteration.  Also clears the nzero
+// words at `zero` (maxima that the next centroid preparation takes).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void scan_clusters_kernel(const int32_t* __restrict__ counts,
                                                              int k, int64_t* __restrict__ offsets,
                                                              int32_t* __restrict__ chunk_base,
                                                              int32_t* __restrict__ empty_list,
-                                                             int32_t* __restrict__ meta) {
+                                                             int32_t* __restrict__ meta,
+                                                             const int32_t* __restrict__ changed,
+                                                             unsigned long long* __restrict__ zero, int nzero) {
     __shared__ int64_t s_off[1024];
     __shared__ int32_t s_chk[1024];
     __shared__ int32_t s_emp[1024];
     __shared__ int64_t carry_off;
     __shared__ int32_t carry_chk, carry_emp;
     const int t = threadIdx.x;
+    if (t < nzero) zero[t] = 0ull;
     if (t == 0) {
         carry_off = 0;
         carry_chk = 0;
@@ -146,8 +161,9 @@ __global__ __launch_bounds__(1024) void scan_clusters_kernel(const int32_t* __re
     for (int base = 0; base < k; base += 1024) {
         const int j = base + t;
         const int32_t c = j < k ? counts[j] : 0;
+        const int32_t nchk = j < k && changed[j] ? (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK : 0;
         s_off[t] = c;
-        s_chk[t] = j < k ? (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK : 0;
+        s_chk[t] = nchk;
         s_emp[t] = (j < k && c == 0) ? 1 : 0;
         __syncthreads();
         for (int off = 1; off < 1024; off <<= 1) {
@@ -167,7 +183,7 @@ __global__ __launch_bounds__(1024) void scan_clusters_kernel(const int32_t* __re
         if (j < k) {
             const int64_t incl_off = s_off[t];
             offsets[j] = carry_off + incl_off - c;
-            chunk_base[j] = carry_chk + s_chk[t] - (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK;
+            chunk_base[j] = carry_chk + s_chk[t] - nchk;
             if (c == 0) empty_list[carry_emp + s_emp[t] - 1] = j;
         }
         __syncthreads();
@@ -359,18 +375,24 @@ __global__ __launch_bounds__(256) void reduce_chunks_vec_kernel(
 
 // ---------------------------------------------------------------------------
 // merge chunk sums per cluster (chunk order) and divide: C_j = (F)(S1_j / n_j).
-// Empty clusters are left for the ec_* kernels (refilled there).
+// A cluster whose members did not change keeps its centroid (the same sums give
+// the same bits).  Empty clusters are left for the ec_* kernels (refilled there).
 // ---------------------------------------------------------------------------
 template <typename F>
 __global__ __launch_bounds__(256) void finalize_centroids_kernel(
     const double* __restrict__ part, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ chunk_base, int k, int d, F* __restrict__ Cnext) {
+    const int32_t* __restrict__ chunk_base, const int32_t* __restrict__ changed, int k, int d,
+    const F* __restrict__ Ccur, F* __restrict__ Cnext) {
     const int64_t total = int64_t(k) * d;
     for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < total;
          e += int64_t(gridDim.x) * blockDim.x) {
         const int j = int(e / d), f = int(e % d);
         const int32_t cnt = counts[j];
         if (cnt == 0) continue;
+        if (!changed[j]) {
+            Cnext[e] = Ccur[e];
+            continue;
+        }
         double s = 0.0;
         int q = chunk_base[j];
         const int q1 = chunk_base[j + 1];
