@@ -48,8 +48,8 @@ struct top2 {
 
 // Settle one row from its slots (see the file comment).  X = ||x|| rounded up (to
 // a float: ||x|| >= X (1 - 1.2e-7)), C = max_j ||c_j|| rounded up.  With bounds kept
-// (rs.gap), a row settled here leaves its gap; a row sent to a re-score leaves
-// -inf (assigned again by the next pass).
+// (rs.gap), a row settled here leaves its gap; a candidate entry leaves the lower
+// bound of the other centroids for its re-score, which sets the gap.
 template <typename F>
 __device__ __forceinline__ void decide_row(int64_t row, const top2<F>* slots, int nslots,
                                            const band_consts& bc, double X, double C,
@@ -74,20 +74,16 @@ __device__ __forceinline__ void decide_row(int64_t row, const top2<F>* slots, in
             cnt++;
         }
     }
-    if (rs.gap) {
-        float g = -__builtin_inff();
-        if (cert && cnt == 1) {
-            F second = fp_traits<F>::inf;
-            for (int s = 0; s < nslots; ++s) {
-                const F v = slots[s].i1 == bi ? slots[s].m2 : slots[s].m1;
-                second = v < second ? v : second;
-            }
-            const double da = bc.a_xc * X * C + bc.a_cc * C * C;
-            const double X2 = X * X;
-            g = bound_gap(double(best) + da + X2 + (X2 + fabs(double(best))) * 1e-15,
-                          double(second) - da + X2 * (1.0 - 3e-7), rs.gam, rs.base[bi]);
+    const double da = bc.a_xc * X * C + bc.a_cc * C * C;
+    const double X2 = X * X;
+    if (rs.gap && cert && cnt == 1) {
+        F second = fp_traits<F>::inf;
+        for (int s = 0; s < nslots; ++s) {
+            const F v = slots[s].i1 == bi ? slots[s].m2 : slots[s].m1;
+            second = v < second ? v : second;
         }
-        rs.gap[row] = g;
+        rs.gap[row] = bound_gap(double(best) + da + X2 + (X2 + fabs(double(best))) * 1e-15,
+                                double(second) - da + X2 * (1.0 - 3e-7), rs.gam, rs.base[bi]);
     }
     if (cert && cnt == 1) {
         labels[row] = bi;
@@ -95,6 +91,7 @@ __device__ __forceinline__ void decide_row(int64_t row, const top2<F>* slots, in
         const int e = atomicAdd(&L.counters[0], 1);
         L.cand_rows[e] = int32_t(row);
         L.cand_count[e] = cnt;
+        if (rs.gap) L.cand_lo[e] = float_below(T - da + X2 * (1.0 - 3e-7));
         for (int c = 0; c < cnt; ++c) L.cand_ids[int64_t(e) * MAXC + c] = cand[c];
     } else {
         const int e = atomicAdd(&L.counters[1], 1);

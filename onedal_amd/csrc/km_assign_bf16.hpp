@@ -349,6 +349,8 @@ struct seg_lists {
     int32_t* cand_ids;   // MAXC per entry
     int32_t* coll_rows;
     double* coll_T;
+    float* cand_lo;      // lower bounds (refine_lists), null without bounds
+    float* coll_lo;
     int32_t* counts;     // [2 * segment]: candidate entries, [2 * segment + 1]: collect entries
     int64_t cap;
 };
@@ -722,10 +724,14 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
                 cert = cert && (k1[q] > TK || idx_of(k1[q], q < NSL ? h : 1 - h) < k);
             }
             int outcome = 0;  // 1: candidate entry, 2: collect entry
+            // bounds (km_bounds.hpp): the gap of a settled row; for a re-scored one the
+            // lower bound of the centroids outside its list.  Keys' values lie within
+            // da of the true ones.
+            float other = 0.f;
             if (active && rs.gap) {
-                // bounds of a settled row (km_bounds.hpp); the others are assigned
-                // again by the next pass.  Keys' values lie within da of the true ones.
-                float g = -__builtin_inff();
+                const double X2 = double(xnr) * double(xnr);
+                const double da = bf16_row_delta(kc, P, double(xnr), double(xer));
+                const double xlo = X2 * (1.0 - 3e-7) - P.B - da;
                 if (cert && cnt == 1) {
                     uint32_t second = 0xFFFFFFFFu;
 #pragma unroll
@@ -733,14 +739,13 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
                         const bool own = k1[q] == best && (q < NSL ? h : 1 - h) == hb;
                         second = min(second, own ? k2[q] : k1[q]);
                     }
-                    const double X = double(xnr), X2 = X * X;
-                    const double da = bf16_row_delta(kc, P, X, double(xer));
                     const double v1 = double(__uint_as_float(best & kmask));
                     const double v2 = double(__uint_as_float(second & kmask));
-                    g = bound_gap(v1 - P.B + da + X2 + (v1 + X2 + P.B) * 1e-15,
-                                  v2 - P.B - da + X2 * (1.0 - 3e-7), rs.gam, rs.base[idx_of(best, hb)]);
+                    rs.gap[row] = bound_gap(v1 - P.B + da + X2 + (v1 + X2 + P.B) * 1e-15, v2 + xlo, rs.gam,
+                                            rs.base[idx_of(best, hb)]);
+                } else {
+                    other = float_below(Tr + xlo);
                 }
-                rs.gap[row] = g;
             }
             if (active) {
                 if (cert && cnt == 1)
@@ -754,6 +759,7 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
                 const int64_t e = seg_base + n_cand + lanes_below(mc);
                 S.cand_rows[e] = int32_t(row);
                 S.cand_count[e] = cnt;
+                if (rs.gap) S.cand_lo[e] = other;
                 int c = 0;
 #pragma unroll
                 for (int q = 0; q < 2 * NSL; ++q)
@@ -762,6 +768,7 @@ __global__ __launch_bounds__(256, 2) void assign_bf16_kernel(
                 const int64_t e = seg_base + n_coll + lanes_below(ml);
                 S.coll_rows[e] = int32_t(row);
                 S.coll_T[e] = Tr;
+                if (rs.gap) S.coll_lo[e] = other;
             }
             n_cand += int(__popcll(mc));
             n_coll += int(__popcll(ml));
@@ -814,6 +821,7 @@ __global__ __launch_bounds__(256) void compact_lists_kernel(seg_lists S, int nse
     static_assert(MAXC == 8, "an entry's ids are two 16-byte vectors");
     for (int i0 = lane; i0 < nc; i0 += 64 * U) {
         int32_t row[U], cnt[U];
+        float lo[U];
         uintx4 id0[U], id1[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -821,6 +829,7 @@ __global__ __launch_bounds__(256) void compact_lists_kernel(seg_lists S, int nse
             const int64_t src = base + (i < nc ? i : 0);
             row[u] = S.cand_rows[src];
             cnt[u] = S.cand_count[src];
+            lo[u] = S.cand_lo ? S.cand_lo[src] : 0.f;
             id0[u] = *reinterpret_cast<const uintx4*>(S.cand_ids + src * MAXC);
             id1[u] = *reinterpret_cast<const uintx4*>(S.cand_ids + src * MAXC + 4);
         }
@@ -831,6 +840,7 @@ __global__ __launch_bounds__(256) void compact_lists_kernel(seg_lists S, int nse
                 const int64_t dst = int64_t(bc) + i;
                 L.cand_rows[dst] = row[u];
                 L.cand_count[dst] = cnt[u];
+                if (S.cand_lo) L.cand_lo[dst] = lo[u];
                 *reinterpret_cast<uintx4*>(L.cand_ids + dst * MAXC) = id0[u];
                 *reinterpret_cast<uintx4*>(L.cand_ids + dst * MAXC + 4) = id1[u];
             }
@@ -838,6 +848,7 @@ __global__ __launch_bounds__(256) void compact_lists_kernel(seg_lists S, int nse
     }
     for (int i0 = lane; i0 < nl; i0 += 64 * U) {
         int32_t row[U];
+        float lo[U];
         double T[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -845,6 +856,7 @@ __global__ __launch_bounds__(256) void compact_lists_kernel(seg_lists S, int nse
             const int64_t src = base + (i < nl ? i : 0);
             row[u] = S.coll_rows[src];
             T[u] = S.coll_T[src];
+            lo[u] = S.coll_lo ? S.coll_lo[src] : 0.f;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -852,6 +864,7 @@ __global__ __launch_bounds__(256) void compact_lists_kernel(seg_lists S, int nse
             if (i < nl) {
                 L.coll_rows[int64_t(bl) + i] = row[u];
                 L.coll_T[int64_t(bl) + i] = T[u];
+                if (S.coll_lo) L.coll_lo[int64_t(bl) + i] = lo[u];
             }
         }
     }

@@ -717,7 +717,8 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
                                                             const int64_t* __restrict__ pre,
                                                             const int32_t* __restrict__ labels,
                                                             const int32_t* __restrict__ bhist,
-                                                            int32_t* __restrict__ perm, int kcap) {
+                                                            int32_t* __restrict__ perm, int kcap,
+                                                            const int32_t* __restrict__ changed) {
     // LDS: wcnt[4][kcap] (each wave's label counts, then its first local slot per
     // label), ls[kcap] (label's first local slot), gb[kcap] (label's destination),
     // stage[BATCH_CNT_ROWS] (local slot -> label << 16 | row in block)
@@ -726,6 +727,7 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
     int32_t* gb = ls + kcap;
     int32_t* stage = gb + kcap;
     __shared__ int32_t wsum[4];
+    __shared__ uint32_t cbits[BATCH_HIST_MAX / 32];  // changed clusters
     constexpr int G = BATCH_CNT_ROWS / 256;  // groups of 64 rows per wave
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -733,6 +735,14 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
     int32_t* wc = slds + wave * kcap;
     const uint64_t below = (uint64_t(1) << lane) - 1u;
     const int64_t total = pre[B];
+    if (changed) {
+        for (int w = t; w * 32 < kcap; w += 256) {
+            uint32_t m = 0;
+            for (int e = 0; e < 32 && w * 32 + e < kcap; ++e) m |= (changed[w * 32 + e] ? 1u : 0u) << e;
+            cbits[w] = m;
+        }
+        __syncthreads();
+    }
     for (int64_t b = blockIdx.x; b < total; b += gridDim.x) {
         const int ii = batch_find(pre, B, b);
         const batch_inst in = I[ii];
@@ -744,16 +754,41 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
         while ((1 << lbits) < k) ++lbits;
         const int32_t* lab_in = labels + in.row0 + r0;
         const int wr0 = wave * (BATCH_CNT_ROWS / 4);  // the wave's quarter of the block
-        int32_t lab[G], rk[G];
+        int32_t lab[G], rk[G], row[G];
 #pragma unroll
         for (int q = 0; q < G; ++q) {
             const int r = wr0 + q * 64 + lane;
             lab[q] = r < nr ? lab_in[r] : -1;
+            row[q] = r;
+        }
+        int groups = G;  // groups of 64 that hold rows
+        if (changed) {
+            // only the rows of changed clusters, packed in row order through the
+            // wave's part of the staging array (a wave reads its own writes)
+            int32_t* mine = stage + wr0;
+            int cnt = 0;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const bool keep = lab[q] >= 0 && lab[q] < k && ((cbits[lab[q] >> 5] >> (lab[q] & 31)) & 1u);
+                const uint64_t m = __ballot(keep);
+                if (keep) mine[cnt + __popcll(m & below)] = (lab[q] << 16) | row[q];
+                cnt += __popcll(m);
+            }
+            __builtin_amdgcn_wave_barrier();
+            groups = (cnt + 63) / 64;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const int v = q * 64 + lane < cnt ? mine[q * 64 + lane] : -1;
+                lab[q] = v >> 16;
+                row[q] = v & 0xffff;
+            }
         }
         for (int j = lane; j < k; j += 64) wc[j] = 0;
         // 1. rank of each row among the earlier rows of the wave's quarter with its label
 #pragma unroll
         for (int q = 0; q < G; ++q) {
+            rk[q] = -1;
+            if (q >= groups) continue;  // uniform
             const bool ok = lab[q] >= 0 && lab[q] < k;
             uint64_t same = __ballot(ok);
             for (int bit = 0; bit < lbits; ++bit) {
@@ -762,7 +797,6 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
                 same &= on ? m : ~m;
             }
             const int rank = __popcll(same & below);
-            rk[q] = -1;
             if (ok) {
                 rk[q] = wc[lab[q]] + rank;
                 if (rank == 0) wc[lab[q]] = rk[q] + __popcll(same);
@@ -799,7 +833,7 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < G; ++q)
-            if (rk[q] >= 0) stage[wc[lab[q]] + rk[q]] = (lab[q] << 16) | (wr0 + q * 64 + lane);
+            if (rk[q] >= 0) stage[wc[lab[q]] + rk[q]] = (lab[q] << 16) | row[q];
         __syncthreads();
         // 3. the block's rows of each label to their destination run, slot order
         int32_t* out = perm + in.row0;

@@ -47,6 +47,9 @@ __device__ __forceinline__ int64_t select_row(const row_select& s, int64_t e) {
     return s.rows ? int64_t(s.rows[e]) : e;
 }
 
+// the largest float at most v to within two roundings
+__device__ __forceinline__ float float_below(double v) { return float(v - fabs(v) * 1.2e-7); }
+
 // gap of a row settled with squared distances at most up2 (its centroid) and at
 // least lo2 (every other one); the float roundings here are below 1e-6
 __device__ __forceinline__ float bound_gap(double up2, double lo2, double gam, double base) {
@@ -54,7 +57,14 @@ __device__ __forceinline__ float bound_gap(double up2, double lo2, double gam, d
     const float l = sqrtf(float(fmax(lo2, 0.0)));
     if (!(double(u) < BOUND_MAX)) return -__builtin_inff();
     const double g = double(l) * (1.0 - gam) - double(u) * (1.0 + gam) + base;
-    return float(g - fabs(g) * 1.2e-7);
+    return float_below(g);
+}
+
+// gap of a row re-scored exactly: exact-form distances D1 (its centroid) and D2 (the
+// next one re-scored), and a lower bound lo2 of the squared distance to the others;
+// |D - dist^2| <= g dist^2
+__device__ __forceinline__ float bound_gap_exact(double D1, double D2, double lo2, double gam, double base) {
+    return bound_gap(D1 * (1.0 + 2.0 * gam), fmin(D2 * (1.0 - 2.0 * gam), lo2), gam, base);
 }
 
 // Before a pass with moved centroids: base_j += (drift_j + max drift)(1 + g),
@@ -77,39 +87,52 @@ __global__ __launch_bounds__(256) void bound_base_kernel(int k, const double* __
 }
 
 // The rows to assign again, as a dense list.  A workgroup takes runs of
-// SELECT_ROWS rows, counts its open rows with ballots and reserves its part of
-// the list with one atomic; rows keep their order inside a run.  8 bytes read per
-// row: bound by HBM.
+// SELECT_ROWS rows: a lane holds four consecutive rows of each of its wave's groups
+// of 256 (16-byte loads), positions inside the run come from four ballots, and one
+// atomic reserves the run's part of the list; rows keep their order inside a run.
+// 8 bytes read per row: bound by HBM.
 constexpr int SELECT_ROWS = 4096;
 __global__ __launch_bounds__(256) void bound_select_kernel(const int32_t* __restrict__ labels,
                                                            const float* __restrict__ gap,
                                                            const double* __restrict__ base, int64_t n,
                                                            int32_t* __restrict__ rows,
                                                            int32_t* __restrict__ count) {
-    constexpr int U = SELECT_ROWS / 256;
+    typedef int I4 __attribute__((ext_vector_type(4)));
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    constexpr int U = SELECT_ROWS / 1024;
     __shared__ int wtot[4];
     __shared__ int first;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t below = (uint64_t(1) << lane) - 1u;
     const int64_t runs = (n + SELECT_ROWS - 1) / SELECT_ROWS;
     for (int64_t q = blockIdx.x; q < runs; q += gridDim.x) {
-        // a wave's rows are consecutive groups of 64
-        const int64_t r0 = q * SELECT_ROWS + int64_t(wave) * (SELECT_ROWS / 4) + lane;
-        int32_t lab[U];
-        float g[U];
+        const int64_t r0 = q * SELECT_ROWS + int64_t(wave) * (SELECT_ROWS / 4) + 4 * lane;
+        I4 lab[U];
+        F4 g[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t r = r0 + 64 * u;
-            lab[u] = r < n ? labels[r] : 0;
-            g[u] = r < n ? gap[r] : 0.f;
+            const int64_t r = r0 + 256 * u;
+            if (r + 4 <= n) {
+                lab[u] = *reinterpret_cast<const I4*>(labels + r);
+                g[u] = *reinterpret_cast<const F4*>(gap + r);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    lab[u][e] = r + e < n ? labels[r + e] : 0;
+                    g[u][e] = r + e < n ? gap[r + e] : 0.f;
+                }
+            }
         }
-        uint64_t open[U];
+        uint64_t open[U][4];
         int mine = 0;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool settled = double(g[u]) > base[lab[u]] + BOUND_SLACK;
-            open[u] = __ballot(r0 + 64 * u < n && !settled);
-            mine += __popcll(open[u]);
-        }
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool settled = double(g[u][e]) > base[lab[u][e]] + BOUND_SLACK;
+                open[u][e] = __ballot(r0 + 256 * u + e < n && !settled);
+                mine += __popcll(open[u][e]);
+            }
         if (lane == 0) wtot[wave] = mine;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -119,11 +142,17 @@ __global__ __launch_bounds__(256) void bound_select_kernel(const int32_t* __rest
         __syncthreads();
         int at = first;
         for (int w = 0; w < wave; ++w) at += wtot[w];
-        const uint64_t below = (uint64_t(1) << lane) - 1u;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if ((open[u] >> lane) & 1u) rows[at + __popcll(open[u] & below)] = int32_t(r0 + 64 * u);
-            at += __popcll(open[u]);
+            int p = at;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                p += __popcll(open[u][e] & below);
+                at += __popcll(open[u][e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if ((open[u][e] >> lane) & 1u) rows[p++] = int32_t(r0 + 256 * u + e);
         }
         __syncthreads();  // wtot and first are rewritten by the next run
     }

@@ -69,6 +69,10 @@ struct refine_lists {
     double* coll_T;        // their thresholds (shifted value domain)
     int32_t* coll_count;   // ids gathered per entry (may exceed MAXC2: overflow)
     int32_t* coll_ids;     // MAXC2 ids per entry
+    // with bounds kept (km_bounds.hpp), else null: per candidate and per collect entry
+    // a lower bound of the squared distance to every centroid not among its ids
+    float* cand_lo;
+    float* coll_lo;
 };
 
 // Per-iteration centroid statistics used by the error bound.

@@ -141,7 +141,7 @@ struct km_ctx {
     km::dbuf cs_prev, cs_changed;                // its previous labels and changed-cluster flags
     // distance bounds of a training (row_bounds): gap and open rows, per row; base
     // and drift, per cluster
-    km::dbuf b_gap, b_rows, b_count, b_base, b_drift;
+    km::dbuf b_gap, b_rows, b_count, b_base, b_drift, cand_lo, coll_lo, seg_cand_lo, seg_coll_lo;
     // CSR path: values, column indices, row offsets (when uploaded), row squares,
     // transposed centroids, centroid squares, closest distances, structure flag
     km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cs, csr_closest, csr_flag;
@@ -360,6 +360,8 @@ static void launch_bf16(km_ctx* ctx, work<float>& w, bool collect) {
         S.coll_rows = take<int32_t>(ctx, &km_ctx::seg_coll_rows, w.A, ents);
         S.coll_T = take<double>(ctx, &km_ctx::seg_coll_T, w.A, ents);
         S.counts = take<int32_t>(ctx, &km_ctx::seg_counts, w.A, 2 * int64_t(nseg));
+        S.cand_lo = w.sel.gap ? ctx->seg_cand_lo.get<float>(ents) : nullptr;
+        S.coll_lo = w.sel.gap ? ctx->seg_coll_lo.get<float>(ents) : nullptr;
         auto kern = assign_bf16_kernel<DPB, NB, false>;
         KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    int(lds)));
@@ -388,14 +390,14 @@ static void launch_bf16(km_ctx* ctx, work<float>& w, bool collect) {
 template <typename F>
 static void refine_pairs(km_ctx* ctx, work<F>& w, const F* C, const int32_t* rows,
                          const int32_t* counts, const int32_t* ids, int stride,
-                         const int32_t* count_p) {
+                         const int32_t* count_p, const float* others) {
     const int64_t row_bytes = int64_t(refine_row_stride<F>(w.d)) * sizeof(F);
     const int rb = int(std::max<int64_t>(1, std::min<int64_t>(16, 16384 / row_bytes)));
     const size_t lds = size_t(4) * rb * row_bytes;
     auto kern = refine_pairs_kernel<F>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(kern, dim3(ctx->cu_count * 4), dim3(256), lds, ctx->stream, w.X, w.d, C, rows,
-                       counts, ids, stride, count_p, rb, w.L.full_rows, w.L.counters + 1, w.labels);
+                       counts, ids, stride, count_p, rb, w.L.full_rows, w.L.counters + 1, w.labels, others, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -451,7 +453,8 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
     }
     ctx->stats.assign_launches++;
     const int rgrid = ctx->cu_count * 4;
-    refine_pairs<F>(ctx, w, C, w.L.cand_rows, w.L.cand_count, w.L.cand_ids, MAXC, w.L.counters + 0);
+    refine_pairs<F>(ctx, w, C, w.L.cand_rows, w.L.cand_count, w.L.cand_ids, MAXC, w.L.counters + 0,
+                    w.L.cand_lo);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
             switch (w.dpad) {
@@ -461,16 +464,16 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
                 default: launch_bf16<256>(ctx, w, true); break;
             }
             refine_pairs<F>(ctx, w, C, w.L.coll_rows, w.L.coll_count, w.L.coll_ids, MAXC2,
-                            w.L.counters + 2);
+                            w.L.counters + 2, w.L.coll_lo);
         }
     }
     if (w.d % 4 == 0 && reinterpret_cast<uintptr_t>(w.X) % (4 * sizeof(F)) == 0 &&
         reinterpret_cast<uintptr_t>(C) % (4 * sizeof(F)) == 0)
         hipLaunchKernelGGL(refine_full_vec_kernel<F>, dim3(rgrid), dim3(256), 0, ctx->stream, w.X,
-                           w.d, C, w.k, w.L, w.labels);
+                           w.d, C, w.k, w.L, w.labels, w.sel);
     else
         hipLaunchKernelGGL(refine_full_kernel<F>, dim3(rgrid), dim3(256), 0, ctx->stream, w.X, w.d,
-                           C, w.k, w.L, w.labels);
+                           C, w.k, w.L, w.labels, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -644,7 +647,7 @@ static void label_group(km_ctx* ctx, const label_sort& ls, const int32_t* labels
     KM_LAUNCH_CHECK();
     const int grid = int(std::min<int64_t>(ls.nb, int64_t(ctx->cu_count) * 8));
     hipLaunchKernelGGL(batch_scatter_kernel, dim3(grid), dim3(256), batch_scatter_lds_bytes(ls.k), ctx->stream,
-                       ls.I, 1, ls.pre, labels, ls.bhist, perm, ls.k);
+                       ls.I, 1, ls.pre, labels, ls.bhist, perm, ls.k, ls.changed);
     KM_LAUNCH_CHECK();
 }
 
@@ -814,6 +817,8 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
         open_rows = ctx->b_rows.get<int32_t>(n);
         open_count = ctx->b_count.get<int32_t>(1);
         w.sel.gap = ctx->b_gap.get<float>(n);
+        w.L.cand_lo = ctx->cand_lo.get<float>(n);
+        if (path == 3) w.L.coll_lo = ctx->coll_lo.get<float>(n);
         w.sel.base = base;
         w.sel.gam = make_band<F>(d).g_canon + 1e-6;
     }
@@ -1651,7 +1656,8 @@ static void plan_iteration(km_ctx* ctx, batch_plan& p, hipEvent_t asg_start = nu
     if (p.csort) {
         hipLaunchKernelGGL(batch_scatter_kernel, dim3(g(p.P(BP::P_CNT, B))), dim3(256),
                            batch_scatter_lds_bytes(p.maxk),
-                           ctx->stream, p.dI, B, p.DP(BP::P_CNT), p.labels, p.bhist, p.perm, p.maxk);
+                           ctx->stream, p.dI, B, p.DP(BP::P_CNT), p.labels, p.bhist, p.perm, p.maxk,
+                           (const int32_t*)nullptr);
         KM_LAUNCH_CHECK();
     } else {
         rocprim::counting_iterator<int32_t> ids(0);
@@ -2244,7 +2250,8 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->init_d2, &ctx->init_chunks, &ctx->init_chosen, &ctx->init_ids,
                         &ctx->gt_d, &ctx->stat_acc, &ctx->coop_wcnt, &ctx->cs_inst, &ctx->cs_pre,
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
-                        &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
+                        &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
+                        &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
                         &ctx->csr_ct, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();

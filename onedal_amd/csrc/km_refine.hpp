@@ -7,6 +7,7 @@
 // as in select_min_distance (kernels_fp_impl.hpp:198-202).
 #pragma once
 
+#include "km_bounds.hpp"
 #include "km_common.hpp"
 
 namespace km {
@@ -20,7 +21,9 @@ namespace km {
 // different banks), the (row, id) pairs are spread over the lanes, each lane
 // forms the exact distance of its pair (features in order), reading the centroid
 // one 32-feature chunk ahead of the sum, and lane r keeps the minimum of entry r
-// (ties to the lowest id).
+// (ties to the lowest id), and with bounds kept (rs.gap) the second smallest: the
+// exact distances and the entry's bound of the other centroids (others) give the
+// row's gap, so a row between two centroids stays settled while they hardly move.
 template <typename F>
 __host__ __device__ inline int refine_row_stride(int d) {
     return d + int(16 / sizeof(F));
@@ -31,7 +34,8 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(
     const F* __restrict__ X, int d, const F* __restrict__ C, const int32_t* __restrict__ rows,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ ids, int stride,
     const int32_t* __restrict__ count_p, int rb, int32_t* __restrict__ full_rows,
-    int32_t* __restrict__ full_counter, int32_t* __restrict__ labels) {
+    int32_t* __restrict__ full_counter, int32_t* __restrict__ labels, const float* __restrict__ others,
+    row_select rs) {
     typedef F F4 __attribute__((ext_vector_type(4)));
     constexpr int CH = 32 / int(sizeof(F));  // 4-vectors per prefetched centroid chunk
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -88,7 +92,7 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(
         const int npairs = __shfl(incl, 63);
         pstart[wave][lane] = my_start;
         __builtin_amdgcn_wave_barrier();
-        F best = fp_traits<F>::inf;
+        F best = fp_traits<F>::inf, second = fp_traits<F>::inf;
         int bj = 0x7fffffff;
         for (int p0 = 0; p0 < npairs; p0 += 64) {
             const int p = p0 + lane;
@@ -146,14 +150,22 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(
                     const F v = pd[wave][q - p0];
                     const int jj = pj[wave][q - p0];
                     if (v < best || (v == best && jj < bj)) {
+                        second = best;
                         best = v;
                         bj = jj;
+                    } else if (v < second) {
+                        second = v;
                     }
                 }
             }
             __builtin_amdgcn_wave_barrier();
         }
-        if (lane < nr && my_cnt > 0) labels[my_row] = bj;
+        if (lane < nr && my_cnt > 0) {
+            labels[my_row] = bj;
+            if (rs.gap)
+                rs.gap[my_row] = bound_gap_exact(double(best), double(second), double(others[e0 + lane]), rs.gam,
+                                                 rs.base[bj]);
+        }
         __builtin_amdgcn_wave_barrier();
     }
 }
@@ -168,7 +180,7 @@ template <typename F>
 __global__ __launch_bounds__(256) void refine_full_kernel(const F* __restrict__ X, int d,
                                                           const F* __restrict__ C, int k,
                                                           const refine_lists L,
-                                                          int32_t* __restrict__ labels) {
+                                                          int32_t* __restrict__ labels, row_select rs) {
     constexpr int KT = 64, RW = 4, RB = 4 * RW;
     constexpr int FT = sizeof(F) == 4 ? 112 : 56;
     __shared__ F Ct[FT][KT + 1];
@@ -180,7 +192,7 @@ __global__ __launch_bounds__(256) void refine_full_kernel(const F* __restrict__ 
     const int nbatch = (total + RB - 1) / RB;
     for (int b = blockIdx.x; b < nbatch; b += gridDim.x) {
         int64_t rows[RW];
-        F best[RW];
+        F best[RW], second[RW];
         int bi[RW];
         bool nan0[RW];
 #pragma unroll
@@ -188,6 +200,7 @@ __global__ __launch_bounds__(256) void refine_full_kernel(const F* __restrict__ 
             const int e = b * RB + wave * RW + r;
             rows[r] = e < total ? int64_t(L.full_rows[e]) : -1;
             best[r] = fp_traits<F>::inf;
+            second[r] = fp_traits<F>::inf;
             bi[r] = 0x7fffffff;
             nan0[r] = false;
         }
@@ -225,51 +238,69 @@ __global__ __launch_bounds__(256) void refine_full_kernel(const F* __restrict__ 
                 for (int r = 0; r < RW; ++r) {
                     if (j == 0 && acc[r] != acc[r]) nan0[r] = true;
                     if (acc[r] < best[r]) {
+                        second[r] = best[r];
                         best[r] = acc[r];
                         bi[r] = j;
+                    } else if (acc[r] < second[r]) {
+                        second[r] = acc[r];
                     }
                 }
             }
         }
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
-            F bv = best[r];
+            F bv = best[r], sv = second[r];
             int bj = bi[r];
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) {
-                const F ob = __shfl_xor(bv, off);
+                const F ob = __shfl_xor(bv, off), os = __shfl_xor(sv, off);
                 const int oi = __shfl_xor(bj, off);
+                sv = fmin(fmin(sv, os), bv < ob ? ob : bv);
                 if (ob < bv || (ob == bv && oi < bj)) {
                     bv = ob;
                     bj = oi;
                 }
             }
             const bool n0 = __shfl(nan0[r] ? 1 : 0, 0) != 0;
-            if (lane == 0 && rows[r] >= 0) labels[rows[r]] = (n0 || bj == 0x7fffffff) ? 0 : bj;
+            if (lane == 0 && rows[r] >= 0) {
+                const bool none = n0 || bj == 0x7fffffff;
+                labels[rows[r]] = none ? 0 : bj;
+                if (rs.gap)
+                    rs.gap[rows[r]] = none ? -__builtin_inff()
+                                           : bound_gap_exact(double(bv), double(sv), __builtin_inf(), rs.gam, rs.base[bj]);
+            }
         }
     }
 }
 
-// refine_full_kernel for d % 4 == 0 with 4-vector aligned X and C.  A workgroup
-// takes 32 listed rows (8 per wave), staged in LDS as 4-vectors (feature chunks of
-// 32 KB when the rows do not fit); lane l carries centroid j0 + l of a 64-centroid
-// tile with its features in registers, a register chunk of 32 bytes per feature
-// group loaded one chunk ahead of use, and forms the exact-form sums of the
-// wave's 8 rows in feature order, reading the rows as LDS broadcasts.  Same scan
-// semantics as refine_full_kernel.
+// refine_full_kernel for d % 4 == 0 with 4-vector aligned X and C.  Listed rows are
+// staged in LDS as 4-vectors (feature chunks of 32 KB when they do not fit); lane l
+// carries centroid j0 + l of a 64-centroid tile with its features in registers, a
+// register chunk of 32 bytes per feature group loaded one chunk ahead of use, and
+// forms the exact-form sums of 8 rows in feature order, reading the rows as LDS
+// broadcasts.  Same scan semantics as refine_full_kernel.
+// The list is usually short, so the kernel is bound by one wave's chain of
+// centroid reads, not by their volume: WS waves of a workgroup share 8 rows and
+// take every WS-th tile (WS = 4 for k > 128, where one wave alone took the 16 tiles
+// of k = 1024, d = 128 in 0.23 ms a pass), and their results meet in LDS.
 template <typename F>
 __global__ __launch_bounds__(256) void refine_full_vec_kernel(const F* __restrict__ X, int d,
                                                               const F* __restrict__ C, int k,
                                                               const refine_lists L,
-                                                              int32_t* __restrict__ labels) {
+                                                              int32_t* __restrict__ labels, row_select rs) {
     typedef F F4 __attribute__((ext_vector_type(4)));
-    constexpr int RW = 8, RB = 4 * RW;
-    constexpr int VT = 32768 / (RB * int(sizeof(F4)));  // 4-vectors per staged row chunk
-    constexpr int CQ = 32 / int(sizeof(F));             // 4-vectors per register chunk
-    __shared__ F4 Xs[RB][VT];
+    constexpr int RW = 8;
+    constexpr int VT = 32768 / (4 * RW * int(sizeof(F4)));  // 4-vectors per staged row chunk
+    constexpr int CQ = 32 / int(sizeof(F));                 // 4-vectors per register chunk
+    __shared__ F4 Xs[4 * RW][VT];
+    __shared__ F w_best[4][RW], w_second[4][RW];
+    __shared__ int w_id[4][RW];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
+    const int WS = k > 128 ? 4 : k > 64 ? 2 : 1;  // waves per row group
+    const int RB = RW * (4 / WS);                 // rows per workgroup
+    const int rg = wave / WS, cw = wave % WS;     // this wave's row group and tile phase
     const int total = L.counters[1];
     const int nbatch = (total + RB - 1) / RB;
     const int nv = d / 4;
@@ -284,25 +315,23 @@ __global__ __launch_bounds__(256) void refine_full_vec_kernel(const F* __restric
         }
     };
     for (int b = blockIdx.x; b < nbatch; b += gridDim.x) {
-        int64_t rows[RW];
-        F best[RW];
+        F best[RW], second[RW];
         int bi[RW];
         bool nan0[RW];
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
-            const int e = b * RB + wave * RW + r;
-            rows[r] = e < total ? int64_t(L.full_rows[e]) : -1;
             best[r] = fp_traits<F>::inf;
+            second[r] = fp_traits<F>::inf;
             bi[r] = 0x7fffffff;
             nan0[r] = false;
         }
+        __syncthreads();  // the previous batch's LDS reads are done
         if (one_chunk) {
-            __syncthreads();
             stage(b, 0, nv);
             __syncthreads();
         }
-        for (int j0 = 0; j0 < k; j0 += 64) {
-            const int j = j0 + lane;
+        for (int j0 = 0; j0 < k; j0 += 64 * WS) {
+            const int j = j0 + 64 * cw + lane;
             const F4* c = reinterpret_cast<const F4*>(C + int64_t(j < k ? j : 0) * d);
             F acc[RW];
 #pragma unroll
@@ -326,7 +355,7 @@ __global__ __launch_bounds__(256) void refine_full_vec_kernel(const F* __restric
                         if (u0 + q < vt) {
 #pragma unroll
                             for (int r = 0; r < RW; ++r) {
-                                const F4 x4 = Xs[wave * RW + r][u0 + q];
+                                const F4 x4 = Xs[rg * RW + r][u0 + q];
 #pragma unroll
                                 for (int t = 0; t < 4; ++t) {
                                     const F diff = x4[t] - cur[q][t];
@@ -345,27 +374,58 @@ __global__ __launch_bounds__(256) void refine_full_vec_kernel(const F* __restric
                 for (int r = 0; r < RW; ++r) {
                     if (j == 0 && acc[r] != acc[r]) nan0[r] = true;
                     if (acc[r] < best[r]) {
+                        second[r] = best[r];
                         best[r] = acc[r];
                         bi[r] = j;
+                    } else if (acc[r] < second[r]) {
+                        second[r] = acc[r];
                     }
                 }
             }
         }
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
-            F bv = best[r];
+            F bv = best[r], sv = second[r];
             int bj = bi[r];
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) {
-                const F ob = __shfl_xor(bv, off);
+                const F ob = __shfl_xor(bv, off), os = __shfl_xor(sv, off);
                 const int oi = __shfl_xor(bj, off);
+                sv = fmin(fmin(sv, os), bv < ob ? ob : bv);
                 if (ob < bv || (ob == bv && oi < bj)) {
                     bv = ob;
                     bj = oi;
                 }
             }
+            // a NaN distance to centroid 0 (seen by phase 0's lane 0) keeps label 0
             const bool n0 = __shfl(nan0[r] ? 1 : 0, 0) != 0;
-            if (lane == 0 && rows[r] >= 0) labels[rows[r]] = (n0 || bj == 0x7fffffff) ? 0 : bj;
+            if (lane == 0) {
+                w_best[wave][r] = bv;
+                w_second[wave][r] = sv;
+                w_id[wave][r] = n0 ? -1 : bj;
+            }
+        }
+        __syncthreads();
+        if (tid < RB && b * RB + tid < total) {
+            const int g = tid / RW, r = tid - g * RW;
+            F bv = w_best[g * WS][r], sv = w_second[g * WS][r];
+            int bj = w_id[g * WS][r];
+            bool none = bj < 0;
+            for (int w = 1; w < WS; ++w) {
+                const F ob = w_best[g * WS + w][r], os = w_second[g * WS + w][r];
+                const int oi = w_id[g * WS + w][r];
+                sv = fmin(fmin(sv, os), bv < ob ? ob : bv);
+                if (ob < bv || (ob == bv && oi < bj)) {
+                    bv = ob;
+                    bj = oi;
+                }
+            }
+            none = none || bj == 0x7fffffff;
+            const int64_t row = L.full_rows[b * RB + tid];
+            labels[row] = none ? 0 : bj;
+            if (rs.gap)
+                rs.gap[row] = none ? -__builtin_inff()
+                                   : bound_gap_exact(double(bv), double(sv), __builtin_inf(), rs.gam, rs.base[bj]);
         }
     }
 }
