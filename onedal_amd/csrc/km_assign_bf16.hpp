@@ -178,83 +178,14 @@ __global__ __launch_bounds__(256) void convert_rows_bf16_kernel(
     }
 }
 
-// ---------------------------------------------------------------------------
-// centroids -> bf16(-2 c) padded rows, ||c||^2 (F), maxima of ||c||,
-// ||bf16(c)||, ||c - bf16(c)||, and with bounds kept how far the centroid moved.
-// One wave per centroid.  Rows k .. kp-1
-// (kp = bf16_padded_k(k)) are zero, so the last centroid blocks read defined
-// values without clamping.
-// max_bits: [0] C, [1] Ch, [2] Ec
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void centroid_prep_bf16_kernel(
-    const float* __restrict__ C, int k, int kp, int d, int dpb, uint16_t* __restrict__ Cb,
-    float* __restrict__ cn, unsigned long long* __restrict__ max_bits, drift_out dr) {
-    const int lane = threadIdx.x & 63;
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int nwaves = (gridDim.x * blockDim.x) >> 6;
-    for (int j = k + wave; j < kp; j += nwaves)
-        for (int f = lane; f < dpb; f += 64) Cb[int64_t(j) * dpb + f] = 0;
-    unsigned long long b0 = 0, b1 = 0, b2 = 0, b3 = 0;  // lane 0: this wave's maxima
-    for (int j = wave; j < k; j += nwaves) {
-        double s = 0.0, sh = 0.0, se = 0.0;
-        for (int f = lane; f < dpb; f += 64) {
-            const float v = f < d ? C[int64_t(j) * d + f] : 0.f;
-            const uint16_t b = f2bf(v);
-            Cb[int64_t(j) * dpb + f] = f2bf(-2.0f * bf2f(b));  // exact: -2 * bf16(c)
-            const double dv = double(v), dh = double(bf2f(b)), de = dv - dh;
-            s = fma(dv, dv, s);
-            sh = fma(dh, dh, sh);
-            se = fma(de, de, se);
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            s += __shfl_xor(s, off);
-            sh += __shfl_xor(sh, off);
-            se += __shfl_xor(se, off);
-        }
-        if (lane == 0) {
-            cn[j] = float(s);
-            const double up = 1.0 + 1e-12;
-            b0 = max(b0, (unsigned long long)__double_as_longlong(sqrt(s) * up));
-            b1 = max(b1, (unsigned long long)__double_as_longlong(sqrt(sh) * up));
-            b2 = max(b2, (unsigned long long)__double_as_longlong(sqrt(se) * up + 1e-30));
-        }
-        if (dr.cold) {
-            const double m = wave_drift<float>(C + int64_t(j) * d, static_cast<const float*>(dr.cold) + int64_t(j) * d,
-                                               d, lane);
-            if (lane == 0) dr.drift[j] = m;
-            b3 = max(b3, (unsigned long long)__double_as_longlong(m));
-        }
-    }
-    // one atomic per bound and workgroup (the maxima of non-negative doubles, or
-    // NaN, taken on their bit patterns as before)
-    __shared__ unsigned long long wb[4][4];
-    const int w = threadIdx.x >> 6;
-    if (lane == 0) {
-        wb[w][0] = b0;
-        wb[w][1] = b1;
-        wb[w][2] = b2;
-        wb[w][3] = b3;
-    }
-    __syncthreads();
-    if (threadIdx.x < 4) {
-        const int q = threadIdx.x;
-        const unsigned long long m = max(max(wb[0][q], wb[1][q]), max(wb[2][q], wb[3][q]));
-        if (m) atomicMax(q < 3 ? &max_bits[q] : dr.max_drift, m);
-    }
-}
-
-// B and the bound parameters for this pass (one thread).
-__global__ void bf16_params_kernel(const unsigned long long* __restrict__ cmax_bits,
-                                   const unsigned long long* __restrict__ xmax_bits,
-                                   bf16_consts kc, bf16_params* __restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// B and the bound parameters of a pass, from the maxima of ||c||, ||bf16(c)||,
+// ||c - bf16(c)|| and of the rows' ||x||, ||x - bf16(x)||
+__device__ __forceinline__ bf16_params make_bf16_params(double C, double Ch, double Ec, double X, double ex,
+                                                        const bf16_consts& kc) {
     bf16_params p;
-    p.C = __longlong_as_double((long long)cmax_bits[0]);
-    p.Ch = __longlong_as_double((long long)cmax_bits[1]);
-    p.Ec = __longlong_as_double((long long)cmax_bits[2]);
-    const double X = __longlong_as_double((long long)xmax_bits[0]);
-    const double ex = __longlong_as_double((long long)xmax_bits[1]);
+    p.C = C;
+    p.Ch = Ch;
+    p.Ec = Ec;
     // B >= max ||x||^2 + the largest value error, so every v_j stays positive;
     // the error terms that scale with B are below 2^-12 B, hence the 1.01 factor
     p.B = 0.0;
@@ -264,16 +195,7 @@ __global__ void bf16_params_kernel(const unsigned long long* __restrict__ cmax_b
     float fb = float(B);
     if (double(fb) < B) fb = __uint_as_float(__float_as_uint(fb) + 1u);
     p.B = double(fb);
-    *out = p;
-}
-
-// cnB_j = ||c_j||^2 + B rounded up (v_j keeps its lower bound); padded ids get
-// a huge start value so they are never chosen.  kp = bf16_padded_k(k) entries.
-__global__ void cnb_kernel(const float* __restrict__ cn, int k, int kp,
-                           const bf16_params* __restrict__ params_p, float* __restrict__ cnb) {
-    const float Bf = float(params_p->B);
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < kp; j += gridDim.x * blockDim.x)
-        cnb[j] = j < k ? add_round_up(cn[j], Bf) : __uint_as_float(0x7F000000u);
+    return p;
 }
 
 // Centroid blocks live in a ring of LDS slots, filled ahead of use with
@@ -310,13 +232,15 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // avoids the hazards itself: the base SGPRs typically come from v_readfirstlane
 // just before, and a VMEM read of an SGPR written by a VALU op needs 5 wait
 // states (otherwise the load may use the register's previous contents as the
-// address).  The load therefore reads a copy made by a scalar move (no wait
-// states after an SALU write), and that move is also the one wait state that an
-// M0 write -> LDS DMA needs.
+// address).  The load therefore reads a copy made by a scalar move, and the move and
+// the no-op are the five wait states for whatever VALU op (also the reload of a
+// spilled SGPR into the copy's registers) the compiler puts before the asm; they
+// cover the one that an M0 write -> LDS DMA needs.
 __device__ __forceinline__ void lds_dma16(const void* gbase, uint32_t voff, uint32_t lds_base) {
     uint64_t base;
     asm volatile(
         "s_mov_b64 %0, %3\n\t"
+        "s_nop 3\n\t"
         "global_load_lds_dwordx4 %1, %0"
         : "=&s"(base)
         : "v"(voff), "{m0}"(lds_base), "s"(gbase)
@@ -335,6 +259,7 @@ __device__ __forceinline__ void lds_dma4(const void* gbase, uint32_t voff, uint3
     uint64_t base;
     asm volatile(
         "s_mov_b64 %0, %3\n\t"
+        "s_nop 3\n\t"
         "global_load_lds_dword %1, %0"
         : "=&s"(base)
         : "v"(voff), "{m0}"(lds_base), "s"(gbase)

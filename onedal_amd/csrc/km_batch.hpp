@@ -667,18 +667,6 @@ __global__ __launch_bounds__(256) void sort_group_sums_kernel(const int32_t* __r
     gsum[e] = s;
 }
 
-// counts[j] = label j's count over every block (the column sums of gsum), in
-// place of one global atomic per (block, label)
-__global__ __launch_bounds__(256) void sort_counts_kernel(const int32_t* __restrict__ gsum, int k, int G,
-                                                          int32_t* __restrict__ counts) {
-    const int j = int(blockIdx.x) * 256 + int(threadIdx.x);
-    if (j >= k) return;
-    int32_t s = 0;
-#pragma unroll 16
-    for (int g = 0; g < G; ++g) s += gsum[int64_t(g) * k + j];
-    counts[j] = s;
-}
-
 __global__ __launch_bounds__(256) void sort_block_bases_kernel(int32_t* __restrict__ bhist, int64_t nb, int k,
                                                                int G, int GB, const int32_t* __restrict__ gsum,
                                                                const int64_t* __restrict__ offsets) {

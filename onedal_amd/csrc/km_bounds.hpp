@@ -67,25 +67,6 @@ __device__ __forceinline__ float bound_gap_exact(double D1, double D2, double lo
     return bound_gap(D1 * (1.0 + 2.0 * gam), fmin(D2 * (1.0 - 2.0 * gam), lo2), gam, base);
 }
 
-// Before a pass with moved centroids: base_j += (drift_j + max drift)(1 + g),
-// rounded up; the changed-cluster flags and the pass's counters (selected rows,
-// re-score lists) start at zero.
-__global__ __launch_bounds__(256) void bound_base_kernel(int k, const double* __restrict__ drift,
-                                                         const unsigned long long* __restrict__ max_drift,
-                                                         double gam, double* __restrict__ base,
-                                                         int32_t* __restrict__ changed,
-                                                         int32_t* __restrict__ sel_count,
-                                                         int32_t* __restrict__ counters) {
-    const double m = __longlong_as_double((long long)*max_drift);
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < k; j += gridDim.x * blockDim.x) {
-        const double b = (base[j] + (drift[j] + m) * (1.0 + gam)) * (1.0 + 1e-15);
-        base[j] = b < BOUND_MAX ? b : __builtin_inf();
-        changed[j] = 0;
-    }
-    if (blockIdx.x == 0 && threadIdx.x < 3) counters[threadIdx.x] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 3) *sel_count = 0;
-}
-
 // The rows to assign again, as a dense list.  A workgroup takes runs of
 // SELECT_ROWS rows: a lane holds four consecutive rows of each of its wave's groups
 // of 256 (16-byte loads), positions inside the run come from four ballots, and one
@@ -156,28 +137,6 @@ __global__ __launch_bounds__(256) void bound_select_kernel(const int32_t* __rest
         }
         __syncthreads();  // wtot and first are rewritten by the next run
     }
-}
-
-// Centroid movement, taken by the preparation kernels (one wave per centroid): lane
-// partials of ||cnew - cold||^2, reduced over the wave and rounded up.  Its maximum is
-// kept as the bits of a non-negative double (a NaN wins).
-struct drift_out {
-    const void* cold;  // previous centroids (null: no bounds kept)
-    double* drift;     // k
-    unsigned long long* max_drift;
-};
-
-template <typename F>
-__device__ __forceinline__ double wave_drift(const F* __restrict__ cnew, const F* __restrict__ cold, int d,
-                                             int lane) {
-    double s = 0.0;
-    for (int f = lane; f < d; f += 64) {
-        const double v = double(cnew[f]) - double(cold[f]);
-        s = fma(v, v, s);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    return sqrt(s) * (1.0 + 1e-12);
 }
 
 }  // namespace km

@@ -260,9 +260,7 @@ template <typename F>
 __global__ __launch_bounds__(256) void csr_objective_chunks_kernel(const F* __restrict__ closest,
                                                                    int64_t n,
                                                                    double* __restrict__ d64_out,
-                                                                   double* __restrict__ chunk_sums,
-                                                                   const int32_t* __restrict__ gate) {
-    if (gate && gate[0] == 0) return;  // gated off (no empty clusters this iteration)
+                                                                   double* __restrict__ chunk_sums) {
     __shared__ double part[256];
     const int t = threadIdx.x;
     const int64_t nchunks = (n + OBJ_CHUNK - 1) / OBJ_CHUNK;

@@ -5,12 +5,13 @@
 // (cluster_updater.hpp:82-179) and infer_kernel_gpu (infer_kernel_dpc.cpp:36-107).
 //
 // One Lloyd iteration on the context's stream:
-//   centroid_prep -> assign (+ exact re-score) -> count -> scan -> stable sort of
-//   row ids by label -> chunk sums (FP64) -> merge/divide [-> objective]
-//   -> one small D2H (empty-cluster count, objective) and a stream sync
-//   [-> empty-cluster refill].
-// The reference syncs twice per iteration (cluster_updater.hpp:135-136 and
-// kernels_integral_dpc.cpp:148); this driver syncs once.
+//   open rows (km_bounds.hpp) -> assign (+ exact re-score) -> counts, scan and stable
+//   grouping of row ids by label -> chunk sums (FP64) of the changed clusters
+//   [-> objective] -> centroid step (merge, divide, preparation of the next pass,
+//   bounds) [-> empty-cluster refill].
+// The reference waits for the device twice per iteration (cluster_updater.hpp:135-136
+// and kernels_integral_dpc.cpp:148); here the scan and the objective write what the
+// host decides by to host memory, and the stream is not waited for.
 
 #include <hip/hip_runtime.h>
 
@@ -43,6 +44,7 @@
 #include "km_probe.hpp"
 #include "km_rng.hpp"
 #include "km_refine.hpp"
+#include "km_step.hpp"
 #include "km_update.hpp"
 
 namespace km {
@@ -136,7 +138,7 @@ struct km_ctx {
     km::dbuf tune_x, tune_c, tune_l;  // autotuner inputs (released after tuning)
     km::dbuf init_d2, init_chunks, init_chosen, init_ids;  // initialisation
     km::dbuf gt_d;  // empty-cluster candidates' d64
-    km::dbuf stat_acc, coop_wcnt;  // device-side statistics; per-workgroup counts of ec_count_kernel
+    km::dbuf stat_acc, ec_wcnt;  // device-side statistics; per-workgroup counts of ec_count_kernel
     km::dbuf cs_inst, cs_pre, cs_hist, cs_gsum;  // single-instance counting sort (label_sort)
     km::dbuf cs_prev, cs_changed;                // its previous labels and changed-cluster flags
     // distance bounds of a training (row_bounds): gap and open rows, per row; base
@@ -145,7 +147,13 @@ struct km_ctx {
     // CSR path: values, column indices, row offsets (when uploaded), row squares,
     // transposed centroids, centroid squares, closest distances, structure flag
     km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cs, csr_closest, csr_flag;
-    int32_t* pinned = nullptr;  // small pinned host staging: meta[2], counters[2], obj (as 2 ints)
+    // step_ticket: zero between launches; step_max: centroid_step_kernel's workspace.
+    // Both live from the context's creation on.
+    km::dbuf step_ticket, step_max;
+    int32_t* pinned = nullptr;  // small pinned host staging, then the kernels' reports
+    km::host_report* report = nullptr;          // host address
+    km::objective_report* obj_report = nullptr;
+    uint32_t seq = 0;  // of the last report asked for
     // this device's copy of the scratch array (null if its address is unknown)
     void* scratch = nullptr;
     std::string scratch_err;
@@ -214,7 +222,7 @@ struct work {
     refine_lists L{};
     F* cn = nullptr;
     F* cpad = nullptr;
-    unsigned long long* cmax_bits = nullptr;  // [0] max ||c|| ([1], [2]: BF16 path), [3] max drift
+    double* maxima = nullptr;  // [0] max ||c||, BF16 path: [1] max ||bf16(c)||, [2] max ||c - bf16(c)||
     // BF16 path
     uint16_t* Xb = nullptr;       // n x dpad bf16 rows
     float* enorm = nullptr;       // ||x - bf16(x)|| (up)
@@ -224,6 +232,14 @@ struct work {
     bf16_params* params = nullptr;
     // rows of the next assignment pass, and where their bounds go
     row_select sel{nullptr, nullptr, nullptr, nullptr, 0.0};
+    // training: centroid movement and bounds per cluster, changed clusters, the open
+    // rows' count, and the re-score counters summed over the passes
+    double* drift = nullptr;
+    double* base = nullptr;
+    int32_t* changed = nullptr;
+    int32_t* open_rows = nullptr;
+    int32_t* open_count = nullptr;
+    unsigned long long* acc = nullptr;
     // workspace source: a fixed arena, or (null) the context's buffers
     arena* A = nullptr;
 };
@@ -273,34 +289,57 @@ static bf16_consts make_bf16_consts(int d, int k) {
     return c;
 }
 
-// per-centroid prep: ||c||^2, padded copy, max ||c||; with dr.cold (a training
-// iteration after the first, whose scan has cleared the maxima) the centroids'
-// movement too
+// chunk sums that a centroid step merges
+struct chunk_sums {
+    const double* part;
+    const int32_t* counts;
+    const int32_t* chunk_base;
+};
+
+// The centroid step before an assignment pass (km_step.hpp): C from the chunk sums
+// (when given), its preparation for the path, and with cold (the previous
+// centroids) the bounds.  The re-score counters are clear afterwards.
 template <typename F>
-static void centroid_prep(km_ctx* ctx, work<F>& w, const F* C, int path,
-                          const drift_out& dr = {nullptr, nullptr, nullptr}) {
-    if (!dr.cold) fill<unsigned long long>(ctx, w.cmax_bits, 4, 0ull);
+static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* cold = nullptr,
+                           const chunk_sums& m = {nullptr, nullptr, nullptr}) {
+    centroid_step<F> s{};
+    s.part = m.part;
+    s.counts = m.counts;
+    s.chunk_base = m.chunk_base;
+    s.C = C;
+    s.cold = cold;
+    s.k = w.k;
+    s.d = w.d;
+    s.dpad = w.dpad;
+    s.cn = w.cn;
+    s.cpad = path == 2 ? w.cpad : nullptr;
+    s.kp = w.k;
+    s.maxima = w.maxima;
+    s.drift = w.drift;
+    s.base = w.base;
+    s.gam = w.sel.gam;
+    s.changed = w.changed;
+    s.sel_count = w.open_count;
+    s.counters = w.L.counters;
+    s.acc = cold ? w.acc : nullptr;
+    s.ticket = ctx->step_ticket.get<uint32_t>(1);
+    s.wgmax = ctx->step_max.get<unsigned long long>(4 * STEP_MAX_GRID);
+    const int grid = std::min(w.k, STEP_MAX_GRID);
+    const size_t lds = size_t(w.d) * sizeof(F);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
-            const int kp = bf16_padded_k(w.k);
-            // four centroids per wave, so few workgroups add to the three maxima
-            const int grid = grid_for(ctx, int64_t(kp) * 16, 256, 4);
-            hipLaunchKernelGGL(centroid_prep_bf16_kernel, dim3(grid), dim3(256), 0, ctx->stream, C,
-                               w.k, kp, w.d, w.dpad, w.Cb, w.cn, w.cmax_bits, dr);
-            KM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(bf16_params_kernel, dim3(1), dim3(64), 0, ctx->stream, w.cmax_bits,
-                               w.xmax_bits, make_bf16_consts(w.d, w.k), w.params);
-            KM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(cnb_kernel, dim3(grid_for(ctx, kp, 256, 1)), dim3(256), 0, ctx->stream,
-                               w.cn, w.k, kp, w.params, w.cnb);
+            s.Cb = w.Cb;
+            s.kp = bf16_padded_k(w.k);
+            s.xmax_bits = w.xmax_bits;
+            s.kc = make_bf16_consts(w.d, w.k);
+            s.params = w.params;
+            s.cnb = w.cnb;
+            hipLaunchKernelGGL((centroid_step_kernel<float, true>), dim3(grid), dim3(256), lds, ctx->stream, s);
             KM_LAUNCH_CHECK();
             return;
         }
     }
-    const bool need_pad = path == 2;
-    const int grid = grid_for(ctx, int64_t(w.k) * 64, 256, 4);
-    hipLaunchKernelGGL(centroid_prep_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, C, w.k, w.d,
-                       w.dpad, w.cn, need_pad ? w.cpad : (F*)nullptr, w.cmax_bits, dr);
+    hipLaunchKernelGGL((centroid_step_kernel<F, false>), dim3(grid), dim3(256), lds, ctx->stream, s);
     KM_LAUNCH_CHECK();
 }
 
@@ -310,7 +349,7 @@ static void launch_mfma_f32_mode(km_ctx* ctx, work<float>& w, const band_consts&
     auto kern = assign_mfma_f32_kernel<DP, NB, RES>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.Xv, w.ldx, w.n, w.d, w.cpad,
-                       w.k, w.cn, w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L, w.sel);
+                       w.k, w.cn, w.xnorm, w.maxima, bc, w.labels, w.L, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -336,7 +375,7 @@ static void launch_mfma_f64(km_ctx* ctx, work<double>& w, const band_consts& bc)
     auto kern = assign_mfma_f64_kernel<DP, NB>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.Xv, w.ldx, w.n, w.d, w.cpad, w.k, w.cn,
-                       w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L, w.sel);
+                       w.xnorm, w.maxima, bc, w.labels, w.L, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -388,24 +427,20 @@ static void launch_bf16(km_ctx* ctx, work<float>& w, bool collect) {
 
 // exact re-score of a list of (row, candidate ids) entries; overflow -> full list
 template <typename F>
-static void refine_pairs(km_ctx* ctx, work<F>& w, const F* C, const int32_t* rows,
-                         const int32_t* counts, const int32_t* ids, int stride,
-                         const int32_t* count_p, const float* others) {
+static void refine_pairs(km_ctx* ctx, work<F>& w, const F* C, const pair_list& list) {
     const int64_t row_bytes = int64_t(refine_row_stride<F>(w.d)) * sizeof(F);
     const int rb = int(std::max<int64_t>(1, std::min<int64_t>(16, 16384 / row_bytes)));
     const size_t lds = size_t(4) * rb * row_bytes;
     auto kern = refine_pairs_kernel<F>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL(kern, dim3(ctx->cu_count * 4), dim3(256), lds, ctx->stream, w.X, w.d, C, rows,
-                       counts, ids, stride, count_p, rb, w.L.full_rows, w.L.counters + 1, w.labels, others, w.sel);
+    hipLaunchKernelGGL(kern, dim3(ctx->cu_count * 4), dim3(256), lds, ctx->stream, w.X, w.d, C, list,
+                       rb, w.L.full_rows, w.L.counters + 1, w.labels, w.sel);
     KM_LAUNCH_CHECK();
 }
 
-// assignment of the selected rows against w.X/C (centroid_prep already done for C);
-// a selected pass starts with cleared counters (bound_base_kernel)
+// assignment of the selected rows against w.X/C (after step_centroids for C)
 template <typename F>
 static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
-    if (!w.sel.rows) fill<int32_t>(ctx, w.L.counters, 3, 0);
     const band_consts bc = make_band<F>(w.d);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing) {
@@ -445,7 +480,7 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
         const int64_t tiles = (w.n + 63) / 64;
         const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * 4)));
         hipLaunchKernelGGL(assign_generic_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, w.X, w.n,
-                           w.d, C, w.k, w.cn, w.xnorm, (const double*)w.cmax_bits, bc, w.labels, w.L, w.sel);
+                           w.d, C, w.k, w.cn, w.xnorm, w.maxima, bc, w.labels, w.L, w.sel);
         KM_LAUNCH_CHECK();
     }
     if (ctx->timing) {
@@ -453,8 +488,8 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
     }
     ctx->stats.assign_launches++;
     const int rgrid = ctx->cu_count * 4;
-    refine_pairs<F>(ctx, w, C, w.L.cand_rows, w.L.cand_count, w.L.cand_ids, MAXC, w.L.counters + 0,
-                    w.L.cand_lo);
+    refine_pairs<F>(ctx, w, C,
+                    {w.L.cand_rows, w.L.cand_count, w.L.cand_ids, w.L.cand_lo, w.L.counters + 0, MAXC});
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
             switch (w.dpad) {
@@ -463,8 +498,8 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
                 case 128: launch_bf16<128>(ctx, w, true); break;
                 default: launch_bf16<256>(ctx, w, true); break;
             }
-            refine_pairs<F>(ctx, w, C, w.L.coll_rows, w.L.coll_count, w.L.coll_ids, MAXC2,
-                            w.L.counters + 2, w.L.coll_lo);
+            refine_pairs<F>(ctx, w, C,
+                            {w.L.coll_rows, w.L.coll_count, w.L.coll_ids, w.L.coll_lo, w.L.counters + 2, MAXC2});
         }
     }
     if (w.d % 4 == 0 && reinterpret_cast<uintptr_t>(w.X) % (4 * sizeof(F)) == 0 &&
@@ -477,29 +512,52 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
     KM_LAUNCH_CHECK();
 }
 
-// objective chunk sums (objective_chunks_kernel)
+// d64 of every row against its label's centroid
 template <typename F>
-static void launch_objective(km_ctx* ctx, int grid, const F* X, int64_t n, int d, const F* C,
-                             const int32_t* labels, double* d64_out, double* chunks,
-                             const int32_t* gate = nullptr) {
-    const size_t lds = objective_lds_bytes<F>();
-    hipLaunchKernelGGL(objective_chunks_kernel<F>, dim3(grid), dim3(256), lds, ctx->stream, X, n, d, C, labels,
-                       d64_out, chunks, gate);
+static void launch_d64(km_ctx* ctx, const F* X, int64_t n, int d, const F* C, const int32_t* labels, double* d64) {
+    hipLaunchKernelGGL(row_d64_kernel<F>, dim3(grid_for(ctx, n, D64_ROWS, 8)), dim3(256), 0, ctx->stream, X, n, d, C,
+                       labels, d64);
     KM_LAUNCH_CHECK();
 }
 
-// objective of the current labels against C; optional per-row d64 output
+// the objective from the rows' d64, onto *start (null: 0), into *out and (seq not 0)
+// the context's report with the re-scored rows
+static void launch_objective_sum(km_ctx* ctx, const double* d64, int64_t n, double* chunks, const double* start,
+                                 double* out, const int32_t* counters, const unsigned long long* acc, uint32_t seq) {
+    const int64_t nchunks = (n + OBJ_CHUNK - 1) / OBJ_CHUNK;
+    hipLaunchKernelGGL(objective_sum_kernel, dim3(grid_for(ctx, nchunks, 1, 4)), dim3(256), 0, ctx->stream, d64, n,
+                       chunks, start, out, seq ? ctx->obj_report : (objective_report*)nullptr, seq, counters, acc,
+                       ctx->step_ticket.get<uint32_t>(1));
+    KM_LAUNCH_CHECK();
+}
+
+// objective of the current labels against C; d64 holds the rows' distances afterwards
 template <typename F>
-static double* objective(km_ctx* ctx, work<F>& w, const F* C, double* d64_out) {
-    const int64_t nchunks = (w.n + OBJ_CHUNK - 1) / OBJ_CHUNK;
-    double* chunks = ctx->obj_chunks.get<double>(nchunks);
+static double* objective(km_ctx* ctx, work<F>& w, const F* C, double* d64, uint32_t seq) {
+    double* chunks = ctx->obj_chunks.get<double>((w.n + OBJ_CHUNK - 1) / OBJ_CHUNK);
     double* out = ctx->obj_dev.get<double>(1);
-    const int grid = int(std::min<int64_t>(nchunks, int64_t(ctx->cu_count) * 8));
-    launch_objective<F>(ctx, grid, w.X, w.n, w.d, C, w.labels, d64_out, chunks);
-    KM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sum_sequential_kernel, dim3(1), dim3(64), 0, ctx->stream, chunks, nchunks, out);
-    KM_LAUNCH_CHECK();
+    launch_d64<F>(ctx, w.X, w.n, w.d, C, w.labels, d64);
+    launch_objective_sum(ctx, d64, w.n, chunks, nullptr, out, w.L.counters, w.acc, seq);
     return out;
+}
+
+// Waits until a kernel of the stream has written seq to *word (host memory).  The
+// value precedes the end of the work queued behind that kernel, so the host goes
+// on while the stream is busy; a failed or drained stream ends the wait.
+static void wait_report(km_ctx* ctx, const uint32_t* word, uint32_t seq) {
+    for (uint64_t spin = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) != seq; ++spin) {
+        if (spin % 4096) continue;
+        const hipError_t e = hipStreamQuery(ctx->stream);
+        if (e == hipErrorNotReady) continue;
+        KM_HIP(e);
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != seq)
+            throw status_error(KM_INTERNAL_ERROR, "the stream ended without its report");
+    }
+}
+
+static uint32_t next_seq(km_ctx* ctx) {
+    if (++ctx->seq == 0) ++ctx->seq;  // 0 means no report
+    return ctx->seq;
 }
 
 template <typename F>
@@ -555,14 +613,17 @@ static void sort_by_label(km_ctx* ctx, const int32_t* labels, int64_t n, int k, 
                                      bits, ctx->stream));
 }
 
-// Label counts and the stable grouping of row ids by label for one instance.
-// k <= BATCH_HIST_MAX: the batched path's counting sort on a one-instance table
-// (per-block histograms that also add into counts, block destinations from
-// sort_group_sums_kernel / sort_block_bases_kernel, the LDS-staged scatter);
-// otherwise count_kernel and rocPRIM's radix sort.  Both leave the members of
-// each cluster in ascending row order.
+// Label counts and the stable grouping of row ids by label for one instance: which
+// clusters' members changed, the counts, the scan (offsets, chunks, empty clusters,
+// reported to the host) and the row ids grouped by label (of the changed clusters;
+// the members of each in ascending row order).
+// n <= SMALL_GROUP_ROWS and k <= SMALL_GROUP_K: one workgroup does it all
+// (small_group_kernel).  k <= BATCH_HIST_MAX: the batched path's counting sort on a
+// one-instance table (per-block histograms, block destinations from
+// sort_group_sums_kernel / sort_block_bases_kernel, the LDS-staged scatter).
+// Otherwise count_kernel and rocPRIM's radix sort.
 struct label_sort {
-    bool csort = false;
+    bool small = false, csort = false;
     int64_t n = 0, nb = 0;
     int k = 0, G = 0, GB = 0;
     batch_inst* I = nullptr;
@@ -587,9 +648,15 @@ static label_sort label_sort_setup(km_ctx* ctx, int64_t n, int k) {
     ls.changed = ctx->cs_changed.get<int32_t>(k);
     fill<int32_t>(ctx, ls.changed, k, 0);
     if (k > BATCH_HIST_MAX) return ls;
-    ls.csort = true;
     ls.prev = ctx->cs_prev.get<int32_t>(n);
     fill<int32_t>(ctx, ls.prev, n, -1);
+    if (n <= SMALL_GROUP_ROWS && k <= SMALL_GROUP_K) {
+        ls.small = true;
+        KM_HIP(hipFuncSetAttribute((const void*)small_group_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   int(small_group_lds_bytes(SMALL_GROUP_K))));
+        return ls;
+    }
+    ls.csort = true;
     ls.nb = (n + BATCH_CNT_ROWS - 1) / BATCH_CNT_ROWS;
     ls.G = int(std::min<int64_t>(ls.nb, 64));
     ls.GB = int((ls.nb + ls.G - 1) / ls.G);
@@ -608,100 +675,97 @@ static label_sort label_sort_setup(km_ctx* ctx, int64_t n, int k) {
     return ls;
 }
 
-// counts of the labels (with the counting sort: the block histograms, their
-// group sums, and the counts as the column sums of those) and the flags of the
-// clusters whose members changed (cleared before the call)
-static void label_counts(km_ctx* ctx, const label_sort& ls, const int32_t* labels, int32_t* counts) {
-    if (ls.csort) {
-        const int grid = int(std::min<int64_t>(ls.nb, int64_t(ctx->cu_count) * 8));
-        hipLaunchKernelGGL(label_hist_kernel, dim3(grid), dim3(256), 0, ctx->stream, labels, ls.prev, ls.n, ls.k,
-                           ls.bhist, ls.changed);
-        KM_LAUNCH_CHECK();
-        const int g2 = int((int64_t(ls.G) * ls.k + 255) / 256);
-        hipLaunchKernelGGL(sort_group_sums_kernel, dim3(g2), dim3(256), 0, ctx->stream, ls.bhist, ls.nb, ls.k, ls.G,
-                           ls.GB, ls.gsum);
-        KM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(sort_counts_kernel, dim3((ls.k + 255) / 256), dim3(256), 0, ctx->stream, ls.gsum, ls.k,
-                           ls.G, counts);
-    } else {
-        fill<int32_t>(ctx, ls.changed, ls.k, 1);  // not tracked: every cluster is summed again
-        fill<int32_t>(ctx, counts, ls.k, 0);
-        const bool lds = ls.k <= 16384;
-        hipLaunchKernelGGL(count_kernel, dim3(grid_for(ctx, ls.n, 256, 4)), dim3(256),
-                           lds ? ls.k * sizeof(int32_t) : 0, ctx->stream, labels, ls.n, ls.k, counts, lds ? 1 : 0);
-    }
-    KM_LAUNCH_CHECK();
-}
+// results of label_group
+struct cluster_lists {
+    int32_t* counts;
+    int64_t* offsets;
+    int32_t* chunk_base;
+    int32_t* empty_list;
+    int32_t* meta;
+    int32_t* perm;
+};
 
-// row ids grouped by label (after the scan has set offsets)
-static void label_group(km_ctx* ctx, const label_sort& ls, const int32_t* labels, const int64_t* offsets,
-                        int32_t* perm) {
-    if (!ls.csort) {
-        sort_by_label(ctx, labels, ls.n, ls.k, perm);
+// ls.changed must be clear before the call; the empty clusters are reported with seq
+static void label_group(km_ctx* ctx, const label_sort& ls, const int32_t* labels, const cluster_lists& o,
+                        uint32_t seq) {
+    const int k = ls.k;
+    if (ls.small) {
+        hipLaunchKernelGGL(small_group_kernel, dim3(1), dim3(1024), small_group_lds_bytes(k), ctx->stream, labels,
+                           ls.prev, int(ls.n), k, o.counts, ls.changed, o.offsets, o.chunk_base, o.empty_list, o.meta,
+                           o.perm, ctx->report, seq);
+        KM_LAUNCH_CHECK();
         return;
     }
-    // the group sums are label_counts' (bhist is unchanged since)
-    const int g2 = int((int64_t(ls.G) * ls.k + 255) / 256);
-    hipLaunchKernelGGL(sort_block_bases_kernel, dim3(g2), dim3(256), 0, ctx->stream, ls.bhist, ls.nb, ls.k, ls.G,
-                       ls.GB, ls.gsum, offsets);
-    KM_LAUNCH_CHECK();
     const int grid = int(std::min<int64_t>(ls.nb, int64_t(ctx->cu_count) * 8));
-    hipLaunchKernelGGL(batch_scatter_kernel, dim3(grid), dim3(256), batch_scatter_lds_bytes(ls.k), ctx->stream,
-                       ls.I, 1, ls.pre, labels, ls.bhist, perm, ls.k, ls.changed);
+    const int g2 = int((int64_t(ls.G) * k + 255) / 256);
+    if (ls.csort) {
+        hipLaunchKernelGGL(label_hist_kernel, dim3(grid), dim3(256), 0, ctx->stream, labels, ls.prev, ls.n, k,
+                           ls.bhist, ls.changed);
+        KM_LAUNCH_CHECK();
+        hipLaunchKernelGGL(sort_group_sums_kernel, dim3(g2), dim3(256), 0, ctx->stream, ls.bhist, ls.nb, k, ls.G,
+                           ls.GB, ls.gsum);
+        KM_LAUNCH_CHECK();
+    } else {
+        fill<int32_t>(ctx, ls.changed, k, 1);  // not tracked: every cluster is summed again
+        fill<int32_t>(ctx, o.counts, k, 0);
+        const bool lds = k <= 16384;
+        hipLaunchKernelGGL(count_kernel, dim3(grid_for(ctx, ls.n, 256, 4)), dim3(256),
+                           lds ? k * sizeof(int32_t) : 0, ctx->stream, labels, ls.n, k, o.counts, lds ? 1 : 0);
+        KM_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(scan_clusters_kernel, dim3(1), dim3(1024), 0, ctx->stream, o.counts,
+                       ls.csort ? ls.gsum : (const int32_t*)nullptr, ls.G, k, o.offsets, o.chunk_base, o.empty_list,
+                       o.meta, ls.changed, ctx->report, seq);
+    KM_LAUNCH_CHECK();
+    if (!ls.csort) {
+        sort_by_label(ctx, labels, ls.n, k, o.perm);
+        return;
+    }
+    hipLaunchKernelGGL(sort_block_bases_kernel, dim3(g2), dim3(256), 0, ctx->stream, ls.bhist, ls.nb, k, ls.G, ls.GB,
+                       ls.gsum, o.offsets);
+    KM_LAUNCH_CHECK();
+    hipLaunchKernelGGL(batch_scatter_kernel, dim3(grid), dim3(256), batch_scatter_lds_bytes(k), ctx->stream, ls.I, 1,
+                       ls.pre, labels, ls.bhist, o.perm, k, ls.changed);
     KM_LAUNCH_CHECK();
 }
 
-// Empty clusters of one training iteration, on the device (the ec_* kernels: a
-// fixed sequence of launches, each ending at once when meta[0] = 0): the m rows
-// with the largest d64 (ties: lowest row) go, in that order, to the empty
-// clusters in ascending index order (dense rows X; with X null the picks are
-// left in the context's candidate list for the sparse fill); the objective at
-// objp (when not null) drops by their d64, subtracted in that order.  The
-// sequence also adds the re-score counters (when not null) into acc.  Returns
-// the candidate list.
+static cluster_lists take_cluster_lists(km_ctx* ctx, int64_t n, int k) {
+    return {ctx->counts.get<int32_t>(k),      ctx->offsets.get<int64_t>(k + 1), ctx->chunk_base.get<int32_t>(k + 1),
+            ctx->empty_list.get<int32_t>(k), ctx->meta.get<int32_t>(2),        ctx->perm.get<int32_t>(n)};
+}
+
+// Empty clusters of one training iteration (the ec_* kernels): the m rows with the
+// largest d64 (ties: lowest row) go, in that order, to the m empty clusters in
+// ascending index order (dense rows X; with X null the picks are left in the
+// candidate list for the sparse fill); the objective at objp (when not null) drops
+// by their d64, subtracted in that order.  Returns the candidate list.
 template <typename F>
-static int32_t* launch_empty_clusters(km_ctx* ctx, const F* X, int64_t n, int d, int k, const int32_t* meta,
-                                      const int32_t* empty_list, const int32_t* counters, F* Cnext,
-                                      const double* d64, double* objp, unsigned long long* acc) {
+static int32_t* launch_empty_clusters(km_ctx* ctx, const F* X, int64_t n, int d, int k, const cluster_lists& o,
+                                      F* Cnext, const double* d64, double* objp) {
     const int grid = int(std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, int64_t(ctx->cu_count) * 4)));
     unsigned int* hist = ctx->hist.get<unsigned int>(EC_PASSES * 256);
-    int32_t* wcnt = ctx->coop_wcnt.get<int32_t>(2 * int64_t(grid));
+    int32_t* wcnt = ctx->ec_wcnt.get<int32_t>(2 * int64_t(grid));
     int32_t* gt = ctx->cand_gt.get<int32_t>(k);
     int32_t* eq = ctx->cand_eq.get<int32_t>(k);
     int32_t* cand = ctx->cand_dev.get<int32_t>(k);
     double* cand_d = ctx->gt_d.get<double>(k);
-    hipLaunchKernelGGL(ec_begin_kernel, dim3(1), dim3(256), 0, ctx->stream, meta, counters, acc, hist);
-    KM_LAUNCH_CHECK();
+    fill<unsigned int>(ctx, hist, EC_PASSES * 256, 0u);
     for (int pass = 0; pass < EC_PASSES; ++pass) {
-        hipLaunchKernelGGL(ec_hist_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, n, meta, hist, pass);
+        hipLaunchKernelGGL(ec_hist_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, n, o.meta, hist, pass);
         KM_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(ec_count_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, n, meta, hist, wcnt);
+    hipLaunchKernelGGL(ec_count_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, n, o.meta, hist, wcnt);
     KM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ec_collect_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, n, meta, hist, wcnt, gt,
+    hipLaunchKernelGGL(ec_collect_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, n, o.meta, hist, wcnt, gt,
                        eq);
     KM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ec_order_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, meta, hist, gt, eq, cand,
+    hipLaunchKernelGGL(ec_order_kernel, dim3(grid), dim3(256), 0, ctx->stream, d64, o.meta, hist, gt, eq, cand,
                        cand_d);
     KM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ec_finish_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, X, d, meta, empty_list, cand,
-                       cand_d, Cnext, objp, acc);
+    hipLaunchKernelGGL(ec_finish_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, X, d, o.meta, o.empty_list, cand,
+                       cand_d, Cnext, objp);
     KM_LAUNCH_CHECK();
     return cand;
-}
-
-// Dense rows: the d64 pass first (the objective pass, gated on meta[0] > 0
-// unless objp already ran with d64 out), then launch_empty_clusters.
-template <typename F>
-static void empty_clusters(km_ctx* ctx, work<F>& w, const F* Ccur, F* Cnext, const int32_t* empty_list,
-                           const int32_t* meta, double* objp, double* d64, unsigned long long* acc) {
-    if (!objp) {
-        const int64_t nchunks = (w.n + OBJ_CHUNK - 1) / OBJ_CHUNK;
-        const int ogrid = int(std::min<int64_t>(nchunks, int64_t(ctx->cu_count) * 8));
-        launch_objective<F>(ctx, ogrid, w.X, w.n, w.d, Ccur, w.labels, d64,
-                            ctx->obj_chunks.get<double>(nchunks), meta);
-    }
-    launch_empty_clusters<F>(ctx, w.X, w.n, w.d, w.k, meta, empty_list, w.L.counters, Cnext, d64, objp, acc);
 }
 
 template <typename F>
@@ -723,7 +787,7 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
     w.L.counters = take<int32_t>(ctx, &km_ctx::lists_counters, A, 3);
     w.cn = take<F>(ctx, &km_ctx::cn, A, k);
     w.cpad = take<F>(ctx, &km_ctx::cpad, A, int64_t(k) * w.dpad);
-    w.cmax_bits = take<unsigned long long>(ctx, &km_ctx::cmax, A, 4);
+    w.maxima = take<double>(ctx, &km_ctx::cmax, A, 4);
     // float4-readable view of X for the matrix-core kernels
     w.Xv = Xd;
     w.ldx = d;
@@ -736,8 +800,6 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
         w.Xv = xp;
         w.ldx = ldx;
     }
-    // every label stays a valid cluster id from here on
-    fill<int32_t>(ctx, w.labels, n, 0);
     const int grid = grid_for(ctx, n * 64, 256, 8);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
@@ -762,10 +824,11 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
     KM_LAUNCH_CHECK();
 }
 
-static void collect_refine_stats(km_ctx* ctx, const int32_t* host_counters) {
-    ctx->stats.refined_candidate_rows += host_counters[0];
-    ctx->stats.refined_full_rows += host_counters[1];
-    ctx->stats.refined_collect_rows += host_counters[2];
+// after the stream has passed the report
+static void collect_refine_stats(km_ctx* ctx) {
+    ctx->stats.refined_candidate_rows += int64_t(ctx->obj_report->refined[0]);
+    ctx->stats.refined_full_rows += int64_t(ctx->obj_report->refined[1]);
+    ctx->stats.refined_collect_rows += int64_t(ctx->obj_report->refined[2]);
 }
 
 template <typename F>
@@ -783,62 +846,37 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
     }
     work<F> w;
     const int path = choose_path<F>(ctx, d, k, flags);
-    setup_work<F>(ctx, w, Xd, n, d, k, path);
+    // device labels go straight to the caller's buffer (read as 16-byte vectors by the
+    // row selection)
+    const bool own_labels = !dev || reinterpret_cast<uintptr_t>(labels_out) % 16 != 0;
+    setup_work<F>(ctx, w, Xd, n, d, k, path, nullptr, own_labels ? nullptr : labels_out);
     ctx->stats.assign_path = path;
     F* Ccur = ctx->c_cur.get<F>(int64_t(k) * d);
     F* Cnext = ctx->c_next.get<F>(int64_t(k) * d);
     KM_HIP(hipMemcpyAsync(Ccur, C0, sizeof(F) * k * d,
                           dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-    int32_t* counts = ctx->counts.get<int32_t>(k);
-    int64_t* offsets = ctx->offsets.get<int64_t>(k + 1);
-    int32_t* chunk_base = ctx->chunk_base.get<int32_t>(k + 1);
-    int32_t* empty_list = ctx->empty_list.get<int32_t>(k);
-    int32_t* meta = ctx->meta.get<int32_t>(2);
-    int32_t* perm = ctx->perm.get<int32_t>(n);
+    const cluster_lists o = take_cluster_lists(ctx, n, k);
     double* part = ctx->part.get<double>((n / REDUCE_CHUNK + k + 1) * int64_t(d));
-    int32_t* pin = ctx->pinned;
     const bool need_obj = thr > 0;
-    // re-scored rows (candidate, full, collect) and refill events, summed on the device
-    unsigned long long* acc = ctx->stat_acc.get<unsigned long long>(4);
-    fill<unsigned long long>(ctx, acc, 4, 0ull);
-    double* d64 = ctx->d64.get<double>(n);  // per-row d64 for empty clusters
+    double* d64 = ctx->d64.get<double>(n);
     const label_sort lsort = label_sort_setup(ctx, n, k);
     // bounds (km_bounds.hpp): every pass after the first assigns only the rows
     // whose label could have changed
-    double* base = nullptr;
-    drift_out drift{nullptr, nullptr, nullptr};
-    int32_t* open_rows = nullptr;
-    int32_t* open_count = nullptr;
     if (max_iter > 0) {
-        base = ctx->b_base.get<double>(k);
-        fill<double>(ctx, base, k, 0.0);
-        drift.drift = ctx->b_drift.get<double>(k);
-        drift.max_drift = w.cmax_bits + 3;
-        open_rows = ctx->b_rows.get<int32_t>(n);
-        open_count = ctx->b_count.get<int32_t>(1);
+        w.base = ctx->b_base.get<double>(k);
+        fill<double>(ctx, w.base, k, 0.0);
+        w.drift = ctx->b_drift.get<double>(k);
+        w.changed = lsort.changed;
+        w.open_rows = ctx->b_rows.get<int32_t>(n);
+        w.open_count = ctx->b_count.get<int32_t>(1);
+        w.acc = ctx->stat_acc.get<unsigned long long>(3);
+        fill<unsigned long long>(ctx, w.acc, 3, 0ull);
         w.sel.gap = ctx->b_gap.get<float>(n);
         w.L.cand_lo = ctx->cand_lo.get<float>(n);
         if (path == 3) w.L.coll_lo = ctx->coll_lo.get<float>(n);
-        w.sel.base = base;
+        w.sel.base = w.base;
         w.sel.gam = make_band<F>(d).g_canon + 1e-6;
     }
-    // centroid preparation and the rows of the next pass (first: all of them)
-    auto open_pass = [&](const F* C, const F* Cold, bool first) {
-        if (first) {
-            centroid_prep<F>(ctx, w, C, path);
-            return;
-        }
-        drift.cold = Cold;
-        centroid_prep<F>(ctx, w, C, path, drift);
-        hipLaunchKernelGGL(bound_base_kernel, dim3(grid_for(ctx, k, 256, 1)), dim3(256), 0, ctx->stream, k,
-                           drift.drift, drift.max_drift, w.sel.gam, base, lsort.changed, open_count, w.L.counters);
-        KM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(bound_select_kernel, dim3(grid_for(ctx, n, SELECT_ROWS, 8)), dim3(256), 0, ctx->stream,
-                           w.labels, w.sel.gap, base, n, open_rows, open_count);
-        KM_LAUNCH_CHECK();
-        w.sel.rows = open_rows;
-        w.sel.count = open_count;
-    };
 
     hipEvent_t loop0 = nullptr, loop1 = nullptr;
     ctx->ev_used = 0;
@@ -847,63 +885,63 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
         loop1 = ctx->event();
         KM_HIP(hipEventRecord(loop0, ctx->stream));
     }
+    step_centroids<F>(ctx, w, path, Ccur);
     double prev = double(std::numeric_limits<F>::max());
     int64_t iter = 0;
     for (iter = 0; iter < max_iter; ++iter) {
-        open_pass(Ccur, Cnext, iter == 0);  // Cnext: the previous centroids
         assign<F>(ctx, w, Ccur, path);
-        label_counts(ctx, lsort, w.labels, counts);
-        hipLaunchKernelGGL(scan_clusters_kernel, dim3(1), dim3(1024), 0, ctx->stream, counts, k,
-                           offsets, chunk_base, empty_list, meta, lsort.changed, w.cmax_bits, 4);
-        KM_LAUNCH_CHECK();
-        label_group(ctx, lsort, w.labels, offsets, perm);
-        launch_reduce<F>(ctx, w, perm, offsets, chunk_base, meta, part);
-        {
-            const int grid = grid_for(ctx, int64_t(k) * d, 256, 4);
-            hipLaunchKernelGGL(finalize_centroids_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream,
-                               part, counts, chunk_base, lsort.changed, k, d, Ccur, Cnext);
-            KM_LAUNCH_CHECK();
-        }
+        const uint32_t seq = next_seq(ctx);
+        label_group(ctx, lsort, w.labels, o, seq);
+        launch_reduce<F>(ctx, w, o.perm, o.offsets, o.chunk_base, o.meta, part);
         double* objp = nullptr;
-        if (need_obj) objp = objective<F>(ctx, w, Ccur, d64);
-        // empty clusters and the statistics stay on the device: with no stop
-        // threshold an iteration needs no host round trip
-        empty_clusters<F>(ctx, w, Ccur, Cnext, empty_list, meta, objp, d64, acc);
+        if (need_obj) objp = objective<F>(ctx, w, Ccur, d64, seq);
+        step_centroids<F>(ctx, w, path, Cnext, Ccur, {part, o.counts, o.chunk_base});
+        // The scan has told the host by now whether there are empty clusters (the
+        // stream still works on the sums behind it): the refill's launches are left
+        // out when there are none.  Queued unconditionally, its 14 launches cost 45 to
+        // 110 us an iteration.
+        wait_report(ctx, &ctx->report->seq, seq);
+        const bool refill = ctx->report->empties > 0;
+        if (refill) {
+            if (!need_obj) launch_d64<F>(ctx, w.X, n, d, Ccur, w.labels, d64);
+            launch_empty_clusters<F>(ctx, w.X, n, d, k, o, Cnext, d64, objp);
+            step_centroids<F>(ctx, w, path, Cnext, Ccur);  // norms and bounds of the refilled
+            ctx->stats.empty_cluster_events++;
+        }
         std::swap(Ccur, Cnext);
+        bool stop = false;
         if (need_obj) {
             double obj = 0.0;
-            KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-            KM_HIP(hipStreamSynchronize(ctx->stream));
-            std::memcpy(&obj, pin + 6, sizeof(double));
-            if (obj + thr > prev) {
-                iter++;
-                break;
+            if (refill) {
+                KM_HIP(hipMemcpyAsync(&obj, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+                KM_HIP(hipStreamSynchronize(ctx->stream));
+            } else {
+                wait_report(ctx, &ctx->obj_report->seq, seq);
+                obj = ctx->obj_report->value;
             }
+            stop = obj + thr > prev;
             prev = obj;
+        }
+        hipLaunchKernelGGL(bound_select_kernel, dim3(grid_for(ctx, n, SELECT_ROWS, 8)), dim3(256), 0, ctx->stream,
+                           w.labels, w.sel.gap, w.base, n, w.open_rows, w.open_count);
+        KM_LAUNCH_CHECK();
+        w.sel.rows = w.open_rows;
+        w.sel.count = w.open_count;
+        if (stop) {
+            iter++;
+            break;
         }
     }
     // final assignment with the final centroids and the objective
-    open_pass(Ccur, Cnext, iter == 0);
     assign<F>(ctx, w, Ccur, path);
-    double* objp = objective<F>(ctx, w, Ccur, nullptr);
+    objective<F>(ctx, w, Ccur, d64, next_seq(ctx));
     if (ctx->timing) KM_HIP(hipEventRecord(loop1, ctx->stream));
-    KM_HIP(hipMemcpyAsync(pin + 2, w.L.counters, 3 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    unsigned long long acc_h[4];
-    KM_HIP(hipMemcpyAsync(acc_h, acc, sizeof(acc_h), hipMemcpyDeviceToHost, ctx->stream));
     const hipMemcpyKind out_kind = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     KM_HIP(hipMemcpyAsync(C_out, Ccur, sizeof(F) * k * d, out_kind, ctx->stream));
-    KM_HIP(hipMemcpyAsync(labels_out, w.labels, sizeof(int32_t) * n, out_kind, ctx->stream));
+    if (own_labels) KM_HIP(hipMemcpyAsync(labels_out, w.labels, sizeof(int32_t) * n, out_kind, ctx->stream));
     KM_HIP(hipStreamSynchronize(ctx->stream));
-    collect_refine_stats(ctx, pin + 2);
-    ctx->stats.refined_candidate_rows += int64_t(acc_h[0]);
-    ctx->stats.refined_full_rows += int64_t(acc_h[1]);
-    ctx->stats.refined_collect_rows += int64_t(acc_h[2]);
-    ctx->stats.empty_cluster_events += int64_t(acc_h[3]);
-    double obj;
-    std::memcpy(&obj, pin + 6, sizeof(double));
-    if (obj_out) *obj_out = obj;
+    collect_refine_stats(ctx);
+    if (obj_out) *obj_out = ctx->obj_report->value;
     if (iters_out) *iters_out = iter;
     if (ctx->timing) {
         float ms = 0.f;
@@ -934,26 +972,30 @@ static void infer(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C, 
     }
     work<F> w;
     const int path = choose_path<F>(ctx, d, k, flags);
-    setup_work<F>(ctx, w, Xd, n, d, k, path);
+    // device centroids and labels are used in place
+    setup_work<F>(ctx, w, Xd, n, d, k, path, nullptr, dev ? labels_out : nullptr);
     ctx->stats.assign_path = path;
-    F* Cd = ctx->c_cur.get<F>(int64_t(k) * d);
-    KM_HIP(hipMemcpyAsync(Cd, C, sizeof(F) * k * d,
-                          dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-    centroid_prep<F>(ctx, w, Cd, path);
-    assign<F>(ctx, w, Cd, path);
-    int32_t* pin = ctx->pinned;
-    const bool want_obj = flags & KM_FLAG_EXACT_OBJECTIVE;
-    if (want_obj) {
-        double* objp = objective<F>(ctx, w, Cd, nullptr);
-        KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    F* Cd = const_cast<F*>(C);  // only read (step_centroids without chunk sums)
+    if (!dev) {
+        Cd = ctx->c_cur.get<F>(int64_t(k) * d);
+        KM_HIP(hipMemcpyAsync(Cd, C, sizeof(F) * k * d, hipMemcpyHostToDevice, ctx->stream));
     }
-    KM_HIP(hipMemcpyAsync(pin + 2, w.L.counters, 3 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    KM_HIP(hipMemcpyAsync(labels_out, w.labels, sizeof(int32_t) * n,
-                          dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, ctx->stream));
+    step_centroids<F>(ctx, w, path, Cd);
+    assign<F>(ctx, w, Cd, path);
+    const bool want_obj = flags & KM_FLAG_EXACT_OBJECTIVE;
+    const uint32_t seq = next_seq(ctx);
+    if (want_obj) {
+        objective<F>(ctx, w, Cd, ctx->d64.get<double>(n), seq);
+    } else {
+        hipLaunchKernelGGL(refine_report_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->obj_report, w.L.counters,
+                           (const unsigned long long*)nullptr, seq);
+        KM_LAUNCH_CHECK();
+    }
+    if (!dev)
+        KM_HIP(hipMemcpyAsync(labels_out, w.labels, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx->stream));
     KM_HIP(hipStreamSynchronize(ctx->stream));
-    collect_refine_stats(ctx, pin + 2);
-    if (want_obj && obj_out) std::memcpy(obj_out, pin + 6, sizeof(double));
+    collect_refine_stats(ctx);
+    if (want_obj && obj_out) *obj_out = ctx->obj_report->value;
     if (ctx->timing) {
         double tot = 0.0;
         for (size_t i = 0; i + 1 < ctx->ev_used; i += 2) {
@@ -1035,35 +1077,32 @@ static void infer_noalloc(km_ctx* ctx, const float* X, int64_t n, int64_t d64_, 
     unsigned char* base = static_cast<unsigned char*>(ctx->scratch);
     double* acc = reinterpret_cast<double*>(base);
     if (want_obj) fill<double>(ctx, acc, 1, 0.0);
-    int32_t* pin = ctx->pinned;
     for (int64_t r0 = 0; r0 < n; r0 += R) {
         const int64_t rows = std::min<int64_t>(R, n - r0);
         arena A{base + 256, cap, 0};
         work<F> w;
         setup_work<F>(ctx, w, X + r0 * d, rows, d, k, path, &A, labels_out + r0);
-        centroid_prep<F>(ctx, w, C, path);
+        step_centroids<F>(ctx, w, path, const_cast<F*>(C));  // only read
         assign<F>(ctx, w, C, path);
+        const uint32_t seq = next_seq(ctx);
         if (want_obj) {
-            const int64_t nchunks = (rows + OBJ_CHUNK - 1) / OBJ_CHUNK;
-            double* chunks = A.get<double>(nchunks);
-            const int grid = int(std::min<int64_t>(nchunks, int64_t(ctx->cu_count) * 8));
-            launch_objective<F>(ctx, grid, w.X, w.n, w.d, C, w.labels, nullptr, chunks);
-            hipLaunchKernelGGL(sum_sequential_into_kernel, dim3(1), dim3(64), 0, ctx->stream, chunks,
-                               nchunks, acc);
+            // the rows' d64 take the candidate ids' place (re-scored by now)
+            static_assert(MAXC * sizeof(int32_t) >= sizeof(double), "d64 fits the candidate ids");
+            double* d64 = reinterpret_cast<double*>(w.L.cand_ids);
+            double* chunks = A.get<double>((rows + OBJ_CHUNK - 1) / OBJ_CHUNK);
+            launch_d64<F>(ctx, w.X, w.n, w.d, C, w.labels, d64);
+            launch_objective_sum(ctx, d64, w.n, chunks, acc, acc, w.L.counters, nullptr, seq);
+        } else {
+            hipLaunchKernelGGL(refine_report_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->obj_report,
+                               w.L.counters, (const unsigned long long*)nullptr, seq);
             KM_LAUNCH_CHECK();
         }
         // the next block reuses the arena: its pieces are stream-ordered after this
-        // block's kernels, and the counters are read before they are cleared again
-        KM_HIP(hipMemcpyAsync(pin + 2, w.L.counters, 3 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                              ctx->stream));
+        // block's kernels, and the report is read before it is written again
         KM_HIP(hipStreamSynchronize(ctx->stream));
-        collect_refine_stats(ctx, pin + 2);
+        collect_refine_stats(ctx);
     }
-    if (want_obj) {
-        KM_HIP(hipMemcpyAsync(pin + 6, acc, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        KM_HIP(hipStreamSynchronize(ctx->stream));
-        if (obj_out) std::memcpy(obj_out, pin + 6, sizeof(double));
-    }
+    if (want_obj && obj_out) *obj_out = ctx->obj_report->value;  // the last block's: all of them added
 }
 
 // ---------------------------------------------------------------------------
@@ -1162,17 +1201,15 @@ static void csr_assign(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, con
 
 // objective = sum of closest (as double) in the fixed order; d64 per row if asked
 template <typename F>
-static double* csr_objective(km_ctx* ctx, const F* closest, int64_t n, double* d64_out,
-                             const int32_t* gate = nullptr) {
+static double* csr_objective(km_ctx* ctx, const F* closest, int64_t n, double* d64_out) {
     const int64_t nchunks = (n + OBJ_CHUNK - 1) / OBJ_CHUNK;
     double* chunks = ctx->obj_chunks.get<double>(nchunks);
     double* out = ctx->obj_dev.get<double>(1);
     const int grid = int(std::min<int64_t>(nchunks, int64_t(ctx->cu_count) * 8));
     hipLaunchKernelGGL(csr_objective_chunks_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream,
-                       closest, n, d64_out, chunks, gate);
+                       closest, n, d64_out, chunks);
     KM_LAUNCH_CHECK();
-    if (gate) return nullptr;  // the d64 pass of the empty-cluster refill only
-    hipLaunchKernelGGL(sum_sequential_kernel, dim3(1), dim3(64), 0, ctx->stream, chunks, nchunks, out);
+    hipLaunchKernelGGL(sum_sequential_kernel, dim3(1), dim3(256), 0, ctx->stream, chunks, nchunks, out);
     KM_LAUNCH_CHECK();
     return out;
 }
@@ -1212,12 +1249,7 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     F* Cnext = ctx->c_next.get<F>(int64_t(k) * d);
     KM_HIP(hipMemcpyAsync(Ccur, C0, sizeof(F) * k * d,
                           dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-    int32_t* counts = ctx->counts.get<int32_t>(k);
-    int64_t* offsets = ctx->offsets.get<int64_t>(k + 1);
-    int32_t* chunk_base = ctx->chunk_base.get<int32_t>(k + 1);
-    int32_t* empty_list = ctx->empty_list.get<int32_t>(k);
-    int32_t* meta = ctx->meta.get<int32_t>(2);
-    int32_t* perm = ctx->perm.get<int32_t>(n);
+    const cluster_lists o = take_cluster_lists(ctx, n, k);
     double* part = ctx->part.get<double>((n / REDUCE_CHUNK + k + 1) * int64_t(d));
     int32_t* pin = ctx->pinned;
     const bool need_obj = thr > 0;
@@ -1226,8 +1258,6 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     double* d64 = ctx->d64.get<double>(n);  // refill candidates' keys
     const label_sort lsort = label_sort_setup(ctx, n, k);
-    unsigned long long* acc = ctx->stat_acc.get<unsigned long long>(4);  // [3]: refill events
-    fill<unsigned long long>(ctx, acc, 4, 0ull);
     if (ctx->timing) KM_HIP(hipEventRecord(loop0, ctx->stream));
 
     double prev = double(std::numeric_limits<F>::max());
@@ -1235,32 +1265,27 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     for (iter = 0; iter < max_iter; ++iter) {
         csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest);
         if (iter > 0) fill<int32_t>(ctx, lsort.changed, k, 0);
-        label_counts(ctx, lsort, labels, counts);
-        hipLaunchKernelGGL(scan_clusters_kernel, dim3(1), dim3(1024), 0, ctx->stream, counts, k,
-                           offsets, chunk_base, empty_list, meta, lsort.changed, (unsigned long long*)nullptr, 0);
-        KM_LAUNCH_CHECK();
-        label_group(ctx, lsort, labels, offsets, perm);
+        const uint32_t seq = next_seq(ctx);
+        label_group(ctx, lsort, labels, o, seq);
         const int64_t max_chunks = n / REDUCE_CHUNK + k + 1;
         hipLaunchKernelGGL(csr_chunk_sums_kernel<F>, dim3(grid_for(ctx, max_chunks * 64, 64, 16)),
-                           dim3(64), lds, ctx->stream, x.vals, x.cols, x.offs, x.base, d, k, perm,
-                           offsets, chunk_base, meta, part);
+                           dim3(64), lds, ctx->stream, x.vals, x.cols, x.offs, x.base, d, k, o.perm,
+                           o.offsets, o.chunk_base, o.meta, part);
         KM_LAUNCH_CHECK();
         hipLaunchKernelGGL(finalize_centroids_kernel<F>, dim3(grid_for(ctx, int64_t(k) * d, 256, 4)),
-                           dim3(256), 0, ctx->stream, part, counts, chunk_base, lsort.changed, k, d, Ccur, Cnext);
+                           dim3(256), 0, ctx->stream, part, o.counts, o.chunk_base, lsort.changed, k, d, Ccur, Cnext);
         KM_LAUNCH_CHECK();
-        // empty clusters on the device (d64 pass gated on the empty count, the
-        // selection kernels, the sparse fill): no host round trip without a
-        // stop threshold
         double* objp = nullptr;
-        if (need_obj)
-            objp = csr_objective<F>(ctx, closest, n, d64);
-        else
-            csr_objective<F>(ctx, closest, n, d64, meta);
-        int32_t* cand = launch_empty_clusters<F>(ctx, (const F*)nullptr, n, d, k, meta, empty_list,
-                                                 (const int32_t*)nullptr, Cnext, d64, objp, acc);
-        hipLaunchKernelGGL(csr_fill_empty_kernel<F>, dim3(std::min(k, ctx->cu_count * 4)), dim3(64), 0,
-                           ctx->stream, x.vals, x.cols, x.offs, x.base, d, empty_list, cand, meta, Cnext);
-        KM_LAUNCH_CHECK();
+        if (need_obj) objp = csr_objective<F>(ctx, closest, n, d64);
+        wait_report(ctx, &ctx->report->seq, seq);  // as in train()
+        if (ctx->report->empties > 0) {
+            if (!need_obj) csr_objective<F>(ctx, closest, n, d64);
+            int32_t* cand = launch_empty_clusters<F>(ctx, (const F*)nullptr, n, d, k, o, Cnext, d64, objp);
+            hipLaunchKernelGGL(csr_fill_empty_kernel<F>, dim3(std::min(k, ctx->cu_count * 4)), dim3(64), 0,
+                               ctx->stream, x.vals, x.cols, x.offs, x.base, d, o.empty_list, cand, o.meta, Cnext);
+            KM_LAUNCH_CHECK();
+            ctx->stats.empty_cluster_events++;
+        }
         std::swap(Ccur, Cnext);
         if (need_obj) {
             double obj = 0.0;
@@ -1278,13 +1303,10 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     double* objp = csr_objective<F>(ctx, closest, n, nullptr);
     if (ctx->timing) KM_HIP(hipEventRecord(loop1, ctx->stream));
     KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    unsigned long long acc_h[4];
-    KM_HIP(hipMemcpyAsync(acc_h, acc, sizeof(acc_h), hipMemcpyDeviceToHost, ctx->stream));
     const hipMemcpyKind out_kind = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     KM_HIP(hipMemcpyAsync(C_out, Ccur, sizeof(F) * k * d, out_kind, ctx->stream));
     KM_HIP(hipMemcpyAsync(labels_out, labels, sizeof(int32_t) * n, out_kind, ctx->stream));
     KM_HIP(hipStreamSynchronize(ctx->stream));
-    ctx->stats.empty_cluster_events += int64_t(acc_h[3]);
     double obj;
     std::memcpy(&obj, pin + 6, sizeof(double));
     if (obj_out) *obj_out = obj;
@@ -2221,12 +2243,24 @@ km_status km_context_create(int device, km_ctx** out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->cu_count = prop.multiProcessorCount;
     void* pin = nullptr;
-    if (hipHostMalloc(&pin, 64, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&pin, 256, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) {
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return KM_HOST_BAD_ALLOC;
     }
+    std::memset(pin, 0, 256);
     ctx->pinned = static_cast<int32_t*>(pin);
+    ctx->report = reinterpret_cast<km::host_report*>(ctx->pinned + 16);
+    ctx->obj_report = reinterpret_cast<km::objective_report*>(ctx->pinned + 32);
+    const km_status ws = km::guarded(ctx, [&] {
+        km::fill<uint32_t>(ctx, ctx->step_ticket.get<uint32_t>(1), 1, 0u);
+        (void)ctx->step_max.get<unsigned long long>(4 * km::STEP_MAX_GRID);
+        KM_HIP(hipStreamSynchronize(ctx->stream));
+    });
+    if (ws != KM_OK) {
+        (void)km_context_destroy(ctx);
+        return ws;
+    }
     // the device is current: resolve its copy of the no-allocation scratch array
     ctx->scratch = km::scratch_address(device, &ctx->scratch_err);
     *out = ctx;
@@ -2248,10 +2282,10 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->seg_cand_cnt, &ctx->seg_cand_ids, &ctx->seg_coll_rows, &ctx->seg_coll_T,
                         &ctx->seg_counts, &ctx->tune_x, &ctx->tune_c, &ctx->tune_l,
                         &ctx->init_d2, &ctx->init_chunks, &ctx->init_chosen, &ctx->init_ids,
-                        &ctx->gt_d, &ctx->stat_acc, &ctx->coop_wcnt, &ctx->cs_inst, &ctx->cs_pre,
+                        &ctx->gt_d, &ctx->stat_acc, &ctx->ec_wcnt, &ctx->cs_inst, &ctx->cs_pre,
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
                         &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
-                        &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
+                        &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->step_ticket, &ctx->step_max, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
                         &ctx->csr_ct, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();

@@ -22,19 +22,28 @@ namespace km {
 // forms the exact distance of its pair (features in order), reading the centroid
 // one 32-feature chunk ahead of the sum, and lane r keeps the minimum of entry r
 // (ties to the lowest id), and with bounds kept (rs.gap) the second smallest: the
-// exact distances and the entry's bound of the other centroids (others) give the
+// exact distances and the entry's bound of the other centroids give the
 // row's gap, so a row between two centroids stays settled while they hardly move.
 template <typename F>
 __host__ __device__ inline int refine_row_stride(int d) {
     return d + int(16 / sizeof(F));
 }
 
+// entries of a re-score list: row, number of ids and ids of each (stride apart), and
+// with bounds kept a lower bound of the squared distance to the other centroids
+struct pair_list {
+    const int32_t* rows;
+    const int32_t* counts;
+    const int32_t* ids;
+    const float* others;
+    const int32_t* count;  // number of entries
+    int stride;
+};
+
 template <typename F>
 __global__ __launch_bounds__(256) void refine_pairs_kernel(
-    const F* __restrict__ X, int d, const F* __restrict__ C, const int32_t* __restrict__ rows,
-    const int32_t* __restrict__ counts, const int32_t* __restrict__ ids, int stride,
-    const int32_t* __restrict__ count_p, int rb, int32_t* __restrict__ full_rows,
-    int32_t* __restrict__ full_counter, int32_t* __restrict__ labels, const float* __restrict__ others,
+    const F* __restrict__ X, int d, const F* __restrict__ C, pair_list list, int rb,
+    int32_t* __restrict__ full_rows, int32_t* __restrict__ full_counter, int32_t* __restrict__ labels,
     row_select rs) {
     typedef F F4 __attribute__((ext_vector_type(4)));
     constexpr int CH = 32 / int(sizeof(F));  // 4-vectors per prefetched centroid chunk
@@ -47,7 +56,9 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(
     const int wave = threadIdx.x >> 6;
     const int ds = refine_row_stride<F>(d);
     F* xs = reinterpret_cast<F*>(smem_raw) + size_t(wave) * rb * ds;
-    const int total = *count_p;
+    const int32_t* __restrict__ ids = list.ids;
+    const int stride = list.stride;
+    const int total = *list.count;
     const int nbatch = (total + rb - 1) / rb;
     const int gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int nw = (gridDim.x * blockDim.x) >> 6;
@@ -59,8 +70,8 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(
         const int nr = min(rb, total - e0);
         int my_row = 0, my_cnt = 0;
         if (lane < nr) {
-            my_row = rows[e0 + lane];
-            my_cnt = counts[e0 + lane];
+            my_row = list.rows[e0 + lane];
+            my_cnt = list.counts[e0 + lane];
             if (my_cnt > stride || my_cnt <= 0) {
                 full_rows[atomicAdd(full_counter, 1)] = my_row;
                 my_cnt = 0;
@@ -163,8 +174,8 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(
         if (lane < nr && my_cnt > 0) {
             labels[my_row] = bj;
             if (rs.gap)
-                rs.gap[my_row] = bound_gap_exact(double(best), double(second), double(others[e0 + lane]), rs.gam,
-                                                 rs.base[bj]);
+                rs.gap[my_row] = bound_gap_exact(double(best), double(second), double(list.others[e0 + lane]),
+                                                 rs.gam, rs.base[bj]);
         }
         __builtin_amdgcn_wave_barrier();
     }

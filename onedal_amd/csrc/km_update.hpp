@@ -67,45 +67,6 @@ __global__ __launch_bounds__(256) void row_norm_kernel(const F* __restrict__ X, 
 }
 
 // ---------------------------------------------------------------------------
-// centroid preparation for one assignment pass: ||c_j||^2 in F (from a double
-// sum), max ||c_j|| (rounded up) and a zero-padded copy for the matrix-core
-// kernel, and with bounds kept how far the centroid moved.  One wave per centroid.
-// ---------------------------------------------------------------------------
-template <typename F>
-__global__ __launch_bounds__(256) void centroid_prep_kernel(const F* __restrict__ C, int k, int d,
-                                                            int dpad, F* __restrict__ cn,
-                                                            F* __restrict__ cpad,
-                                                            unsigned long long* __restrict__ cmax_bits,
-                                                            drift_out dr) {
-    const int lane = threadIdx.x & 63;
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int nwaves = (gridDim.x * blockDim.x) >> 6;
-    for (int j = wave; j < k; j += nwaves) {
-        double s = 0.0;
-        for (int f = lane; f < d; f += 64) {
-            const double v = double(C[int64_t(j) * d + f]);
-            s = fma(v, v, s);
-        }
-        if (cpad)
-            for (int f = lane; f < dpad; f += 64) cpad[int64_t(j) * dpad + f] = f < d ? C[int64_t(j) * d + f] : F(0);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-        if (lane == 0) {
-            cn[j] = F(s);
-            const double r = sqrt(s) * (1.0 + 1e-12);
-            atomicMax(cmax_bits, (unsigned long long)__double_as_longlong(r));
-        }
-        if (dr.cold) {
-            const double m = wave_drift<F>(C + int64_t(j) * d, static_cast<const F*>(dr.cold) + int64_t(j) * d, d, lane);
-            if (lane == 0) {
-                dr.drift[j] = m;
-                atomicMax(dr.max_drift, (unsigned long long)__double_as_longlong(m));
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // label histogram (count_clusters)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void count_kernel(const int32_t* __restrict__ labels, int64_t n,
@@ -135,70 +96,98 @@ __global__ __launch_bounds__(256) void count_kernel(const int32_t* __restrict__ 
 // single-workgroup scan over clusters: member offsets, chunk offsets and the
 // ascending list of empty clusters.  meta[0] = #empty, meta[1] = #chunks.  A
 // cluster whose members did not change (changed[j] = 0) has no chunks: its sums,
-// and so its centroid, are those of the previous iteration.  Also clears the nzero
-// words at `zero` (maxima that the next centroid preparation takes).
+// and so its centroid, are those of the previous iteration.  With gsum (the counting
+// sort) the counts are first taken as its column sums over G groups.  The number
+// of empty clusters also goes to host memory (report), followed by seq, so the
+// host can leave out the refill's launches without waiting for the stream.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void scan_clusters_kernel(const int32_t* __restrict__ counts,
-                                                             int k, int64_t* __restrict__ offsets,
+struct host_report {
+    int32_t empties;
+    uint32_t seq;
+};
+
+__device__ __forceinline__ void report_empties(host_report* report, int32_t empties, uint32_t seq) {
+    if (!report) return;
+    __hip_atomic_store(&report->empties, empties, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&report->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// inclusive scans of three values over a workgroup of 1024 threads (sums: 16 x 3
+// LDS words, rewritten by every call); returns this thread's inclusive values
+__device__ __forceinline__ void scan3_1024(int32_t& a, int32_t& b, int32_t& c, int32_t (*sums)[16]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t pa = __shfl_up(a, off), pb = __shfl_up(b, off), pc = __shfl_up(c, off);
+        if (lane >= off) {
+            a += pa;
+            b += pb;
+            c += pc;
+        }
+    }
+    __syncthreads();  // the previous call's readers are done
+    if (lane == 63) {
+        sums[0][wave] = a;
+        sums[1][wave] = b;
+        sums[2][wave] = c;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) {
+        a += sums[0][w];
+        b += sums[1][w];
+        c += sums[2][w];
+    }
+}
+
+__global__ __launch_bounds__(1024) void scan_clusters_kernel(int32_t* __restrict__ counts,
+                                                             const int32_t* __restrict__ gsum, int G,
+                                                             int k,
+                                                             int64_t* __restrict__ offsets,
                                                              int32_t* __restrict__ chunk_base,
                                                              int32_t* __restrict__ empty_list,
                                                              int32_t* __restrict__ meta,
                                                              const int32_t* __restrict__ changed,
-                                                             unsigned long long* __restrict__ zero, int nzero) {
-    __shared__ int64_t s_off[1024];
-    __shared__ int32_t s_chk[1024];
-    __shared__ int32_t s_emp[1024];
-    __shared__ int64_t carry_off;
-    __shared__ int32_t carry_chk, carry_emp;
+                                                             host_report* report, uint32_t seq) {
+    __shared__ int32_t sums[3][16];
+    __shared__ int32_t last[3];
     const int t = threadIdx.x;
-    if (t < nzero) zero[t] = 0ull;
-    if (t == 0) {
-        carry_off = 0;
-        carry_chk = 0;
-        carry_emp = 0;
-    }
-    __syncthreads();
+    int32_t c_off = 0, c_chk = 0, c_emp = 0;  // of the earlier blocks of 1024 clusters
     for (int base = 0; base < k; base += 1024) {
         const int j = base + t;
-        const int32_t c = j < k ? counts[j] : 0;
-        const int32_t nchk = j < k && changed[j] ? (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK : 0;
-        s_off[t] = c;
-        s_chk[t] = nchk;
-        s_emp[t] = (j < k && c == 0) ? 1 : 0;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            int64_t a = 0;
-            int32_t b = 0, e = 0;
-            if (t >= off) {
-                a = s_off[t - off];
-                b = s_chk[t - off];
-                e = s_emp[t - off];
-            }
-            __syncthreads();
-            s_off[t] += a;
-            s_chk[t] += b;
-            s_emp[t] += e;
-            __syncthreads();
-        }
+        int32_t c = 0;
         if (j < k) {
-            const int64_t incl_off = s_off[t];
-            offsets[j] = carry_off + incl_off - c;
-            chunk_base[j] = carry_chk + s_chk[t] - nchk;
-            if (c == 0) empty_list[carry_emp + s_emp[t] - 1] = j;
+            if (gsum) {
+#pragma unroll 16
+                for (int g = 0; g < G; ++g) c += gsum[int64_t(g) * k + j];
+                counts[j] = c;
+            } else {
+                c = counts[j];
+            }
         }
-        __syncthreads();
+        const int32_t nchk = j < k && changed[j] ? (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK : 0;
+        int32_t so = c, sc = nchk, se = (j < k && c == 0) ? 1 : 0;  // the row count is below 2^31
+        scan3_1024(so, sc, se, sums);
+        if (j < k) {
+            offsets[j] = int64_t(c_off) + so - c;
+            chunk_base[j] = c_chk + sc - nchk;
+            if (c == 0) empty_list[c_emp + se - 1] = j;
+        }
         if (t == 1023) {
-            carry_off += s_off[1023];
-            carry_chk += s_chk[1023];
-            carry_emp += s_emp[1023];
+            last[0] = so;
+            last[1] = sc;
+            last[2] = se;
         }
         __syncthreads();
+        c_off += last[0];
+        c_chk += last[1];
+        c_emp += last[2];
     }
     if (t == 0) {
-        offsets[k] = carry_off;
-        chunk_base[k] = carry_chk;
-        meta[0] = carry_emp;
-        meta[1] = carry_chk;
+        offsets[k] = c_off;
+        chunk_base[k] = c_chk;
+        meta[0] = c_emp;
+        meta[1] = c_chk;
+        report_empties(report, c_emp, seq);
     }
 }
 
@@ -236,7 +225,21 @@ __global__ __launch_bounds__(256) void reduce_chunks_kernel(
 #pragma unroll
         for (int c = 0; c < CPL; ++c) acc[c] = 0.0;
         if (small) {
-            for (int64_t m = m_begin; m < m_end; m += G) {
+            int64_t m = m_begin;
+            // eight steps of G members: ids and values loaded first, added in order
+            for (; m + 8 * G <= m_end; m += 8 * G) {
+                if (active) {
+                    int64_t r[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) r[u] = perm[m + u * G + g];
+                    double v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = double(X[r[u] * d + f0]);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc[0] = acc[0] + v[u];
+                }
+            }
+            for (; m < m_end; m += G) {
                 const int64_t mm = m + g;
                 if (active && mm < m_end) {
                     const int64_t row = perm[mm];
@@ -410,90 +413,148 @@ __global__ __launch_bounds__(256) void finalize_centroids_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// objective: d64 per row against its label's centroid.  Order (fixed): rows in
-// chunks of OBJ_CHUNK; thread t of a chunk sums rows t, t+256, t+512, ... in
-// order; the 256 partials are combined by the tree p[t] += p[t+s], s = 128..1;
-// chunk sums are added in chunk order by sum_sequential_kernel.
+// objective: d64 per row against its label's centroid (row_d64_kernel), then, in a
+// fixed order: rows in chunks of OBJ_CHUNK; thread t of a chunk sums rows t, t+256,
+// t+512, ... in order; the 256 partials are combined by the tree p[t] += p[t+s],
+// s = 128..1; chunk sums are added in chunk order.
 // ---------------------------------------------------------------------------
-// Thread t reads its rows directly, two rows (t + 256 j and t + 256 (j + 1)) at a
-// time so their loads overlap: one 128-byte line of each row and of its
-// centroid per step (16-byte loads), each row's squares added in feature order;
-// the two rows' d64 then enter the thread's sum in row order.  No LDS.
+// d64 of one row, features in order: 16-byte loads, a 128-byte line of the row and of
+// the centroid per step, when vec (whole 16-byte pieces, 16-byte aligned)
 template <typename F>
-__host__ inline size_t objective_lds_bytes() {
-    return 0;
+__device__ __forceinline__ double row_d64(const F* __restrict__ x, const F* __restrict__ c, int d, bool vec) {
+    typedef F V __attribute__((ext_vector_type(16 / int(sizeof(F)))));
+    constexpr int N = 16 / int(sizeof(F));  // elements per 16 bytes
+    double acc = 0.0;
+    int f = 0;
+    if (vec) {
+        for (; f + 8 * N <= d; f += 8 * N) {
+            V xv[8], cv[8];
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+                xv[v] = *reinterpret_cast<const V*>(x + f + N * v);
+                cv[v] = *reinterpret_cast<const V*>(c + f + N * v);
+            }
+#pragma unroll
+            for (int v = 0; v < 8; ++v)
+#pragma unroll
+                for (int e = 0; e < N; ++e) {
+                    const double diff = double(xv[v][e]) - double(cv[v][e]);
+                    const double sq = diff * diff;
+                    acc = acc + sq;
+                }
+        }
+        for (; f < d; f += N) {
+            const V xv = *reinterpret_cast<const V*>(x + f);
+            const V cv = *reinterpret_cast<const V*>(c + f);
+#pragma unroll
+            for (int e = 0; e < N; ++e) {
+                const double diff = double(xv[e]) - double(cv[e]);
+                const double sq = diff * diff;
+                acc = acc + sq;
+            }
+        }
+    }
+    for (; f < d; ++f) {
+        const double diff = double(x[f]) - double(c[f]);
+        const double sq = diff * diff;
+        acc = acc + sq;
+    }
+    return acc;
 }
 
+// One row per thread, 256 rows per workgroup.  Rows that allow 16-byte reads are read
+// directly.  The others (odd widths) are contiguous in memory as a block: the
+// workgroup copies up to FT features of its 256 rows to LDS in consecutive
+// elements and each thread then walks its own row there (row stride odd, so the
+// lanes meet different banks), the centroid from the cache.
+constexpr int D64_ROWS = 256;
 template <typename F>
-__global__ __launch_bounds__(256) void objective_chunks_kernel(
-    const F* __restrict__ X, int64_t n, int d, const F* __restrict__ C,
-    const int32_t* __restrict__ labels, double* __restrict__ d64_out,
-    double* __restrict__ chunk_sums, const int32_t* __restrict__ gate) {
-    if (gate && gate[0] == 0) return;  // gated off (no empty clusters this iteration)
-    constexpr int RPT = 2;                           // rows in flight per thread
-    constexpr int LV = 128 / (4 * int(sizeof(F)));   // 4-vectors per 128-byte line
-    __shared__ double part[256];
+__global__ __launch_bounds__(256) void row_d64_kernel(const F* __restrict__ X, int64_t n, int d,
+                                                      const F* __restrict__ C,
+                                                      const int32_t* __restrict__ labels,
+                                                      double* __restrict__ d64) {
+    constexpr int FT = 96 / int(sizeof(F));  // staged features: 24 float, 12 double
+    constexpr int ST = FT | 1;
+    __shared__ F Xs[D64_ROWS * ST];
     const int t = threadIdx.x;
-    const bool vec = (d % 4) == 0 && (reinterpret_cast<uintptr_t>(X) % (4 * sizeof(F))) == 0 &&
-                     (reinterpret_cast<uintptr_t>(C) % (4 * sizeof(F))) == 0;
-    typedef F F4 __attribute__((ext_vector_type(4)));
+    constexpr int N = 16 / int(sizeof(F));
+    const bool vec = (d % N) == 0 && (reinterpret_cast<uintptr_t>(X) % 16) == 0 &&
+                     (reinterpret_cast<uintptr_t>(C) % 16) == 0;
+    for (int64_t r0 = int64_t(blockIdx.x) * D64_ROWS; r0 < n; r0 += int64_t(gridDim.x) * D64_ROWS) {
+        const int nr = int(min<int64_t>(D64_ROWS, n - r0));
+        const F* c = C + int64_t(t < nr ? labels[r0 + t] : 0) * d;
+        if (vec) {
+            if (t < nr) d64[r0 + t] = row_d64<F>(X + (r0 + t) * d, c, d, true);
+            continue;
+        }
+        double acc = 0.0;
+        for (int f0 = 0; f0 < d; f0 += FT) {
+            const int ft = min(FT, d - f0);
+            __syncthreads();
+            if (ft == d) {  // whole rows: one contiguous run
+                for (int e = t; e < nr * d; e += 256) {
+                    const int r = e / d;
+                    Xs[r * ST + (e - r * d)] = X[r0 * d + e];
+                }
+            } else {
+                for (int e = t; e < nr * FT; e += 256) {
+                    const int r = e / FT, f = e - r * FT;
+                    if (f < ft) Xs[r * ST + f] = X[(r0 + r) * d + f0 + f];
+                }
+            }
+            __syncthreads();
+            if (t < nr) {
+                for (int f = 0; f < ft; ++f) {
+                    const double diff = double(Xs[t * ST + f]) - double(c[f0 + f]);
+                    const double sq = diff * diff;
+                    acc = acc + sq;
+                }
+            }
+        }
+        if (t < nr) d64[r0 + t] = acc;
+    }
+}
+
+// Chunk sums of d64 and, by the last workgroup to finish (a ticket that it resets), the
+// objective: the chunk sums added one at a time in chunk order onto `start` (null:
+// 0).  The sum is bound by its chain of dependent adds, so the chunk sums are
+// staged in LDS first.  The result also goes to host memory, when given: with the
+// re-scored rows (counters, plus acc when not null), followed by seq.
+struct objective_report {
+    double value;
+    unsigned long long refined[3];  // re-scored rows: candidate, full, collect
+    uint32_t seq;
+};
+__device__ __forceinline__ void report_objective(objective_report* report, double value, const int32_t* counters,
+                                                 const unsigned long long* acc, uint32_t seq) {
+    __hip_atomic_store(&report->value, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (int q = 0; q < 3; ++q)
+        __hip_atomic_store(&report->refined[q], (unsigned long long)counters[q] + (acc ? acc[q] : 0ull),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&report->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(256) void objective_sum_kernel(const double* __restrict__ d64, int64_t n,
+                                                            double* __restrict__ chunk_sums,
+                                                            const double* start, double* out,
+                                                            objective_report* report, uint32_t seq,
+                                                            const int32_t* __restrict__ counters,
+                                                            const unsigned long long* __restrict__ acc,
+                                                            uint32_t* __restrict__ ticket) {
+    __shared__ double part[256];
+    __shared__ bool s_last;
+    const int t = threadIdx.x;
     const int64_t nchunks = (n + OBJ_CHUNK - 1) / OBJ_CHUNK;
     for (int64_t q = blockIdx.x; q < nchunks; q += gridDim.x) {
         const int64_t r0 = q * OBJ_CHUNK;
         const int rows = int(min<int64_t>(OBJ_CHUNK, n - r0));
-        double p = 0.0;
-        // thread t owns chunk rows t, t+256, ... and adds them in that order
-        for (int r = t; r < rows; r += 256 * RPT) {
-            double acc[RPT];
-            const F* xs[RPT];
-            const F* cs[RPT];
-            bool ok[RPT];
+        constexpr int RPT = OBJ_CHUNK / 256;
+        double v[RPT], p = 0.0;
 #pragma unroll
-            for (int u = 0; u < RPT; ++u) {
-                const int rr = r + 256 * u;
-                ok[u] = rr < rows;
-                const int64_t row = r0 + (ok[u] ? rr : r);
-                xs[u] = X + row * d;
-                cs[u] = C + int64_t(labels[row]) * d;
-                acc[u] = 0.0;
-            }
-            int f = 0;
-            if (vec) {
-                for (; f + 4 * LV <= d; f += 4 * LV) {
-                    F4 xv[RPT][LV], cv[RPT][LV];
+        for (int u = 0; u < RPT; ++u) v[u] = t + 256 * u < rows ? d64[r0 + t + 256 * u] : 0.0;
 #pragma unroll
-                    for (int u = 0; u < RPT; ++u)
-#pragma unroll
-                        for (int v = 0; v < LV; ++v) {
-                            xv[u][v] = *reinterpret_cast<const F4*>(xs[u] + f + 4 * v);
-                            cv[u][v] = *reinterpret_cast<const F4*>(cs[u] + f + 4 * v);
-                        }
-#pragma unroll
-                    for (int u = 0; u < RPT; ++u)
-#pragma unroll
-                        for (int v = 0; v < LV; ++v)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const double diff = double(xv[u][v][e]) - double(cv[u][v][e]);
-                                const double sq = diff * diff;
-                                acc[u] = acc[u] + sq;
-                            }
-                }
-            }
-            for (; f < d; ++f)
-#pragma unroll
-                for (int u = 0; u < RPT; ++u) {
-                    const double diff = double(xs[u][f]) - double(cs[u][f]);
-                    const double sq = diff * diff;
-                    acc[u] = acc[u] + sq;
-                }
-#pragma unroll
-            for (int u = 0; u < RPT; ++u)
-                if (ok[u]) {
-                    if (d64_out) d64_out[r0 + r + 256 * u] = acc[u];
-                    p = p + acc[u];
-                }
-        }
+        for (int u = 0; u < RPT; ++u)
+            if (t + 256 * u < rows) p = p + v[u];
         part[t] = p;
         __syncthreads();
         for (int s = 128; s > 0; s >>= 1) {
@@ -503,43 +564,66 @@ __global__ __launch_bounds__(256) void objective_chunks_kernel(
         if (t == 0) chunk_sums[q] = part[0];
         __syncthreads();
     }
-}
-
-__global__ void sum_sequential_kernel(const double* __restrict__ v, int64_t count,
-                                      double* __restrict__ out) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        double s = 0.0;
-        int64_t i = 0;
-        for (; i + 16 <= count; i += 16) {
-            double w[16];
+    if (t == 0) {
+        __threadfence();  // this workgroup's chunk sums before its ticket
+        s_last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    __threadfence();
+    double sum = start ? *start : 0.0;
+    for (int64_t b = 0; b < nchunks; b += 256) {
+        __syncthreads();
+        if (b + t < nchunks) part[t] = chunk_sums[b + t];
+        __syncthreads();
+        if (t == 0) {
+            const int m = int(min<int64_t>(256, nchunks - b));
+            int i = 0;
+            for (; i + 16 <= m; i += 16) {
+                double w[16];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) w[u] = v[i + u];
+                for (int u = 0; u < 16; ++u) w[u] = part[i + u];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) s = s + w[u];
+                for (int u = 0; u < 16; ++u) sum = sum + w[u];
+            }
+            for (; i < m; ++i) sum = sum + part[i];
         }
-        for (; i < count; ++i) s = s + v[i];
-        *out = s;
+    }
+    if (t == 0) {
+        *out = sum;
+        *ticket = 0u;
+        if (report) report_objective(report, sum, counters, acc, seq);
     }
 }
 
-// *acc += v[0] + ... + v[count-1], added one at a time in order: a sum over row
-// blocks processed one after another equals sum_sequential_kernel over all
-// chunks at once (acc starts at 0, and 0 + v0 = v0).
-__global__ void sum_sequential_into_kernel(const double* __restrict__ v, int64_t count,
-                                           double* __restrict__ acc) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        double s = *acc;
-        for (int64_t i = 0; i < count; ++i) s = s + v[i];
-        *acc = s;
+// the report alone (no objective asked for)
+__global__ void refine_report_kernel(objective_report* report, const int32_t* counters,
+                                     const unsigned long long* acc, uint32_t seq) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) report_objective(report, 0.0, counters, acc, seq);
+}
+
+// *out = v[0] + ... + v[count-1], added one at a time in order (one workgroup, the
+// values staged in LDS)
+__global__ __launch_bounds__(256) void sum_sequential_kernel(const double* __restrict__ v, int64_t count,
+                                                             double* __restrict__ out) {
+    __shared__ double part[256];
+    double sum = 0.0;
+    for (int64_t b = 0; b < count; b += 256) {
+        const int m = int(min<int64_t>(256, count - b));
+        __syncthreads();
+        if (int(threadIdx.x) < m) part[threadIdx.x] = v[b + threadIdx.x];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+#pragma unroll 16
+            for (int i = 0; i < m; ++i) sum = sum + part[i];
+        }
     }
+    if (threadIdx.x == 0) *out = sum;
 }
 
 // ---------------------------------------------------------------------------
-// Empty clusters on the device, as a fixed sequence of ordinary launches per
-// iteration, each of which ends at once when meta[0] = 0 (no empty cluster):
-//   ec_begin_kernel     adds the iteration's re-score counters into acc[0..2];
-//                       with m = meta[0] > 0 empty clusters, zeroes the
-//                       histograms;
+// Empty clusters on the device, as a sequence of ordinary launches in the iterations
+// that have any (m = meta[0] > 0; the host launches it when the scan reported some):
 //   ec_hist_kernel x 8  radix select of the m-th largest d64, 8 bits a pass from
 //                       the top (keys: the raw bits of the non-negative doubles,
 //                       which order like the values); every workgroup derives
@@ -553,11 +637,9 @@ __global__ void sum_sequential_into_kernel(const double* __restrict__ v, int64_t
 //                       d64, ties to the lowest row;
 //   ec_finish_kernel    pick e fills the e-th empty cluster (ascending index) of
 //                       Cnext (dense rows; sparse rows are filled by
-//                       csr_fill_empty_kernel from cand), the objective (when
-//                       given) drops by the picks' d64 in pick order, and acc[3]
-//                       counts the iteration.
-// The d64 of every row against its label's centroid comes in from the
-// objective pass (gated on the same count).
+//                       csr_fill_empty_kernel from cand), and the objective (when
+//                       given) drops by the picks' d64 in pick order.
+// The d64 of every row against its label's centroid comes in (row_d64_kernel).
 // ---------------------------------------------------------------------------
 constexpr int EC_PASSES = 8;
 
@@ -602,19 +684,6 @@ __device__ __forceinline__ void ec_state_shared(const unsigned int* __restrict__
 
 __device__ __forceinline__ unsigned long long ec_key(double v) {
     return (unsigned long long)__double_as_longlong(v);
-}
-
-__global__ __launch_bounds__(256) void ec_begin_kernel(const int32_t* __restrict__ meta,
-                                                       const int32_t* __restrict__ counters,
-                                                       unsigned long long* __restrict__ acc,
-                                                       unsigned int* __restrict__ hist) {
-    if (threadIdx.x == 0 && counters) {
-        acc[0] += (unsigned long long)counters[0];
-        acc[1] += (unsigned long long)counters[1];
-        acc[2] += (unsigned long long)counters[2];
-    }
-    if (meta[0] <= 0) return;
-    for (int i = threadIdx.x; i < EC_PASSES * 256; i += blockDim.x) hist[i] = 0u;
 }
 
 __global__ __launch_bounds__(256) void ec_hist_kernel(const double* __restrict__ d64, int64_t n,
@@ -776,8 +845,7 @@ __global__ __launch_bounds__(256) void ec_finish_kernel(const F* __restrict__ X,
                                                         const int32_t* __restrict__ empty_list,
                                                         const int32_t* __restrict__ cand,
                                                         const double* __restrict__ cand_d, F* __restrict__ Cnext,
-                                                        double* __restrict__ obj,
-                                                        unsigned long long* __restrict__ acc) {
+                                                        double* __restrict__ obj) {
     const int m = meta[0];
     if (m <= 0) return;
     const int64_t gtid = int64_t(blockIdx.x) * 256 + threadIdx.x, gsize = int64_t(gridDim.x) * 256;
@@ -786,13 +854,10 @@ __global__ __launch_bounds__(256) void ec_finish_kernel(const F* __restrict__ X,
             const int q = int(e / d), f = int(e - int64_t(q) * d);
             Cnext[int64_t(empty_list[q]) * d + f] = X[int64_t(cand[q]) * d + f];
         }
-    if (gtid == 0) {
-        if (obj) {
-            double o = *obj;
-            for (int e = 0; e < m; ++e) o = o - cand_d[e];
-            *obj = o;
-        }
-        acc[3] += 1ull;
+    if (gtid == 0 && obj) {
+        double o = *obj;
+        for (int e = 0; e < m; ++e) o = o - cand_d[e];
+        *obj = o;
     }
 }
 

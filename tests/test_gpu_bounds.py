@@ -15,7 +15,7 @@ CASES = [
     # name, n, d, k, iterations, scale, threshold: run to the fixed point (nothing
     # left to assign), the edges of the 4096-row runs, squares near underflow and
     # distances past the bounds' largest (every row assigned again), the stop rule,
-    # and k above the counting sort's (clusters not tracked)
+    # k above the counting sort's (clusters not tracked)
     ("to_fixed_point", 30011, 17, 23, 30, 1.0, 0.0),
     ("one_run_exact", 4096, 8, 5, 12, 1.0, 0.0),
     ("one_run_and_a_row", 4097, 33, 40, 12, 1.0, 0.0),
@@ -24,6 +24,11 @@ CASES = [
     ("offset_rows", 20000, 20, 16, 10, 1.0, 0.0),
     ("stop_rule", 12001, 64, 30, 40, 1.0, 1e-3),
     ("k_above_counting_sort", 9000, 4, 4500, 3, 1.0, 0.0),
+    # the largest grouping in one workgroup and the first past it; rows staged for
+    # their d64 in several pieces (odd widths)
+    ("small_group_largest", 16384, 3, 1024, 4, 1.0, 0.0),
+    ("small_group_past", 16385, 3, 1025, 4, 1.0, 0.0),
+    ("d64_pieces", 5001, 51, 7, 4, 1.0, 1e-3),
 ]
 
 
