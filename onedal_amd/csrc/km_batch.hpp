@@ -19,6 +19,7 @@
 
 #include "km_assign.hpp"
 #include "km_common.hpp"
+#include "km_update.hpp"
 
 namespace km {
 
@@ -243,13 +244,13 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
 
 // ---------------------------------------------------------------------------
 // Certified FP32 matrix-core assignment (tile variant 7) for instances with
-// d <= DP (DP in {16, 32, 64, 128}) and k <= 128.  A work item is BATCH_MFMA_ROWS
-// rows of one instance.  The item loads the instance's centroids into LDS once
+// d <= DP (DP in {16, 32, 64, 128}) and k <= 128.  A work item is item_rows (whole
+// tiles, at most BATCH_MFMA_ROWS) rows of one instance.  The item loads the instance's centroids into LDS once
 // (zero-padded to DP features and to whole blocks of 32), with ||c_j||^2 (double
 // sum rounded to float) and max ||c_j|| rounded up.  Then each 128-row tile puts
 // a row in the registers of a lane pair (feature halves), runs
-// v_mfma_f32_32x32x2f32 against every block of 32 centroids and keeps four top-2
-// slots per row, as the single-instance FP32 kernel does (km_assign.hpp).  The
+// v_mfma_f32_32x32x2f32 against every block of 32 centroids and keeps a top-2 slot
+// per lane and block, as the single-instance FP32 kernel does (km_assign.hpp).  The
 // settle uses that kernel's error band: v_j = ||c_j||^2 - 2 x.c_j is within the
 // band of the exact-form distance minus ||x||^2, so every centroid that can be
 // the exact-form argmin has v_j <= T.  Rows with one such centroid are settled.
@@ -258,7 +259,8 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
 // finite, gets the exact scan of select_min_distance (kernels_fp_impl.hpp:198-202).
 // So labels equal the exact-form kernel's.
 // ---------------------------------------------------------------------------
-constexpr int BATCH_MFMA_ROWS = 1024;  // rows per work item
+constexpr int BATCH_MFMA_ROWS = 1024;  // most rows per work item
+constexpr int BATCH_MFMA_TILE = 128;   // rows per tile; an item is whole tiles
 constexpr int BATCH_MFMA_MAXK = 128;
 __host__ __device__ constexpr size_t batch_mfma_lds_bytes(int dp) {
     return size_t(BATCH_MFMA_MAXK) * (dp + 4) * 4 + BATCH_MFMA_MAXK * 4 + 4 * 8;
@@ -279,13 +281,14 @@ __device__ __forceinline__ band_consts batch_band_f32(int d) {
 template <int DP>
 __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_inst* __restrict__ I,
                                                                    const int32_t* __restrict__ sel, int nsel,
-                                                                   const int64_t* __restrict__ pre,
+                                                                   const int64_t* __restrict__ pre, int item_rows,
                                                                    const float* __restrict__ C,
                                                                    int32_t* __restrict__ labels,
                                                                    uint32_t* __restrict__ skeys, int lbits,
                                                                    int to_user) {
     constexpr int HALF = DP / 2;
     constexpr int CST = DP + 4;  // LDS row stride in floats
+    constexpr int NSL = BATCH_MFMA_MAXK / 32;
     extern __shared__ __align__(16) float smem[];
     float* Cs = smem;                                                   // BATCH_MFMA_MAXK x CST
     float* Cn = smem + BATCH_MFMA_MAXK * CST;                           // BATCH_MFMA_MAXK
@@ -302,42 +305,74 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
         const batch_inst in = I[sel[si]];
         const int d = in.d, k = in.k;
         if (d > DP || k > BATCH_MFMA_MAXK) continue;  // never planned so; keeps LDS in bounds
-        const int64_t rb = (b - pre[si]) * BATCH_MFMA_ROWS;
-        const int64_t re = min<int64_t>(in.n, rb + BATCH_MFMA_ROWS);
+        const int64_t rb = (b - pre[si]) * item_rows;
+        const int64_t re = min<int64_t>(in.n, rb + item_rows);
         const float* Ci = C + in.c0;
         const int mblocks = (k + 31) / 32;
         const int kp = mblocks * 32;
         __syncthreads();  // the previous item's LDS reads are done
-        for (int e = tid; e < kp * DP; e += 256) {
-            const int j = e / DP, f = e - j * DP;
-            Cs[j * CST + f] = (j < k && f < d) ? Ci[int64_t(j) * d + f] : 0.f;
+        // centroids: 16-byte pieces when rows allow them (c0 is a multiple of 4 floats),
+        // eight loads of a thread in flight
+        if ((d & 3) == 0) {
+            constexpr int Q = DP / 4;
+            for (int e0 = tid; e0 < kp * Q; e0 += 256 * 8) {
+                floatx4 v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int e = e0 + 256 * u, j = e / Q, f = (e - j * Q) * 4;
+                    v[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    if (j < k && f < d) v[u] = *reinterpret_cast<const floatx4*>(Ci + int64_t(j) * d + f);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int e = e0 + 256 * u, j = e / Q, f = (e - j * Q) * 4;
+                    if (j < kp) *reinterpret_cast<floatx4*>(&Cs[j * CST + f]) = v[u];
+                }
+            }
+        } else {
+            for (int e = tid; e < kp * DP; e += 256) {
+                const int j = e / DP, f = e - j * DP;
+                Cs[j * CST + f] = (j < k && f < d) ? Ci[int64_t(j) * d + f] : 0.f;
+            }
         }
         __syncthreads();
-        // ||c_j||^2 and the largest of them: one wave per centroid; a centroid
-        // that is not finite sends every row of the item to the exact scan
+        // ||c_j||^2 and the largest of them: two threads per centroid, half of the
+        // features each; a centroid that is not finite sends every row of the item to
+        // the exact scan
         double wm = 0.0;
         bool wbad = false;
-        for (int j = wave; j < kp; j += 4) {
+        {
+            const int j = tid >> 1, hf = tid & 1;
             double sq = 0.0;
-            for (int f = lane; f < DP; f += 64) {
-                const double v = double(Cs[j * CST + f]);
-                sq = fma(v, v, sq);
-            }
+            if (j < kp) {
+                const float* c = &Cs[j * CST + hf * HALF];
+#pragma unroll 4
+                for (int f = 0; f < HALF; f += 4) {
+                    const floatx4 v4 = *reinterpret_cast<const floatx4*>(c + f);
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off);
-            if (lane == 0) Cn[j] = j < k ? float(sq) : finf;
+                    for (int q = 0; q < 4; ++q) {
+                        const double v = double(v4[q]);
+                        sq = fma(v, v, sq);
+                    }
+                }
+            }
+            sq += __shfl_xor(sq, 1);
+            if (j < kp && hf == 0) Cn[j] = j < k ? float(sq) : finf;
             if (j < k) {
                 if (!(sq < 1.0e300)) wbad = true;  // NaN or overflow
-                wm = fmax(wm, sq);
+                wm = sq;
             }
         }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) wm = fmax(wm, __shfl_xor(wm, off));
+        wbad = __any(wbad);
         if (lane == 0) wmax[wave] = wbad ? -1.0 : wm;
         __syncthreads();
         const bool cbad = wmax[0] < 0.0 || wmax[1] < 0.0 || wmax[2] < 0.0 || wmax[3] < 0.0;
         const double cmax =
             sqrt(fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]))) * (1.0 + 1e-12);
         const band_consts bc = batch_band_f32(d);
-        for (int64_t t0 = rb; t0 < re; t0 += 128) {
+        for (int64_t t0 = rb; t0 < re; t0 += BATCH_MFMA_TILE) {
             const int64_t row = t0 + wave * 32 + r32;
             const bool ok = row < re;
             const float* xrow = in.X + (ok ? row : rb) * int64_t(d);
@@ -370,11 +405,11 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
             xs += __shfl_xor(xs, 32);
             const double Xup = sqrt(xs) * (1.0 + 1e-12);
 
-            top2<float> st[2];
-            st[0].init();
-            st[1].init();
-            // block mb into slot sl (even blocks slot 0, odd blocks slot 1; the
-            // slot is a compile-time index, so the slots stay in registers)
+            // one slot per block of 32 centroids, so near centroids seldom share one (the
+            // slot is a compile-time index: the slots stay in registers)
+            top2<float> st[NSL];
+#pragma unroll
+            for (int q = 0; q < NSL; ++q) st[q].init();
             auto block = [&](int mb, top2<float>& slot) {
                 floatx16 acc;
 #pragma unroll
@@ -396,20 +431,18 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                         slot.push(__builtin_fmaf(-2.f, acc[4 * q + t], c4[t]), mb * 32 + 8 * q + 4 * h + t);
                 }
             };
-            for (int mb = 0; mb < mblocks; mb += 2) {
-                block(mb, st[0]);
-                if (mb + 1 < mblocks) block(mb + 1, st[1]);
-            }
-            // lane r32 (h = 0) holds the row's four slots: its two and lane r32 + 32's
-            top2<float> sl[4];
-            sl[0] = st[0];
-            sl[1] = st[1];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                sl[2 + q].m1 = __shfl_xor(st[q].m1, 32);
-                sl[2 + q].m2 = __shfl_xor(st[q].m2, 32);
-                sl[2 + q].i1 = __shfl_xor(st[q].i1, 32);
-                sl[2 + q].i2 = __shfl_xor(st[q].i2, 32);
+            for (int mb = 0; mb < NSL; ++mb)
+                if (mb < mblocks) block(mb, st[mb]);
+            // lane r32 (h = 0) holds the row's slots: its own and lane r32 + 32's
+            top2<float> sl[2 * NSL];
+#pragma unroll
+            for (int q = 0; q < NSL; ++q) {
+                sl[q] = st[q];
+                sl[NSL + q].m1 = __shfl_xor(st[q].m1, 32);
+                sl[NSL + q].m2 = __shfl_xor(st[q].m2, 32);
+                sl[NSL + q].i1 = __shfl_xor(st[q].i1, 32);
+                sl[NSL + q].i2 = __shfl_xor(st[q].i2, 32);
             }
             int lab = 0;
             bool need_scan = false;
@@ -417,7 +450,7 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                 float best = finf;
                 int bi = -1;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < 2 * NSL; ++q) {
                     if (sl[q].m1 < best || (sl[q].m1 == best && sl[q].i1 >= 0 && sl[q].i1 < bi)) {
                         best = sl[q].m1;
                         bi = sl[q].i1;
@@ -427,7 +460,7 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                 bool cert = !cbad && bi >= 0 && bi < k && T < double(finf);
                 int cnt = 0;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < 2 * NSL; ++q) {
                     if (double(sl[q].m2) <= T) cert = false;
                     if (sl[q].i1 >= 0 && double(sl[q].m1) <= T) {
                         if (sl[q].i1 >= k) cert = false;
@@ -443,7 +476,7 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                     float bd = finf;
                     lab = k;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
+                    for (int q = 0; q < 2 * NSL; ++q) {
                         if (sl[q].i1 >= 0 && double(sl[q].m1) <= T) {
                             const int j = sl[q].i1;
                             const float D = canon_dist<float>(xrow, Cs + j * CST, d);
@@ -857,10 +890,8 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
                                                           int64_t* __restrict__ dpre,
                                                           uint32_t* __restrict__ ticket) {
     __shared__ int64_t s_off[1024];
-    __shared__ int32_t s_chk[1024];
-    __shared__ int32_t s_emp[1024];
-    __shared__ int64_t carry_off;
-    __shared__ int32_t carry_chk, carry_emp;
+    __shared__ int32_t sums[3][16];
+    __shared__ int32_t last[3];
     __shared__ bool s_last;
     const int t = threadIdx.x;
     for (int ii = blockIdx.x; ii < B; ii += gridDim.x) {
@@ -871,13 +902,7 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
         int32_t* cb = chunk_base + in.k0 + ii;
         int32_t* emp = empty_list + in.k0;
         const int64_t nb = (in.n + BATCH_CNT_ROWS - 1) / BATCH_CNT_ROWS;
-        __syncthreads();
-        if (t == 0) {
-            carry_off = 0;
-            carry_chk = 0;
-            carry_emp = 0;
-        }
-        __syncthreads();
+        int32_t carry_off = 0, carry_chk = 0, carry_emp = 0;  // an instance has below 2^31 rows
         for (int base = 0; base < k; base += 1024) {
             const int j = base + t;
             int32_t c = 0;
@@ -885,10 +910,12 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
                 if (bhist) {
                     const int32_t* h = bhist + in.h0 + j;
                     int64_t lb = 0;
-                    for (; lb + 4 <= nb; lb += 4) {
-                        const int32_t h0 = h[lb * k], h1 = h[(lb + 1) * k], h2 = h[(lb + 2) * k],
-                                      h3 = h[(lb + 3) * k];
-                        c += h0 + h1 + h2 + h3;
+                    for (; lb + 8 <= nb; lb += 8) {
+                        int32_t v[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) v[u] = h[(lb + u) * k];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) c += v[u];
                     }
                     for (; lb < nb; ++lb) c += h[lb * k];
                     cnt[j] = c;
@@ -896,46 +923,44 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
                     c = cnt[j];
                 }
             }
-            s_off[t] = c;
-            s_chk[t] = j < k ? (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK : 0;
-            s_emp[t] = (j < k && c == 0) ? 1 : 0;
-            __syncthreads();
-            for (int o = 1; o < 1024; o <<= 1) {
-                int64_t a = 0;
-                int32_t bch = 0, e = 0;
-                if (t >= o) {
-                    a = s_off[t - o];
-                    bch = s_chk[t - o];
-                    e = s_emp[t - o];
-                }
-                __syncthreads();
-                s_off[t] += a;
-                s_chk[t] += bch;
-                s_emp[t] += e;
-                __syncthreads();
-            }
+            const int32_t nchk = (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK;
+            int32_t so = c, sc = nchk, se = (j < k && c == 0) ? 1 : 0;
+            scan3_1024(so, sc, se, sums);
             if (j < k) {
-                const int64_t first = carry_off + s_off[t] - c;
+                const int32_t first = carry_off + so - c;
                 off[j] = first;
-                cb[j] = carry_chk + s_chk[t] - (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK;
-                if (c == 0) emp[carry_emp + s_emp[t] - 1] = j;
+                cb[j] = carry_chk + sc - nchk;
+                if (c == 0) emp[carry_emp + se - 1] = j;
                 if (bhist) {
                     int32_t* h = bhist + in.h0 + j;
-                    int32_t dst = int32_t(first);
-                    for (int64_t lb = 0; lb < nb; ++lb) {
+                    int32_t dst = first;
+                    int64_t lb = 0;
+                    for (; lb + 8 <= nb; lb += 8) {
+                        int32_t v[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) v[u] = h[(lb + u) * k];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            h[(lb + u) * k] = dst;
+                            dst += v[u];
+                        }
+                    }
+                    for (; lb < nb; ++lb) {
                         const int32_t hc = h[lb * k];
                         h[lb * k] = dst;
                         dst += hc;
                     }
                 }
             }
-            __syncthreads();
             if (t == 1023) {
-                carry_off += s_off[1023];
-                carry_chk += s_chk[1023];
-                carry_emp += s_emp[1023];
+                last[0] = so;
+                last[1] = sc;
+                last[2] = se;
             }
             __syncthreads();
+            carry_off += last[0];
+            carry_chk += last[1];
+            carry_emp += last[2];
         }
         if (t == 0) {
             off[k] = carry_off;
@@ -992,6 +1017,10 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
 // the same members in the same order as batch_reduce_kernel's and the partials
 // are identical.  Waves take runs of consecutive chunks (up to RUN), round
 // robin; member ids are loaded one step ahead of the row reads.
+// U members' rows in flight per lane: 8 fill HBM when there are chunks for every wave;
+// with few chunks a chunk's chain of 256 / U round trips is the kernel's time, so U
+// is 32 then.
+template <int U>
 __global__ __launch_bounds__(256) void batch_reduce_vec_kernel(const batch_inst* __restrict__ I, int B,
                                                                const int64_t* __restrict__ qpre,
                                                                const int32_t* __restrict__ perm,
@@ -1000,7 +1029,6 @@ __global__ __launch_bounds__(256) void batch_reduce_vec_kernel(const batch_inst*
                                                                double* __restrict__ part) {
     typedef float F4 __attribute__((ext_vector_type(4)));
     constexpr int RUN = 16;
-    constexpr int U = 8;
     const int lane = threadIdx.x & 63;
     const int64_t gw = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
     const int64_t nw = (int64_t(gridDim.x) * blockDim.x) >> 6;
@@ -1072,14 +1100,21 @@ __global__ __launch_bounds__(256) void batch_reduce_vec_kernel(const batch_inst*
 #pragma unroll
                     for (int u = 0; u < U; ++u) r[u] = rn[u];
                 }
-                for (; m < m_end; m += Sm) {
-                    const int64_t mm = m + g;
-                    if (mm < m_end) {
-                        const int64_t row = int64_t(pm[mm]) - in.row0;
-                        const F4 x4 = *reinterpret_cast<const F4*>(in.X + row * d + 4 * f4);
+                // the rest (fewer than U steps): loads together, the valid ones added
+                if (m < m_end) {
+                    F4 xv[U];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[e] = acc[e] + double(x4[e]);
+                    for (int u = 0; u < U; ++u) {
+                        const int64_t mm = m + u * Sm + g;
+                        const int64_t row = int64_t(pm[mm < m_end ? mm : m_begin]) - in.row0;
+                        xv[u] = *reinterpret_cast<const F4*>(in.X + row * d + 4 * f4);
                     }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (m + u * Sm + g < m_end) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[e] = acc[e] + double(xv[u][e]);
+                        }
                 }
             }
             // every lane reaches the shuffles: group partials into group 0, in
@@ -1327,14 +1362,15 @@ __global__ __launch_bounds__(256) void batch_d64_kernel(const batch_inst* __rest
 // e-th empty cluster (ascending index) receives that row -- the policy of
 // empty_cluster_handling_dpc.cpp:26-114 with its tie order pinned.  An empty
 // cluster left without a row (every remaining d64 is NaN) keeps its centroid.
-__global__ __launch_bounds__(256) void batch_fill_empty_kernel(const batch_inst* __restrict__ I, int B,
+__global__ __launch_bounds__(1024) void batch_fill_empty_kernel(const batch_inst* __restrict__ I, int B,
                                                                const int32_t* __restrict__ meta,
                                                                const int32_t* __restrict__ empty_list,
                                                                const double* __restrict__ d64,
                                                                const float* __restrict__ Ccur,
                                                                float* __restrict__ Cnext) {
-    __shared__ double sd[256];
-    __shared__ int64_t sr[256];
+    constexpr int T = 1024, U = 8;  // threads, rows of a thread in flight
+    __shared__ double sd[T];
+    __shared__ int64_t sr[T];
     const int t = threadIdx.x;
     for (int ii = blockIdx.x; ii < B; ii += gridDim.x) {
         const int m = meta[2 * ii];
@@ -1346,18 +1382,26 @@ __global__ __launch_bounds__(256) void batch_fill_empty_kernel(const batch_inst*
         for (int e = 0; e < m; ++e) {
             double bd = -1.0;
             int64_t br = -1;
-            for (int64_t r = t; r < in.n; r += 256) {
-                const double v = dd[r];
-                const bool after = v < pd || (v == pd && r > pr);
-                if (after && (br < 0 || v > bd)) {  // rows ascend per thread: first max wins
-                    bd = v;
-                    br = r;
+            for (int64_t r0 = t; r0 < in.n; r0 += T * U) {
+                double w[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) w[u] = r0 + T * u < in.n ? dd[r0 + T * u] : 0.0;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int64_t r = r0 + T * u;
+                    if (r >= in.n) continue;
+                    const double v = w[u];
+                    const bool after = v < pd || (v == pd && r > pr);
+                    if (after && (br < 0 || v > bd)) {  // rows ascend per thread: first max wins
+                        bd = v;
+                        br = r;
+                    }
                 }
             }
             sd[t] = bd;
             sr[t] = br;
             __syncthreads();
-            for (int s = 128; s > 0; s >>= 1) {
+            for (int s = T / 2; s > 0; s >>= 1) {
                 if (t < s) {
                     const double od = sd[t + s];
                     const int64_t orr = sr[t + s];
@@ -1372,7 +1416,7 @@ __global__ __launch_bounds__(256) void batch_fill_empty_kernel(const batch_inst*
             const int64_t wr = sr[0];
             __syncthreads();
             const int j = empty_list[in.k0 + e];
-            for (int f = t; f < in.d; f += 256)
+            for (int f = t; f < in.d; f += T)
                 Cnext[in.c0 + int64_t(j) * in.d + f] =
                     wr >= 0 ? in.X[wr * in.d + f] : Ccur[in.c0 + int64_t(j) * in.d + f];
             pd = wd;

@@ -1366,6 +1366,7 @@ struct batch_plan {
     // (asel[sel_off ..]) and the prefix of their workgroup counts (apre[pre_off ..])
     struct asg_launch {
         int v;
+        int rows;  // per work item
         int nsel;
         int64_t sel_off, pre_off, batches;
     };
@@ -1425,15 +1426,30 @@ static int tile_bucket(int64_t d, int64_t k) {
     return db * 6 + kb;
 }
 
-// untuned choice: the narrowest centroid tile that still holds k
-static int default_tile(int64_t k) { return k <= 8 ? 4 : k <= 16 ? 3 : k <= 32 ? 2 : 0; }
-
 static bool mfma_tile_ok(int64_t d, int64_t k) { return d <= 128 && k <= BATCH_MFMA_MAXK; }
+
+// untuned choice per (d, k) bucket: what the tuner picks on this chip (the fastest of
+// the eight variants at each bucket's largest shape).  The matrix cores win from
+// d = 17 on wherever they apply, except for k <= 8 at d <= 64, where 32 centroid
+// columns are mostly padding; narrow VALU tiles win elsewhere.
+static int default_tile(int64_t d, int64_t k) {
+    static const int8_t best[KM_BATCH_TILE_BUCKETS] = {
+        4, 4, 4, 4, 4, 4,  // d <= 8:   (8, 8)
+        4, 4, 4, 4, 7, 4,  // d <= 16:  matrix cores for k in 65..128
+        7, 7, 7, 7, 7, 3,  // d <= 32
+        4, 7, 7, 7, 7, 3,  // d <= 64
+        7, 7, 7, 7, 7, 2,  // d <= 128
+        4, 6, 2, 0, 0, 0,  // d <= 256: (8, 8), (16, 4), (32, 8), (64, 8)
+        4, 3, 2, 0, 0, 0,  // more
+    };
+    const int t = best[tile_bucket(d, k)];
+    return t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k) ? 4 : t;
+}
 
 // tile variant of an instance (the matrix-core variant only where it applies)
 static int tile_for(const km_ctx* ctx, int64_t d, int64_t k) {
     int t = ctx->tile_force > 0 ? ctx->tile_force - 1 : ctx->tile_table[tile_bucket(d, k)];
-    if (t < 0 || (t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k))) t = default_tile(k);
+    if (t < 0 || (t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k))) t = default_tile(d, k);
     return t;
 }
 
@@ -1530,8 +1546,18 @@ static void plan_build(batch_plan& p, const km_ctx* ctx, const km_batch_instance
     p.apre.clear();
     p.launches.clear();
     for (int v = 0; v < BATCH_LAUNCH_KINDS; ++v) {
-        batch_plan::asg_launch L{v, 0, int64_t(p.asel.size()), int64_t(p.apre.size()), 0};
-        const int64_t rb = batch_kind_rows(v);
+        batch_plan::asg_launch L{v, batch_kind_rows(v), 0, int64_t(p.asel.size()), int64_t(p.apre.size()), 0};
+        if (v >= BATCH_TILE_MFMA) {
+            // A work item loads its instance's centroids once, so items are long when
+            // there are rows for four per CU, and down to one tile when there are not
+            // (30000 rows in items of 1024 keep 30 of 256 CUs busy)
+            int64_t rows = 0;
+            for (int i = 0; i < B; ++i)
+                if (var[i] == v) rows += inst[i].n;
+            const int64_t fit = rows / (int64_t(ctx->cu_count) * 4) / BATCH_MFMA_TILE * BATCH_MFMA_TILE;
+            L.rows = int(std::min<int64_t>(BATCH_MFMA_ROWS, std::max<int64_t>(BATCH_MFMA_TILE, fit)));
+        }
+        const int64_t rb = L.rows;
         p.apre.push_back(0);
         for (int i = 0; i < B; ++i) {
             if (var[i] != v) continue;
@@ -1625,7 +1651,7 @@ static void plan_assign(km_ctx* ctx, const batch_plan& p, int32_t* labels, uint3
                        p.Ccur, labels, skeys, lb, to_user)
 #define KM_BATCH_MFMA(DP)                                                                          \
     hipLaunchKernelGGL((batch_assign_mfma_kernel<DP>), grid, block, batch_mfma_lds_bytes(DP), ctx->stream, \
-                       p.dI, sel, L.nsel, pre, p.Ccur, labels, skeys, lb, to_user)
+                       p.dI, sel, L.nsel, pre, L.rows, p.Ccur, labels, skeys, lb, to_user)
         switch (L.v) {
             case 0: KM_BATCH_ASSIGN(64, 8); break;
             case 1: KM_BATCH_ASSIGN(64, 4); break;
@@ -1688,8 +1714,13 @@ static void plan_iteration(km_ctx* ctx, batch_plan& p, hipEvent_t asg_start = nu
                                          unsigned(p.rows), 0, p.kbits, ctx->stream));
     }
     if (p.any_vec) {
-        hipLaunchKernelGGL(batch_reduce_vec_kernel, dim3(cap), dim3(256), 0, ctx->stream, p.dI, B, p.qpre,
-                           p.perm, p.offsets, p.cb, p.part);
+        // at most rows / REDUCE_CHUNK + clusters chunks, four to a wave at d <= 64
+        if (p.rows / REDUCE_CHUNK + p.kk <= int64_t(cap) * 4)
+            hipLaunchKernelGGL((batch_reduce_vec_kernel<32>), dim3(cap), dim3(256), 0, ctx->stream, p.dI, B, p.qpre,
+                               p.perm, p.offsets, p.cb, p.part);
+        else
+            hipLaunchKernelGGL((batch_reduce_vec_kernel<8>), dim3(cap), dim3(256), 0, ctx->stream, p.dI, B, p.qpre,
+                               p.perm, p.offsets, p.cb, p.part);
         KM_LAUNCH_CHECK();
     }
     if (p.any_scalar) {
@@ -1704,7 +1735,7 @@ static void plan_iteration(km_ctx* ctx, batch_plan& p, hipEvent_t asg_start = nu
     hipLaunchKernelGGL(batch_d64_kernel, dim3(g(p.P(BP::P_D64, B))), dim3(256), 0, ctx->stream, p.dI, B,
                        p.d64pre, p.meta, p.Ccur, p.labels, p.d64);
     KM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(batch_fill_empty_kernel, dim3(g(B)), dim3(256), 0, ctx->stream, p.dI, B, p.meta,
+    hipLaunchKernelGGL(batch_fill_empty_kernel, dim3(g(B)), dim3(1024), 0, ctx->stream, p.dI, B, p.meta,
                        p.empty, p.d64, p.Ccur, p.Cnext);
     KM_LAUNCH_CHECK();
     // every centroid of Cnext is written (finalize: counted clusters; fill:
@@ -1915,7 +1946,7 @@ static void batch_autotune(km_ctx* ctx, int32_t* table_out, int64_t table_len) {
             for (int i = 0; i < NI; ++i)
                 q[i] = km_batch_instance_f32{X + i * n * d, C + int64_t(i) * k * d, nullptr, lab + i * n, n, d, k};
             float best_ms = std::numeric_limits<float>::infinity();
-            int best_v = default_tile(k);
+            int best_v = default_tile(d, k);
             for (int v = 0; v < BATCH_TILES; ++v) {
                 if (v == BATCH_TILE_MFMA && !mfma_tile_ok(d, k)) continue;
                 ctx->tile_force = v + 1;

@@ -351,15 +351,24 @@ __global__ __launch_bounds__(256) void reduce_chunks_vec_kernel(
 #pragma unroll
             for (int u = 0; u < 8; ++u) r[u] = rn[u];
         }
-        for (; m < m_end; ++m) {
-            const int64_t r0 = perm[m];
+        // the rest (fewer than eight): loads together, the valid ones added
+        if (m < m_end) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) r[u] = perm[m + u < m_end ? m + u : m_begin];
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 const int c4 = sl + lpc * v;
                 if (c4 < d4) {
-                    const F4 x4 = *reinterpret_cast<const F4*>(X + r0 * d + 4 * c4);
+                    F4 xv[8];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[v][e] = acc[v][e] + double(x4[e]);
+                    for (int u = 0; u < 8; ++u)
+                        xv[u] = *reinterpret_cast<const F4*>(X + int64_t(r[u]) * d + 4 * c4);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (m + u < m_end) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[v][e] = acc[v][e] + double(xv[u][e]);
+                        }
                 }
             }
         }
