@@ -36,6 +36,7 @@
 #include "km_args.hpp"
 #include "km_assign.hpp"
 #include "km_assign_bf16.hpp"
+#include "km_assign_split.hpp"
 #include "km_batch.hpp"
 #include "km_bounds.hpp"
 #include "km_common.hpp"
@@ -150,6 +151,7 @@ struct km_ctx {
     // step_ticket: zero between launches; step_max: centroid_step_kernel's workspace.
     // Both live from the context's creation on.
     km::dbuf step_ticket, step_max;
+    km::dbuf c_split, c_pieces;  // centroid operands of the split path
     int32_t* pinned = nullptr;  // small pinned host staging, then the kernels' reports
     km::host_report* report = nullptr;          // host address
     km::objective_report* obj_report = nullptr;
@@ -230,6 +232,10 @@ struct work {
     uint16_t* Cb = nullptr;       // k x dpad bf16(-2 c)
     float* cnb = nullptr;         // ||c||^2 + B (rounded up), 32 * ceil(k / 32) entries
     bf16_params* params = nullptr;
+    // split path (path 2, float): both bf16 halves of -2 c, and the norm pieces
+    bool split = false;
+    uint16_t* Csp = nullptr;  // bf16_padded_k(k) x 2 dpad
+    uint16_t* cnp = nullptr;  // bf16_padded_k(k) x 16
     // rows of the next assignment pass, and where their bounds go
     row_select sel{nullptr, nullptr, nullptr, nullptr, 0.0};
     // training: centroid movement and bounds per cluster, changed clusters, the open
@@ -262,6 +268,11 @@ static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
     if (ctx->assign_path_opt == 1) return 1;
     return 2;
 }
+
+// float data on path 2: split BF16 products (km_assign_split.hpp) where a row's halves
+// fit a lane's registers and the key's index bits leave the band narrow; FP32
+// products past that.  double data: never.
+static bool use_split(int path, int d, int k) { return path == 2 && d <= 128 && k <= SPLIT_MAX_K; }
 
 template <typename F>
 static band_consts make_band(int d) {
@@ -312,8 +323,10 @@ static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* col
     s.d = w.d;
     s.dpad = w.dpad;
     s.cn = w.cn;
-    s.cpad = path == 2 ? w.cpad : nullptr;
-    s.kp = w.k;
+    s.cpad = path == 2 && !w.split ? w.cpad : nullptr;
+    s.Csp = w.Csp;
+    s.cnp = w.cnp;
+    s.kp = w.split ? bf16_padded_k(w.k) : w.k;
     s.maxima = w.maxima;
     s.drift = w.drift;
     s.base = w.base;
@@ -364,6 +377,33 @@ static void launch_mfma_f32(km_ctx* ctx, work<float>& w, const band_consts& bc) 
         launch_mfma_f32_mode<DP, NB, true>(ctx, w, bc, grid, res_lds);
     else
         launch_mfma_f32_mode<DP, NB, false>(ctx, w, bc, grid, mfma_f32_lds_bytes(DP, w.k, false));
+}
+
+static split_consts make_split_consts(int d, int k) {
+    split_consts c;
+    int mbits = 0;
+    while ((1 << mbits) < bf16_padded_k(k) / 32) mbits++;
+    c.ib = 4 + mbits;
+    const double ua = fp_traits<float>::u_acc;
+    c.xc = float(std::ldexp(6.02, -18) + gamma_m(2.0 * d, ua) * 2.02 / 256.0 + gamma_m(double(d), ua) * 2.04);
+    c.sum = float(gamma_m(8.0, ua) * 1.02);
+    c.trunc = float(std::ldexp(1.0, c.ib - 23));
+    const double g = gamma_m(double(d + 2), fp_traits<float>::u);
+    c.g_canon = float(g / (1.0 - g)) * (1.0f + 2.4e-7f);
+    return c;
+}
+
+template <int DP, int NB>
+static void launch_split(km_ctx* ctx, work<float>& w) {
+    constexpr int ROWS_PER_WG = 4 * 32 * NB;
+    const int64_t tiles = (w.n + ROWS_PER_WG - 1) / ROWS_PER_WG;
+    const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * 2)));
+    const size_t lds = split_lds_bytes(DP);
+    auto kern = assign_split_kernel<DP, NB>;
+    KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.X, w.n, w.d, w.Csp, w.cnp, w.k, w.maxima,
+                       make_split_consts(w.d, w.k), w.labels, w.L, w.sel);
+    KM_LAUNCH_CHECK();
 }
 
 template <int DP, int NB>
@@ -449,7 +489,13 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
         KM_HIP(hipEventRecord(e0, ctx->stream));
     }
     if constexpr (std::is_same<F, float>::value) {
-        if (path == 2) {
+        if (w.split) {
+            switch (w.dpad) {
+                case 32: launch_split<32, 2>(ctx, w); break;
+                case 64: launch_split<64, 2>(ctx, w); break;
+                default: launch_split<128, 1>(ctx, w); break;
+            }
+        } else if (path == 2) {
             switch (w.dpad) {
                 case 32: launch_mfma_f32<32, 2>(ctx, w, bc); break;
                 case 64: launch_mfma_f32<64, 2>(ctx, w, bc); break;
@@ -771,7 +817,8 @@ static int32_t* launch_empty_clusters(km_ctx* ctx, const F* X, int64_t n, int d,
 template <typename F>
 static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, int k,
                        int path, arena* A = nullptr, int32_t* labels_into = nullptr) {
-    const bool vec_view = path == 2;
+    w.split = std::is_same<F, float>::value && use_split(path, d, k);
+    const bool vec_view = path == 2 && !w.split;
     w.n = n;
     w.d = d;
     w.k = k;
@@ -786,7 +833,12 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
     w.L.full_rows = take<int32_t>(ctx, &km_ctx::lists_full, A, n);
     w.L.counters = take<int32_t>(ctx, &km_ctx::lists_counters, A, 3);
     w.cn = take<F>(ctx, &km_ctx::cn, A, k);
-    w.cpad = take<F>(ctx, &km_ctx::cpad, A, int64_t(k) * w.dpad);
+    if (w.split) {
+        w.Csp = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(bf16_padded_k(k)) * 2 * w.dpad);
+        w.cnp = take<uint16_t>(ctx, &km_ctx::c_pieces, A, int64_t(bf16_padded_k(k)) * 16);
+    } else {
+        w.cpad = take<F>(ctx, &km_ctx::cpad, A, int64_t(k) * w.dpad);
+    }
     w.maxima = take<double>(ctx, &km_ctx::cmax, A, 4);
     // float4-readable view of X for the matrix-core kernels
     w.Xv = Xd;
@@ -820,6 +872,7 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
             return;
         }
     }
+    if (w.split) return;  // its kernel forms the norms itself
     hipLaunchKernelGGL(row_norm_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, Xd, n, d, w.xnorm);
     KM_LAUNCH_CHECK();
 }
@@ -1025,7 +1078,9 @@ static size_t noalloc_block_bytes(const km_ctx* ctx, int path, int64_t R, int d,
     const int64_t dpad = pad_dim(d);
     int64_t b = R * (4 + 4 + 4 + 4 * int64_t(MAXC) + 4) + 16 + int64_t(sizeof(F)) * k +
                 int64_t(sizeof(F)) * k * dpad + 32;
-    if (path == 2 && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
+    const bool split = use_split(path, d, k);
+    if (split) b += 36 * int64_t(bf16_padded_k(k)) + 4 * int64_t(bf16_padded_k(k) - k) * dpad;
+    if (path == 2 && !split && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
     if (path == 3) {
         const int64_t kp = bf16_padded_k(k);
         b += R * (2 * dpad + 4 + 4 + 8 + 4 + 4 * int64_t(MAXC2)) + 16 + 2 * kp * dpad + 4 * kp + 64;
@@ -2316,7 +2371,7 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->gt_d, &ctx->stat_acc, &ctx->ec_wcnt, &ctx->cs_inst, &ctx->cs_pre,
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
                         &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
-                        &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->step_ticket, &ctx->step_max, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
+                        &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->step_ticket, &ctx->step_max, &ctx->c_split, &ctx->c_pieces, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
                         &ctx->csr_ct, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();

@@ -10,6 +10,7 @@
 #pragma once
 
 #include "km_assign_bf16.hpp"
+#include "km_assign_split.hpp"
 #include "km_bounds.hpp"
 #include "km_common.hpp"
 #include "km_update.hpp"
@@ -32,6 +33,10 @@ struct centroid_step {
     F* cn;
     F* cpad;
     uint16_t* Cb;
+    // or (Csp) rows of both bf16 halves of -2 c and (cnp) the pieces of ||c_j||^2 for the
+    // norm step of assign_split_kernel, kp rows
+    uint16_t* Csp;
+    uint16_t* cnp;
     int kp;
     double* maxima;  // [0] max ||c||, BF16: [1] max ||bf16(c)||, [2] max ||c - bf16(c)||
     // BF16: value shift and start values
@@ -102,6 +107,14 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
         if constexpr (BF16) {
             for (int f = t; f < dpad; f += 256)  // exact: -2 * bf16(c)
                 s.Cb[int64_t(j) * dpad + f] = f < d ? f2bf(-2.0f * bf2f(f2bf(float(row[f])))) : uint16_t(0);
+        } else if (s.Csp) {
+            uint16_t* o2 = s.Csp + int64_t(j) * 2 * dpad;
+            for (int f = t; f < dpad; f += 256) {
+                const float v = f < d ? -2.0f * float(row[f]) : 0.f;
+                const uint16_t hi = f2bf(v);
+                o2[f] = hi;
+                o2[dpad + f] = f2bf(v - bf2f(hi));
+            }
         } else if (s.cpad) {
             for (int f = t; f < dpad; f += 256) s.cpad[int64_t(j) * dpad + f] = f < d ? row[f] : F(0);
         }
@@ -133,6 +146,13 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
                 const double up = 1.0 + 1e-12;
                 auto bits = [](double v) { return (unsigned long long)__double_as_longlong(v); };
                 s.cn[j] = F(sq);
+                if (s.cnp) {
+                    uint32_t hm, l;
+                    split3(float(sq), hm, l);
+                    uintx4* o4 = reinterpret_cast<uintx4*>(s.cnp + int64_t(j) * 16);
+                    o4[0] = uintx4{hm, l | 0x3F800000u, 0x3F803F80u, 0u};
+                    o4[1] = uintx4{0u, 0u, 0u, 0u};
+                }
                 mx[0] = max(mx[0], bits(sqrt(sq) * up));
                 if constexpr (BF16) {
                     mx[1] = max(mx[1], bits(sqrt(sh) * up));
@@ -150,6 +170,12 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
     if constexpr (BF16) {
         for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x)
             for (int f = t; f < dpad; f += 256) s.Cb[int64_t(j) * dpad + f] = 0;
+    }
+    if (s.Csp) {  // padding: zero rows with a norm of 2^127, which no threshold reaches
+        for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x) {
+            for (int f = t; f < 2 * dpad; f += 256) s.Csp[int64_t(j) * 2 * dpad + f] = 0;
+            if (t < 16) s.cnp[int64_t(j) * 16 + t] = t == 0 ? uint16_t(0x7F00u) : uint16_t(0);
+        }
     }
     if (t == 0) {
 #pragma unroll
