@@ -57,6 +57,32 @@ struct fp_traits<double> {
 // Candidate ids gathered per row by the BF16 collect pass.
 constexpr int MAXC2 = 32;
 
+// Results that the last workgroup of a launch reads from the others: stored and loaded
+// past the XCDs' caches (agent scope).  A __threadfence() before the ticket would
+// also write back everything else the XCD's L2 holds, which took 2 ms where a
+// launch did it for 10000 workgroups.
+template <typename T>
+__device__ __forceinline__ void agent_store(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T agent_load(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True in every thread of the launch's last workgroup to get here; what the others
+// stored with agent_store before is then visible to agent_load.  Every thread calls
+// it; the ticket is 0 before the launch and must be reset by the last workgroup.
+__device__ __forceinline__ bool last_workgroup(uint32_t* ticket) {
+    __shared__ bool s_last;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores have arrived
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    return s_last;
+}
+
 // Device-side work lists filled by the assignment kernels.
 struct refine_lists {
     int32_t* cand_rows;    // rows with 2..MAXC certified candidates

@@ -137,7 +137,7 @@ struct km_ctx {
     // batched training and steps: the iterated set, and the finished set of a step
     km::batch_ws bws, bws_fin;
     km::dbuf tune_x, tune_c, tune_l;  // autotuner inputs (released after tuning)
-    km::dbuf init_d2, init_chunks, init_chosen, init_ids;  // initialisation
+    km::dbuf init_d2, init_chunks, init_chosen, init_ids, init_near, init_cnew, init_thr;  // initialisation
     km::dbuf gt_d;  // empty-cluster candidates' d64
     km::dbuf stat_acc, ec_wcnt;  // device-side statistics; per-workgroup counts of ec_count_kernel
     km::dbuf cs_inst, cs_pre, cs_hist, cs_gsum;  // single-instance counting sort (label_sort)
@@ -2060,6 +2060,9 @@ static std::vector<int64_t> init_random_rows(uint64_t seed, int64_t n, int64_t k
     return ids;
 }
 
+// bytes of rows from which a k-means++ step keeps bounds (init_step_kernel)
+constexpr double INIT_BOUND_BYTES = 32e6;
+
 static void init_check_args(const void* X, int64_t n, int64_t d, int64_t k, int method, const void* C_out) {
     if (X == nullptr || n <= 0 || d <= 0) throw status_error(KM_DOMAIN_ERROR, "Input data is empty");
     if (k <= 0) throw status_error(KM_DOMAIN_ERROR, "Cluster count is lower than or equal to zero");
@@ -2104,28 +2107,50 @@ static void init_centroids(km_ctx* ctx, const F* X, int64_t n, int64_t d, int64_
         KM_HIP(hipStreamSynchronize(ctx->stream));  // ids is read by the copy above
     } else {
         // k-means++ (D^2 sampling), every step on the device without host syncs
-        double* D2 = ctx->init_d2.get<double>(n);
         const int64_t nchunks = (n + OBJ_CHUNK - 1) / OBJ_CHUNK;
-        double* chunks = ctx->init_chunks.get<double>(nchunks);
-        int64_t* chosen = ctx->init_chosen.get<int64_t>(1);
+        const int dp = int((d + 31) / 32 * 32);  // whole pieces of init_step_kernel
+        init_step<F> s{};
+        s.X = Xd;
+        s.n = n;
+        s.d = di;
+        s.D2 = ctx->init_d2.get<double>(n);
+        s.chunk_sums = ctx->init_chunks.get<double>(nchunks);
+        s.cnew = ctx->init_cnew.get<double>(dp);
+        // The bound needs each centroid's distance to the new one, a launch of 5 us: less
+        // than the reads it saves once the rows no longer fit the caches of the
+        // chip (n=50000, d=33, k=64, 6.6 MB: 2.1 ms without, 3.5 ms with it)
+        double* thr = nullptr;
+        if (double(n) * double(d) * sizeof(F) >= INIT_BOUND_BYTES) {
+            thr = ctx->init_thr.get<double>(k);
+            s.near = ctx->init_near.get<int32_t>(n);
+        }
+        s.thr = thr;
+        s.C = Cd;
+        s.ticket = ctx->step_ticket.get<uint32_t>(1);
         const int64_t first = int64_t(rng_index(seed, RNG_STREAM_PLUS_PLUS, 0, uint64_t(n)));
-        hipLaunchKernelGGL(init_copy_row_kernel<F>, dim3(1), dim3(256), 0, ctx->stream, Xd, di, nullptr, first,
-                           Cd, int64_t(0));
+        hipLaunchKernelGGL(init_first_kernel<F>, dim3(1), dim3(256), 0, ctx->stream, Xd, di, first, Cd, s.cnew, dp);
         KM_LAUNCH_CHECK();
-        const int d2_grid = grid_for(ctx, n, 256, 8);
-        const int ch_grid = grid_for(ctx, nchunks, 1, 8);
+        const int grid = grid_for(ctx, n, INIT_PART, 4);
+        const int vectors = int((d * int64_t(sizeof(F)) + 15) / 16);  // 16-byte vectors of a row
         for (int64_t t = 1; t < k; ++t) {
-            hipLaunchKernelGGL(init_d2_kernel<F>, dim3(d2_grid), dim3(256), 0, ctx->stream, Xd, n, di,
-                               Cd + (t - 1) * d, D2, t == 1 ? 1 : 0);
+            s.t = t;
+            s.u = rng_uniform01(seed, RNG_STREAM_PLUS_PLUS, uint64_t(t));
+#define KM_INIT_STEP(PP_) \
+    hipLaunchKernelGGL((init_step_kernel<F, PP_>), dim3(grid), dim3(256), 0, ctx->stream, s)
+            if (vectors <= 1) KM_INIT_STEP(1);
+            else if (vectors <= 2) KM_INIT_STEP(2);
+            else if (vectors <= 4) KM_INIT_STEP(4);
+            else KM_INIT_STEP(8);
+#undef KM_INIT_STEP
             KM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(init_chunk_sums_kernel, dim3(ch_grid), dim3(256), 0, ctx->stream, D2, n, chunks);
+            hipLaunchKernelGGL(init_pick_kernel<F>, dim3(grid_for(ctx, nchunks, 1, 2)), dim3(256), 0, ctx->stream, s,
+                               dp);
             KM_LAUNCH_CHECK();
-            const double u = rng_uniform01(seed, RNG_STREAM_PLUS_PLUS, uint64_t(t));
-            hipLaunchKernelGGL(init_select_kernel, dim3(1), dim3(256), 0, ctx->stream, D2, n, chunks, u, chosen);
-            KM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(init_copy_row_kernel<F>, dim3(1), dim3(256), 0, ctx->stream, Xd, di, chosen,
-                               int64_t(0), Cd, t);
-            KM_LAUNCH_CHECK();
+            if (thr && t + 1 < k) {
+                hipLaunchKernelGGL(init_pairs_kernel<F>, dim3(grid_for(ctx, t, 4, 4)), dim3(256), 0, ctx->stream, Cd,
+                                   s.cnew, t, di, thr);
+                KM_LAUNCH_CHECK();
+            }
         }
     }
     if (!dev) KM_HIP(hipMemcpyAsync(C_out, Cd, sizeof(F) * k * d, hipMemcpyDeviceToHost, ctx->stream));
@@ -2367,7 +2392,7 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->cand_dev, &ctx->c_out_dev, &ctx->seg_cand_rows,
                         &ctx->seg_cand_cnt, &ctx->seg_cand_ids, &ctx->seg_coll_rows, &ctx->seg_coll_T,
                         &ctx->seg_counts, &ctx->tune_x, &ctx->tune_c, &ctx->tune_l,
-                        &ctx->init_d2, &ctx->init_chunks, &ctx->init_chosen, &ctx->init_ids,
+                        &ctx->init_d2, &ctx->init_chunks, &ctx->init_chosen, &ctx->init_ids, &ctx->init_near, &ctx->init_cnew, &ctx->init_thr,
                         &ctx->gt_d, &ctx->stat_acc, &ctx->ec_wcnt, &ctx->cs_inst, &ctx->cs_pre,
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
                         &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,

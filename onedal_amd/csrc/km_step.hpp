@@ -69,7 +69,6 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
     extern __shared__ __align__(16) unsigned char step_raw[];
     F* row = reinterpret_cast<F*>(step_raw);  // [d]
     __shared__ unsigned long long red[4][4];
-    __shared__ bool s_last;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int k = s.k, d = s.d, dpad = s.dpad;
     unsigned long long mx[4] = {0ull, 0ull, 0ull, 0ull};  // wave 0, lane 0
@@ -145,7 +144,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
             if (lane == 0) {
                 const double up = 1.0 + 1e-12;
                 auto bits = [](double v) { return (unsigned long long)__double_as_longlong(v); };
-                s.cn[j] = F(sq);
+                agent_store(s.cn + j, F(sq));
                 if (s.cnp) {
                     uint32_t hm, l;
                     split3(float(sq), hm, l);
@@ -160,7 +159,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
                 }
                 if (s.cold) {
                     const double m = sqrt(sd) * up;
-                    s.drift[j] = m;
+                    agent_store(s.drift + j, m);
                     mx[3] = max(mx[3], bits(m));
                 }
             }
@@ -179,21 +178,14 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
     }
     if (t == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s.wgmax[4 * blockIdx.x + q] = mx[q];
+        for (int q = 0; q < 4; ++q) agent_store(s.wgmax + 4 * blockIdx.x + q, mx[q]);
     }
-    __syncthreads();
-    if (t == 0) {
-        __threadfence();  // this workgroup's results before its ticket
-        s_last = atomicAdd(s.ticket, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
+    if (!last_workgroup(s.ticket)) return;
     // joint maxima
     unsigned long long m[4] = {0ull, 0ull, 0ull, 0ull};
     for (int b = t; b < int(gridDim.x); b += 256)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) m[q] = max(m[q], s.wgmax[4 * b + q]);
+        for (int q = 0; q < 4; ++q) m[q] = max(m[q], agent_load(s.wgmax + 4 * b + q));
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
@@ -214,12 +206,12 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
         // cnB_j = ||c_j||^2 + B rounded up (v_j keeps its lower bound); padded ids get
         // a huge start value so they are never chosen
         for (int j = t; j < s.kp; j += 256)
-            s.cnb[j] = j < k ? add_round_up(float(s.cn[j]), float(p.B)) : __uint_as_float(0x7F000000u);
+            s.cnb[j] = j < k ? add_round_up(float(agent_load(s.cn + j)), float(p.B)) : __uint_as_float(0x7F000000u);
     }
     if (s.cold) {
         const double top = value(3);
         for (int j = t; j < k; j += 256) {
-            const double b = (s.base[j] + (s.drift[j] + top) * (1.0 + s.gam)) * (1.0 + 1e-15);
+            const double b = (s.base[j] + (agent_load(s.drift + j) + top) * (1.0 + s.gam)) * (1.0 + 1e-15);
             s.base[j] = b < BOUND_MAX ? b : __builtin_inf();
             s.changed[j] = 0;
         }

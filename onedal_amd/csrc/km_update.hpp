@@ -551,7 +551,6 @@ __global__ __launch_bounds__(256) void objective_sum_kernel(const double* __rest
                                                             const unsigned long long* __restrict__ acc,
                                                             uint32_t* __restrict__ ticket) {
     __shared__ double part[256];
-    __shared__ bool s_last;
     const int t = threadIdx.x;
     const int64_t nchunks = (n + OBJ_CHUNK - 1) / OBJ_CHUNK;
     for (int64_t q = blockIdx.x; q < nchunks; q += gridDim.x) {
@@ -570,20 +569,14 @@ __global__ __launch_bounds__(256) void objective_sum_kernel(const double* __rest
             if (t < s) part[t] = part[t] + part[t + s];
             __syncthreads();
         }
-        if (t == 0) chunk_sums[q] = part[0];
+        if (t == 0) agent_store(chunk_sums + q, part[0]);
         __syncthreads();
     }
-    if (t == 0) {
-        __threadfence();  // this workgroup's chunk sums before its ticket
-        s_last = atomicAdd(ticket, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
+    if (!last_workgroup(ticket)) return;
     double sum = start ? *start : 0.0;
     for (int64_t b = 0; b < nchunks; b += 256) {
         __syncthreads();
-        if (b + t < nchunks) part[t] = chunk_sums[b + t];
+        if (b + t < nchunks) part[t] = agent_load(chunk_sums + b + t);
         __syncthreads();
         if (t == 0) {
             const int m = int(min<int64_t>(256, nchunks - b));
