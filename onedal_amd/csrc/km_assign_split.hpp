@@ -27,6 +27,15 @@
 //   rounding of ||c_j||^2, s: 2^-22 (X^2 + C^2); underflow of halves and products:
 //                 1e-32 (X + C) + 2e-35
 // Padding features are exact zeros and add nothing.
+//
+// TERMS = 1 keeps xh.ch alone: the BF16 form for rows that are assigned once
+// (inference), straight from the float rows.  Its band is the BF16 one,
+//   2 (X Ec + ex C (1 + 2^-8)) + gamma_d 2.04 X C + gamma_8 1.02 (X + C)^2 + ...
+// with Ec = max ||c - bf16(c)|| and ex = ||x - bf16(x)|| formed in the kernel; rows that
+// its slots cannot settle go through the three-term kernel, a list of rows.  A BF16
+// copy of the rows would be written and read once for nothing: at n=5e6, d=128, k=512
+// the conversion took 0.91 ms of a 1.57 ms call.  Training keeps the copy
+// (assign_bf16_kernel): its passes read the rows again and again.
 #pragma once
 
 #include "km_assign.hpp"
@@ -50,10 +59,13 @@ struct split_consts {
     int ib;
 };
 
-// value error of a row with squared norm at most X2
-__device__ __forceinline__ float split_delta(const split_consts& kc, float X2, float C) {
+// value error of a row with squared norm at most X2 (one term: Ec, and ex2 = ex^2)
+template <int TERMS>
+__device__ __forceinline__ float split_delta(const split_consts& kc, float X2, float C, float Ec, float ex2) {
     const float X = sqrtf(X2), m = X + C;
-    return 1.03f * (kc.xc * X * C + kc.sum * m * m + 2.4e-7f * (X2 + C * C) + 1e-32f * m + 2e-35f);
+    float e = kc.xc * X * C + kc.sum * m * m + 2.4e-7f * (X2 + C * C) + 1e-32f * m + 2e-35f;
+    if (TERMS == 1) e += 2.0f * (X * Ec + sqrtf(ex2) * C * 1.004f);
+    return 1.03f * e;
 }
 
 // (hi, lo) bf16 halves of two floats, packed
@@ -79,30 +91,40 @@ __device__ __forceinline__ void split3(float v, uint32_t& hm, uint32_t& l) {
 // Ring of 4 LDS slots: a block of 32 centroids with both halves is 128 DP bytes, and
 // 1 KB of norm pieces (DP = 128: 68 KB, two workgroups per CU)
 constexpr int SPLIT_RING = 4;
-__host__ inline size_t split_lds_bytes(int dp) { return size_t(SPLIT_RING) * (size_t(128) * dp + 1024); }
+__host__ inline size_t split_lds_bytes(int dp, int terms) {
+    const size_t ring = size_t(SPLIT_RING) * (size_t(terms == 3 ? 128 : 64) * dp + 1024);
+    return ring > 16384 ? ring : 16384;  // rows are transposed in it, 4 KB a wave
+}
 
 // Workgroup = 4 waves of NB x 32 rows (B operand, both halves in registers for the
 // whole pass); blocks of 32 centroids (A operand) stream through the LDS ring by
 // direct-to-LDS copies, one barrier per block, as in assign_bf16_kernel: 16-byte
-// chunk c of a row sits at chunk c ^ (row & SWZ).  Lane l = 32 h + r holds features
-// [h DP/2, (h+1) DP/2) of row r.  Cs: rows of [hi DP | lo DP] bf16 of -2 c_j, and
+// chunk c of a row sits at chunk c ^ (row & SWZ).  Lane l = 32 h + r holds row r's
+// features 32 p + 16 h .. + 15 of every 128-byte piece p.  Rows are read as whole
+// pieces (eight lanes a piece, so every load is full lines; a lane reading its own row
+// 16 bytes at a time fetched each line from L2 again and again: 1.25 ms a launch at
+// n=5e6, d=128, k=512) and pass through the ring's memory to their lanes before the
+// ring is filled.  Cs: rows of [hi DP | lo DP] bf16 of -2 c_j, and
 // cnp: 16 bf16 per row (the norm step's operand), both padded to whole groups of
 // four blocks (padding: zero rows with a huge norm).  Slots and settling as in
-// assign_bf16_kernel; rows without a certain candidate set go to the full list.
-template <int DP, int NB>
+// assign_bf16_kernel; rows without a certain candidate set go to the full list (one
+// term: to the collect rows, for the three-term kernel).
+template <int DP, int NB, int TERMS>
 __global__ __launch_bounds__(256, 2) void assign_split_kernel(
     const float* __restrict__ X, int64_t n, int d, const uint16_t* __restrict__ Cs,
     const uint16_t* __restrict__ cnp, int k, const double* __restrict__ cmax_p, split_consts kc,
     int32_t* __restrict__ labels, refine_lists L, row_select rs) {
     constexpr int HALF = DP / 2;
     constexpr int STEPS = HALF / 8;
+    constexpr int PIECES = DP / 32;  // 128-byte pieces of a row
     constexpr int ROWS_PER_WAVE = 32 * NB;
     constexpr int ROWS_PER_WG = 4 * ROWS_PER_WAVE;
-    constexpr int CPR = DP / 4;                     // 16-byte chunks per centroid row
+    constexpr int ROWB = TERMS == 3 ? DP * 4 : DP * 2;  // bytes of a centroid row in LDS
+    constexpr int CPR = ROWB / 16;                  // 16-byte chunks of it
     constexpr int SWZ = (CPR < 16 ? CPR : 16) - 1;  // chunk swizzle mask
-    constexpr int ROWB = DP * 4;
     constexpr int BLKB = 32 * ROWB;
-    constexpr int DPW = BLKB / 4096;                // 1 KB copies per wave per block
+    constexpr int NDATA = BLKB / 1024;              // 1 KB copies per block
+    constexpr int DPW = NDATA >= 4 ? NDATA / 4 : 1;  // of each wave (2 KB blocks: two waves copy the same)
     constexpr int CPW = DPW + 1;                    // + the block's norm pieces
     constexpr int NSL = 4;
     constexpr int RING = SPLIT_RING;
@@ -118,7 +140,8 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
     const int r32 = lane & 31;
     const int h = lane >> 5;
     const int mblocks = bf16_padded_k(k) / 32;  // a multiple of 4
-    const float C = float(*cmax_p) * (1.0f + 2.4e-7f);
+    const float C = float(cmax_p[0]) * (1.0f + 2.4e-7f);
+    const float Ec = TERMS == 1 ? float(cmax_p[2]) * (1.0f + 2.4e-7f) : 0.f;
     const uint32_t kmask = 0x7FFFFFFFu & ~((1u << kc.ib) - 1u);
     const int64_t nrows = select_rows(rs, n);
     const int64_t ntiles = (nrows + ROWS_PER_WG - 1) / ROWS_PER_WG;
@@ -129,16 +152,16 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
     uint32_t voff[DPW], moff[DPW];
 #pragma unroll
     for (int c = 0; c < DPW; ++c) {
-        const int q = wave + 4 * c;
+        const int q = NDATA >= 4 ? wave + 4 * c : wave % NDATA;
         const int p = q * 64 + lane;
         const int prow = p / CPR, pc = p % CPR;
-        voff[c] = uint32_t(prow * ROWB + (pc ^ (prow & SWZ)) * 16);
+        voff[c] = uint32_t(prow * DP * 4 + (pc ^ (prow & SWZ)) * 16);  // both halves in memory
         moff[c] = lds_addr(ring + q * 1024);
     }
     const uint32_t voff_cn = uint32_t(lane * 16);
     const uint32_t moff_cn = lds_addr(ring_cn);
     auto issue_block = [&](int mb, int slot) {
-        const void* gb = uniform_ptr(reinterpret_cast<const unsigned char*>(Cs) + size_t(mb) * BLKB);
+        const void* gb = uniform_ptr(reinterpret_cast<const unsigned char*>(Cs) + size_t(mb) * (128 * DP));
 #pragma unroll
         for (int c = 0; c < DPW; ++c) lds_dma16(gb, voff[c], moff[c] + slot * BLKB);
         const void* gc = uniform_ptr(reinterpret_cast<const unsigned char*>(cnp) + size_t(mb) * 1024);
@@ -147,61 +170,94 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
 
     // rows of a tile: loaded as floats while the previous tile settles, then split into
     // both halves, the norm step's operand, and what the settle needs
-    uintx4 xh[NB][STEPS], xl[NB][STEPS];
+    uintx4 xh[NB][STEPS], xl[NB][TERMS == 3 ? STEPS : 1];
     uintx4 xs_op[NB];
-    floatx4 raw[NB][2 * STEPS];
+    floatx4 raw[NB][PIECES][4];
     int64_t rows[NB];
     float x2[NB], xs[NB], da[NB];
     auto load_tile = [&](int64_t tile) {
         const int64_t w0 = tile * ROWS_PER_WG + int64_t(wave) * ROWS_PER_WAVE;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            const int64_t e = w0 + nb * 32 + r32;
-            const bool ok = e < nrows;
-            const int64_t row = ok ? select_row(rs, e) : 0;
-            rows[nb] = ok ? row : -1;
-            const float* src = X + row * d + h * HALF;
-            const int left = ok ? d - h * HALF : 0;  // features of this half
-            // 16-byte loads need dword alignment only, so any width takes them.  The last
-            // piece of an odd width also reads the next row's first features (masked
-            // in split_tile); the last row of X, which has none, is read by elements.
-            const int64_t avail = (n - row) * d - h * HALF;  // floats from src to the end of X
+            const int64_t own = w0 + nb * 32 + r32;
+            rows[nb] = own < nrows ? select_row(rs, own) : -1;
+            // this lane's 16 bytes of rows lane / 8 + 8 i
 #pragma unroll
-            for (int q = 0; q < 2 * STEPS; ++q) {
-                floatx4 t = {0.f, 0.f, 0.f, 0.f};
-                if (4 * q < left) {
-                    if (4 * q + 4 <= avail) {
-                        t = *reinterpret_cast<const floatx4u*>(src + 4 * q);
-                    } else {
-                        t[0] = src[4 * q];
-                        if (4 * q + 1 < left) t[1] = src[4 * q + 1];
-                        if (4 * q + 2 < left) t[2] = src[4 * q + 2];
+            for (int i = 0; i < 4; ++i) {
+                const int64_t e = w0 + nb * 32 + 8 * i + (lane >> 3);
+                const bool ok = e < nrows;
+                const int64_t row = ok ? select_row(rs, e) : 0;
+                const float* src = X + row * d + 4 * (lane & 7);
+                // 16-byte loads need dword alignment only, so any width takes them.  The
+                // last vector of an odd width also reads the next row's first features
+                // (masked in split_tile); the last row of X has none: by elements.
+                const int left = ok ? d - 4 * (lane & 7) : 0;               // features from src on
+                const int64_t avail = (n - row) * d - 4 * (lane & 7);  // floats from src to the end of X
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) {
+                    floatx4 t = {0.f, 0.f, 0.f, 0.f};
+                    if (32 * p < left) {
+                        if (32 * p + 4 <= avail) {
+                            t = *reinterpret_cast<const floatx4u*>(src + 32 * p);
+                        } else {
+                            t[0] = src[32 * p];
+                            if (32 * p + 1 < left) t[1] = src[32 * p + 1];
+                            if (32 * p + 2 < left) t[2] = src[32 * p + 2];
+                        }
                     }
+                    raw[nb][p][i] = t;
                 }
-                raw[nb][q] = t;
             }
         }
+    };
+    // each row's pieces to the lanes that hold it (the ring is empty; a wave uses 4 KB of
+    // it, and its LDS operations run in order)
+    auto transpose_tile = [&]() {
+        unsigned char* mine = ring + wave * 4096;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = 8 * i + (lane >> 3);
+                    *reinterpret_cast<floatx4*>(mine + r * 128 + (((lane & 7) ^ (r & 7)) * 16)) = raw[nb][p][i];
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    raw[nb][p][q] =
+                        *reinterpret_cast<const floatx4*>(mine + r32 * 128 + (((4 * h + q) ^ (r32 & 7)) * 16));
+                __builtin_amdgcn_wave_barrier();
+            }
     };
     auto split_tile = [&]() {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            float sq[4] = {0.f, 0.f, 0.f, 0.f};
+            float sq[4] = {0.f, 0.f, 0.f, 0.f}, se[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int q = 0; q < 2 * STEPS; ++q) {
-                floatx4 v = raw[nb][q];
+            for (int q = 0; q < 2 * STEPS; ++q) {  // vector q: features 32 (q / 4) + 16 h + 4 (q % 4) ..
+                floatx4 v = raw[nb][q >> 2][q & 3];
                 if (d & 3) {
-                    const int left = d - h * HALF;
+                    const int left = d - 32 * (q >> 2) - 16 * h - 4 * (q & 3);
 #pragma unroll
-                    for (int u = 1; u < 4; ++u) v[u] = 4 * q + u < left ? v[u] : 0.f;
+                    for (int u = 1; u < 4; ++u) v[u] = u < left ? v[u] : 0.f;
                 }
 #pragma unroll
                 for (int u = 0; u < 4; ++u) sq[u] = __builtin_fmaf(v[u], v[u], sq[u]);
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
                     uint32_t hi, lo;
-                    split2(v[2 * u], v[2 * u + 1], hi, lo);
+                    split2(v[2 * u], v[2 * u + 1], hi, lo);  // one term: lo is not used
                     xh[nb][q >> 1][2 * (q & 1) + u] = hi;
-                    xl[nb][q >> 1][2 * (q & 1) + u] = lo;
+                    if constexpr (TERMS == 3) {
+                        xl[nb][q >> 1][2 * (q & 1) + u] = lo;
+                    } else {
+                        const float e0 = v[2 * u] - __uint_as_float(hi << 16);
+                        const float e1 = v[2 * u + 1] - __uint_as_float(hi & 0xFFFF0000u);
+                        se[2 * u] = __builtin_fmaf(e0, e0, se[2 * u]);
+                        se[2 * u + 1] = __builtin_fmaf(e1, e1, se[2 * u + 1]);
+                    }
                 }
             }
             // ||x||^2: chains of at most DP / 8 additions, so the relative error is
@@ -210,7 +266,12 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
             t += __shfl_xor(t, 32);
             x2[nb] = t;
             const float up = t * (1.0f + 2.4e-6f);
-            da[nb] = split_delta(kc, up, C);
+            float ex2 = 0.f;
+            if constexpr (TERMS == 1) {
+                ex2 = (se[0] + se[1]) + (se[2] + se[3]);
+                ex2 = (ex2 + __shfl_xor(ex2, 32)) * (1.0f + 2.4e-6f);
+            }
+            da[nb] = split_delta<TERMS>(kc, up, C, Ec, ex2);
             xs[nb] = (up + da[nb]) * (1.0f + 2.4e-7f);
             uint32_t hm, l;
             split3(xs[nb], hm, l);
@@ -233,35 +294,38 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
             const unsigned char* arow = ring + slot * BLKB + r32 * ROWB;
             const bf16x8 an = __builtin_bit_cast(
                 bf16x8, *reinterpret_cast<const uintx4*>(ring_cn + slot * 1024 + r32 * 32 + h * 16));
-            bf16x8 ah[STEPS], al[STEPS];
+            bf16x8 ah[STEPS], al[TERMS == 3 ? STEPS : 1];
 #pragma unroll
             for (int s = 0; s < STEPS; ++s) {
-                const int c = h * STEPS + s;
+                const int c = 4 * (s >> 1) + 2 * h + (s & 1);  // step s: features 8 c .. 8 c + 7
                 ah[s] = __builtin_bit_cast(
                     bf16x8, *reinterpret_cast<const uintx4*>(arow + ((c ^ (r32 & SWZ)) * 16)));
-                al[s] = __builtin_bit_cast(
-                    bf16x8, *reinterpret_cast<const uintx4*>(arow + (((DP / 8 + c) ^ (r32 & SWZ)) * 16)));
+                if constexpr (TERMS == 3)
+                    al[s] = __builtin_bit_cast(
+                        bf16x8, *reinterpret_cast<const uintx4*>(arow + (((DP / 8 + c) ^ (r32 & SWZ)) * 16)));
             }
             // the small products first, then xh.ch, then the norms (the error bound
             // counts on this order)
             const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if constexpr (TERMS == 3) {
 #pragma unroll
-            for (int s = 0; s < STEPS; ++s) {
+                for (int s = 0; s < STEPS; ++s) {
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        ah[s], __builtin_bit_cast(bf16x8, xl[nb][s]), s == 0 ? zero : acc[nb], 0, 0, 0);
+                    for (int nb = 0; nb < NB; ++nb)
+                        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            ah[s], __builtin_bit_cast(bf16x8, xl[nb][s]), s == 0 ? zero : acc[nb], 0, 0, 0);
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        al[s], __builtin_bit_cast(bf16x8, xh[nb][s]), acc[nb], 0, 0, 0);
+                    for (int nb = 0; nb < NB; ++nb)
+                        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            al[s], __builtin_bit_cast(bf16x8, xh[nb][s]), acc[nb], 0, 0, 0);
+                }
             }
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
                     acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        ah[s], __builtin_bit_cast(bf16x8, xh[nb][s]), acc[nb], 0, 0, 0);
+                        ah[s], __builtin_bit_cast(bf16x8, xh[nb][s]), TERMS == 1 && s == 0 ? zero : acc[nb], 0, 0, 0);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
                 acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(an, __builtin_bit_cast(bf16x8, xs_op[nb]), acc[nb],
@@ -299,6 +363,8 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
         // row loads complete here; the previous tile's last readers are done before
         // the prologue refills the ring
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        __syncthreads();
+        transpose_tile();
         __syncthreads();
 #pragma unroll
         for (int b = 0; b < AHEAD; ++b) issue_block(min(b, mblocks - 1), b);
@@ -412,9 +478,9 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
         }
         if (ml) {
             int e0 = 0;
-            if (lane == 0) e0 = atomicAdd(&L.counters[1], int(__popcll(ml)));
+            if (lane == 0) e0 = atomicAdd(&L.counters[TERMS == 3 ? 1 : 2], int(__popcll(ml)));
             e0 = __builtin_amdgcn_readfirstlane(e0);
-            if (outcome == 2) L.full_rows[e0 + lanes_below(ml)] = int32_t(row);
+            if (outcome == 2) (TERMS == 3 ? L.full_rows : L.coll_rows)[e0 + lanes_below(ml)] = int32_t(row);
         }
     }
 }

@@ -232,7 +232,8 @@ struct work {
     uint16_t* Cb = nullptr;       // k x dpad bf16(-2 c)
     float* cnb = nullptr;         // ||c||^2 + B (rounded up), 32 * ceil(k / 32) entries
     bf16_params* params = nullptr;
-    // split path (path 2, float): both bf16 halves of -2 c, and the norm pieces
+    // split path (path 2, float; and path 3 for rows assigned once): both bf16 halves of
+    // -2 c, and the norm pieces
     bool split = false;
     uint16_t* Csp = nullptr;  // bf16_padded_k(k) x 2 dpad
     uint16_t* cnp = nullptr;  // bf16_padded_k(k) x 16
@@ -269,10 +270,13 @@ static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
     return 2;
 }
 
-// float data on path 2: split BF16 products (km_assign_split.hpp) where a row's halves
-// fit a lane's registers and the key's index bits leave the band narrow; FP32
-// products past that.  double data: never.
-static bool use_split(int path, int d, int k) { return path == 2 && d <= 128 && k <= SPLIT_MAX_K; }
+// float data on path 2, and on path 3 for rows assigned once (inference): split BF16
+// products (km_assign_split.hpp) where a row's halves fit a lane's registers and the
+// key's index bits leave the band narrow.  Path 2 takes FP32 products past that, path
+// 3 a BF16 copy of the rows.  double data: never.
+static bool use_split(int path, int d, int k, bool once) {
+    return (path == 2 || (path == 3 && once)) && d <= 128 && k <= SPLIT_MAX_K;
+}
 
 template <typename F>
 static band_consts make_band(int d) {
@@ -340,7 +344,7 @@ static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* col
     const int grid = std::min(w.k, STEP_MAX_GRID);
     const size_t lds = size_t(w.d) * sizeof(F);
     if constexpr (std::is_same<F, float>::value) {
-        if (path == 3) {
+        if (path == 3 && !w.split) {
             s.Cb = w.Cb;
             s.kp = bf16_padded_k(w.k);
             s.xmax_bits = w.xmax_bits;
@@ -379,13 +383,15 @@ static void launch_mfma_f32(km_ctx* ctx, work<float>& w, const band_consts& bc) 
         launch_mfma_f32_mode<DP, NB, false>(ctx, w, bc, grid, mfma_f32_lds_bytes(DP, w.k, false));
 }
 
+template <int TERMS>
 static split_consts make_split_consts(int d, int k) {
     split_consts c;
     int mbits = 0;
     while ((1 << mbits) < bf16_padded_k(k) / 32) mbits++;
     c.ib = 4 + mbits;
     const double ua = fp_traits<float>::u_acc;
-    c.xc = float(std::ldexp(6.02, -18) + gamma_m(2.0 * d, ua) * 2.02 / 256.0 + gamma_m(double(d), ua) * 2.04);
+    c.xc = float(gamma_m(double(d), ua) * 2.04);
+    if (TERMS == 3) c.xc += float(std::ldexp(6.02, -18) + gamma_m(2.0 * d, ua) * 2.02 / 256.0);
     c.sum = float(gamma_m(8.0, ua) * 1.02);
     c.trunc = float(std::ldexp(1.0, c.ib - 23));
     const double g = gamma_m(double(d + 2), fp_traits<float>::u);
@@ -393,17 +399,27 @@ static split_consts make_split_consts(int d, int k) {
     return c;
 }
 
-template <int DP, int NB>
-static void launch_split(km_ctx* ctx, work<float>& w) {
+// terms 3, or 1 (BF16 distances of rows assigned once); sel: the rows
+template <int DP, int NB, int TERMS>
+static void launch_split(km_ctx* ctx, work<float>& w, const row_select& sel) {
     constexpr int ROWS_PER_WG = 4 * 32 * NB;
     const int64_t tiles = (w.n + ROWS_PER_WG - 1) / ROWS_PER_WG;
     const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * 2)));
-    const size_t lds = split_lds_bytes(DP);
-    auto kern = assign_split_kernel<DP, NB>;
+    const size_t lds = split_lds_bytes(DP, TERMS);
+    auto kern = assign_split_kernel<DP, NB, TERMS>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.X, w.n, w.d, w.Csp, w.cnp, w.k, w.maxima,
-                       make_split_consts(w.d, w.k), w.labels, w.L, w.sel);
+                       make_split_consts<TERMS>(w.d, w.k), w.labels, w.L, sel);
     KM_LAUNCH_CHECK();
+}
+
+template <int TERMS>
+static void launch_split(km_ctx* ctx, work<float>& w, const row_select& sel) {
+    switch (w.dpad) {
+        case 32: launch_split<32, 2, TERMS>(ctx, w, sel); break;
+        case 64: launch_split<64, 2, TERMS>(ctx, w, sel); break;
+        default: launch_split<128, TERMS == 3 ? 1 : 2, TERMS>(ctx, w, sel); break;
+    }
 }
 
 template <int DP, int NB>
@@ -489,12 +505,12 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
         KM_HIP(hipEventRecord(e0, ctx->stream));
     }
     if constexpr (std::is_same<F, float>::value) {
-        if (w.split) {
-            switch (w.dpad) {
-                case 32: launch_split<32, 2>(ctx, w); break;
-                case 64: launch_split<64, 2>(ctx, w); break;
-                default: launch_split<128, 1>(ctx, w); break;
-            }
+        if (w.split && path == 3) {
+            // rows that one term leaves open: three terms
+            launch_split<1>(ctx, w, w.sel);
+            launch_split<3>(ctx, w, {w.L.coll_rows, w.L.counters + 2, nullptr, nullptr, 0.0});
+        } else if (w.split) {
+            launch_split<3>(ctx, w, w.sel);
         } else if (path == 2) {
             switch (w.dpad) {
                 case 32: launch_mfma_f32<32, 2>(ctx, w, bc); break;
@@ -503,7 +519,7 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
                 default: launch_mfma_f32<256, 1>(ctx, w, bc); break;
             }
         }
-        if (path == 3) {
+        if (path == 3 && !w.split) {
             switch (w.dpad) {
                 case 32: launch_bf16<32>(ctx, w, false); break;
                 case 64: launch_bf16<64>(ctx, w, false); break;
@@ -537,7 +553,7 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
     refine_pairs<F>(ctx, w, C,
                     {w.L.cand_rows, w.L.cand_count, w.L.cand_ids, w.L.cand_lo, w.L.counters + 0, MAXC});
     if constexpr (std::is_same<F, float>::value) {
-        if (path == 3) {
+        if (path == 3 && !w.split) {
             switch (w.dpad) {
                 case 32: launch_bf16<32>(ctx, w, true); break;
                 case 64: launch_bf16<64>(ctx, w, true); break;
@@ -816,8 +832,8 @@ static int32_t* launch_empty_clusters(km_ctx* ctx, const F* X, int64_t n, int d,
 
 template <typename F>
 static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, int k,
-                       int path, arena* A = nullptr, int32_t* labels_into = nullptr) {
-    w.split = std::is_same<F, float>::value && use_split(path, d, k);
+                       int path, bool once, arena* A = nullptr, int32_t* labels_into = nullptr) {
+    w.split = std::is_same<F, float>::value && use_split(path, d, k, once);
     const bool vec_view = path == 2 && !w.split;
     w.n = n;
     w.d = d;
@@ -852,6 +868,10 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
         w.Xv = xp;
         w.ldx = ldx;
     }
+    if (w.split) {  // its kernel forms the norms itself
+        if (path == 3) w.L.coll_rows = take<int32_t>(ctx, &km_ctx::coll_rows, A, n);
+        return;
+    }
     const int grid = grid_for(ctx, n * 64, 256, 8);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
@@ -872,7 +892,6 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
             return;
         }
     }
-    if (w.split) return;  // its kernel forms the norms itself
     hipLaunchKernelGGL(row_norm_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, Xd, n, d, w.xnorm);
     KM_LAUNCH_CHECK();
 }
@@ -902,7 +921,7 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
     // device labels go straight to the caller's buffer (read as 16-byte vectors by the
     // row selection)
     const bool own_labels = !dev || reinterpret_cast<uintptr_t>(labels_out) % 16 != 0;
-    setup_work<F>(ctx, w, Xd, n, d, k, path, nullptr, own_labels ? nullptr : labels_out);
+    setup_work<F>(ctx, w, Xd, n, d, k, path, false, nullptr, own_labels ? nullptr : labels_out);
     ctx->stats.assign_path = path;
     F* Ccur = ctx->c_cur.get<F>(int64_t(k) * d);
     F* Cnext = ctx->c_next.get<F>(int64_t(k) * d);
@@ -1026,7 +1045,7 @@ static void infer(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C, 
     work<F> w;
     const int path = choose_path<F>(ctx, d, k, flags);
     // device centroids and labels are used in place
-    setup_work<F>(ctx, w, Xd, n, d, k, path, nullptr, dev ? labels_out : nullptr);
+    setup_work<F>(ctx, w, Xd, n, d, k, path, true, nullptr, dev ? labels_out : nullptr);
     ctx->stats.assign_path = path;
     F* Cd = const_cast<F*>(C);  // only read (step_centroids without chunk sums)
     if (!dev) {
@@ -1078,10 +1097,11 @@ static size_t noalloc_block_bytes(const km_ctx* ctx, int path, int64_t R, int d,
     const int64_t dpad = pad_dim(d);
     int64_t b = R * (4 + 4 + 4 + 4 * int64_t(MAXC) + 4) + 16 + int64_t(sizeof(F)) * k +
                 int64_t(sizeof(F)) * k * dpad + 32;
-    const bool split = use_split(path, d, k);
+    const bool split = use_split(path, d, k, true);
     if (split) b += 36 * int64_t(bf16_padded_k(k)) + 4 * int64_t(bf16_padded_k(k) - k) * dpad;
     if (path == 2 && !split && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
-    if (path == 3) {
+    if (path == 3 && split) b += 4 * R;
+    if (path == 3 && !split) {
         const int64_t kp = bf16_padded_k(k);
         b += R * (2 * dpad + 4 + 4 + 8 + 4 + 4 * int64_t(MAXC2)) + 16 + 2 * kp * dpad + 4 * kp + 64;
         const int64_t rows_per_wg = dpad >= 256 ? 128 : 256;  // launch_bf16: 4 waves x 32 x NB
@@ -1136,7 +1156,7 @@ static void infer_noalloc(km_ctx* ctx, const float* X, int64_t n, int64_t d64_, 
         const int64_t rows = std::min<int64_t>(R, n - r0);
         arena A{base + 256, cap, 0};
         work<F> w;
-        setup_work<F>(ctx, w, X + r0 * d, rows, d, k, path, &A, labels_out + r0);
+        setup_work<F>(ctx, w, X + r0 * d, rows, d, k, path, true, &A, labels_out + r0);
         step_centroids<F>(ctx, w, path, const_cast<F*>(C));  // only read
         assign<F>(ctx, w, C, path);
         const uint32_t seq = next_seq(ctx);

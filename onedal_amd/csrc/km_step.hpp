@@ -38,7 +38,7 @@ struct centroid_step {
     uint16_t* Csp;
     uint16_t* cnp;
     int kp;
-    double* maxima;  // [0] max ||c||, BF16: [1] max ||bf16(c)||, [2] max ||c - bf16(c)||
+    double* maxima;  // [0] max ||c||, with Cb or Csp: [1] max ||bf16(c)||, [2] max ||c - bf16(c)||
     // BF16: value shift and start values
     const unsigned long long* xmax_bits;
     bf16_consts kc;
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
             for (int f = lane; f < d; f += 64) {
                 const double v = double(row[f]);
                 sq = fma(v, v, sq);
-                if constexpr (BF16) {
+                if (BF16 || s.Csp) {
                     const double vh = double(bf2f(f2bf(float(row[f])))), ve = v - vh;
                     sh = fma(vh, vh, sh);
                     se = fma(ve, ve, se);
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) {
                 sq += __shfl_xor(sq, off);
-                if constexpr (BF16) {
+                if (BF16 || s.Csp) {
                     sh += __shfl_xor(sh, off);
                     se += __shfl_xor(se, off);
                 }
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
                     o4[1] = uintx4{0u, 0u, 0u, 0u};
                 }
                 mx[0] = max(mx[0], bits(sqrt(sq) * up));
-                if constexpr (BF16) {
+                if (BF16 || s.Csp) {
                     mx[1] = max(mx[1], bits(sqrt(sh) * up));
                     mx[2] = max(mx[2], bits(sqrt(se) * up + 1e-30));
                 }
