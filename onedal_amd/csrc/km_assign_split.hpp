@@ -131,6 +131,7 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
     constexpr int AHEAD = RING - 1;
     static_assert(DPW >= 1, "block copy layout");
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ int open_cnt[2][4], open_base[2];  // the tile's list entries per wave, and where they go
     unsigned char* ring = smem_raw;                          // [RING][BLKB]
     unsigned char* ring_cn = smem_raw + size_t(RING) * BLKB;  // [RING][1024]
 
@@ -461,10 +462,24 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
         }
         const uint64_t mc = __ballot(outcome == 1);
         const uint64_t ml = __ballot(outcome == 2);
+        // one reservation per list and tile: every wave's atomics on the two counters
+        // were the time of a pass over few rows (1M open rows of n=1e7: 0.39 ms)
+        if (lane == 0) {
+            open_cnt[0][wave] = int(__popcll(mc));
+            open_cnt[1][wave] = int(__popcll(ml));
+        }
+        __syncthreads();
+        const int tc = open_cnt[0][0] + open_cnt[0][1] + open_cnt[0][2] + open_cnt[0][3];
+        const int tl = open_cnt[1][0] + open_cnt[1][1] + open_cnt[1][2] + open_cnt[1][3];
+        if (tc + tl == 0) continue;  // uniform over the workgroup
+        if (tid < 2) open_base[tid] = atomicAdd(&L.counters[tid == 0 ? 0 : TERMS == 3 ? 1 : 2], tid == 0 ? tc : tl);
+        __syncthreads();
+        int e0 = open_base[0], f0 = open_base[1];
+        for (int w = 0; w < wave; ++w) {
+            e0 += open_cnt[0][w];
+            f0 += open_cnt[1][w];
+        }
         if (mc) {
-            int e0 = 0;
-            if (lane == 0) e0 = atomicAdd(&L.counters[0], int(__popcll(mc)));
-            e0 = __builtin_amdgcn_readfirstlane(e0);
             if (outcome == 1) {
                 const int e = e0 + lanes_below(mc);
                 L.cand_rows[e] = int32_t(row);
@@ -476,12 +491,7 @@ __global__ __launch_bounds__(256, 2) void assign_split_kernel(
                     if (k1[q] <= TK) L.cand_ids[int64_t(e) * MAXC + c++] = idx_of(k1[q], q < NSL ? h : 1 - h);
             }
         }
-        if (ml) {
-            int e0 = 0;
-            if (lane == 0) e0 = atomicAdd(&L.counters[TERMS == 3 ? 1 : 2], int(__popcll(ml)));
-            e0 = __builtin_amdgcn_readfirstlane(e0);
-            if (outcome == 2) (TERMS == 3 ? L.full_rows : L.coll_rows)[e0 + lanes_below(ml)] = int32_t(row);
-        }
+        if (outcome == 2) (TERMS == 3 ? L.full_rows : L.coll_rows)[f0 + lanes_below(ml)] = int32_t(row);
     }
 }
 
