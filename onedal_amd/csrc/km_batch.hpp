@@ -18,6 +18,7 @@
 #pragma once
 
 #include "km_assign.hpp"
+#include "km_bounds.hpp"
 #include "km_common.hpp"
 #include "km_update.hpp"
 
@@ -46,6 +47,27 @@ struct batch_inst {
     int32_t index;
     int32_t vec;  // d % 4 == 0 and X 16-byte aligned
 };
+
+// Rows of an assignment pass over a batch: with bounds (km_bounds.hpp) the open rows of
+// each instance (rows[row0 ..], count[index] of them, as rows of the instance), else
+// (null rows) all; and where the bounds of the assigned rows go (null gap: none).
+struct batch_select {
+    const int32_t* rows;
+    const int32_t* count;
+    float* gap;          // at row0
+    const double* base;  // at k0
+};
+__device__ __forceinline__ int64_t batch_rows(const batch_select& s, const batch_inst& in) {
+    return s.rows ? int64_t(s.count[in.index]) : in.n;
+}
+__device__ __forceinline__ int64_t batch_row(const batch_select& s, const batch_inst& in, int64_t e) {
+    return s.rows ? int64_t(s.rows[in.row0 + e]) : e;
+}
+// g of bound_gap: the exact form's gamma_{d+2}, with room for the float roundings
+__device__ __forceinline__ double batch_gam(int d) {
+    const double g = gamma_m(double(d + 2), fp_traits<float>::u);
+    return g / (1.0 - g) + 1e-6;
+}
 
 constexpr int BATCH_CNT_ROWS = 4096;      // rows per histogram workgroup
 constexpr int BATCH_D64_ROWS = 256;       // rows per d64 workgroup
@@ -93,14 +115,16 @@ __host__ __device__ constexpr int batch_tile_rw(int v) {
 // rows per workgroup
 __host__ __device__ constexpr int batch_tile_rows(int v) { return 4 * batch_tile_rw(v) * (64 / batch_tile_ct(v)); }
 
-template <int CT, int RW>
+// BND: rows and bounds of a selected pass (the second smallest distance costs two ops
+// per distance, so passes without bounds leave it out).
+template <int CT, int RW, bool BND>
 __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __restrict__ I,
                                                            const int32_t* __restrict__ sel, int nsel,
                                                            const int64_t* __restrict__ pre,
                                                            const float* __restrict__ C,
                                                            int32_t* __restrict__ labels,
                                                            uint32_t* __restrict__ skeys, int lbits,
-                                                           int to_user) {
+                                                           int to_user, batch_select bs) {
     constexpr int G = 64 / CT;    // row groups per wave
     constexpr int RWW = RW * G;   // rows per wave
     constexpr int RB = 4 * RWW;   // rows per workgroup
@@ -109,6 +133,7 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
     static_assert(FT % 4 == 0 && FT >= 4, "feature chunk");
     typedef float F4 __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) float Xs[RB][FT];
+    __shared__ int32_t srow[BND ? RB : 1];  // the staged rows
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -121,15 +146,23 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
         const batch_inst in = I[sel[si]];
         const int d = in.d, k = in.k;
         const int64_t r0 = (b - pre[si]) * RB;
-        const int nr = int(min<int64_t>(RB, in.n - r0));
+        const int64_t open = BND ? batch_rows(bs, in) : in.n;
+        if (BND && r0 >= open) continue;  // uniform: the instance has fewer open rows
+        const int nr = int(min<int64_t>(RB, open - r0));
+        if constexpr (BND) {
+            __syncthreads();  // the previous item's readers are done
+            for (int r = tid; r < nr; r += 256) srow[r] = int32_t(batch_row(bs, in, r0 + r));
+        }
+        auto row_of = [&](int r) { return BND ? int64_t(srow[r]) : r0 + r; };
         const float* Ci = C + in.c0;
         const bool vec = in.vec != 0;
-        float best[RW];
+        float best[RW], second[RW];
         int bi[RW];
         bool nan0[RW];
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
             best[r] = __builtin_inff();
+            second[r] = __builtin_inff();
             bi[r] = 0x7fffffff;
             nan0[r] = false;
         }
@@ -141,13 +174,13 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
                 for (int e = tid; e < RB * nv; e += 256) {
                     const int r = e / nv, q = e - r * nv;
                     F4 v = F4{0.f, 0.f, 0.f, 0.f};
-                    if (r < nr) v = *reinterpret_cast<const F4*>(in.X + (r0 + r) * d + f0 + 4 * q);
+                    if (r < nr) v = *reinterpret_cast<const F4*>(in.X + row_of(r) * d + f0 + 4 * q);
                     *reinterpret_cast<F4*>(&Xs[r][4 * q]) = v;
                 }
             } else {
                 for (int e = tid; e < RB * ft; e += 256) {
                     const int r = e / ft, q = e - r * ft;
-                    Xs[r][q] = r < nr ? in.X[(r0 + r) * d + f0 + q] : 0.f;
+                    Xs[r][q] = r < nr ? in.X[row_of(r) * d + f0 + q] : 0.f;
                 }
             }
             __syncthreads();
@@ -208,20 +241,24 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
                 for (int r = 0; r < RW; ++r) {
                     if (j == 0 && acc[r] != acc[r]) nan0[r] = true;
                     if (acc[r] < best[r]) {
+                        if (BND) second[r] = best[r];
                         best[r] = acc[r];
                         bi[r] = j;
+                    } else if (BND && acc[r] < second[r]) {
+                        second[r] = acc[r];
                     }
                 }
             }
         }
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
-            float bv = best[r];
+            float bv = best[r], sv = second[r];
             int bj = bi[r];
 #pragma unroll
             for (int off = CT / 2; off > 0; off >>= 1) {
                 const float ob = __shfl_xor(bv, off);
                 const int oi = __shfl_xor(bj, off);
+                if (BND) sv = fminf(fminf(sv, __shfl_xor(sv, off)), bv < ob ? ob : bv);
                 if (ob < bv || (ob == bv && oi < bj)) {
                     bv = ob;
                     bj = oi;
@@ -230,12 +267,19 @@ __global__ __launch_bounds__(256) void batch_assign_kernel(const batch_inst* __r
             const bool n0 = __shfl(nan0[r] ? 1 : 0, rg * CT) != 0;
             const int rr = rbase + r;
             if (cl == 0 && rr < nr) {
-                const int lab = (n0 || bj == 0x7fffffff) ? 0 : bj;
+                const bool none = n0 || bj == 0x7fffffff;
+                const int lab = none ? 0 : bj;
+                const int64_t row = row_of(rr);
                 if (to_user) {
-                    in.labels_out[r0 + rr] = lab;
+                    in.labels_out[row] = lab;
                 } else {
-                    labels[in.row0 + r0 + rr] = lab;
-                    if (skeys) skeys[in.row0 + r0 + rr] = (uint32_t(in.index) << lbits) | uint32_t(lab);
+                    labels[in.row0 + row] = lab;
+                    if (skeys) skeys[in.row0 + row] = (uint32_t(in.index) << lbits) | uint32_t(lab);
+                    if (BND && bs.gap)
+                        bs.gap[in.row0 + row] =
+                            none ? -__builtin_inff()
+                                 : bound_gap_exact(double(bv), double(sv), __builtin_inf(), batch_gam(d),
+                                                   bs.base[in.k0 + lab]);
                 }
             }
         }
@@ -285,7 +329,7 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                                                                    const float* __restrict__ C,
                                                                    int32_t* __restrict__ labels,
                                                                    uint32_t* __restrict__ skeys, int lbits,
-                                                                   int to_user) {
+                                                                   int to_user, batch_select bs) {
     constexpr int HALF = DP / 2;
     constexpr int CST = DP + 4;  // LDS row stride in floats
     constexpr int NSL = BATCH_MFMA_MAXK / 32;
@@ -305,8 +349,13 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
         const batch_inst in = I[sel[si]];
         const int d = in.d, k = in.k;
         if (d > DP || k > BATCH_MFMA_MAXK) continue;  // never planned so; keeps LDS in bounds
-        const int64_t rb = (b - pre[si]) * item_rows;
-        const int64_t re = min<int64_t>(in.n, rb + item_rows);
+        // the instance's open rows, spread over its items in whole tiles
+        const int64_t open = batch_rows(bs, in), items = pre[si + 1] - pre[si];
+        const int64_t per = bs.rows ? ((open + items - 1) / items + BATCH_MFMA_TILE - 1) / BATCH_MFMA_TILE * BATCH_MFMA_TILE
+                                    : int64_t(item_rows);
+        const int64_t rb = (b - pre[si]) * per;
+        const int64_t re = min<int64_t>(open, rb + per);
+        if (rb >= re) continue;  // uniform: no rows left for this item
         const float* Ci = C + in.c0;
         const int mblocks = (k + 31) / 32;
         const int kp = mblocks * 32;
@@ -372,10 +421,12 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
         const double cmax =
             sqrt(fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]))) * (1.0 + 1e-12);
         const band_consts bc = batch_band_f32(d);
+        const double gam = batch_gam(d);
         for (int64_t t0 = rb; t0 < re; t0 += BATCH_MFMA_TILE) {
-            const int64_t row = t0 + wave * 32 + r32;
-            const bool ok = row < re;
-            const float* xrow = in.X + (ok ? row : rb) * int64_t(d);
+            const int64_t entry = t0 + wave * 32 + r32;
+            const bool ok = entry < re;
+            const int64_t row = batch_row(bs, in, ok ? entry : rb);
+            const float* xrow = in.X + row * int64_t(d);
             float xr[HALF];
             if (in.vec) {
 #pragma unroll
@@ -445,6 +496,7 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                 sl[NSL + q].i2 = __shfl_xor(st[q].i2, 32);
             }
             int lab = 0;
+            float gap = -__builtin_inff();
             bool need_scan = false;
             if (h == 0 && ok) {
                 float best = finf;
@@ -467,13 +519,24 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                         ++cnt;
                     }
                 }
+                const double da = bc.a_xc * Xup * cmax + bc.a_cc * cmax * cmax, X2 = Xup * Xup;
                 if (cert && cnt == 1) {
                     lab = bi;
+                    if (bs.gap) {
+                        float second = finf;
+#pragma unroll
+                        for (int q = 0; q < 2 * NSL; ++q) {
+                            const float v = sl[q].i1 == bi ? sl[q].m2 : sl[q].m1;
+                            second = v < second ? v : second;
+                        }
+                        gap = bound_gap(double(best) + da + X2 + (X2 + fabs(double(best))) * 1e-15,
+                                        double(second) - da + X2 * (1.0 - 3e-12), gam, bs.base[in.k0 + bi]);
+                    }
                 } else if (cert) {
                     // exact form over the candidates (the slot minima inside T, in
                     // slot order; slots are visited by a fixed unrolled loop, so no
                     // candidate array is indexed at run time), ties to the lowest index
-                    float bd = finf;
+                    float bd = finf, sd = finf;
                     lab = k;
 #pragma unroll
                     for (int q = 0; q < 2 * NSL; ++q) {
@@ -481,12 +544,19 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                             const int j = sl[q].i1;
                             const float D = canon_dist<float>(xrow, Cs + j * CST, d);
                             if (D < bd || (D == bd && j < lab)) {
+                                sd = bd;
                                 bd = D;
                                 lab = j;
+                            } else if (D < sd) {
+                                sd = D;
                             }
                         }
                     }
                     if (lab >= k) lab = bi;
+                    // the others lie above T
+                    if (bs.gap)
+                        gap = bound_gap_exact(double(bd), double(sd), T - da + X2 * (1.0 - 3e-12), gam,
+                                              bs.base[in.k0 + lab]);
                 } else {
                     need_scan = true;
                 }
@@ -499,29 +569,38 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
             while (scan_rows) {
                 const int src = __ffsll((unsigned long long)scan_rows) - 1;  // a lane with h = 0
                 scan_rows &= scan_rows - 1;
-                const float* fx = in.X + (t0 + wave * 32 + src) * int64_t(d);
-                float bv = finf;
+                const float* fx = in.X + __shfl(row, src) * int64_t(d);
+                float bv = finf, sv = finf;
                 int bj = 0x7fffffff;
                 bool nan0 = false;
                 for (int j = lane; j < k; j += 64) {
                     const float D = canon_dist<float>(fx, Cs + j * CST, d);
                     if (j == 0 && D != D) nan0 = true;
                     if (D < bv) {
+                        sv = bv;
                         bv = D;
                         bj = j;
+                    } else if (D < sv) {
+                        sv = D;
                     }
                 }
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) {
-                    const float ob = __shfl_xor(bv, off);
+                    const float ob = __shfl_xor(bv, off), os = __shfl_xor(sv, off);
                     const int oj = __shfl_xor(bj, off);
+                    sv = fminf(fminf(sv, os), bv < ob ? ob : bv);
                     if (ob < bv || (ob == bv && oj < bj)) {
                         bv = ob;
                         bj = oj;
                     }
                 }
                 const bool n0 = __shfl(nan0 ? 1 : 0, 0) != 0;
-                if (lane == src) lab = (n0 || bj == 0x7fffffff) ? 0 : bj;
+                if (lane == src) {
+                    const bool none = n0 || bj == 0x7fffffff;
+                    lab = none ? 0 : bj;
+                    if (bs.gap && !none)
+                        gap = bound_gap_exact(double(bv), double(sv), __builtin_inf(), gam, bs.base[in.k0 + bj]);
+                }
             }
             if (h == 0 && ok) {
                 if (to_user) {
@@ -529,6 +608,7 @@ __global__ __launch_bounds__(256, 2) void batch_assign_mfma_kernel(const batch_i
                 } else {
                     labels[in.row0 + row] = lab;
                     if (skeys) skeys[in.row0 + row] = (uint32_t(in.index) << lbits) | uint32_t(lab);
+                    if (bs.gap) bs.gap[in.row0 + row] = gap;
                 }
             }
         }
@@ -575,12 +655,16 @@ __global__ void batch_tune_fill_kernel(float* __restrict__ p, int64_t count, uin
 }
 
 // label histogram: BATCH_CNT_ROWS rows of one instance per workgroup, added to
-// counts (when not null) and written per block to bhist (when not null)
+// counts (when not null) and written per block to bhist (when not null).  With prev
+// (the labels at the previous call, -1 before the first), the clusters whose members
+// changed are flagged and prev takes the new labels.
 __global__ __launch_bounds__(256) void batch_count_kernel(const batch_inst* __restrict__ I, int B,
                                                           const int64_t* __restrict__ pre,
                                                           const int32_t* __restrict__ labels,
                                                           int32_t* __restrict__ counts,
-                                                          int32_t* __restrict__ bhist) {
+                                                          int32_t* __restrict__ bhist,
+                                                          int32_t* __restrict__ prev,
+                                                          int32_t* __restrict__ changed) {
     __shared__ int hist[BATCH_HIST_MAX];
     const int64_t total = pre[B];
     for (int64_t b = blockIdx.x; b < total; b += gridDim.x) {
@@ -595,16 +679,22 @@ __global__ __launch_bounds__(256) void batch_count_kernel(const batch_inst* __re
         __syncthreads();
         // every label of the thread loaded before the first atomic
         constexpr int RPT = BATCH_CNT_ROWS / 256;
-        int lv[RPT];
+        int lv[RPT], pv[RPT];
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
             const int r = threadIdx.x + 256 * u;
             lv[u] = r < nr ? labels[in.row0 + r0 + r] : -1;
+            pv[u] = prev && r < nr ? prev[in.row0 + r0 + r] : -1;
         }
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
             const int lab = lv[u];
             if (lab >= 0 && lab < in.k) {
+                if (prev && lab != pv[u]) {
+                    changed[in.k0 + lab] = 1;
+                    if (pv[u] >= 0) changed[in.k0 + pv[u]] = 1;
+                    prev[in.row0 + r0 + threadIdx.x + 256 * u] = lab;
+                }
                 if (lds) atomicAdd(&hist[lab], 1);
                 else atomicAdd(&counts[in.k0 + lab], 1);
             }
@@ -673,7 +763,8 @@ __global__ __launch_bounds__(256) void label_hist_kernel(const int32_t* __restri
 //    slot in the block's label-ordered LDS staging array, and the staging array
 //    is written out in slot order, so each label's rows of the block leave as
 //    one contiguous run.  Labels outside [0, k) are skipped, as the histogram
-//    skips them.
+//    skips them; with changed, so are the clusters whose members did not change
+//    (nobody reads their runs).
 // ---------------------------------------------------------------------------
 // One large instance (the single-instance engine): its block destinations in
 // two parallel steps instead of batch_scan_kernel's per-label walk over every
@@ -756,18 +847,22 @@ __global__ __launch_bounds__(256) void batch_scatter_kernel(const batch_inst* __
     int32_t* wc = slds + wave * kcap;
     const uint64_t below = (uint64_t(1) << lane) - 1u;
     const int64_t total = pre[B];
-    if (changed) {
-        for (int w = t; w * 32 < kcap; w += 256) {
-            uint32_t m = 0;
-            for (int e = 0; e < 32 && w * 32 + e < kcap; ++e) m |= (changed[w * 32 + e] ? 1u : 0u) << e;
-            cbits[w] = m;
-        }
-        __syncthreads();
-    }
+    int held = -1;  // the instance whose flags cbits holds
     for (int64_t b = blockIdx.x; b < total; b += gridDim.x) {
         const int ii = batch_find(pre, B, b);
         const batch_inst in = I[ii];
         const int k = in.k;
+        if (changed && ii != held) {
+            __syncthreads();
+            const int32_t* chg = changed + in.k0;
+            for (int w = t; w * 32 < k; w += 256) {
+                uint32_t m = 0;
+                for (int e = 0; e < 32 && w * 32 + e < k; ++e) m |= (chg[w * 32 + e] ? 1u : 0u) << e;
+                cbits[w] = m;
+            }
+            __syncthreads();
+            held = ii;
+        }
         const int64_t lb = b - pre[ii];
         const int64_t r0 = lb * BATCH_CNT_ROWS;
         const int nr = int(min<int64_t>(BATCH_CNT_ROWS, in.n - r0));
@@ -888,7 +983,8 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
                                                           int32_t* __restrict__ meta,
                                                           int64_t* __restrict__ qpre,
                                                           int64_t* __restrict__ dpre,
-                                                          uint32_t* __restrict__ ticket) {
+                                                          uint32_t* __restrict__ ticket,
+                                                          const int32_t* __restrict__ changed) {
     __shared__ int64_t s_off[1024];
     __shared__ int32_t sums[3][16];
     __shared__ int32_t last[3];
@@ -923,7 +1019,8 @@ __global__ __launch_bounds__(1024) void batch_scan_kernel(const batch_inst* __re
                     c = cnt[j];
                 }
             }
-            const int32_t nchk = (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK;
+            // a cluster whose members did not change has no chunks (it keeps its centroid)
+            const int32_t nchk = !changed || (j < k && changed[in.k0 + j]) ? (c + REDUCE_CHUNK - 1) / REDUCE_CHUNK : 0;
             int32_t so = c, sc = nchk, se = (j < k && c == 0) ? 1 : 0;
             scan3_1024(so, sc, se, sums);
             if (j < k) {
@@ -1041,7 +1138,7 @@ __global__ __launch_bounds__(256) void batch_reduce_vec_kernel(const batch_inst*
         int ii = batch_find(qpre, B, q0);
         int64_t q = q0;
         while (q < q1) {
-            while (q >= qpre[ii + 1]) ++ii;  // every instance has chunks
+            while (q >= qpre[ii + 1]) ++ii;  // instances without chunks are passed over
             const batch_inst in = I[ii];
             const int64_t inst_end = min<int64_t>(q1, qpre[ii + 1]);
             const int d = in.d;
@@ -1158,7 +1255,7 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(const batch_inst* __r
         int ii = batch_find(qpre, B, q0);
         int j = -1;
         for (int64_t q = q0; q < q1; ++q) {
-            while (q >= qpre[ii + 1]) {  // next instance (every instance has chunks)
+            while (q >= qpre[ii + 1]) {  // next instance (those without chunks are passed over)
                 ++ii;
                 j = -1;
             }
@@ -1253,6 +1350,8 @@ __global__ __launch_bounds__(256) void batch_finalize_kernel(const batch_inst* _
                                                              const int32_t* __restrict__ counts,
                                                              const int32_t* __restrict__ chunk_base,
                                                              const double* __restrict__ part,
+                                                             const int32_t* __restrict__ changed,
+                                                             const float* __restrict__ Ccur,
                                                              float* __restrict__ Cnext) {
     const int64_t total = pre[B];
     for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
@@ -1263,6 +1362,10 @@ __global__ __launch_bounds__(256) void batch_finalize_kernel(const batch_inst* _
         const int j = int(le / in.d), f = int(le - int64_t(j) * in.d);
         const int32_t cnt = counts[in.k0 + j];
         if (cnt == 0) continue;
+        if (changed && !changed[in.k0 + j]) {  // the same members: the same bits
+            Cnext[in.c0 + le] = Ccur[in.c0 + le];
+            continue;
+        }
         const int32_t* cb = chunk_base + in.k0 + ii;
         const double* pp = part + in.p0;
         double s = 0.0;
@@ -1422,6 +1525,116 @@ __global__ __launch_bounds__(1024) void batch_fill_empty_kernel(const batch_inst
             pd = wd;
             pr = wr;
         }
+    }
+}
+
+// Bounds of one instance per workgroup after its centroids have moved: drift_j =
+// ||Cnext_j - Ccur_j|| (one wave per centroid), its maximum, base_j advanced by (drift_j + max drift)(1 + g) and the changed
+// flags cleared (km_step.hpp does the same for one instance).
+__global__ __launch_bounds__(1024) void batch_bound_kernel(const batch_inst* __restrict__ I, int B,
+                                                          const float* __restrict__ Ccur,
+                                                          const float* __restrict__ Cnext,
+                                                          double* __restrict__ drift, double* __restrict__ base,
+                                                          int32_t* __restrict__ changed,
+                                                          int32_t* __restrict__ count) {
+    __shared__ unsigned long long wmax[16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    for (int ii = blockIdx.x; ii < B; ii += gridDim.x) {
+        const batch_inst in = I[ii];
+        unsigned long long mx = 0;
+        for (int j = wave; j < in.k; j += 16) {
+            const float* a = Cnext + in.c0 + int64_t(j) * in.d;
+            const float* o = Ccur + in.c0 + int64_t(j) * in.d;
+            double s = 0.0;
+            for (int f = lane; f < in.d; f += 64) {
+                const double v = double(a[f]) - double(o[f]);
+                s = fma(v, v, s);
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+            const double r = sqrt(s) * (1.0 + 1e-12);
+            if (lane == 0) drift[in.k0 + j] = r;
+            mx = max(mx, (unsigned long long)__double_as_longlong(r));
+        }
+        if (lane == 0) wmax[wave] = mx;
+        __syncthreads();
+        for (int w = 0; w < 16; ++w) mx = max(mx, wmax[w]);
+        const double top = __longlong_as_double((long long)mx);
+        const double gam = batch_gam(in.d);
+        for (int j = t; j < in.k; j += 1024) {
+            const double v = (base[in.k0 + j] + (drift[in.k0 + j] + top) * (1.0 + gam)) * (1.0 + 1e-15);
+            base[in.k0 + j] = v < BOUND_MAX ? v : __builtin_inf();
+            changed[in.k0 + j] = 0;
+        }
+        if (t == 0) count[in.index] = 0;
+        __syncthreads();
+    }
+}
+
+// the open rows of every instance (bound_select_kernel): BATCH_CNT_ROWS rows of one
+// instance per workgroup
+__global__ __launch_bounds__(256) void batch_select_kernel(const batch_inst* __restrict__ I, int B,
+                                                           const int64_t* __restrict__ pre,
+                                                           const int32_t* __restrict__ labels,
+                                                           const float* __restrict__ gap,
+                                                           const double* __restrict__ base,
+                                                           int32_t* __restrict__ rows,
+                                                           int32_t* __restrict__ count) {
+    constexpr int U = BATCH_CNT_ROWS / 256;
+    __shared__ int wtot[4];
+    __shared__ int first;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t below = (uint64_t(1) << lane) - 1u;
+    const int64_t total = pre[B];
+    for (int64_t b = blockIdx.x; b < total; b += gridDim.x) {
+        const int ii = batch_find(pre, B, b);
+        const batch_inst in = I[ii];
+        const int64_t r0 = (b - pre[ii]) * BATCH_CNT_ROWS + int64_t(wave) * (BATCH_CNT_ROWS / 4) + lane;
+        int lab[U];
+        float g[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t r = r0 + 64 * u;
+            lab[u] = r < in.n ? labels[in.row0 + r] : 0;
+            g[u] = r < in.n ? gap[in.row0 + r] : 0.f;
+        }
+        uint64_t open[U];
+        int mine = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool settled = double(g[u]) > base[in.k0 + lab[u]] + BOUND_SLACK;
+            open[u] = __ballot(r0 + 64 * u < in.n && !settled);
+            mine += __popcll(open[u]);
+        }
+        if (lane == 0) wtot[wave] = mine;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int sum = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+            first = sum ? atomicAdd(&count[in.index], sum) : 0;
+        }
+        __syncthreads();
+        int at = first;
+        for (int w = 0; w < wave; ++w) at += wtot[w];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if ((open[u] >> lane) & 1u) rows[in.row0 + at + __popcll(open[u] & below)] = int32_t(r0 + 64 * u);
+            at += __popcll(open[u]);
+        }
+        __syncthreads();  // wtot and first are rewritten by the next block
+    }
+}
+
+// concatenated labels to every instance's output
+__global__ __launch_bounds__(256) void batch_labels_out_kernel(const batch_inst* __restrict__ I, int B,
+                                                               const int64_t* __restrict__ pre,
+                                                               const int32_t* __restrict__ labels) {
+    const int64_t total = pre[B];
+    for (int64_t b = blockIdx.x; b < total; b += gridDim.x) {
+        const int ii = batch_find(pre, B, b);
+        const batch_inst in = I[ii];
+        const int64_t r0 = (b - pre[ii]) * BATCH_CNT_ROWS;
+        const int64_t r1 = min<int64_t>(in.n, r0 + BATCH_CNT_ROWS);
+        for (int64_t r = r0 + threadIdx.x; r < r1; r += 256) in.labels_out[r] = labels[in.row0 + r];
     }
 }
 

@@ -98,9 +98,10 @@ struct dbuf {
 // per-row, per-cluster and per-chunk arrays, sort scratch
 struct batch_ws {
     dbuf inst, pre, labels, keys, perm, d64, ccur, cnext, counts, offsets, cb, empty, meta, qpre,
-        part, objc, obj, sort_tmp, asel, apre, bhist, ticket;
+        part, objc, obj, sort_tmp, asel, apre, bhist, ticket, prev, changed, gap, rows, count, base, drift;
     void release() {
-        dbuf* all[] = {&inst, &pre,  &labels, &keys, &perm,     &d64,  &ccur, &cnext, &counts, &offsets, &cb,
+        dbuf* all[] = {&prev, &changed, &gap, &rows, &count, &base, &drift,
+                       &inst, &pre,  &labels, &keys, &perm,     &d64,  &ccur, &cnext, &counts, &offsets, &cb,
                        &empty, &meta, &qpre,  &part, &objc, &obj, &sort_tmp, &asel, &apre, &bhist, &ticket};
         for (dbuf* b : all) b->release();
     }
@@ -1483,6 +1484,15 @@ struct batch_plan {
     double* part = nullptr;
     double* objc = nullptr;
     double* objd = nullptr;
+    // bounds (km_bounds.hpp), kept when enough iterations follow
+    bool bounds = false;
+    int32_t* prev = nullptr;
+    int32_t* changed = nullptr;
+    double* drift = nullptr;
+    int32_t* rows_open = nullptr;
+    int32_t* count_open = nullptr;
+    double* base = nullptr;
+    batch_select sel{nullptr, nullptr, nullptr, nullptr};
     void* tmp = nullptr;
     size_t tmp_bytes = 0;
 
@@ -1656,8 +1666,23 @@ static int batch_grid(const km_ctx* ctx, int64_t items) {
 
 // Device workspace of the plan and the table upload (stream-ordered: the host
 // tables must stay alive until the stream has passed the copies).
-static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p) {
+static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p, int64_t iterations = 0) {
     const int B = p.B;
+    // Bounds pay from the fourth iteration on, when most rows are certain; fewer
+    // iterations would only add their two launches each
+    p.bounds = p.train && p.csort && iterations >= 5;
+    if (p.bounds) {
+        p.prev = ws.prev.get<int32_t>(p.rows);
+        fill<int32_t>(ctx, p.prev, p.rows, -1);
+        p.changed = ws.changed.get<int32_t>(p.kk);
+        fill<int32_t>(ctx, p.changed, p.kk, 0);
+        p.base = ws.base.get<double>(p.kk);
+        fill<double>(ctx, p.base, p.kk, 0.0);
+        p.drift = ws.drift.get<double>(p.kk);
+        p.rows_open = ws.rows.get<int32_t>(p.rows);
+        p.count_open = ws.count.get<int32_t>(B);
+        p.sel = {nullptr, nullptr, ws.gap.get<float>(p.rows), p.base};
+    }
     p.dI = ws.inst.get<batch_inst>(B);
     p.dpre = ws.pre.get<int64_t>(p.pre.size());
     p.Ccur = ws.ccur.get<float>(p.cfl);
@@ -1715,18 +1740,23 @@ static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p) {
 }
 
 // exact assignment of every instance of the plan, one launch per tile variant in use
-static void plan_assign(km_ctx* ctx, const batch_plan& p, int32_t* labels, uint32_t* skeys, int to_user) {
+static void plan_assign(km_ctx* ctx, const batch_plan& p, int32_t* labels, uint32_t* skeys, int to_user,
+                        const batch_select& bs) {
     for (const batch_plan::asg_launch& L : p.launches) {
         const dim3 grid(batch_grid(ctx, L.batches)), block(256);
         const int32_t* sel = p.d_asel + L.sel_off;
         const int64_t* pre = p.d_apre + L.pre_off;
         const int lb = int(p.lbits);
 #define KM_BATCH_ASSIGN(CT, RW)                                                                      \
-    hipLaunchKernelGGL((batch_assign_kernel<CT, RW>), grid, block, 0, ctx->stream, p.dI, sel, L.nsel, pre, \
-                       p.Ccur, labels, skeys, lb, to_user)
+    if (bs.gap)                                                                                      \
+        hipLaunchKernelGGL((batch_assign_kernel<CT, RW, true>), grid, block, 0, ctx->stream, p.dI, sel, L.nsel, pre, \
+                           p.Ccur, labels, skeys, lb, to_user, bs);                                  \
+    else                                                                                             \
+        hipLaunchKernelGGL((batch_assign_kernel<CT, RW, false>), grid, block, 0, ctx->stream, p.dI, sel, L.nsel, \
+                           pre, p.Ccur, labels, skeys, lb, to_user, bs)
 #define KM_BATCH_MFMA(DP)                                                                          \
     hipLaunchKernelGGL((batch_assign_mfma_kernel<DP>), grid, block, batch_mfma_lds_bytes(DP), ctx->stream, \
-                       p.dI, sel, L.nsel, pre, L.rows, p.Ccur, labels, skeys, lb, to_user)
+                       p.dI, sel, L.nsel, pre, L.rows, p.Ccur, labels, skeys, lb, to_user, bs)
         switch (L.v) {
             case 0: KM_BATCH_ASSIGN(64, 8); break;
             case 1: KM_BATCH_ASSIGN(64, 4); break;
@@ -1764,23 +1794,23 @@ static void plan_iteration(km_ctx* ctx, batch_plan& p, hipEvent_t asg_start = nu
     const int cap = ctx->cu_count * 8;
     auto g = [&](int64_t items) { return batch_grid(ctx, items); };
     if (asg_start) KM_HIP(hipEventRecord(asg_start, ctx->stream));
-    plan_assign(ctx, p, p.labels, p.csort ? nullptr : p.skeys, 0);
+    plan_assign(ctx, p, p.labels, p.csort ? nullptr : p.skeys, 0, p.sel);
     if (asg_end) KM_HIP(hipEventRecord(asg_end, ctx->stream));
     if (!p.csort) fill<int32_t>(ctx, p.counts, p.kk, 0);
     // counting sort: per-block histograms only (the scan sums them into the counts)
     hipLaunchKernelGGL(batch_count_kernel, dim3(g(p.P(BP::P_CNT, B))), dim3(256), 0, ctx->stream, p.dI, B,
                        p.DP(BP::P_CNT), p.labels, p.csort ? (int32_t*)nullptr : p.counts,
-                       p.csort ? p.bhist : (int32_t*)nullptr);
+                       p.csort ? p.bhist : (int32_t*)nullptr, p.prev, p.changed);
     KM_LAUNCH_CHECK();
     hipLaunchKernelGGL(batch_scan_kernel, dim3(g(B)), dim3(1024), 0, ctx->stream, p.dI, B, p.counts,
                        p.csort ? p.bhist : (int32_t*)nullptr, p.offsets, p.cb, p.empty, p.meta, p.qpre,
-                       p.d64pre, p.ticket);
+                       p.d64pre, p.ticket, p.changed);
     KM_LAUNCH_CHECK();
     if (p.csort) {
         hipLaunchKernelGGL(batch_scatter_kernel, dim3(g(p.P(BP::P_CNT, B))), dim3(256),
                            batch_scatter_lds_bytes(p.maxk),
                            ctx->stream, p.dI, B, p.DP(BP::P_CNT), p.labels, p.bhist, p.perm, p.maxk,
-                           (const int32_t*)nullptr);
+                           p.changed);
         KM_LAUNCH_CHECK();
     } else {
         rocprim::counting_iterator<int32_t> ids(0);
@@ -1804,7 +1834,7 @@ static void plan_iteration(km_ctx* ctx, batch_plan& p, hipEvent_t asg_start = nu
         KM_LAUNCH_CHECK();
     }
     hipLaunchKernelGGL(batch_finalize_kernel, dim3(g((p.P(BP::P_EL, B) + 255) / 256)), dim3(256), 0,
-                       ctx->stream, p.dI, B, p.DP(BP::P_EL), p.counts, p.cb, p.part, p.Cnext);
+                       ctx->stream, p.dI, B, p.DP(BP::P_EL), p.counts, p.cb, p.part, p.changed, p.Ccur, p.Cnext);
     KM_LAUNCH_CHECK();
     // blocks of the instances with empty clusters only (the scan's prefix)
     hipLaunchKernelGGL(batch_d64_kernel, dim3(g(p.P(BP::P_D64, B))), dim3(256), 0, ctx->stream, p.dI, B,
@@ -1813,6 +1843,16 @@ static void plan_iteration(km_ctx* ctx, batch_plan& p, hipEvent_t asg_start = nu
     hipLaunchKernelGGL(batch_fill_empty_kernel, dim3(g(B)), dim3(1024), 0, ctx->stream, p.dI, B, p.meta,
                        p.empty, p.d64, p.Ccur, p.Cnext);
     KM_LAUNCH_CHECK();
+    if (p.bounds) {
+        hipLaunchKernelGGL(batch_bound_kernel, dim3(g(B)), dim3(1024), 0, ctx->stream, p.dI, B, p.Ccur, p.Cnext,
+                           p.drift, p.base, p.changed, p.count_open);
+        KM_LAUNCH_CHECK();
+        hipLaunchKernelGGL(batch_select_kernel, dim3(g(p.P(BP::P_CNT, B))), dim3(256), 0, ctx->stream, p.dI, B,
+                           p.DP(BP::P_CNT), p.labels, p.sel.gap, p.base, p.rows_open, p.count_open);
+        KM_LAUNCH_CHECK();
+        p.sel.rows = p.rows_open;
+        p.sel.count = p.count_open;
+    }
     // every centroid of Cnext is written (finalize: counted clusters; fill:
     // empty ones): the next iteration reads it, and this one's input becomes
     // the next output buffer
@@ -1825,7 +1865,14 @@ static void plan_finish(km_ctx* ctx, const batch_plan& p) {
     using BP = batch_plan;
     const int B = p.B;
     auto g = [&](int64_t items) { return batch_grid(ctx, items); };
-    plan_assign(ctx, p, nullptr, nullptr, 1);
+    if (p.sel.rows) {  // after iterations with bounds: the open rows, then every label out
+        plan_assign(ctx, p, p.labels, nullptr, 0, p.sel);
+        hipLaunchKernelGGL(batch_labels_out_kernel, dim3(g(p.P(BP::P_CNT, B))), dim3(256), 0, ctx->stream, p.dI, B,
+                           p.DP(BP::P_CNT), p.labels);
+        KM_LAUNCH_CHECK();
+    } else {
+        plan_assign(ctx, p, nullptr, nullptr, 1, {nullptr, nullptr, nullptr, nullptr});
+    }
     // every row's d64 (against its final label), then the chunk sums in order
     hipLaunchKernelGGL(batch_d64_kernel, dim3(g(p.P(BP::P_D64, B))), dim3(256), 0, ctx->stream, p.dI, B,
                        p.DP(BP::P_D64), (const int32_t*)nullptr, p.Ccur, (const int32_t*)nullptr, p.d64);
@@ -1848,7 +1895,7 @@ static void batch_train(km_ctx* ctx, const km_batch_instance_f32* inst, int64_t 
     batch_plan p;
     plan_build(p, ctx, inst, count, true);
     ctx->stats = km_stats{};
-    plan_upload(ctx, ctx->bws, p);
+    plan_upload(ctx, ctx->bws, p, max_iter);
     KM_HIP(hipStreamSynchronize(ctx->stream));  // the host tables may be released from here on
     plan_copy_centroids(ctx, p, 0);
 
@@ -2029,11 +2076,11 @@ static void batch_autotune(km_ctx* ctx, int32_t* table_out, int64_t table_len) {
                 plan_build(p, ctx, q.data(), NI, false);
                 plan_upload(ctx, ctx->bws_fin, p);
                 plan_copy_centroids(ctx, p, 0);
-                plan_assign(ctx, p, nullptr, nullptr, 1);  // warm-up
+                plan_assign(ctx, p, nullptr, nullptr, 1, p.sel);  // warm-up
                 float ms_v = std::numeric_limits<float>::infinity();
                 for (int rep = 0; rep < 3; ++rep) {
                     KM_HIP(hipEventRecord(e0, ctx->stream));
-                    plan_assign(ctx, p, nullptr, nullptr, 1);
+                    plan_assign(ctx, p, nullptr, nullptr, 1, p.sel);
                     KM_HIP(hipEventRecord(e1, ctx->stream));
                     KM_HIP(hipEventSynchronize(e1));
                     float ms = 0.f;
