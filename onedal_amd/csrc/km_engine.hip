@@ -37,6 +37,7 @@
 #include "km_assign.hpp"
 #include "km_assign_bf16.hpp"
 #include "km_assign_split.hpp"
+#include "km_assign_wide.hpp"
 #include "km_batch.hpp"
 #include "km_bounds.hpp"
 #include "km_common.hpp"
@@ -238,6 +239,11 @@ struct work {
     bool split = false;
     uint16_t* Csp = nullptr;  // bf16_padded_k(k) x 2 dpad
     uint16_t* cnp = nullptr;  // bf16_padded_k(k) x 16
+    // wide rows (path 2, float, d > 128): both halves chunk by chunk, kpw rows, and norms
+    bool wide = false;
+    int nwc = 0, kpw = 0;
+    uint16_t* Cw = nullptr;
+    float* cnw = nullptr;
     // rows of the next assignment pass, and where their bounds go
     row_select sel{nullptr, nullptr, nullptr, nullptr, 0.0};
     // training: centroid movement and bounds per cluster, changed clusters, the open
@@ -258,13 +264,14 @@ static int pad_dim(int d) {
     return p;
 }
 
-// 1 generic tile kernel, 2 matrix cores of the data's precision (FP32 or FP64),
-// 3 BF16 matrix cores + exact re-score.  BF16 applies to float data with
-// d <= 256; double data takes path 2 for d <= 256, else path 1.
+// 1 generic tile kernel, 2 matrix cores with the precision of the data's (float:
+// split BF16 products, or FP32), 3 BF16 matrix cores + exact re-score.  BF16 applies to
+// float data with d <= 256; double data takes path 2 for d <= 256, else path 1; float
+// data takes path 1 past 256 columns and the limits of use_wide, or when asked to.
 template <typename F>
 static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
     if (std::is_same<F, double>::value) return (d <= 256 && ctx->assign_path_opt != 1) ? 2 : 1;
-    if (d > 256) return 1;
+    if (d > 256) return ctx->assign_path_opt == 1 || k > SPLIT_MAX_K ? 1 : 2;
     // keys carry (block, register) in at most 15 low bits: k <= 65536
     if ((flags & KM_FLAG_BF16_REFINE) && k <= 65536) return 3;
     if (ctx->assign_path_opt == 1) return 1;
@@ -278,6 +285,14 @@ static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
 static bool use_split(int path, int d, int k, bool once) {
     return (path == 2 || (path == 3 && once)) && d <= 128 && k <= SPLIT_MAX_K;
 }
+
+// float data on path 2 with wider rows: split products in chunks (km_assign_wide.hpp).
+// From the first width past the split kernel's row registers and for any n and k: a call
+// on (n, d, k) took (500, 300, 5) 134 -> 96 us, (2000, 129, 3) 91 -> 66, (1e6, 300, 5)
+// 1463 -> 459, (1e5, 130, 2000) 2084 -> 1056, (2e4, 4000, 50) 1431 -> 965 (the whole
+// inference call, which other kernels made faster as well).
+static bool use_wide(int path, int d, int k) { return path == 2 && d > 128 && k <= SPLIT_MAX_K; }
+static int wide_columns(int k) { return k <= 128 ? 2 : 4; }  // waves across the centroids
 
 template <typename F>
 static band_consts make_band(int d) {
@@ -328,10 +343,12 @@ static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* col
     s.d = w.d;
     s.dpad = w.dpad;
     s.cn = w.cn;
-    s.cpad = path == 2 && !w.split ? w.cpad : nullptr;
+    s.cpad = path == 2 && !w.split && !w.wide ? w.cpad : nullptr;
     s.Csp = w.Csp;
     s.cnp = w.cnp;
-    s.kp = w.split ? bf16_padded_k(w.k) : w.k;
+    s.Cw = w.Cw;
+    s.cnw = w.cnw;
+    s.kp = w.split ? bf16_padded_k(w.k) : w.wide ? w.kpw : w.k;
     s.maxima = w.maxima;
     s.drift = w.drift;
     s.base = w.base;
@@ -400,6 +417,16 @@ static split_consts make_split_consts(int d, int k) {
     return c;
 }
 
+static split_consts make_wide_consts(int d, int k, int kp) {
+    split_consts c = make_split_consts<3>(d, k);
+    int mbits = 0;
+    while ((1 << mbits) < kp / 32) mbits++;
+    c.ib = 4 + mbits;
+    c.trunc = float(std::ldexp(1.0, c.ib - 23));
+    c.xc = float(std::ldexp(6.02, -18) + gamma_m(3.0 * d, fp_traits<float>::u_acc) * 2.04);
+    return c;
+}
+
 // terms 3, or 1 (BF16 distances of rows assigned once); sel: the rows
 template <int DP, int NB, int TERMS>
 static void launch_split(km_ctx* ctx, work<float>& w, const row_select& sel) {
@@ -421,6 +448,18 @@ static void launch_split(km_ctx* ctx, work<float>& w, const row_select& sel) {
         case 64: launch_split<64, 2, TERMS>(ctx, w, sel); break;
         default: launch_split<128, TERMS == 3 ? 1 : 2, TERMS>(ctx, w, sel); break;
     }
+}
+
+template <int NWC>
+static void launch_wide(km_ctx* ctx, work<float>& w) {
+    const int64_t tiles = (w.n + WIDE_ROWS - 1) / WIDE_ROWS;
+    const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * (NWC == 2 ? 2 : 1))));
+    const size_t lds = wide_lds_bytes(NWC);
+    auto kern = assign_wide_kernel<NWC>;
+    KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(128 * NWC), lds, ctx->stream, w.X, w.n, w.d, w.Cw, w.cnw, w.k, w.kpw,
+                       w.maxima, make_wide_consts(w.d, w.k, w.kpw), w.labels, w.L, w.sel);
+    KM_LAUNCH_CHECK();
 }
 
 template <int DP, int NB>
@@ -512,6 +551,9 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
             launch_split<3>(ctx, w, {w.L.coll_rows, w.L.counters + 2, nullptr, nullptr, 0.0});
         } else if (w.split) {
             launch_split<3>(ctx, w, w.sel);
+        } else if (w.wide) {
+            if (w.nwc == 2) launch_wide<2>(ctx, w);
+            else launch_wide<4>(ctx, w);
         } else if (path == 2) {
             switch (w.dpad) {
                 case 32: launch_mfma_f32<32, 2>(ctx, w, bc); break;
@@ -833,9 +875,10 @@ static int32_t* launch_empty_clusters(km_ctx* ctx, const F* X, int64_t n, int d,
 
 template <typename F>
 static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, int k,
-                       int path, bool once, arena* A = nullptr, int32_t* labels_into = nullptr) {
+                       int path, bool once, arena* A = nullptr, int32_t* labels_into = nullptr, bool wide = true) {
     w.split = std::is_same<F, float>::value && use_split(path, d, k, once);
-    const bool vec_view = path == 2 && !w.split;
+    w.wide = std::is_same<F, float>::value && wide && use_wide(path, d, k);
+    const bool vec_view = path == 2 && !w.split && !w.wide;
     w.n = n;
     w.d = d;
     w.k = k;
@@ -853,6 +896,11 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
     if (w.split) {
         w.Csp = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(bf16_padded_k(k)) * 2 * w.dpad);
         w.cnp = take<uint16_t>(ctx, &km_ctx::c_pieces, A, int64_t(bf16_padded_k(k)) * 16);
+    } else if (w.wide) {
+        w.nwc = wide_columns(k);
+        w.kpw = wide_kp(k, w.nwc);
+        w.Cw = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(w.kpw) * wide_chunks(d) * 64);
+        w.cnw = take<float>(ctx, &km_ctx::c_pieces, A, w.kpw);
     } else {
         w.cpad = take<F>(ctx, &km_ctx::cpad, A, int64_t(k) * w.dpad);
     }
@@ -873,6 +921,7 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
         if (path == 3) w.L.coll_rows = take<int32_t>(ctx, &km_ctx::coll_rows, A, n);
         return;
     }
+    if (w.wide) return;
     const int grid = grid_for(ctx, n * 64, 256, 8);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
@@ -1094,13 +1143,14 @@ constexpr int64_t NOALLOC_SLACK = 16384;  // alignment of the arena's pieces
 // objective chunks); the arena itself refuses anything beyond its end
 template <typename F>
 static size_t noalloc_block_bytes(const km_ctx* ctx, int path, int64_t R, int d, int k, bool pad_x,
-                                  bool want_obj) {
+                                  bool want_obj, bool wide) {
     const int64_t dpad = pad_dim(d);
     int64_t b = R * (4 + 4 + 4 + 4 * int64_t(MAXC) + 4) + 16 + int64_t(sizeof(F)) * k +
-                int64_t(sizeof(F)) * k * dpad + 32;
+                (wide ? int64_t(wide_kp(k, wide_columns(k))) * (wide_chunks(d) * 128 + 4) : int64_t(sizeof(F)) * k * dpad) +
+                32;
     const bool split = use_split(path, d, k, true);
     if (split) b += 36 * int64_t(bf16_padded_k(k)) + 4 * int64_t(bf16_padded_k(k) - k) * dpad;
-    if (path == 2 && !split && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
+    if (path == 2 && !split && !wide && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
     if (path == 3 && split) b += 4 * R;
     if (path == 3 && !split) {
         const int64_t kp = bf16_padded_k(k);
@@ -1126,20 +1176,25 @@ static void infer_noalloc(km_ctx* ctx, const float* X, int64_t n, int64_t d64_, 
         throw status_error(KM_INTERNAL_ERROR,
                            "the fixed scratch buffer is not available on this device: " + ctx->scratch_err);
     ctx->stats = km_stats{};
-    const int path = choose_path<F>(ctx, d, k, flags);
+    int path = choose_path<F>(ctx, d, k, flags);
     const bool want_obj = flags & KM_FLAG_EXACT_OBJECTIVE;
     const bool pad_x = (d % 4) != 0 || (reinterpret_cast<uintptr_t>(X) % 16) != 0;
     const size_t cap = NOALLOC_BYTES - 256;  // the objective accumulator sits in front
+    // the padded operand of the wide kernel, where it fits; else the older kernels (the
+    // generic one past 256 columns)
+    const int64_t least = std::min<int64_t>(n, OBJ_CHUNK);
+    const bool wide = use_wide(path, d, k) && noalloc_block_bytes<F>(ctx, path, least, d, k, pad_x, want_obj, true) <= cap;
+    if (!wide && path == 2 && d > 256) path = 1;
     // largest block: a multiple of OBJ_CHUNK rows (or all rows) that fits
     int64_t R = std::min<int64_t>(n, int64_t(1) << 22);
     R = R < n ? R / OBJ_CHUNK * OBJ_CHUNK : R;
-    while (R > OBJ_CHUNK && noalloc_block_bytes<F>(ctx, path, R, d, k, pad_x, want_obj) > cap)
+    while (R > OBJ_CHUNK && noalloc_block_bytes<F>(ctx, path, R, d, k, pad_x, want_obj, wide) > cap)
         R = (R - 1) / OBJ_CHUNK * OBJ_CHUNK;
-    if (noalloc_block_bytes<F>(ctx, path, R, d, k, pad_x, want_obj) > cap)
+    if (noalloc_block_bytes<F>(ctx, path, R, d, k, pad_x, want_obj, wide) > cap)
         throw status_error(KM_INVALID_ARGUMENT,
                            "k x d too large for km_lloyd_infer_f32_noalloc: one block of " +
                                std::to_string(R) + " rows needs " +
-                               std::to_string(noalloc_block_bytes<F>(ctx, path, R, d, k, pad_x, want_obj)) +
+                               std::to_string(noalloc_block_bytes<F>(ctx, path, R, d, k, pad_x, want_obj, wide)) +
                                " bytes of the " + std::to_string(NOALLOC_BYTES) +
                                "-byte scratch buffer");
     // no timing events here: creating one may allocate
@@ -1157,7 +1212,7 @@ static void infer_noalloc(km_ctx* ctx, const float* X, int64_t n, int64_t d64_, 
         const int64_t rows = std::min<int64_t>(R, n - r0);
         arena A{base + 256, cap, 0};
         work<F> w;
-        setup_work<F>(ctx, w, X + r0 * d, rows, d, k, path, true, &A, labels_out + r0);
+        setup_work<F>(ctx, w, X + r0 * d, rows, d, k, path, true, &A, labels_out + r0, wide);
         step_centroids<F>(ctx, w, path, const_cast<F*>(C));  // only read
         assign<F>(ctx, w, C, path);
         const uint32_t seq = next_seq(ctx);

@@ -11,6 +11,7 @@
 
 #include "km_assign_bf16.hpp"
 #include "km_assign_split.hpp"
+#include "km_assign_wide.hpp"
 #include "km_bounds.hpp"
 #include "km_common.hpp"
 #include "km_update.hpp"
@@ -37,6 +38,9 @@ struct centroid_step {
     // norm step of assign_split_kernel, kp rows
     uint16_t* Csp;
     uint16_t* cnp;
+    // or (Cw) both halves chunk by chunk for assign_wide_kernel, kp rows, and their norms
+    uint16_t* Cw;
+    float* cnw;
     int kp;
     double* maxima;  // [0] max ||c||, with Cb or Csp: [1] max ||bf16(c)||, [2] max ||c - bf16(c)||
     // BF16: value shift and start values
@@ -114,6 +118,14 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
                 o2[f] = hi;
                 o2[dpad + f] = f2bf(v - bf2f(hi));
             }
+        } else if (s.Cw) {
+            for (int f = t; f < 32 * wide_chunks(d); f += 256) {
+                const float v = f < d ? -2.0f * float(row[f]) : 0.f;
+                const uint16_t hi = f2bf(v);
+                uint16_t* o2 = s.Cw + (int64_t(f >> 5) * s.kp + j) * 64 + (f & 31);
+                o2[0] = hi;
+                o2[32] = f2bf(v - bf2f(hi));
+            }
         } else if (s.cpad) {
             for (int f = t; f < dpad; f += 256) s.cpad[int64_t(j) * dpad + f] = f < d ? row[f] : F(0);
         }
@@ -145,6 +157,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
                 const double up = 1.0 + 1e-12;
                 auto bits = [](double v) { return (unsigned long long)__double_as_longlong(v); };
                 agent_store(s.cn + j, F(sq));
+                if (s.cnw) s.cnw[j] = float(sq);
                 if (s.cnp) {
                     uint32_t hm, l;
                     split3(float(sq), hm, l);
@@ -169,6 +182,16 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
     if constexpr (BF16) {
         for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x)
             for (int f = t; f < dpad; f += 256) s.Cb[int64_t(j) * dpad + f] = 0;
+    }
+    if (s.Cw) {
+        for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x) {
+            for (int f = t; f < 32 * wide_chunks(d); f += 256) {
+                uint16_t* o2 = s.Cw + (int64_t(f >> 5) * s.kp + j) * 64 + (f & 31);
+                o2[0] = 0;
+                o2[32] = 0;
+            }
+            if (t == 0) s.cnw[j] = __uint_as_float(0x7F000000u);
+        }
     }
     if (s.Csp) {  // padding: zero rows with a norm of 2^127, which no threshold reaches
         for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x) {
