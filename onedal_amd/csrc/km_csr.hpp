@@ -7,7 +7,7 @@
 //   assign_clusters (sparse gemm, select, complete_closest_distances)
 //                                   :118-187  -> csr_assign_kernel
 //   calc_objective_function         :193-203  -> csr_objective_chunks_kernel
-//   update_centroids (local atomics):219-322  -> csr_chunk_sums_kernel + finalize_centroids_kernel
+//   update_centroids (local atomics):219-322  -> csr_chunk_sums_kernel + centroid_step_kernel
 //   copy_candidates_from_data       empty_cluster_handling_dpc.cpp:152-189 -> csr_fill_empty_kernel
 //
 // Arithmetic (fixed order, so results are identical run to run and equal to the
@@ -25,70 +25,130 @@
 // one in stored order (sums) or overwrite in stored order (empty-cluster fill).
 #pragma once
 
+#include <type_traits>
+
+#include "km_bounds.hpp"
 #include "km_common.hpp"
 
 namespace km {
 
+// A workgroup's 256 rows, one per thread, walked through LDS: the rows' entries [lo, hi) are
+// one run of memory, read CSR_WINDOW at a time by all threads (stage(e, p): entry p to
+// slot e), then each thread takes its row's part [x, y) of the window (use), in stored
+// order.  A thread reading its own row from memory touches a line per entry and lane:
+// n=1e6, 20 entries a row, the three kernels that do this took 144, 90 and 124 us,
+// now 36, 66 and 82 us.
+constexpr int CSR_WINDOW = 4096;
+template <typename Stage, typename Use>
+__device__ __forceinline__ void csr_walk(int64_t lo, int64_t hi, int64_t o0, int64_t o1, Stage stage, Use use) {
+    for (int64_t w0 = lo; w0 < hi; w0 += CSR_WINDOW) {
+        const int cnt = int(min<int64_t>(CSR_WINDOW, hi - w0));
+        __syncthreads();  // the previous window's readers are done
+#pragma unroll 4
+        for (int e = threadIdx.x; e < cnt; e += 256) stage(e, w0 + e);
+        __syncthreads();
+        const int x = int(max(o0, w0) - w0);
+        const int y = int(min<int64_t>(o1 - w0, cnt));
+        if (x < y) use(x, y);
+    }
+}
+
 // Structure check: row offsets non-decreasing from `base` to base + nnz, every
-// column index in [base, base + d).  Each thread reads a row's entries only after
-// its own offsets passed the check.  flag bit 1: bad offsets, bit 2: bad column,
+// column index in [base, base + d).  A workgroup reads its rows' entries only after
+// all their offsets passed the check.  flag bit 1: bad offsets, bit 2: bad column,
 // bit 4: a row whose column indices do not increase strictly (unsorted or
-// repeated; allowed, reported for the initialisation's feature-order walk).
+// repeated; allowed, reported for the initialisation's feature-order walk and for
+// the assignment's bounds).
 __global__ __launch_bounds__(256) void csr_check_kernel(const int64_t* __restrict__ cols,
                                                         const int64_t* __restrict__ offs,
                                                         int64_t base, int64_t n, int64_t d,
                                                         int64_t nnz, int32_t* __restrict__ flag) {
-    for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * blockDim.x) {
-        const int64_t o0 = offs[i] - base, o1 = offs[i + 1] - base;
-        bool ok = o0 >= 0 && o1 >= o0 && o1 <= nnz;
-        if (i == 0 && o0 != 0) ok = false;
-        if (i == n - 1 && o1 != nnz) ok = false;
-        if (!ok) {
-            atomicOr(flag, 1);
-            continue;
+    __shared__ int32_t sc[CSR_WINDOW];
+    for (int64_t r0 = blockIdx.x * int64_t(256); r0 < n; r0 += int64_t(gridDim.x) * 256) {
+        const int64_t i = r0 + threadIdx.x;
+        int64_t o0 = 0, o1 = 0;
+        bool ok = true;
+        if (i < n) {
+            o0 = offs[i] - base;
+            o1 = offs[i + 1] - base;
+            ok = o0 >= 0 && o1 >= o0 && o1 <= nnz;
+            if (i == 0 && o0 != 0) ok = false;
+            if (i == n - 1 && o1 != nnz) ok = false;
+            if (!ok) atomicOr(flag, 1);
         }
-        int64_t prev = -1;
-        bool inc = true;
-        for (int64_t p = o0; p < o1; ++p) {
-            const int64_t c = cols[p] - base;
-            if (c < 0 || c >= d) {
-                atomicOr(flag, 2);
-                break;
-            }
-            inc = inc && c > prev;
-            prev = c;
-        }
+        if (!__syncthreads_and(ok)) continue;
+        int prev = -1;
+        bool inc = true, in = true;
+        csr_walk(
+            offs[r0] - base, offs[min(r0 + 256, n)] - base, o0, o1,
+            [&](int e, int64_t p) {
+                const int64_t c = cols[p] - base;
+                in = in && c >= 0 && c < d;
+                sc[e] = int32_t(c);
+            },
+            [&](int x, int y) {
+                for (int p = x; p < y; ++p) {
+                    const int c = sc[p];
+                    inc = inc && c > prev;
+                    prev = c;
+                }
+            });
+        if (!in) atomicOr(flag, 2);
         if (!inc) atomicOr(flag, 4);
     }
 }
 
-// xs_i: squares of a row's stored entries, summed in stored order
+// xs_i: squares of a row's stored entries, summed in stored order; and (when given) the
+// bits of the largest as a double (a NaN wins)
 template <typename F>
 __global__ __launch_bounds__(256) void csr_row_squares_kernel(const F* __restrict__ vals,
                                                               const int64_t* __restrict__ offs,
                                                               int64_t base, int64_t n,
-                                                              F* __restrict__ xs) {
-    for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * blockDim.x) {
-        const int64_t o0 = offs[i] - base, o1 = offs[i + 1] - base;
+                                                              F* __restrict__ xs,
+                                                              unsigned long long* __restrict__ xmax) {
+    __shared__ F sv[CSR_WINDOW];
+    unsigned long long top = 0ull;
+    for (int64_t r0 = blockIdx.x * int64_t(256); r0 < n; r0 += int64_t(gridDim.x) * 256) {
+        const int64_t i = r0 + threadIdx.x;
+        const int64_t o0 = i < n ? offs[i] - base : 0, o1 = i < n ? offs[i + 1] - base : 0;
         F acc(0);
-        for (int64_t p = o0; p < o1; ++p) {
-            const F v = vals[p];
-            const F sq = v * v;
-            acc = acc + sq;
+        csr_walk(
+            offs[r0] - base, offs[min(r0 + 256, n)] - base, o0, o1,
+            [&](int e, int64_t p) {
+                const F v = vals[p];
+                sv[e] = v * v;
+            },
+            [&](int x, int y) {
+                for (int p = x; p < y; ++p) acc = acc + sv[p];
+            });
+        if (i < n) {
+            xs[i] = acc;
+            top = max(top, (unsigned long long)__double_as_longlong(double(acc)));
         }
-        xs[i] = acc;
     }
+    if (!xmax) return;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) top = max(top, (unsigned long long)__shfl_xor((long long)top, off));
+    if ((threadIdx.x & 63) == 0) atomicMax(xmax, top);
+}
+
+// power of two that brings values up to cmax to at most 2^15
+__device__ __forceinline__ double csr_half_scale(double cmax) {
+    int x = 0;
+    frexp(cmax < BOUND_MAX ? cmax : 1.0, &x);
+    return ldexp(1.0, min(15 - x, 120));
 }
 
 // Ct (d x kp) = C^T, rows padded with zeros to kp (a multiple of the 16-byte
-// vector), for coalesced vector reads over centroids: 64 x 64 tiles through LDS
+// vector), and (when given) Cth, the same in half precision times csr_half_scale, for coalesced vector reads over centroids: 64 x 64 tiles through LDS
 // (grid: ceil(d/64) x up to 65535 workgroups of 256 threads, striding over k)
 template <typename F>
 __global__ __launch_bounds__(256) void csr_transpose_kernel(const F* __restrict__ C, int64_t k,
-                                                            int64_t kp, int64_t d, F* __restrict__ Ct) {
+                                                            int64_t kp, int64_t d, F* __restrict__ Ct,
+                                                            _Float16* __restrict__ Cth,
+                                                            const double* __restrict__ cmax) {
     __shared__ F tile[64][65];
+    const F scale = Cth ? F(csr_half_scale(*cmax)) : F(1);
     const int64_t f0 = int64_t(blockIdx.x) * 64;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     for (int64_t j0 = int64_t(blockIdx.y) * 64; j0 < kp; j0 += int64_t(gridDim.y) * 64) {
@@ -99,44 +159,55 @@ __global__ __launch_bounds__(256) void csr_transpose_kernel(const F* __restrict_
         __syncthreads();
         for (int r = ty; r < 64; r += 4) {
             const int64_t f = f0 + r, j = j0 + tx;
-            if (j < kp && f < d) Ct[f * kp + j] = j < k ? tile[tx][r] : F(0);
+            if (j < kp && f < d) {
+                const F v = j < k ? tile[tx][r] : F(0);
+                Ct[f * kp + j] = v;
+                if (Cth) Cth[f * kp + j] = _Float16(float(v * scale));
+            }
         }
         __syncthreads();
     }
 }
 
-// cs_j = |c_j|^2, features in order: one wave per centroid copies the row to LDS
-// (coalesced), then lane 0 adds the squares in feature order
+// cs_j = |c_j|^2, features in order: one wave per centroid copies the squares to LDS
+// (coalesced; zeros up to a multiple of 32, which add nothing), then lane 0 adds them in
+// feature order, 32 read ahead of their additions.  One serial chain of d additions.
+constexpr int CSR_SQ = 32;
+__host__ __device__ inline int csr_sq_len(int d) { return (d + CSR_SQ - 1) / CSR_SQ * CSR_SQ; }
+
 template <typename F>
 __global__ __launch_bounds__(64) void csr_centroid_squares_kernel(const F* __restrict__ C, int64_t k,
                                                                   int d, F* __restrict__ cs) {
-    extern __shared__ unsigned char sq_raw[];
-    F* row = reinterpret_cast<F*>(sq_raw);  // [d]
+    typedef F F4 __attribute__((ext_vector_type(4)));
+    extern __shared__ __align__(32) unsigned char sq_raw[];
+    F* row = reinterpret_cast<F*>(sq_raw);  // [csr_sq_len(d)]
+    const int len = csr_sq_len(d);
     for (int64_t j = blockIdx.x; j < k; j += gridDim.x) {
-        for (int f = threadIdx.x; f < d; f += 64) row[f] = C[j * d + f];
+        for (int f = threadIdx.x; f < len; f += 64) {
+            const F c = f < d ? C[j * d + f] : F(0);
+            row[f] = c * c;
+        }
         __syncthreads();
         if (threadIdx.x == 0) {
+            const F4* r4 = reinterpret_cast<const F4*>(row);
             F acc(0);
-            for (int f = 0; f < d; ++f) {
-                const F c = row[f];
-                const F sq = c * c;
-                acc = acc + sq;
+            F4 cur[CSR_SQ / 4], nxt[CSR_SQ / 4];
+#pragma unroll
+            for (int u = 0; u < CSR_SQ / 4; ++u) cur[u] = r4[u];
+            for (int f = 0; f < len; f += CSR_SQ) {
+                const int g = f + CSR_SQ < len ? f + CSR_SQ : 0;  // past the end: read, not used
+#pragma unroll
+                for (int u = 0; u < CSR_SQ / 4; ++u) nxt[u] = r4[g / 4 + u];
+#pragma unroll
+                for (int u = 0; u < CSR_SQ / 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc = acc + cur[u][e];
+#pragma unroll
+                for (int u = 0; u < CSR_SQ / 4; ++u) cur[u] = nxt[u];
             }
             cs[j] = acc;
         }
         __syncthreads();
-    }
-}
-
-// (s, j) candidate order: the smaller s wins, equal values go to the lower j;
-// NaN never wins (has == false stands for "no candidate yet")
-template <typename F>
-__device__ __forceinline__ void csr_take(F& bs, int& bj, bool& has, F s, int j) {
-    if (s != s) return;
-    if (!has || s < bs || (s == bs && j < bj)) {
-        bs = s;
-        bj = j;
-        has = true;
     }
 }
 
@@ -149,6 +220,56 @@ __device__ __forceinline__ double lane_value(double x, int u) {
     const int lo = __builtin_amdgcn_readlane(int(b & 0xFFFFFFFFll), u);
     const int hi = __builtin_amdgcn_readlane(int(b >> 32), u);
     return __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
+}
+
+__device__ __forceinline__ int64_t lane_value(int64_t x, int u) {
+    const int lo = __builtin_amdgcn_readlane(int(x & 0xFFFFFFFFll), u);
+    const int hi = __builtin_amdgcn_readlane(int(x >> 32), u);
+    return int64_t((unsigned long long)(unsigned(lo)) | ((unsigned long long)(unsigned(hi)) << 32));
+}
+__device__ __forceinline__ int lane_value(int x, int u) { return __builtin_amdgcn_readlane(x, u); }
+
+// smallest value of the wave's 64 lanes (DPP: six steps without LDS; NaN never wins)
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T dpp_from(T x) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "lane values");
+    if constexpr (sizeof(T) == 4) {
+        const int v = __builtin_bit_cast(int, x);
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false));
+    } else {
+        const long long v = __builtin_bit_cast(long long, x);
+        const int lo = int(v & 0xFFFFFFFFll), hi = int(v >> 32);
+        const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+        const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+        return __builtin_bit_cast(T, (long long)(unsigned(l2)) | ((long long)h2 << 32));
+    }
+}
+__device__ __forceinline__ float lower(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ double lower(double a, double b) { return fmin(a, b); }
+__device__ __forceinline__ int lower(int a, int b) { return min(a, b); }
+template <typename T>
+__device__ __forceinline__ T wave_lowest(T x) {
+    x = lower(x, dpp_from<0x111, 0xf>(x));  // row_shr 1, 2, 4, 8: lane 15 of each row of 16
+    x = lower(x, dpp_from<0x112, 0xf>(x));
+    x = lower(x, dpp_from<0x114, 0xf>(x));
+    x = lower(x, dpp_from<0x118, 0xf>(x));
+    x = lower(x, dpp_from<0x142, 0xa>(x));  // row_bcast 15, 31: lane 63
+    x = lower(x, dpp_from<0x143, 0xc>(x));
+    return lane_value(x, 63);
+}
+// the same steps as one instruction each (the compiler's form takes five: a copy, the
+// move, and two operands made canonical); a DPP operand is read two cycles after a write
+template <>
+__device__ __forceinline__ float wave_lowest<float>(float x) {
+    asm("s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "+v"(x));
+    return lane_value(x, 63);
 }
 
 // 16-byte vectors of F
@@ -165,17 +286,33 @@ struct csr_vec<double> {
     typedef double type __attribute__((ext_vector_type(2)));
 };
 
+// (s, j) candidate order: the smaller s wins, equal values go to the lower j;
+// NaN never wins (has == false stands for "no candidate yet")
+template <typename F>
+__device__ __forceinline__ void csr_take(F& bs, int& bj, bool& has, F s, int j) {
+    if (s != s) return;
+    if (!has || s < bs || (s == bs && j < bj)) {
+        bs = s;
+        bj = j;
+        has = true;
+    }
+}
+
+// The exact dots for k past 128 VEC centroids (without FAST), several blocks of them.
 // One wave per row.  Lane l accumulates the dots of the VEC consecutive
 // centroids jb + VEC (l + 64 t) + e (t < JT, e < VEC) over the row's entries,
 // which are loaded 64 at a time and taken in stored order from their lanes;
-// each entry reads one 16-byte vector of its transposed-centroid row per t.
+// each entry reads one 16-byte vector of its transposed-centroid row per t.  Few
+// registers, so that eight waves a SIMD hide the reads, which miss the L2 here: k = 1000 in
+// double, n=3e5, 20 entries takes 3.8 ms, 4.5 ms with csr_assign_kernel's runs of rows.
 // Then each lane's best and a wave reduction (ties to the lower j).
-template <typename F, int JT>
-__global__ __launch_bounds__(256) void csr_assign_kernel(
+template <typename F>
+__global__ __launch_bounds__(256) void csr_assign_blocks_kernel(
     const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs,
     int64_t base, int64_t n, int k, int kp, const F* __restrict__ Ct, const F* __restrict__ cs,
     const F* __restrict__ xs, int32_t* __restrict__ labels, F* __restrict__ closest) {
     constexpr int VEC = csr_vec<F>::N;
+    constexpr int JT = 4;
     typedef typename csr_vec<F>::type V;
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
@@ -253,6 +390,369 @@ __global__ __launch_bounds__(256) void csr_assign_kernel(
     }
 }
 
+// reads through a buffer descriptor: a lane's byte offset and the wave's, no 64-bit address
+// arithmetic
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+template <typename V>
+__device__ __forceinline__ V buffer_read(__amdgpu_buffer_rsrc_t r, int lane_off, int wave_off) {
+    if constexpr (sizeof(V) == 4)
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, wave_off, 0));
+    else if constexpr (sizeof(V) == 8)
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, wave_off, 0));
+    else
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, wave_off, 0));
+}
+
+// Bounds (km_bounds.hpp) for rows whose columns increase strictly (so that the stored
+// entries are a vector).  The label is the smallest computed s_ij, whose error is
+//     |s_ij - (||c_j||^2 - 2 x.c_j)| <= g (||c_j||^2 + 2 ||x|| ||c_j||) <= 3 g M^2,
+// g = gamma_{d+4} and M the largest norm of a row or centroid: not relative to the
+// distance, as the dense form's.  With d_j - d_a >= G > 0 for every other centroid,
+// d_j^2 - d_a^2 >= G^2, so a row stays settled while G > sqrt(2 * 3 g M^2): that part is
+// taken off its gap when it is settled.  M may be taken at that time: later centroids
+// are means of rows, rows, or unchanged.
+struct csr_bounds {
+    const unsigned long long* xmax;  // csr_row_squares_kernel
+    const double* cmax;              // max ||c_j||, rounded up
+    double g;    // gamma_{d+4}
+    float g32;   // in FP32 (FAST)
+    int32_t* open;  // [4] this pass's open rows and rows, the previous pass's
+};
+
+// Rows are taken in runs of up to 16 per wave (their offsets read and their results written
+// together, by lanes), one wave per row.  Lane l accumulates the dots of the VEC consecutive
+// centroids VEC (l + 64 t) + e (t < JT, e < VEC: one block holds k) over the row's entries,
+// which are loaded 64 at a time (a row's first ones during the row before) and taken in
+// stored order from their lanes; each entry reads one 16-byte vector of its
+// transposed-centroid row per t, U in flight.  Then each lane's best and a wave
+// reduction (ties to the lower j).
+//
+// FAST (columns that increase strictly): the same dots from a
+// half-precision copy of the centroids (scaled by a power of two), half the bytes and one
+// v_fma_mix_f32 a product, in FP32:
+//     |s'_ij - s_ij| <= B = 2 X C (1.02 2^-11 + gamma_{d+4}) + 2^-21 (C^2 + 2 X C) + 3 g M^2 + 1e-34
+// (X the row's norm, C = max ||c_j||; the last term covers underflow).  One centroid with
+// s' <= min s' + 2 B is the label; otherwise the lanes that hold such centroids form their
+// exact dots from Ct.  closest is not written: csr_closest_kernel forms it where it is
+// needed, for one centroid a row.
+//
+// Bound by a row's instructions, not by bytes (n=1e6, 20 entries, k=256: about 300 vector
+// instructions a row, a third of them products): 0.8 ms for all rows, 1.3 ms for the exact
+// dots.  The bookkeeping matters as much as the reads: with the bounds' double arithmetic
+// done per row by a whole wave, FAST took 1.43 ms, with a read at a time for a row's last
+// entries 1.3 ms.
+//
+// Rough distances that leave most rows open are work for nothing (random columns, n=1e5,
+// 50 entries, k=256: 8 iterations took 3.90 ms, 3.75 so): kb.open counts a pass's rows with more
+// than one candidate, and the next pass over fewer than twice as many rows as that goes
+// straight to the exact dots.
+template <typename F, int JT, bool FAST>
+__global__ __launch_bounds__(256) void csr_assign_kernel(
+    const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs,
+    int64_t base, int64_t n, int d, int k, int kp, const F* __restrict__ Ct, const _Float16* __restrict__ Cth,
+    const F* __restrict__ cs, const F* __restrict__ xs, int32_t* __restrict__ labels, F* __restrict__ closest,
+    row_select rs, csr_bounds kb) {
+    constexpr int VEC = csr_vec<F>::N;
+    constexpr int U = FAST ? 16 / JT : 8 / JT;  // entries whose vectors are in flight together
+    static_assert(U >= 4, "groups of U, U / 2 and U / 4 entries");
+    typedef typename csr_vec<F>::type V;
+    typedef _Float16 VH __attribute__((ext_vector_type(VEC)));
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+    const int64_t nwaves = (int64_t(gridDim.x) * blockDim.x) >> 6;
+    const int64_t nsel = select_rows(rs, n);
+    const int per = int(max<int64_t>(1, min<int64_t>(16, nsel / nwaves)));
+    const int64_t nruns = (nsel + per - 1) / per;
+    double band = 0.0, C = 0.0;  // g M^2, and the largest centroid norm
+    float unscale = 1.0f;        // -2 / csr_half_scale
+    if (FAST) {
+        C = *kb.cmax;
+        const double M = fmax(sqrt(__longlong_as_double((long long)*kb.xmax)) * (1.0 + kb.g), C) * (1.0 + 1e-6);
+        band = kb.g * M * M;
+        if (!(M < BOUND_MAX) || !(C < BOUND_MAX)) band = __builtin_inf();  // NaN as well
+        unscale = float(-2.0 / csr_half_scale(C));
+    }
+    const bool rough = FAST && (!kb.open || kb.open[2] <= kb.open[3] / 2);
+    int opened = 0;
+    // (k <= 1024 and d <= 4096: at most 32 MB)
+    const auto half_rsrc = FAST ? buffer_of(Cth, int(2 * int64_t(d) * kp)) : buffer_of(nullptr, 0);
+    const auto full_rsrc = FAST ? buffer_of(Ct, int(int64_t(sizeof(F)) * d * kp)) : buffer_of(nullptr, 0);
+    F csv[JT][VEC];  // the same for every row
+#pragma unroll
+    for (int t = 0; t < JT; ++t)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const int j = VEC * (64 * t + lane) + e;
+            csv[t][e] = j < k ? cs[j] : F(0);
+        }
+    for (int64_t run = wave; run < nruns; run += nwaves) {
+        const int64_t e0 = run * per;
+        const int rows = int(min<int64_t>(per, nsel - e0));
+        // lane q holds row q of the run, and its results
+        int64_t my_row = 0, my_o0 = 0, my_o1 = 0;
+        F my_xs(0), my_best(0), my_second = fp_traits<F>::inf;
+        float my_B = 0.f, my_rest = __builtin_inff();
+        int my_lab = 0;
+        bool my_rough = false, my_none = false;
+        if (lane < rows) {
+            my_row = select_row(rs, e0 + lane);
+            my_o0 = offs[my_row] - base;
+            my_o1 = offs[my_row + 1] - base;
+            my_xs = xs[my_row];
+        }
+        if (FAST) {
+            const double X = sqrt(double(my_xs)) * (1.0 + kb.g);
+            const double B = 2.0 * X * C * (1.02 / 2048.0 + double(kb.g32)) + 4.8e-7 * (C * C + 2.0 * X * C) +
+                             3.0 * band + 1e-34;
+            my_B = float(B * (1.0 + 1e-6));
+        }
+        auto fetch = [&](int64_t p0, int64_t o1, int& c, F& v) {
+            c = 0;  // a column index (< d <= 4096), FAST: the byte offset of its row of Cth
+            v = F(0);
+            if (p0 + lane < o1) {
+                c = int(cols[p0 + lane] - base) * (FAST ? 2 * kp : 1);
+                v = vals[p0 + lane];
+            }
+        };
+        int next_c;
+        F next_v;
+        fetch(lane_value(my_o0, 0), lane_value(my_o1, 0), next_c, next_v);
+        for (int q = 0; q < rows; ++q) {
+            const int64_t o0 = lane_value(my_o0, q), o1 = lane_value(my_o1, q);
+            const int first_c = next_c;
+            const F first_v = next_v;
+            if (q + 1 < rows) fetch(lane_value(my_o0, q + 1), lane_value(my_o1, q + 1), next_c, next_v);
+            // the row's entries in stored order, U at a time: add(columns, values, first
+            // lane, entries left, group)
+            auto entries = [&](auto&& add) {
+                for (int64_t p0 = o0; p0 < o1; p0 += 64) {
+                    const int cnt = int(min<int64_t>(64, o1 - p0));
+                    int my_c = first_c;
+                    F my_v = first_v;
+                    if (p0 != o0) fetch(p0, o1, my_c, my_v);
+                    // whole groups, then the smallest group that holds the rest: past the
+                    // last entry the column is 0, and add() leaves the value out
+                    int u = 0;
+                    for (; cnt - u > U / 2; u += U) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U>());
+                    if (cnt - u > U / 4) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U / 2>());
+                    else if (cnt > u) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U / 4>());
+                }
+            };
+            uint64_t holders = ~0ull;  // lanes whose centroids may hold the label
+            float rest = __builtin_inff();  // FAST: smallest s' of a centroid that does not
+            if (rough) {
+                float acc[JT][VEC];
+#pragma unroll
+                for (int t = 0; t < JT; ++t)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) acc[t][e] = 0.f;
+                int off[JT];  // a lane past k reads the last vector, for nothing
+#pragma unroll
+                for (int t = 0; t < JT; ++t) off[t] = min(VEC * (64 * t + lane), kp - VEC) * 2;
+                entries([&](int c_of, F v_of, int u0, int left, auto count) {
+                    constexpr int N = decltype(count)::value;
+                    (void)left;
+                    VH cv[N][JT];
+#pragma unroll
+                    for (int u = 0; u < N; ++u) {
+                        const int crow = lane_value(c_of, u0 + u);
+#pragma unroll
+                        for (int t = 0; t < JT; ++t) cv[u][t] = buffer_read<VH>(half_rsrc, off[t], crow);
+                    }
+#pragma unroll
+                    for (int u = 0; u < N; ++u) {
+                        const float v = float(lane_value(v_of, u0 + u));  // 0 past the last entry
+#pragma unroll
+                        for (int t = 0; t < JT; ++t)
+#pragma unroll
+                            for (int e = 0; e < VEC; ++e)
+                                acc[t][e] = __builtin_fmaf(v, float(cv[u][t][e]), acc[t][e]);
+                    }
+                });
+                float low = __builtin_inff();
+#pragma unroll
+                for (int t = 0; t < JT; ++t)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        acc[t][e] = __builtin_fmaf(unscale, acc[t][e], float(csv[t][e]));
+                        low = VEC * (64 * t + lane) + e < k ? fminf(low, acc[t][e]) : low;
+                    }
+                const float top = wave_lowest(low);
+                const float lim = top + 2.0f * lane_value(my_B, q);
+                const float T = lim + fabsf(lim) * 2.4e-7f;  // not a number: every centroid stays
+                int mine = 0, at = 0;
+#pragma unroll
+                for (int t = 0; t < JT; ++t)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        const int j = VEC * (64 * t + lane) + e;
+                        const bool out = acc[t][e] > T;
+                        const bool in = j < k && !out;
+                        mine += in ? 1 : 0;
+                        at = in ? j : at;
+                        rest = j < k && out ? fminf(rest, acc[t][e]) : rest;
+                    }
+                holders = __ballot(mine > 0);
+                const int src = int(__builtin_ctzll(holders | (uint64_t(1) << 63)));
+                if ((holders & (holders - 1)) == 0 && lane_value(mine, src) == 1) {
+                    const float r = rs.gap ? wave_lowest(rest) : rest;
+                    const int lab = lane_value(at, src);
+                    if (lane == q) {
+                        my_lab = lab;
+                        my_best = F(top);
+                        my_rest = r;
+                        my_rough = true;
+                    }
+                    continue;
+                }
+            }
+            ++opened;
+            const bool act = (holders >> lane) & 1u;
+            const int spare = int(__builtin_ctzll(holders | (uint64_t(1) << 63)));  // read by idle lanes
+            F bs(0), b2 = fp_traits<F>::inf;  // best and second best of this lane
+            int bj = 0;
+            bool has = false;
+            F s0(0);  // s of centroid 0 (lane 0)
+            F acc[JT][VEC];
+#pragma unroll
+            for (int t = 0; t < JT; ++t)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) acc[t][e] = F(0);
+            int off[JT];
+#pragma unroll
+            for (int t = 0; t < JT; ++t) off[t] = min(VEC * (64 * t + (act ? lane : spare)), kp - VEC);
+            entries([&](int c_of, F v_of, int u0, int left, auto count) {
+                constexpr int N = decltype(count)::value;
+                V cv[N][JT];
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    const int at_c = lane_value(c_of, u0 + u);
+#pragma unroll
+                    for (int t = 0; t < JT; ++t) {
+                        if constexpr (FAST)
+                            cv[u][t] = buffer_read<V>(full_rsrc, off[t] * int(sizeof(F)), at_c * int(sizeof(F) / 2));
+                        else
+                            cv[u][t] = *reinterpret_cast<const V*>(Ct + int64_t(at_c) * kp + off[t]);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    const F v = lane_value(v_of, u0 + u);
+                    if (u >= left) break;  // nothing added: a centroid may be infinite
+#pragma unroll
+                    for (int t = 0; t < JT; ++t)
+#pragma unroll
+                        for (int e = 0; e < VEC; ++e) {
+                            const F pr = v * cv[u][t][e];
+                            acc[t][e] = acc[t][e] + pr;
+                        }
+                }
+            });
+#pragma unroll
+            for (int t = 0; t < JT; ++t)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    const int j = VEC * (64 * t + lane) + e;
+                    const F two_dot = F(2) * acc[t][e];
+                    const F s = csv[t][e] - two_dot;
+                    if (j == 0) s0 = s;
+                    // ascending j in a lane: an equal value is the later one
+                    const bool in = act && j < k && s == s;
+                    const bool win = in && (!has || s < bs);
+                    if (FAST && in) b2 = win ? (has ? bs : b2) : lower(b2, s);
+                    bs = win ? s : bs;
+                    bj = win ? j : bj;
+                    has = has || win;
+                }
+            // the smallest s, then the lowest j that has it; every s NaN, or s_i0 (when it
+            // can matter: idle lanes' centroids are finite): label 0
+            const F best = wave_lowest(has ? bs : fp_traits<F>::inf);
+            const int lab = wave_lowest(has && bs == best ? bj : 0x7fffffff);
+            s0 = lane_value(s0, 0);
+            const bool none = lab == 0x7fffffff || ((holders & 1u) && s0 != s0);
+            F second = fp_traits<F>::inf;
+            if (FAST && rs.gap) {
+                second = wave_lowest(!has ? fp_traits<F>::inf : bj == lab ? b2 : bs);
+                rest = wave_lowest(rest);
+            }
+            if (lane == q) {
+                my_lab = none ? 0 : lab;
+                my_best = none ? s0 : best;
+                my_second = second;
+                my_rest = rest;
+                my_none = none;
+            }
+        }
+        if (lane < rows) {
+            labels[my_row] = my_lab;
+            if (!FAST) closest[my_row] = my_best + my_xs;
+            if (FAST && rs.gap) {
+                float gap = -__builtin_inff();
+                if (!my_none && band < BOUND_MAX) {
+                    const double x2 = double(my_xs), rough = double(my_B) + 1.5 * band;
+                    const double up2 = double(my_best) + x2 + (my_rough ? rough : 4.5 * band);
+                    const double lo2 = fmin(double(my_second) - 4.5 * band, double(my_rest) - rough) + x2;
+                    gap = float_below(double(bound_gap(up2, lo2, rs.gam, rs.base[my_lab])) - sqrt(6.3 * band));
+                }
+                rs.gap[my_row] = gap;
+            }
+        }
+    }
+    if (FAST && kb.open && lane == 0) {
+        if (opened) atomicAdd(kb.open, opened);
+        if (wave == 0) kb.open[1] = int32_t(nsel);
+    }
+}
+
+// closest_i of every row with its label known (no pass with FAST writes it): the
+// arithmetic of csr_assign_kernel for one centroid, a lane per row
+template <typename F>
+__global__ __launch_bounds__(256) void csr_closest_kernel(
+    const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs, int64_t base,
+    int64_t n, int d, const F* __restrict__ C, const F* __restrict__ cs, const F* __restrict__ xs,
+    const int32_t* __restrict__ labels, F* __restrict__ closest) {
+    constexpr int U = 8;  // gathers in flight
+    __shared__ int32_t sc[CSR_WINDOW];
+    __shared__ F sv[CSR_WINDOW];
+    for (int64_t r0 = blockIdx.x * int64_t(256); r0 < n; r0 += int64_t(gridDim.x) * 256) {
+        const int64_t i = r0 + threadIdx.x;
+        const int64_t o0 = i < n ? offs[i] - base : 0, o1 = i < n ? offs[i + 1] - base : 0;
+        const int lab = i < n ? labels[i] : 0;
+        const F* c = C + int64_t(lab) * d;
+        F acc(0);
+        csr_walk(
+            offs[r0] - base, offs[min(r0 + 256, n)] - base, o0, o1,
+            [&](int e, int64_t p) {
+                sc[e] = int32_t(cols[p] - base);
+                sv[e] = vals[p];
+            },
+            [&](int x, int y) {
+                for (int p = x; p < y; p += U) {
+                    F v[U], w[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int q = min(p + u, y - 1);
+                        v[u] = sv[q];
+                        w[u] = c[sc[q]];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const F pr = v[u] * w[u];
+                        const F t = acc + pr;
+                        acc = p + u < y ? t : acc;
+                    }
+                }
+            });
+        if (i < n) {
+            const F two_dot = F(2) * acc;
+            const F s = cs[lab] - two_dot;
+            closest[i] = s + xs[i];
+        }
+    }
+}
+
 // objective over closest_i (as double) in the dense objective's order; also
 // writes the per-row keys used to pick empty-cluster candidates (and subtracted
 // from the objective for each one taken)
@@ -289,11 +789,13 @@ __global__ __launch_bounds__(256) void csr_objective_chunks_kernel(const F* __re
 // members whose entries are loaded together by the chunk-sum kernel
 constexpr int CSR_AHEAD = 8;
 
-__device__ __forceinline__ int64_t lane_value(int64_t x, int u) {
-    const int lo = __builtin_amdgcn_readlane(int(x & 0xFFFFFFFFll), u);
-    const int hi = __builtin_amdgcn_readlane(int(x >> 32), u);
-    return int64_t((unsigned long long)(unsigned(lo)) | ((unsigned long long)(unsigned(hi)) << 32));
+// *p += v in LDS.  float: one ds_add_f64 (sums of floats are never denormal doubles, so no
+// mode changes their bits), which the next member's add does not wait for as it waits
+// for a read and a write
+__device__ __forceinline__ void csr_add(double* p, float v) {
+    __hip_atomic_fetch_add(p, double(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ void csr_add(double* p, double v) { *p = *p + v; }
 
 // Chunk sums of the CSR rows: one single-wave workgroup per chunk of
 // REDUCE_CHUNK members, G = reduce_groups(d) partial vectors of d doubles in LDS
@@ -303,9 +805,12 @@ __device__ __forceinline__ int64_t lane_value(int64_t x, int u) {
 // order and, inside a row, in stored order.  Partials are added in g order.
 // The wave's LDS operations execute in issue order, so a member's adds see the
 // previous member's.  Groups of 64 members whose rows all hold at most 64
-// entries load CSR_AHEAD rows' entries at a time from registers (the offsets of
-// the whole group first); other groups go member by member.
-template <typename F>
+// entries load CSR_AHEAD rows' entries at a time into registers (the offsets of
+// the whole group first), the next ones while these are added; other groups go member
+// by member.  INC: every row's columns are known to increase, nothing is compared.
+// n=1e6, 20 entries, d=2000: 304 us for all rows, 340 us with the comparison and
+// without the loads ahead.
+template <typename F, bool INC>
 __global__ __launch_bounds__(64) void csr_chunk_sums_kernel(
     const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs,
     int64_t base, int d, int k, const int32_t* __restrict__ perm,
@@ -340,42 +845,51 @@ __global__ __launch_bounds__(64) void csr_chunk_sums_kernel(
             if (__all(my_len <= 64)) {
                 // every row fits the lanes: the entries of CSR_AHEAD members are
                 // loaded together, then added member by member
-                for (int u0 = 0; u0 < cnt; u0 += CSR_AHEAD) {
-                    int cc[CSR_AHEAD], ln[CSR_AHEAD];
-                    F vv[CSR_AHEAD];
+                int cc[2][CSR_AHEAD];
+                F vv[2][CSR_AHEAD];
+                auto load = [&](int u0, int (&c)[CSR_AHEAD], F (&v)[CSR_AHEAD]) {
 #pragma unroll
                     for (int q = 0; q < CSR_AHEAD; ++q) {
-                        cc[q] = 0;
-                        vv[q] = F(0);
-                        ln[q] = 0;
-                        if (u0 + q < cnt) {
-                            ln[q] = __builtin_amdgcn_readlane(my_len, u0 + q);
-                            const int64_t o0 = lane_value(my_o0, u0 + q);
-                            if (lane < ln[q]) {
-                                cc[q] = int(cols[o0 + lane] - base);
-                                vv[q] = vals[o0 + lane];
+                        const int m = min(u0 + q, cnt - 1);
+                        const int64_t o0 = lane_value(my_o0, m);
+                        c[q] = 0;
+                        v[q] = F(0);
+                        if (lane < __builtin_amdgcn_readlane(my_len, m)) {
+                            c[q] = int(cols[o0 + lane] - base);
+                            v[q] = vals[o0 + lane];
+                        }
+                    }
+                };
+                auto add = [&](int u0, const int (&c)[CSR_AHEAD], const F (&v)[CSR_AHEAD]) {
+#pragma unroll
+                    for (int q = 0; q < CSR_AHEAD; ++q) {
+                        if (u0 + q >= cnt) break;  // uniform
+                        const int len = __builtin_amdgcn_readlane(my_len, u0 + q);
+                        double* pg = acc + int((m0 + u0 + q - m_begin) % G) * d;
+                        bool inc = true;
+                        if (!INC) {
+                            const int prev = __shfl_up(c[q], 1);
+                            inc = __all(lane == 0 || lane >= len || prev < c[q]);
+                        }
+                        if (inc) {
+                            // strictly increasing columns: distinct, added at once
+                            if (lane < len) csr_add(pg + c[q], v[q]);
+                        } else {
+                            for (int e = 0; e < len; ++e) {
+                                const int ce = __builtin_amdgcn_readlane(c[q], e);
+                                const F ve = lane_value(v[q], e);
+                                if (lane == 0) pg[ce] = pg[ce] + double(ve);
                             }
                         }
                     }
-#pragma unroll
-                    for (int q = 0; q < CSR_AHEAD; ++q) {
-                        if (u0 + q < cnt) {
-                            const int len = ln[q];
-                            double* pg = acc + int((m0 + u0 + q - m_begin) % G) * d;
-                            const int prev = __shfl_up(cc[q], 1);
-                            const bool inc = lane == 0 || lane >= len || prev < cc[q];
-                            if (__all(inc)) {
-                                // strictly increasing columns: distinct, added at once
-                                if (lane < len) pg[cc[q]] = pg[cc[q]] + double(vv[q]);
-                            } else {
-                                for (int e = 0; e < len; ++e) {
-                                    const int c = __builtin_amdgcn_readlane(cc[q], e);
-                                    const F v = lane_value(vv[q], e);
-                                    if (lane == 0) pg[c] = pg[c] + double(v);
-                                }
-                            }
-                        }
-                    }
+                };
+                load(0, cc[0], vv[0]);
+                for (int u0 = 0; u0 < cnt; u0 += 2 * CSR_AHEAD) {
+                    if (u0 + CSR_AHEAD < cnt) load(u0 + CSR_AHEAD, cc[1], vv[1]);
+                    add(u0, cc[0], vv[0]);
+                    if (u0 + CSR_AHEAD >= cnt) break;
+                    if (u0 + 2 * CSR_AHEAD < cnt) load(u0 + 2 * CSR_AHEAD, cc[0], vv[0]);
+                    add(u0 + CSR_AHEAD, cc[1], vv[1]);
                 }
                 continue;
             }

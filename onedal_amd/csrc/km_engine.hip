@@ -149,7 +149,7 @@ struct km_ctx {
     km::dbuf b_gap, b_rows, b_count, b_base, b_drift, cand_lo, coll_lo, seg_cand_lo, seg_coll_lo;
     // CSR path: values, column indices, row offsets (when uploaded), row squares,
     // transposed centroids, centroid squares, closest distances, structure flag
-    km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cs, csr_closest, csr_flag;
+    km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cth, csr_open, csr_cs, csr_closest, csr_flag;
     // step_ticket: zero between launches; step_max: centroid_step_kernel's workspace.
     // Both live from the context's creation on.
     km::dbuf step_ticket, step_max;
@@ -254,6 +254,7 @@ struct work {
     int32_t* open_rows = nullptr;
     int32_t* open_count = nullptr;
     unsigned long long* acc = nullptr;
+    int32_t* csr_open = nullptr;  // sparse rows: csr_bounds::open
     // workspace source: a fixed arena, or (null) the context's buffers
     arena* A = nullptr;
 };
@@ -334,7 +335,14 @@ template <typename F>
 static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* cold = nullptr,
                            const chunk_sums& m = {nullptr, nullptr, nullptr}) {
     centroid_step<F> s{};
-    s.part = m.part;
+    if (m.part && w.d > STEP_MERGE_D) {
+        const int64_t items = int64_t(w.k) * ((w.d + 255) / 256);
+        hipLaunchKernelGGL(merge_centroids_kernel<F>, dim3(grid_for(ctx, items, 1, 8)), dim3(256), 0, ctx->stream,
+                           m.part, m.counts, m.chunk_base, w.changed, w.k, w.d, cold, C);
+        KM_LAUNCH_CHECK();
+    } else {
+        s.part = m.part;
+    }
     s.counts = m.counts;
     s.chunk_base = m.chunk_base;
     s.C = C;
@@ -357,6 +365,7 @@ static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* col
     s.sel_count = w.open_count;
     s.counters = w.L.counters;
     s.acc = cold ? w.acc : nullptr;
+    s.csr_open = w.csr_open;
     s.ticket = ctx->step_ticket.get<uint32_t>(1);
     s.wgmax = ctx->step_max.get<unsigned long long>(4 * STEP_MAX_GRID);
     const int grid = std::min(w.k, STEP_MAX_GRID);
@@ -1295,20 +1304,36 @@ static csr_view<F> csr_prepare(km_ctx* ctx, const F* vals, const int64_t* cols,
     return v;
 }
 
-// labels and closest distances of every row against C (k x d)
+// Half-precision distances first (csr_assign_kernel, FAST): rows whose columns increase strictly, and
+// at most one block of centroids.  n=1e6, 20 entries a row, k=256: 0.8 ms a pass
+// against 1.3 ms.  Columns in another order may repeat, and then the entries' norm does
+// not bound the products; past one block the rough values would have to be kept.
+template <typename F>
+static bool csr_fast(int k, bool increasing) {
+    return increasing && k <= 64 * csr_vec<F>::N * 4;
+}
+
+static csr_bounds csr_make_bounds(const unsigned long long* xmax, const double* cmax, int d, double u) {
+    return {xmax, cmax, gamma_m(double(d + 4), u), float(gamma_m(double(d + 4), fp_traits<float>::u) * (1.0 + 1e-6)),
+            nullptr};
+}
+
+// labels of the selected rows against C (k x d), and without fast their closest distances
 template <typename F>
 static void csr_assign(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, const F* xs,
-                       int32_t* labels, F* closest) {
+                       int32_t* labels, F* closest, bool fast, const row_select& sel, const csr_bounds& kb) {
     constexpr int VEC = csr_vec<F>::N;
     const int kp = (k + VEC - 1) / VEC * VEC;  // Ct row stride: whole 16-byte vectors
     F* ct = ctx->csr_ct.get<F>(int64_t(kp) * x.d);
+    _Float16* cth = fast ? ctx->csr_cth.get<_Float16>(int64_t(kp) * x.d) : nullptr;
     F* cs = ctx->csr_cs.get<F>(k);
     hipLaunchKernelGGL(csr_transpose_kernel<F>,
                        dim3(unsigned((x.d + 63) / 64), unsigned(std::min((kp + 63) / 64, 65535))),
-                       dim3(256), 0, ctx->stream, C, int64_t(k), int64_t(kp), x.d, ct);
+                       dim3(256), 0, ctx->stream, C, int64_t(k), int64_t(kp), x.d, ct, cth,
+                       kb.cmax);
     KM_LAUNCH_CHECK();
     hipLaunchKernelGGL(csr_centroid_squares_kernel<F>, dim3(unsigned(std::min(k, ctx->cu_count * 8))),
-                       dim3(64), size_t(x.d) * sizeof(F), ctx->stream, C, int64_t(k), int(x.d), cs);
+                       dim3(64), size_t(csr_sq_len(int(x.d))) * sizeof(F), ctx->stream, C, int64_t(k), int(x.d), cs);
     KM_LAUNCH_CHECK();
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing) {
@@ -1317,17 +1342,36 @@ static void csr_assign(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, con
         KM_HIP(hipEventRecord(e0, ctx->stream));
     }
     const int grid = grid_for(ctx, x.n * 64, 256, 8);
-#define KM_CSRA(JT_)                                                                                \
-    hipLaunchKernelGGL((csr_assign_kernel<F, JT_>), dim3(grid), dim3(256), 0, ctx->stream, x.vals,   \
-                       x.cols, x.offs, x.base, x.n, k, kp, ct, cs, xs, labels, closest)
+#define KM_CSRA(JT_, FAST_)                                                                         \
+    hipLaunchKernelGGL((csr_assign_kernel<F, JT_, FAST_>), dim3(grid), dim3(256), 0, ctx->stream,    \
+                       x.vals, x.cols, x.offs, x.base, x.n, int(x.d), k, kp, ct, cth, cs, xs, labels, closest, \
+                       sel, kb)
     // centroids per lane and block: VEC * JT
-    if (k <= 64 * VEC) KM_CSRA(1);
-    else if (k <= 128 * VEC) KM_CSRA(2);
-    else KM_CSRA(4);
+    if (fast) {
+        if (k <= 64 * VEC) KM_CSRA(1, true);
+        else if (k <= 128 * VEC) KM_CSRA(2, true);
+        else KM_CSRA(4, true);
+    } else if (k <= 64 * VEC) {
+        KM_CSRA(1, false);
+    } else if (k <= 128 * VEC) {
+        KM_CSRA(2, false);
+    } else {
+        hipLaunchKernelGGL(csr_assign_blocks_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, x.vals, x.cols, x.offs,
+                           x.base, x.n, k, kp, ct, cs, xs, labels, closest);
+    }
 #undef KM_CSRA
     KM_LAUNCH_CHECK();
     if (ctx->timing) KM_HIP(hipEventRecord(e1, ctx->stream));
     ctx->stats.assign_launches++;
+}
+
+// closest distances of all rows to their labels' centroids, after csr_assign against C
+template <typename F>
+static void csr_all_closest(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, const F* xs, const int32_t* labels,
+                            F* closest) {
+    hipLaunchKernelGGL(csr_closest_kernel<F>, dim3(grid_for(ctx, x.n, 256, 8)), dim3(256), 0, ctx->stream, x.vals,
+                       x.cols, x.offs, x.base, x.n, int(x.d), C, ctx->csr_cs.get<F>(k), xs, labels, closest);
+    KM_LAUNCH_CHECK();
 }
 
 // objective = sum of closest (as double) in the fixed order; d64 per row if asked
@@ -1355,6 +1399,18 @@ static void csr_timing_stats(km_ctx* ctx, size_t first_pair) {
     ctx->stats.assign_kernel_ms = tot;
 }
 
+// what step_centroids needs of sparse rows (path 1: it prepares nothing else)
+template <typename F>
+static void csr_step_view(km_ctx* ctx, work<F>& w, int64_t n, int d, int k) {
+    w.n = n;
+    w.d = d;
+    w.k = k;
+    w.dpad = d;
+    w.cn = ctx->cn.get<F>(k);
+    w.maxima = ctx->cmax.get<double>(4);
+    w.L.counters = ctx->lists_counters.get<int32_t>(3);
+}
+
 template <typename F>
 static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int64_t* offs,
                       int64_t n, int64_t d64_, int64_t nnz, int32_t indexing, const F* C0,
@@ -1369,12 +1425,15 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
         loop0 = ctx->event();
         loop1 = ctx->event();
     }
-    const csr_view<F> x = csr_prepare<F>(ctx, vals, cols, offs, n, d, nnz, indexing, dev);
+    bool increasing = false;
+    const csr_view<F> x = csr_prepare<F>(ctx, vals, cols, offs, n, d, nnz, indexing, dev, &increasing);
     F* xs = ctx->csr_xs.get<F>(n);
     F* closest = ctx->csr_closest.get<F>(n);
     int32_t* labels = ctx->labels.get<int32_t>(n);
+    unsigned long long* xmax = ctx->xmax.get<unsigned long long>(2);
+    fill<unsigned long long>(ctx, xmax, 2, 0ull);
     hipLaunchKernelGGL(csr_row_squares_kernel<F>, dim3(grid_for(ctx, n, 256, 4)), dim3(256), 0,
-                       ctx->stream, x.vals, x.offs, x.base, n, xs);
+                       ctx->stream, x.vals, x.offs, x.base, n, xs, xmax);
     KM_LAUNCH_CHECK();
     F* Ccur = ctx->c_cur.get<F>(int64_t(k) * d);
     F* Cnext = ctx->c_next.get<F>(int64_t(k) * d);
@@ -1385,39 +1444,68 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     int32_t* pin = ctx->pinned;
     const bool need_obj = thr > 0;
     const size_t lds = size_t(reduce_groups(d)) * d * sizeof(double);
-    KM_HIP(hipFuncSetAttribute((const void*)csr_chunk_sums_kernel<F>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    auto sums = increasing ? csr_chunk_sums_kernel<F, true> : csr_chunk_sums_kernel<F, false>;
+    KM_HIP(hipFuncSetAttribute((const void*)sums, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     double* d64 = ctx->d64.get<double>(n);  // refill candidates' keys
     const label_sort lsort = label_sort_setup(ctx, n, k);
+    // the centroid step's view, and bounds where the rough distances are used
+    work<F> w;
+    csr_step_view(ctx, w, n, d, k);
+    w.base = ctx->b_base.get<double>(k);
+    fill<double>(ctx, w.base, k, 0.0);
+    w.drift = ctx->b_drift.get<double>(k);
+    w.changed = lsort.changed;
+    w.open_count = ctx->b_count.get<int32_t>(1);
+    w.sel.base = w.base;
+    w.sel.gam = 1e-6;
+    csr_bounds kb = csr_make_bounds(xmax, w.maxima, d, fp_traits<F>::u);
+    const bool fast = csr_fast<F>(k, increasing);
+    if (fast) {
+        w.open_rows = ctx->b_rows.get<int32_t>(n);
+        w.sel.gap = ctx->b_gap.get<float>(n);
+    }
+    const int path = 1;  // the step prepares nothing else
     if (ctx->timing) KM_HIP(hipEventRecord(loop0, ctx->stream));
+    step_centroids<F>(ctx, w, path, Ccur);
 
     double prev = double(std::numeric_limits<F>::max());
     int64_t iter = 0;
     for (iter = 0; iter < max_iter; ++iter) {
-        csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest);
-        if (iter > 0) fill<int32_t>(ctx, lsort.changed, k, 0);
+        csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest, fast, w.sel, kb);
         const uint32_t seq = next_seq(ctx);
         label_group(ctx, lsort, labels, o, seq);
         const int64_t max_chunks = n / REDUCE_CHUNK + k + 1;
-        hipLaunchKernelGGL(csr_chunk_sums_kernel<F>, dim3(grid_for(ctx, max_chunks * 64, 64, 16)),
+        hipLaunchKernelGGL(sums, dim3(grid_for(ctx, max_chunks * 64, 64, 16)),
                            dim3(64), lds, ctx->stream, x.vals, x.cols, x.offs, x.base, d, k, o.perm,
                            o.offsets, o.chunk_base, o.meta, part);
         KM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(finalize_centroids_kernel<F>, dim3(grid_for(ctx, int64_t(k) * d, 256, 4)),
-                           dim3(256), 0, ctx->stream, part, o.counts, o.chunk_base, lsort.changed, k, d, Ccur, Cnext);
-        KM_LAUNCH_CHECK();
         double* objp = nullptr;
-        if (need_obj) objp = csr_objective<F>(ctx, closest, n, d64);
+        if (need_obj) {
+            if (fast) csr_all_closest<F>(ctx, x, Ccur, k, xs, labels, closest);
+            objp = csr_objective<F>(ctx, closest, n, d64);
+        }
+        step_centroids<F>(ctx, w, path, Cnext, Ccur, {part, o.counts, o.chunk_base});
         wait_report(ctx, &ctx->report->seq, seq);  // as in train()
         if (ctx->report->empties > 0) {
-            if (!need_obj) csr_objective<F>(ctx, closest, n, d64);
+            if (!need_obj) {
+                if (fast) csr_all_closest<F>(ctx, x, Ccur, k, xs, labels, closest);
+                csr_objective<F>(ctx, closest, n, d64);
+            }
             int32_t* cand = launch_empty_clusters<F>(ctx, (const F*)nullptr, n, d, k, o, Cnext, d64, objp);
             hipLaunchKernelGGL(csr_fill_empty_kernel<F>, dim3(std::min(k, ctx->cu_count * 4)), dim3(64), 0,
                                ctx->stream, x.vals, x.cols, x.offs, x.base, d, o.empty_list, cand, o.meta, Cnext);
             KM_LAUNCH_CHECK();
+            step_centroids<F>(ctx, w, path, Cnext, Ccur);  // bounds of the refilled
             ctx->stats.empty_cluster_events++;
         }
         std::swap(Ccur, Cnext);
+        if (w.sel.gap) {
+            hipLaunchKernelGGL(bound_select_kernel, dim3(grid_for(ctx, n, SELECT_ROWS, 8)), dim3(256), 0, ctx->stream,
+                               labels, w.sel.gap, w.base, n, w.open_rows, w.open_count);
+            KM_LAUNCH_CHECK();
+            w.sel.rows = w.open_rows;
+            w.sel.count = w.open_count;
+        }
         if (need_obj) {
             double obj = 0.0;
             KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1430,7 +1518,8 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
             prev = obj;
         }
     }
-    csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest);
+    csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest, fast, w.sel, kb);
+    if (fast) csr_all_closest<F>(ctx, x, Ccur, k, xs, labels, closest);
     double* objp = csr_objective<F>(ctx, closest, n, nullptr);
     if (ctx->timing) KM_HIP(hipEventRecord(loop1, ctx->stream));
     KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1458,20 +1547,34 @@ static void infer_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     const bool dev = flags & KM_FLAG_DEVICE_POINTERS;
     ctx->stats = km_stats{};
     ctx->ev_used = 0;
-    const csr_view<F> x = csr_prepare<F>(ctx, vals, cols, offs, n, d, nnz, indexing, dev);
+    bool increasing = false;
+    const csr_view<F> x = csr_prepare<F>(ctx, vals, cols, offs, n, d, nnz, indexing, dev, &increasing);
+    // one pass: the rough one has to earn its centroid step and, with the objective, the
+    // closest distances (n=2e4, 30 entries, k=64: 108 us without, 128 with; n=3e5, 40 entries,
+    // k=500: 1585 and 1237)
+    const bool fast = csr_fast<F>(k, increasing) && double(nnz) * k >= 2e9;
+    unsigned long long* xmax = nullptr;
+    if (fast) {
+        xmax = ctx->xmax.get<unsigned long long>(2);
+        fill<unsigned long long>(ctx, xmax, 2, 0ull);
+    }
     F* xs = ctx->csr_xs.get<F>(n);
     F* closest = ctx->csr_closest.get<F>(n);
     int32_t* labels = ctx->labels.get<int32_t>(n);
     hipLaunchKernelGGL(csr_row_squares_kernel<F>, dim3(grid_for(ctx, n, 256, 4)), dim3(256), 0,
-                       ctx->stream, x.vals, x.offs, x.base, n, xs);
+                       ctx->stream, x.vals, x.offs, x.base, n, xs, xmax);
     KM_LAUNCH_CHECK();
     F* Cd = ctx->c_cur.get<F>(int64_t(k) * d);
     KM_HIP(hipMemcpyAsync(Cd, C, sizeof(F) * k * d,
                           dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-    csr_assign<F>(ctx, x, Cd, k, xs, labels, closest);
+    work<F> w;  // the centroid step's view: max ||c_j||
+    csr_step_view(ctx, w, n, d, k);
+    if (fast) step_centroids<F>(ctx, w, 1, Cd);
+    csr_assign<F>(ctx, x, Cd, k, xs, labels, closest, fast, w.sel, csr_make_bounds(xmax, w.maxima, d, fp_traits<F>::u));
     int32_t* pin = ctx->pinned;
     const bool want_obj = flags & KM_FLAG_EXACT_OBJECTIVE;
     if (want_obj) {
+        if (fast) csr_all_closest<F>(ctx, x, Cd, k, xs, labels, closest);
         double* objp = csr_objective<F>(ctx, closest, n, nullptr);
         KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     }
@@ -2519,7 +2622,7 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
                         &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
                         &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->step_ticket, &ctx->step_max, &ctx->c_split, &ctx->c_pieces, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
-                        &ctx->csr_ct, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
+                        &ctx->csr_ct, &ctx->csr_cth, &ctx->csr_open, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();
     ctx->bws_fin.release();

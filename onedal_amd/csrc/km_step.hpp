@@ -20,6 +20,44 @@ namespace km {
 
 constexpr int STEP_MAX_GRID = 256;
 
+// feature f of the chunk sums q0 .. q1 - 1, added in chunk order (loads issued ahead)
+__device__ __forceinline__ double merge_chunks(const double* __restrict__ part, int q0, int q1, int d, int f) {
+    double sum = 0.0;
+    int q = q0;
+    for (; q + 16 <= q1; q += 16) {
+        double w[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) w[u] = part[int64_t(q + u) * d + f];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) sum = sum + w[u];
+    }
+    for (; q < q1; ++q) sum = sum + part[int64_t(q) * d + f];
+    return sum;
+}
+
+// Wide rows (d > STEP_MERGE_D): the merge and the division in a launch of their own, a
+// workgroup per centroid and 256 features, as the step's one workgroup per centroid
+// would read all of a large cluster's chunk sums (d = 2000, a cluster with a third of
+// n=1e6 rows: 480 us in the step, 63 us here; up to two slabs the extra launch costs more
+// than it gives: 5 us).
+constexpr int STEP_MERGE_D = 512;
+template <typename F>
+__global__ __launch_bounds__(256) void merge_centroids_kernel(const double* __restrict__ part,
+                                                              const int32_t* __restrict__ counts,
+                                                              const int32_t* __restrict__ chunk_base,
+                                                              const int32_t* __restrict__ changed, int k, int d,
+                                                              const F* __restrict__ cold, F* __restrict__ C) {
+    const int slabs = (d + 255) / 256;
+    for (int64_t e = blockIdx.x; e < int64_t(k) * slabs; e += gridDim.x) {
+        const int j = int(e / slabs), f = int(e % slabs) * 256 + threadIdx.x;
+        if (f >= d) continue;
+        const int64_t o = int64_t(j) * d + f;
+        const int32_t cnt = counts[j];
+        C[o] = cnt == 0 || !changed[j] ? cold[o]
+                                       : F(merge_chunks(part, chunk_base[j], chunk_base[j + 1], d, f) / double(cnt));
+    }
+}
+
 template <typename F>
 struct centroid_step {
     // new centroids from the chunk sums (null part: C holds them already)
@@ -57,6 +95,7 @@ struct centroid_step {
     // re-score counters: added into acc (when not null), then cleared
     int32_t* counters;
     unsigned long long* acc;
+    int32_t* csr_open;  // sparse rows (csr_bounds::open): the pass's counts become the previous ones
     // workspace of the launch: a ticket (0 between launches) and STEP_MAX_GRID x 4 maxima
     uint32_t* ticket;
     unsigned long long* wgmax;
@@ -83,23 +122,7 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
             const bool keep = cnt == 0 || !s.changed[j];
             const int q0 = s.chunk_base[j], q1 = s.chunk_base[j + 1];
             for (int f = t; f < d; f += 256) {
-                F v;
-                if (keep) {
-                    v = s.cold[o + f];
-                } else {
-                    double sum = 0.0;
-                    int q = q0;
-                    // loads issued ahead, adds kept in chunk order
-                    for (; q + 16 <= q1; q += 16) {
-                        double w[16];
-#pragma unroll
-                        for (int u = 0; u < 16; ++u) w[u] = s.part[int64_t(q + u) * d + f];
-#pragma unroll
-                        for (int u = 0; u < 16; ++u) sum = sum + w[u];
-                    }
-                    for (; q < q1; ++q) sum = sum + s.part[int64_t(q) * d + f];
-                    v = F(sum / double(cnt));
-                }
+                const F v = keep ? s.cold[o + f] : F(merge_chunks(s.part, q0, q1, d, f) / double(cnt));
                 s.C[o + f] = v;
                 row[f] = v;
             }
@@ -243,6 +266,12 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
     if (t < 3) {
         if (s.acc) s.acc[t] += (unsigned long long)s.counters[t];
         s.counters[t] = 0;
+    }
+    if (t == 0 && s.csr_open && s.cold && s.csr_open[1] > 0) {  // not again after a refill
+        s.csr_open[2] = s.csr_open[0];
+        s.csr_open[3] = s.csr_open[1];
+        s.csr_open[0] = 0;
+        s.csr_open[1] = 0;
     }
     if (t == 0) *s.ticket = 0u;
 }

@@ -384,43 +384,6 @@ __global__ __launch_bounds__(256) void reduce_chunks_vec_kernel(
     }
 }
 
-
-// ---------------------------------------------------------------------------
-// merge chunk sums per cluster (chunk order) and divide: C_j = (F)(S1_j / n_j).
-// A cluster whose members did not change keeps its centroid (the same sums give
-// the same bits).  Empty clusters are left for the ec_* kernels (refilled there).
-// ---------------------------------------------------------------------------
-template <typename F>
-__global__ __launch_bounds__(256) void finalize_centroids_kernel(
-    const double* __restrict__ part, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ chunk_base, const int32_t* __restrict__ changed, int k, int d,
-    const F* __restrict__ Ccur, F* __restrict__ Cnext) {
-    const int64_t total = int64_t(k) * d;
-    for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < total;
-         e += int64_t(gridDim.x) * blockDim.x) {
-        const int j = int(e / d), f = int(e % d);
-        const int32_t cnt = counts[j];
-        if (cnt == 0) continue;
-        if (!changed[j]) {
-            Cnext[e] = Ccur[e];
-            continue;
-        }
-        double s = 0.0;
-        int q = chunk_base[j];
-        const int q1 = chunk_base[j + 1];
-        // loads issued ahead, adds kept in chunk order
-        for (; q + 16 <= q1; q += 16) {
-            double v[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) v[u] = part[int64_t(q + u) * d + f];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) s = s + v[u];
-        }
-        for (; q < q1; ++q) s = s + part[int64_t(q) * d + f];
-        Cnext[e] = F(s / double(cnt));
-    }
-}
-
 // ---------------------------------------------------------------------------
 // objective: d64 per row against its label's centroid (row_d64_kernel), then, in a
 // fixed order: rows in chunks of OBJ_CHUNK; thread t of a chunk sums rows t, t+256,
