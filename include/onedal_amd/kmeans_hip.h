@@ -61,10 +61,10 @@ typedef enum {
                                         HIP graph and replay it */
 
 /* context options (km_context_set_option) */
-#define KM_OPT_ASSIGN_PATH 1 /* 0 auto, 1 generic tile kernel, 2 FP32 matrix core */
+#define KM_OPT_ASSIGN_PATH 1 /* 0 auto, 1 generic tile kernel, 2 matrix cores */
 #define KM_OPT_TIMING 2      /* 1: time the assignment kernels with HIP events */
 #define KM_OPT_BATCH_TILE 3  /* batched assignment tile: 0 the context's table (tuned by
-                                km_batch_autotune, else chosen by k), v + 1 force variant v
+                                km_batch_autotune, else the default table), v + 1 force variant v
                                 (0 <= v < KM_BATCH_TILE_VARIANTS) */
 
 /* Tile variants of the batched assignment.  Variants 0..6 compute the exact
@@ -88,7 +88,7 @@ typedef struct {
     int64_t refined_candidate_rows; /* rows settled by the candidate re-score */
     int64_t refined_full_rows;      /* rows re-scored against every centroid */
     int64_t empty_cluster_events;   /* iterations that refilled empty clusters */
-    int32_t assign_path;            /* path used: 1 generic, 2 FP32 MFMA, 3 BF16 MFMA */
+    int32_t assign_path;            /* path used: 1 generic, 2 matrix cores (FP32 results), 3 BF16 */
     int32_t reserved;
     int64_t refined_collect_rows;   /* BF16 path: rows whose candidates were re-collected */
 } km_stats;
