@@ -1639,7 +1639,7 @@ __global__ __launch_bounds__(256) void batch_labels_out_kernel(const batch_inst*
 }
 
 // Objective chunk sums from the rows' d64 (batch_d64_kernel): OBJ_CHUNK rows of
-// one instance per workgroup, in the order of objective_chunks_kernel (thread t
+// one instance per workgroup, in the order of objective_sum_kernel (thread t
 // sums rows t, t+256, ...; tree of the 256 partials).
 __global__ __launch_bounds__(256) void batch_objective_kernel(const batch_inst* __restrict__ I, int B,
                                                               const int64_t* __restrict__ pre,

@@ -11,7 +11,7 @@
 //     inside the bound.
 //   * centroid sums in double, in a fixed order (REDUCE_CHUNK, reduce_groups);
 //     C_j = (F)(S1_j / count_j).
-//   * objective = sum_i d64_i in a fixed order (objective_chunks_kernel), d64 =
+//   * objective = sum_i d64_i in a fixed order (objective_sum_kernel), d64 =
 //     sum_f ((double)x_f - (double)c_f)^2.
 // All code here is compiled with -ffp-contract=off: fused multiply-adds appear
 // only where fma() is written out.
