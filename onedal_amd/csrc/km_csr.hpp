@@ -439,7 +439,7 @@ struct csr_bounds {
 // needed, for one centroid a row.
 //
 // Bound by a row's instructions, not by bytes (n=1e6, 20 entries, k=256: about 300 vector
-// instructions a row, a third of them products): 0.8 ms for all rows, 1.3 ms for the exact
+// instructions a row, a third of them products): 0.8 to 1.0 ms for all rows, 1.3 ms for the exact
 // dots.  The bookkeeping matters as much as the reads: with the bounds' double arithmetic
 // done per row by a whole wave, FAST took 1.43 ms, with a read at a time for a row's last
 // entries 1.3 ms.

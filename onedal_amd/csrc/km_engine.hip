@@ -1305,7 +1305,7 @@ static csr_view<F> csr_prepare(km_ctx* ctx, const F* vals, const int64_t* cols,
 }
 
 // Half-precision distances first (csr_assign_kernel, FAST): rows whose columns increase strictly, and
-// at most one block of centroids.  n=1e6, 20 entries a row, k=256: 0.8 ms a pass
+// at most one block of centroids.  n=1e6, 20 entries a row, k=256: 0.8-1.0 ms a pass
 // against 1.3 ms.  Columns in another order may repeat, and then the entries' norm does
 // not bound the products; past one block the rough values would have to be kept.
 template <typename F>
