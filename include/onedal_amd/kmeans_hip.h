@@ -61,7 +61,8 @@ typedef enum {
                                         HIP graph and replay it */
 
 /* context options (km_context_set_option) */
-#define KM_OPT_ASSIGN_PATH 1 /* 0 auto, 1 generic tile kernel, 2 matrix cores */
+#define KM_OPT_ASSIGN_PATH 1 /* 0 auto, 1 generic tile kernel, 2 FP32 matrix core (float; past
+                                256 columns the generic kernel) */
 #define KM_OPT_TIMING 2      /* 1: time the assignment kernels with HIP events */
 #define KM_OPT_BATCH_TILE 3  /* batched assignment tile: 0 the context's table (tuned by
                                 km_batch_autotune, else the default table), v + 1 force variant v

@@ -268,11 +268,11 @@ static int pad_dim(int d) {
 // 1 generic tile kernel, 2 matrix cores with the precision of the data's (float:
 // split BF16 products, or FP32), 3 BF16 matrix cores + exact re-score.  BF16 applies to
 // float data with d <= 256; double data takes path 2 for d <= 256, else path 1; float
-// data takes path 1 past 256 columns and the limits of use_wide, or when asked to.
+// data takes path 1 past 256 columns where use_wide does not hold, or when asked to.
 template <typename F>
 static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
     if (std::is_same<F, double>::value) return (d <= 256 && ctx->assign_path_opt != 1) ? 2 : 1;
-    if (d > 256) return ctx->assign_path_opt == 1 || k > SPLIT_MAX_K ? 1 : 2;
+    if (d > 256) return ctx->assign_path_opt != 0 || k > SPLIT_MAX_K ? 1 : 2;
     // keys carry (block, register) in at most 15 low bits: k <= 65536
     if ((flags & KM_FLAG_BF16_REFINE) && k <= 65536) return 3;
     if (ctx->assign_path_opt == 1) return 1;
@@ -281,10 +281,12 @@ static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
 
 // float data on path 2, and on path 3 for rows assigned once (inference): split BF16
 // products (km_assign_split.hpp) where a row's halves fit a lane's registers and the
-// key's index bits leave the band narrow.  Path 2 takes FP32 products past that, path
-// 3 a BF16 copy of the rows.  double data: never.
-static bool use_split(int path, int d, int k, bool once) {
-    return (path == 2 || (path == 3 && once)) && d <= 128 && k <= SPLIT_MAX_K;
+// key's index bits leave the band narrow.  Path 2 takes FP32 products past that and where
+// the caller asked for them (KM_OPT_ASSIGN_PATH 2), path 3 a BF16 copy of the rows.
+// double data: never.
+static bool use_split(const km_ctx* ctx, int path, int d, int k, bool once) {
+    if (d > 128 || k > SPLIT_MAX_K) return false;
+    return path == 2 ? ctx->assign_path_opt == 0 : path == 3 && once;
 }
 
 // float data on path 2 with wider rows: split products in chunks (km_assign_wide.hpp).
@@ -292,7 +294,9 @@ static bool use_split(int path, int d, int k, bool once) {
 // on (n, d, k) took (500, 300, 5) 134 -> 96 us, (2000, 129, 3) 91 -> 66, (1e6, 300, 5)
 // 1463 -> 459, (1e5, 130, 2000) 2084 -> 1056, (2e4, 4000, 50) 1431 -> 965 (the whole
 // inference call, which other kernels made faster as well).
-static bool use_wide(int path, int d, int k) { return path == 2 && d > 128 && k <= SPLIT_MAX_K; }
+static bool use_wide(const km_ctx* ctx, int path, int d, int k) {
+    return path == 2 && ctx->assign_path_opt == 0 && d > 128 && k <= SPLIT_MAX_K;
+}
 static int wide_columns(int k) { return k <= 128 ? 2 : 4; }  // waves across the centroids
 
 template <typename F>
@@ -885,8 +889,8 @@ static int32_t* launch_empty_clusters(km_ctx* ctx, const F* X, int64_t n, int d,
 template <typename F>
 static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, int k,
                        int path, bool once, arena* A = nullptr, int32_t* labels_into = nullptr, bool wide = true) {
-    w.split = std::is_same<F, float>::value && use_split(path, d, k, once);
-    w.wide = std::is_same<F, float>::value && wide && use_wide(path, d, k);
+    w.split = std::is_same<F, float>::value && use_split(ctx, path, d, k, once);
+    w.wide = std::is_same<F, float>::value && wide && use_wide(ctx, path, d, k);
     const bool vec_view = path == 2 && !w.split && !w.wide;
     w.n = n;
     w.d = d;
@@ -1157,7 +1161,7 @@ static size_t noalloc_block_bytes(const km_ctx* ctx, int path, int64_t R, int d,
     int64_t b = R * (4 + 4 + 4 + 4 * int64_t(MAXC) + 4) + 16 + int64_t(sizeof(F)) * k +
                 (wide ? int64_t(wide_kp(k, wide_columns(k))) * (wide_chunks(d) * 128 + 4) : int64_t(sizeof(F)) * k * dpad) +
                 32;
-    const bool split = use_split(path, d, k, true);
+    const bool split = use_split(ctx, path, d, k, true);
     if (split) b += 36 * int64_t(bf16_padded_k(k)) + 4 * int64_t(bf16_padded_k(k) - k) * dpad;
     if (path == 2 && !split && !wide && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
     if (path == 3 && split) b += 4 * R;
@@ -1192,7 +1196,7 @@ static void infer_noalloc(km_ctx* ctx, const float* X, int64_t n, int64_t d64_, 
     // the padded operand of the wide kernel, where it fits; else the older kernels (the
     // generic one past 256 columns)
     const int64_t least = std::min<int64_t>(n, OBJ_CHUNK);
-    const bool wide = use_wide(path, d, k) && noalloc_block_bytes<F>(ctx, path, least, d, k, pad_x, want_obj, true) <= cap;
+    const bool wide = use_wide(ctx, path, d, k) && noalloc_block_bytes<F>(ctx, path, least, d, k, pad_x, want_obj, true) <= cap;
     if (!wide && path == 2 && d > 256) path = 1;
     // largest block: a multiple of OBJ_CHUNK rows (or all rows) that fits
     int64_t R = std::min<int64_t>(n, int64_t(1) << 22);
