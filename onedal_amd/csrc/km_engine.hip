@@ -234,12 +234,12 @@ struct work {
     uint16_t* Cb = nullptr;       // k x dpad bf16(-2 c)
     float* cnb = nullptr;         // ||c||^2 + B (rounded up), 32 * ceil(k / 32) entries
     bf16_params* params = nullptr;
-    // split path (path 2, float; and path 3 for rows assigned once): both bf16 halves of
+    // split path (path 2, float; and path 3 for rows assigned once): the bf16 pieces of
     // -2 c, and the norm pieces
     bool split = false;
-    uint16_t* Csp = nullptr;  // bf16_padded_k(k) x 2 dpad
+    uint16_t* Csp = nullptr;  // bf16_padded_k(k) x SPLIT_PIECES dpad
     uint16_t* cnp = nullptr;  // bf16_padded_k(k) x 16
-    // wide rows (path 2, float, d > 128): both halves chunk by chunk, kpw rows, and norms
+    // wide rows (path 2, float, d > 128): the pieces chunk by chunk, kpw rows, and norms
     bool wide = false;
     int nwc = 0, kpw = 0;
     uint16_t* Cw = nullptr;
@@ -265,8 +265,8 @@ static int pad_dim(int d) {
     return p;
 }
 
-// 1 generic tile kernel, 2 matrix cores with the precision of the data's (float:
-// split BF16 products, or FP32), 3 BF16 matrix cores + exact re-score.  BF16 applies to
+// 1 generic tile kernel, 2 matrix cores with the precision of the data's (float: split
+// BF16 products, or FP32 products), 3 BF16 matrix cores + exact re-score.  BF16 applies to
 // float data with d <= 256; double data takes path 2 for d <= 256, else path 1; float
 // data takes path 1 past 256 columns where use_wide does not hold, or when asked to.
 template <typename F>
@@ -280,20 +280,20 @@ static int choose_path(const km_ctx* ctx, int d, int k, uint32_t flags) {
 }
 
 // float data on path 2, and on path 3 for rows assigned once (inference): split BF16
-// products (km_assign_split.hpp) where a row's halves fit a lane's registers and the
-// key's index bits leave the band narrow.  Path 2 takes FP32 products past that and where
+// products (km_assign_split.hpp) where a row's pieces fit a lane's registers, no narrower
+// than SPLIT_MIN_D and up to SPLIT_MAX_K.  Path 2 takes FP32 products past that and where
 // the caller asked for them (KM_OPT_ASSIGN_PATH 2), path 3 a BF16 copy of the rows.
 // double data: never.
 static bool use_split(const km_ctx* ctx, int path, int d, int k, bool once) {
     if (d > 128 || k > SPLIT_MAX_K) return false;
-    return path == 2 ? ctx->assign_path_opt == 0 : path == 3 && once;
+    return path == 2 ? ctx->assign_path_opt == 0 && d >= SPLIT_MIN_D : path == 3 && once;
 }
 
-// float data on path 2 with wider rows: split products in chunks (km_assign_wide.hpp).
-// From the first width past the split kernel's row registers and for any n and k: a call
-// on (n, d, k) took (500, 300, 5) 134 -> 96 us, (2000, 129, 3) 91 -> 66, (1e6, 300, 5)
-// 1463 -> 459, (1e5, 130, 2000) 2084 -> 1056, (2e4, 4000, 50) 1431 -> 965 (the whole
-// inference call, which other kernels made faster as well).
+// float data on path 2 with wider rows: split products in chunks (km_assign_wide.hpp),
+// from the first width past the split kernel's row registers and for any n and k up to
+// SPLIT_MAX_K: an inference call on (n, d, k) takes (500, 300, 5) 112 us, 125 with the kernels
+// before it, (2000, 129, 3) 75 and 88, (1e6, 300, 5) 684 and 1458, (1e5, 130, 2000) 1224 and
+// 2092, (2e4, 4000, 50) 1091 and 1424.
 static bool use_wide(const km_ctx* ctx, int path, int d, int k) {
     return path == 2 && ctx->assign_path_opt == 0 && d > 128 && k <= SPLIT_MAX_K;
 }
@@ -414,64 +414,76 @@ static void launch_mfma_f32(km_ctx* ctx, work<float>& w, const band_consts& bc) 
         launch_mfma_f32_mode<DP, NB, false>(ctx, w, bc, grid, mfma_f32_lds_bytes(DP, w.k, false));
 }
 
-template <int TERMS>
-static split_consts make_split_consts(int d, int k) {
-    split_consts c;
+static bf16_split_consts make_bf16_split_consts(int d, int k) {
+    bf16_split_consts c;
     int mbits = 0;
     while ((1 << mbits) < bf16_padded_k(k) / 32) mbits++;
     c.ib = 4 + mbits;
-    const double ua = fp_traits<float>::u_acc;
-    c.xc = float(gamma_m(double(d), ua) * 2.04);
-    if (TERMS == 3) c.xc += float(std::ldexp(6.02, -18) + gamma_m(2.0 * d, ua) * 2.02 / 256.0);
-    c.sum = float(gamma_m(8.0, ua) * 1.02);
+    c.xc = float(gamma_m(double(d), fp_traits<float>::u_acc) * 2.04);
+    c.sum = float(gamma_m(8.0, fp_traits<float>::u_acc) * 1.02);
     c.trunc = float(std::ldexp(1.0, c.ib - 23));
     const double g = gamma_m(double(d + 2), fp_traits<float>::u);
     c.g_canon = float(g / (1.0 - g)) * (1.0f + 2.4e-7f);
     return c;
 }
 
-static split_consts make_wide_consts(int d, int k, int kp) {
-    split_consts c = make_split_consts<3>(d, k);
-    int mbits = 0;
-    while ((1 << mbits) < kp / 32) mbits++;
-    c.ib = 4 + mbits;
-    c.trunc = float(std::ldexp(1.0, c.ib - 23));
-    c.xc = float(std::ldexp(6.02, -18) + gamma_m(3.0 * d, fp_traits<float>::u_acc) * 2.04);
+// what is left out of the products, the chains of additions, and the rounded norm
+// (km_assign_split.hpp, km_assign_wide.hpp)
+static split_consts make_split_consts(int d, bool wide) {
+    const double u = fp_traits<float>::u, ua = fp_traits<float>::u_acc;
+    split_consts c;
+    c.xc = std::ldexp(1.05, -25) + gamma_m(5.0 * d, ua) * 2.03 / 256.0 + gamma_m(double(d), ua) * 2.02;
+    c.cc = 1.01 * u + gamma_m(double(d), 2.220446049250313e-16);
+    if (wide) {
+        c.xc += 2.0 * u * 2.05;
+        c.cc += u * 1.01;
+        c.tiny = 1e-33;  // up to 6 x 4096 products
+    } else {
+        c.xc += gamma_m(4.0, ua) * 2.05;
+        c.cc += gamma_m(4.0, ua) * 1.01;
+        c.tiny = 2e-35;
+    }
+    const double g = gamma_m(double(d + 2), u);
+    c.g_canon = g / (1.0 - g);
     return c;
 }
 
-// terms 3, or 1 (BF16 distances of rows assigned once); sel: the rows
-template <int DP, int NB, int TERMS>
+// pieces 3, or 1 (BF16 distances of rows assigned once); sel: the rows
+template <int DP, int NB, int PIECES>
 static void launch_split(km_ctx* ctx, work<float>& w, const row_select& sel) {
     constexpr int ROWS_PER_WG = 4 * 32 * NB;
     const int64_t tiles = (w.n + ROWS_PER_WG - 1) / ROWS_PER_WG;
     const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * 2)));
-    const size_t lds = split_lds_bytes(DP, TERMS);
-    auto kern = assign_split_kernel<DP, NB, TERMS>;
+    const size_t lds = split_lds_bytes(DP, PIECES);
+    auto kern = assign_split_kernel<DP, NB, PIECES>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.X, w.n, w.d, w.Csp, w.cnp, w.k, w.maxima,
-                       make_split_consts<TERMS>(w.d, w.k), w.labels, w.L, sel);
+    if constexpr (PIECES == 3)
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.X, w.n, w.d, w.Csp, w.cnp, w.k, w.maxima,
+                           make_split_consts(w.d, false), w.labels, w.L, sel);
+    else
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, ctx->stream, w.X, w.n, w.d, w.Csp, w.cnp, w.k, w.maxima,
+                           make_bf16_split_consts(w.d, w.k), w.labels, w.L, sel);
     KM_LAUNCH_CHECK();
 }
 
-template <int TERMS>
+template <int PIECES>
 static void launch_split(km_ctx* ctx, work<float>& w, const row_select& sel) {
     switch (w.dpad) {
-        case 32: launch_split<32, 2, TERMS>(ctx, w, sel); break;
-        case 64: launch_split<64, 2, TERMS>(ctx, w, sel); break;
-        default: launch_split<128, TERMS == 3 ? 1 : 2, TERMS>(ctx, w, sel); break;
+        case 32: launch_split<32, 2, PIECES>(ctx, w, sel); break;
+        case 64: launch_split<64, 2, PIECES>(ctx, w, sel); break;
+        default: launch_split<128, PIECES == 3 ? 1 : 2, PIECES>(ctx, w, sel); break;
     }
 }
 
 template <int NWC>
 static void launch_wide(km_ctx* ctx, work<float>& w) {
-    const int64_t tiles = (w.n + WIDE_ROWS - 1) / WIDE_ROWS;
-    const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count) * (NWC == 2 ? 2 : 1))));
+    const int64_t tiles = (w.n + wide_rows(NWC) - 1) / wide_rows(NWC);
+    const int grid = int(std::max<int64_t>(1, std::min<int64_t>(tiles, int64_t(ctx->cu_count))));
     const size_t lds = wide_lds_bytes(NWC);
     auto kern = assign_wide_kernel<NWC>;
     KM_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(128 * NWC), lds, ctx->stream, w.X, w.n, w.d, w.Cw, w.cnw, w.k, w.kpw,
-                       w.maxima, make_wide_consts(w.d, w.k, w.kpw), w.labels, w.L, w.sel);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, ctx->stream, w.X, w.n, w.d, w.Cw, w.cnw, w.k, w.kpw,
+                       w.maxima, make_split_consts(w.d, true), w.labels, w.L, w.sel);
     KM_LAUNCH_CHECK();
 }
 
@@ -559,7 +571,7 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
     }
     if constexpr (std::is_same<F, float>::value) {
         if (w.split && path == 3) {
-            // rows that one term leaves open: three terms
+            // rows that one piece leaves open: three pieces
             launch_split<1>(ctx, w, w.sel);
             launch_split<3>(ctx, w, {w.L.coll_rows, w.L.counters + 2, nullptr, nullptr, 0.0});
         } else if (w.split) {
@@ -898,7 +910,8 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
     w.dpad = pad_dim(d);
     w.X = Xd;
     w.A = A;
-    w.xnorm = take<float>(ctx, &km_ctx::xnorm, A, n);
+    const bool norms = !w.split && !w.wide;  // their kernels form the rows' norms themselves
+    if (norms) w.xnorm = take<float>(ctx, &km_ctx::xnorm, A, n);
     w.labels = labels_into ? labels_into : take<int32_t>(ctx, &km_ctx::labels, A, n);
     w.L.cand_rows = take<int32_t>(ctx, &km_ctx::lists_rows, A, n);
     w.L.cand_count = take<int32_t>(ctx, &km_ctx::lists_cnt, A, n);
@@ -907,12 +920,12 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
     w.L.counters = take<int32_t>(ctx, &km_ctx::lists_counters, A, 3);
     w.cn = take<F>(ctx, &km_ctx::cn, A, k);
     if (w.split) {
-        w.Csp = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(bf16_padded_k(k)) * 2 * w.dpad);
+        w.Csp = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(bf16_padded_k(k)) * SPLIT_PIECES * w.dpad);
         w.cnp = take<uint16_t>(ctx, &km_ctx::c_pieces, A, int64_t(bf16_padded_k(k)) * 16);
     } else if (w.wide) {
         w.nwc = wide_columns(k);
         w.kpw = wide_kp(k, w.nwc);
-        w.Cw = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(w.kpw) * wide_chunks(d) * 64);
+        w.Cw = take<uint16_t>(ctx, &km_ctx::c_split, A, int64_t(w.kpw) * wide_chunks(d) * WIDE_ROW);
         w.cnw = take<float>(ctx, &km_ctx::c_pieces, A, w.kpw);
     } else {
         w.cpad = take<F>(ctx, &km_ctx::cpad, A, int64_t(k) * w.dpad);
@@ -930,11 +943,8 @@ static void setup_work(km_ctx* ctx, work<F>& w, const F* Xd, int64_t n, int d, i
         w.Xv = xp;
         w.ldx = ldx;
     }
-    if (w.split) {  // its kernel forms the norms itself
-        if (path == 3) w.L.coll_rows = take<int32_t>(ctx, &km_ctx::coll_rows, A, n);
-        return;
-    }
-    if (w.wide) return;
+    if (w.split && path == 3) w.L.coll_rows = take<int32_t>(ctx, &km_ctx::coll_rows, A, n);
+    if (!norms) return;
     const int grid = grid_for(ctx, n * 64, 256, 8);
     if constexpr (std::is_same<F, float>::value) {
         if (path == 3) {
@@ -1158,11 +1168,11 @@ template <typename F>
 static size_t noalloc_block_bytes(const km_ctx* ctx, int path, int64_t R, int d, int k, bool pad_x,
                                   bool want_obj, bool wide) {
     const int64_t dpad = pad_dim(d);
-    int64_t b = R * (4 + 4 + 4 + 4 * int64_t(MAXC) + 4) + 16 + int64_t(sizeof(F)) * k +
-                (wide ? int64_t(wide_kp(k, wide_columns(k))) * (wide_chunks(d) * 128 + 4) : int64_t(sizeof(F)) * k * dpad) +
-                32;
     const bool split = use_split(ctx, path, d, k, true);
-    if (split) b += 36 * int64_t(bf16_padded_k(k)) + 4 * int64_t(bf16_padded_k(k) - k) * dpad;
+    const int64_t operand = wide    ? int64_t(wide_kp(k, wide_columns(k))) * (wide_chunks(d) * WIDE_ROW * 2 + 4)
+                            : split ? int64_t(bf16_padded_k(k)) * (SPLIT_PIECES * 2 * dpad + 32)
+                                    : int64_t(sizeof(F)) * k * dpad;
+    int64_t b = R * (4 + 4 + 4 + 4 * int64_t(MAXC) + (split || wide ? 0 : 4)) + 16 + int64_t(sizeof(F)) * k + operand + 32;
     if (path == 2 && !split && !wide && pad_x) b += R * ((d + 3) / 4 * 4) * int64_t(sizeof(F));
     if (path == 3 && split) b += 4 * R;
     if (path == 3 && !split) {

@@ -58,6 +58,16 @@ __global__ __launch_bounds__(256) void merge_centroids_kernel(const double* __re
     }
 }
 
+// the bf16 pieces of v, `stride` apart
+__device__ __forceinline__ void split_feature(float v, uint16_t* out, int stride) {
+#pragma unroll
+    for (int p = 0; p < SPLIT_PIECES; ++p) {
+        const uint16_t b = f2bf(v);
+        out[p * stride] = b;
+        v -= bf2f(b);
+    }
+}
+
 template <typename F>
 struct centroid_step {
     // new centroids from the chunk sums (null part: C holds them already)
@@ -72,11 +82,11 @@ struct centroid_step {
     F* cn;
     F* cpad;
     uint16_t* Cb;
-    // or (Csp) rows of both bf16 halves of -2 c and (cnp) the pieces of ||c_j||^2 for the
+    // or (Csp) rows of the three bf16 pieces of -2 c and (cnp) the pieces of ||c_j||^2 for the
     // norm step of assign_split_kernel, kp rows
     uint16_t* Csp;
     uint16_t* cnp;
-    // or (Cw) both halves chunk by chunk for assign_wide_kernel, kp rows, and their norms
+    // or (Cw) the pieces chunk by chunk for assign_wide_kernel, kp rows, and their norms
     uint16_t* Cw;
     float* cnw;
     int kp;
@@ -134,20 +144,12 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
             for (int f = t; f < dpad; f += 256)  // exact: -2 * bf16(c)
                 s.Cb[int64_t(j) * dpad + f] = f < d ? f2bf(-2.0f * bf2f(f2bf(float(row[f])))) : uint16_t(0);
         } else if (s.Csp) {
-            uint16_t* o2 = s.Csp + int64_t(j) * 2 * dpad;
-            for (int f = t; f < dpad; f += 256) {
-                const float v = f < d ? -2.0f * float(row[f]) : 0.f;
-                const uint16_t hi = f2bf(v);
-                o2[f] = hi;
-                o2[dpad + f] = f2bf(v - bf2f(hi));
-            }
+            uint16_t* o3 = s.Csp + int64_t(j) * SPLIT_PIECES * dpad;
+            for (int f = t; f < dpad; f += 256) split_feature(f < d ? -2.0f * float(row[f]) : 0.f, o3 + f, dpad);
         } else if (s.Cw) {
             for (int f = t; f < 32 * wide_chunks(d); f += 256) {
-                const float v = f < d ? -2.0f * float(row[f]) : 0.f;
-                const uint16_t hi = f2bf(v);
-                uint16_t* o2 = s.Cw + (int64_t(f >> 5) * s.kp + j) * 64 + (f & 31);
-                o2[0] = hi;
-                o2[32] = f2bf(v - bf2f(hi));
+                uint16_t* o3 = s.Cw + (int64_t(f >> 5) * s.kp + j) * WIDE_ROW + (f & 31);
+                split_feature(f < d ? -2.0f * float(row[f]) : 0.f, o3, 32);
             }
         } else if (s.cpad) {
             for (int f = t; f < dpad; f += 256) s.cpad[int64_t(j) * dpad + f] = f < d ? row[f] : F(0);
@@ -209,16 +211,15 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
     if (s.Cw) {
         for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x) {
             for (int f = t; f < 32 * wide_chunks(d); f += 256) {
-                uint16_t* o2 = s.Cw + (int64_t(f >> 5) * s.kp + j) * 64 + (f & 31);
-                o2[0] = 0;
-                o2[32] = 0;
+                uint16_t* o3 = s.Cw + (int64_t(f >> 5) * s.kp + j) * WIDE_ROW + (f & 31);
+                for (int p = 0; p < SPLIT_PIECES; ++p) o3[32 * p] = 0;
             }
             if (t == 0) s.cnw[j] = __uint_as_float(0x7F000000u);
         }
     }
     if (s.Csp) {  // padding: zero rows with a norm of 2^127, which no threshold reaches
         for (int j = k + blockIdx.x; j < s.kp; j += gridDim.x) {
-            for (int f = t; f < 2 * dpad; f += 256) s.Csp[int64_t(j) * 2 * dpad + f] = 0;
+            for (int f = t; f < SPLIT_PIECES * dpad; f += 256) s.Csp[int64_t(j) * SPLIT_PIECES * dpad + f] = 0;
             if (t < 16) s.cnp[int64_t(j) * 16 + t] = t == 0 ? uint16_t(0x7F00u) : uint16_t(0);
         }
     }
