@@ -577,8 +577,8 @@ def run_csr(torch, args, wl):
     flops = 2.0 * n * m * k  # one product and sum per stored entry and centroid
     tflops = flops / (avg_ms * 1e-3) / 1e12
     # the assignment's dominant traffic: per stored entry, one centroid column of k
-    # half-precision values gathered through the caches (k*d*2 B, which stay in L2)
-    gather_gbs = n * m * k * 2 / (avg_ms * 1e-3) / 1e9
+    # values gathered through the caches (k*d*4 B, which stay in L2)
+    gather_gbs = n * m * k * 4 / (avg_ms * 1e-3) / 1e9
     cpu = None
     if not args.no_cpu_baseline:
         log("cpu baseline ...")
@@ -613,7 +613,8 @@ def run_csr(torch, args, wl):
                    "iterations": iters, "method": "lloyd_csr"},
         "roofline": {"bound": "valu", "achieved": round(tflops, 2), "peak": PEAK["fp32_vector_tflops"],
                      "unit": "TFLOP/s", "frac": round(tflops / PEAK["fp32_vector_tflops"], 4), "traffic": None,
-                     "kernel": "csr_assign_kernel: 2*nnz*k flops (mixed FMA) of a pass over every row",
+                     "kernel": "csr_assign_kernel: 2*nnz*k flops of a pass over every row (separate multiply "
+                               "and add, so the vector units' ceiling is half the FMA peak)",
                      "full_launch_ms": round(avg_ms, 4),
                      "avg_launch_ms_over_steps": round(asg_ms / max(1, launches), 4), "cache_gather_gbs": round(gather_gbs, 1)},
         "cpu_baseline": cpu,

@@ -132,23 +132,13 @@ __global__ __launch_bounds__(256) void csr_row_squares_kernel(const F* __restric
     if ((threadIdx.x & 63) == 0) atomicMax(xmax, top);
 }
 
-// power of two that brings values up to cmax to at most 2^15
-__device__ __forceinline__ double csr_half_scale(double cmax) {
-    int x = 0;
-    frexp(cmax < BOUND_MAX ? cmax : 1.0, &x);
-    return ldexp(1.0, min(15 - x, 120));
-}
-
 // Ct (d x kp) = C^T, rows padded with zeros to kp (a multiple of the 16-byte
-// vector), and (when given) Cth, the same in half precision times csr_half_scale, for coalesced vector reads over centroids: 64 x 64 tiles through LDS
+// vector), for coalesced vector reads over centroids: 64 x 64 tiles through LDS
 // (grid: ceil(d/64) x up to 65535 workgroups of 256 threads, striding over k)
 template <typename F>
 __global__ __launch_bounds__(256) void csr_transpose_kernel(const F* __restrict__ C, int64_t k,
-                                                            int64_t kp, int64_t d, F* __restrict__ Ct,
-                                                            _Float16* __restrict__ Cth,
-                                                            const double* __restrict__ cmax) {
+                                                            int64_t kp, int64_t d, F* __restrict__ Ct) {
     __shared__ F tile[64][65];
-    const F scale = Cth ? F(csr_half_scale(*cmax)) : F(1);
     const int64_t f0 = int64_t(blockIdx.x) * 64;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     for (int64_t j0 = int64_t(blockIdx.y) * 64; j0 < kp; j0 += int64_t(gridDim.y) * 64) {
@@ -159,11 +149,7 @@ __global__ __launch_bounds__(256) void csr_transpose_kernel(const F* __restrict_
         __syncthreads();
         for (int r = ty; r < 64; r += 4) {
             const int64_t f = f0 + r, j = j0 + tx;
-            if (j < kp && f < d) {
-                const F v = j < k ? tile[tx][r] : F(0);
-                Ct[f * kp + j] = v;
-                if (Cth) Cth[f * kp + j] = _Float16(float(v * scale));
-            }
+            if (j < kp && f < d) Ct[f * kp + j] = j < k ? tile[tx][r] : F(0);
         }
         __syncthreads();
     }
@@ -247,6 +233,8 @@ __device__ __forceinline__ T dpp_from(T x) {
 __device__ __forceinline__ float lower(float a, float b) { return fminf(a, b); }
 __device__ __forceinline__ double lower(double a, double b) { return fmin(a, b); }
 __device__ __forceinline__ int lower(int a, int b) { return min(a, b); }
+__device__ __forceinline__ float higher(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ double higher(double a, double b) { return fmax(a, b); }
 template <typename T>
 __device__ __forceinline__ T wave_lowest(T x) {
     x = lower(x, dpp_from<0x111, 0xf>(x));  // row_shr 1, 2, 4, 8: lane 15 of each row of 16
@@ -298,28 +286,65 @@ __device__ __forceinline__ void csr_take(F& bs, int& bj, bool& has, F s, int j) 
     }
 }
 
-// The exact dots for k past 128 VEC centroids (without FAST), several blocks of them.
+// Bounds (km_bounds.hpp) for rows whose columns increase strictly (so that the stored
+// entries are a vector).  The label is the smallest computed s_ij, whose error is
+//     |s_ij - (||c_j||^2 - 2 x.c_j)| <= g (||c_j||^2 + 2 ||x|| ||c_j||) <= 3 g M^2,
+// g = gamma_{d+4} and M the largest norm of a row or centroid: not relative to the
+// distance, as the dense form's.  With d_j - d_a >= G > 0 for every other centroid,
+// d_j^2 - d_a^2 >= G^2, so a row stays settled while G > sqrt(2 * 3 g M^2): that part is
+// taken off its gap when it is settled.  M may be taken at that time: later centroids
+// are means of rows, rows, or unchanged.
+struct csr_bounds {
+    const unsigned long long* xmax;  // csr_row_squares_kernel
+    const double* cmax;              // max ||c_j||, rounded up
+    double g;                        // gamma_{d+4}
+};
+
+// gap of a row settled with the smallest s (best) and the next one (second, a float at most
+// as large; the wave's lowest float takes a fifth of the instructions of a double), xs its squares;
+// loose: band's worth of rounding in best besides its own
+__device__ __forceinline__ float csr_gap(double best, double second, double xs, double band, double loose,
+                                         const row_select& rs, int lab) {
+    if (!(band < BOUND_MAX) || best != best) return -__builtin_inff();
+    const float g = bound_gap(best + xs + (4.5 + loose) * band, second - 4.5 * band + xs, rs.gam, rs.base[lab]);
+    return float_below(double(g) - sqrt(6.3 * band));
+}
+// g M^2
+__device__ __forceinline__ double csr_band(const csr_bounds& kb) {
+    const double C = *kb.cmax;
+    const double M = fmax(sqrt(__longlong_as_double((long long)*kb.xmax)) * (1.0 + kb.g), C) * (1.0 + 1e-6);
+    return M < BOUND_MAX && C < BOUND_MAX ? kb.g * M * M : __builtin_inf();  // NaN as well
+}
+
+// The dots where csr_assign_kernel's runs of rows are slower: transposed centroids past an
+// XCD's L2, or more than 128 VEC of them.
 // One wave per row.  Lane l accumulates the dots of the VEC consecutive
 // centroids jb + VEC (l + 64 t) + e (t < JT, e < VEC) over the row's entries,
 // which are loaded 64 at a time and taken in stored order from their lanes;
 // each entry reads one 16-byte vector of its transposed-centroid row per t.  Few
-// registers, so that eight waves a SIMD hide the reads, which miss the L2 here: k = 1000 in
-// double, n=3e5, 20 entries takes 3.8 ms, 4.5 ms with csr_assign_kernel's runs of rows.
-// Then each lane's best and a wave reduction (ties to the lower j).
-template <typename F>
-__global__ __launch_bounds__(256) void csr_assign_blocks_kernel(
+// registers, so that eight waves a SIMD hide the reads, which miss the L2 here: k = 500, d = 4000,
+// n=3e5, 40 entries takes 1.51 ms, 1.68 ms with runs of rows (double: 2.8 and 5.0), 2.05 with
+// a lane's four reads issued together.
+// Then each lane's best and a wave reduction (ties to the lower j).  BND: the rows of rs,
+// and the second best of each, from which csr_gap_kernel forms the gaps (3.3 ms a pass in
+// double for the same rows).
+template <typename F, bool BND>
+__global__ __launch_bounds__(256, 8) void csr_assign_blocks_kernel(
     const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs,
     int64_t base, int64_t n, int k, int kp, const F* __restrict__ Ct, const F* __restrict__ cs,
-    const F* __restrict__ xs, int32_t* __restrict__ labels, F* __restrict__ closest) {
+    const F* __restrict__ xs, int32_t* __restrict__ labels, F* __restrict__ closest, row_select rs,
+    float* __restrict__ second) {
     constexpr int VEC = csr_vec<F>::N;
     constexpr int JT = 4;
     typedef typename csr_vec<F>::type V;
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
     const int64_t nwaves = (int64_t(gridDim.x) * blockDim.x) >> 6;
-    for (int64_t i = wave; i < n; i += nwaves) {
+    const int64_t nsel = BND ? select_rows(rs, n) : n;
+    for (int64_t r = wave; r < nsel; r += nwaves) {
+        const int64_t i = BND ? select_row(rs, r) : r;
         const int64_t o0 = offs[i] - base, o1 = offs[i + 1] - base;
-        F bs(0);
+        F bs = fp_traits<F>::inf, b2 = fp_traits<F>::inf;
         int bj = 0;
         bool has = false;
         F s0(0);  // s of centroid 0 (lane 0, first block)
@@ -365,10 +390,19 @@ __global__ __launch_bounds__(256) void csr_assign_blocks_kernel(
                         const F two_dot = F(2) * acc[t][e];
                         const F s = cs[j] - two_dot;
                         if (j == 0) s0 = s;
-                        csr_take(bs, bj, has, s, j);
+                        // ascending j in a lane: an equal value is the later one; bs is
+                        // infinite before the first.  A NaN only lowers b2.
+                        if (BND) b2 = lower(b2, higher(bs, s));
+                        const bool win = s < bs || (!has && s == s);
+                        bs = win ? s : bs;
+                        bj = win ? j : bj;
+                        has = has || win;
                     }
                 }
         }
+        const F mine = bs;
+        const int my_j = bj;
+        const bool mine_has = has;
         // wave reduction of (bs, bj, has)
         for (int off = 32; off > 0; off >>= 1) {
             const F os = __shfl_xor(bs, off);
@@ -387,6 +421,25 @@ __global__ __launch_bounds__(256) void csr_assign_blocks_kernel(
             labels[i] = lab;
             closest[i] = best + xs[i];
         }
+        if (BND) {
+            const float s2 = wave_lowest(!mine_has ? __builtin_inff() : float_below(double(my_j == bj ? b2 : mine)));
+            if (lane == 0) second[i] = s2;
+        }
+    }
+}
+
+// the gaps after csr_assign_blocks_kernel, a thread per row: there they would cost a whole
+// wave's instructions.  best comes back from closest, which rounds twice.
+template <typename F>
+__global__ __launch_bounds__(256) void csr_gap_kernel(int64_t n, const F* __restrict__ xs,
+                                                      const F* __restrict__ closest, const float* __restrict__ second,
+                                                      const int32_t* __restrict__ labels, row_select rs,
+                                                      csr_bounds kb) {
+    const double band = csr_band(kb);
+    const int64_t nsel = select_rows(rs, n);
+    for (int64_t e = blockIdx.x * int64_t(256) + threadIdx.x; e < nsel; e += int64_t(gridDim.x) * 256) {
+        const int64_t i = select_row(rs, e);
+        rs.gap[i] = csr_gap(double(closest[i]) - double(xs[i]), double(second[i]), double(xs[i]), band, 1.0, rs, labels[i]);
     }
 }
 
@@ -405,22 +458,6 @@ __device__ __forceinline__ V buffer_read(__amdgpu_buffer_rsrc_t r, int lane_off,
         return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, wave_off, 0));
 }
 
-// Bounds (km_bounds.hpp) for rows whose columns increase strictly (so that the stored
-// entries are a vector).  The label is the smallest computed s_ij, whose error is
-//     |s_ij - (||c_j||^2 - 2 x.c_j)| <= g (||c_j||^2 + 2 ||x|| ||c_j||) <= 3 g M^2,
-// g = gamma_{d+4} and M the largest norm of a row or centroid: not relative to the
-// distance, as the dense form's.  With d_j - d_a >= G > 0 for every other centroid,
-// d_j^2 - d_a^2 >= G^2, so a row stays settled while G > sqrt(2 * 3 g M^2): that part is
-// taken off its gap when it is settled.  M may be taken at that time: later centroids
-// are means of rows, rows, or unchanged.
-struct csr_bounds {
-    const unsigned long long* xmax;  // csr_row_squares_kernel
-    const double* cmax;              // max ||c_j||, rounded up
-    double g;    // gamma_{d+4}
-    float g32;   // in FP32 (FAST)
-    int32_t* open;  // [4] this pass's open rows and rows, the previous pass's
-};
-
 // Rows are taken in runs of up to 16 per wave (their offsets read and their results written
 // together, by lanes), one wave per row.  Lane l accumulates the dots of the VEC consecutive
 // centroids VEC (l + 64 t) + e (t < JT, e < VEC: one block holds k) over the row's entries,
@@ -429,90 +466,64 @@ struct csr_bounds {
 // transposed-centroid row per t, U in flight.  Then each lane's best and a wave
 // reduction (ties to the lower j).
 //
-// FAST (columns that increase strictly): the same dots from a
-// half-precision copy of the centroids (scaled by a power of two), half the bytes and one
-// v_fma_mix_f32 a product, in FP32:
-//     |s'_ij - s_ij| <= B = 2 X C (1.02 2^-11 + gamma_{d+4}) + 2^-21 (C^2 + 2 X C) + 3 g M^2 + 1e-34
-// (X the row's norm, C = max ||c_j||; the last term covers underflow).  One centroid with
-// s' <= min s' + 2 B is the label; otherwise the lanes that hold such centroids form their
-// exact dots from Ct.  closest is not written: csr_closest_kernel forms it where it is
-// needed, for one centroid a row.
+// BND: the rows of rs, and the second best as well, for the gap of each.
 //
-// Bound by a row's instructions, not by bytes (n=1e6, 20 entries, k=256: about 300 vector
-// instructions a row, a third of them products): 0.8 to 1.0 ms for all rows, 1.3 ms for the exact
-// dots.  The bookkeeping matters as much as the reads: with the bounds' double arithmetic
-// done per row by a whole wave, FAST took 1.43 ms, with a read at a time for a row's last
-// entries 1.3 ms.
-//
-// Rough distances that leave most rows open are work for nothing (random columns, n=1e5,
-// 50 entries, k=256: 8 iterations took 3.90 ms, 3.75 so): kb.open counts a pass's rows with more
-// than one candidate, and the next pass over fewer than twice as many rows as that goes
-// straight to the exact dots.
-template <typename F, int JT, bool FAST>
+// Taken for k up to 128 VEC and transposed centroids up to an XCD's L2 (n=1e6, d=2000, 20
+// entries, k=256 in double, 4 MB: 1.79 ms, 2.29 with a row per wave at a time; past it
+// csr_assign_blocks_kernel is the faster one).
+// Bound by a row's instructions, not by bytes (more reads in flight changed nothing): n=1e6, 20
+// entries, k=256 1.3 ms for all rows.  Dots from a half-precision copy of the centroids
+// first, the others where those left several, took 0.8-1.0 ms, but held the centroids in 16
+// bits, and rows in random columns (n=1e5, 50 entries, k=256) paid for both: 8 iterations
+// to a threshold 4.2 ms, 3.9 ms without.
+constexpr int64_t CSR_RUNS_BYTES = int64_t(4) << 20;
+template <typename F, int JT, bool BND>
 __global__ __launch_bounds__(256) void csr_assign_kernel(
     const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs,
-    int64_t base, int64_t n, int d, int k, int kp, const F* __restrict__ Ct, const _Float16* __restrict__ Cth,
-    const F* __restrict__ cs, const F* __restrict__ xs, int32_t* __restrict__ labels, F* __restrict__ closest,
-    row_select rs, csr_bounds kb) {
+    int64_t base, int64_t n, int d, int k, int kp, const F* __restrict__ Ct, const F* __restrict__ cs,
+    const F* __restrict__ xs, int32_t* __restrict__ labels, F* __restrict__ closest, row_select rs, csr_bounds kb) {
     constexpr int VEC = csr_vec<F>::N;
-    constexpr int U = FAST ? 16 / JT : 8 / JT;  // entries whose vectors are in flight together
-    static_assert(U >= 4, "groups of U, U / 2 and U / 4 entries");
+    constexpr int U = 8 / JT;  // entries whose vectors are in flight together
     typedef typename csr_vec<F>::type V;
-    typedef _Float16 VH __attribute__((ext_vector_type(VEC)));
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
     const int64_t nwaves = (int64_t(gridDim.x) * blockDim.x) >> 6;
-    const int64_t nsel = select_rows(rs, n);
+    const int64_t nsel = BND ? select_rows(rs, n) : n;
     const int per = int(max<int64_t>(1, min<int64_t>(16, nsel / nwaves)));
     const int64_t nruns = (nsel + per - 1) / per;
-    double band = 0.0, C = 0.0;  // g M^2, and the largest centroid norm
-    float unscale = 1.0f;        // -2 / csr_half_scale
-    if (FAST) {
-        C = *kb.cmax;
-        const double M = fmax(sqrt(__longlong_as_double((long long)*kb.xmax)) * (1.0 + kb.g), C) * (1.0 + 1e-6);
-        band = kb.g * M * M;
-        if (!(M < BOUND_MAX) || !(C < BOUND_MAX)) band = __builtin_inf();  // NaN as well
-        unscale = float(-2.0 / csr_half_scale(C));
-    }
-    const bool rough = FAST && (!kb.open || kb.open[2] <= kb.open[3] / 2);
-    int opened = 0;
-    // (k <= 1024 and d <= 4096: at most 32 MB)
-    const auto half_rsrc = FAST ? buffer_of(Cth, int(2 * int64_t(d) * kp)) : buffer_of(nullptr, 0);
-    const auto full_rsrc = FAST ? buffer_of(Ct, int(int64_t(sizeof(F)) * d * kp)) : buffer_of(nullptr, 0);
+    const double band = BND ? csr_band(kb) : 0.0;
+    // (at most CSR_RUNS_BYTES)
+    const auto rsrc = buffer_of(Ct, int(int64_t(sizeof(F)) * d * kp));
     F csv[JT][VEC];  // the same for every row
+    int off[JT];     // a lane past k reads the last vector, for nothing
 #pragma unroll
-    for (int t = 0; t < JT; ++t)
+    for (int t = 0; t < JT; ++t) {
+        off[t] = min(VEC * (64 * t + lane), kp - VEC) * int(sizeof(F));
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             const int j = VEC * (64 * t + lane) + e;
             csv[t][e] = j < k ? cs[j] : F(0);
         }
+    }
     for (int64_t run = wave; run < nruns; run += nwaves) {
         const int64_t e0 = run * per;
         const int rows = int(min<int64_t>(per, nsel - e0));
         // lane q holds row q of the run, and its results
         int64_t my_row = 0, my_o0 = 0, my_o1 = 0;
-        F my_xs(0), my_best(0), my_second = fp_traits<F>::inf;
-        float my_B = 0.f, my_rest = __builtin_inff();
+        F my_xs(0), my_best(0);
+        float my_second = __builtin_inff();
         int my_lab = 0;
-        bool my_rough = false, my_none = false;
         if (lane < rows) {
-            my_row = select_row(rs, e0 + lane);
+            my_row = BND ? select_row(rs, e0 + lane) : e0 + lane;
             my_o0 = offs[my_row] - base;
             my_o1 = offs[my_row + 1] - base;
             my_xs = xs[my_row];
         }
-        if (FAST) {
-            const double X = sqrt(double(my_xs)) * (1.0 + kb.g);
-            const double B = 2.0 * X * C * (1.02 / 2048.0 + double(kb.g32)) + 4.8e-7 * (C * C + 2.0 * X * C) +
-                             3.0 * band + 1e-34;
-            my_B = float(B * (1.0 + 1e-6));
-        }
         auto fetch = [&](int64_t p0, int64_t o1, int& c, F& v) {
-            c = 0;  // a column index (< d <= 4096), FAST: the byte offset of its row of Cth
+            c = 0;  // the byte offset of a column's row of Ct
             v = F(0);
             if (p0 + lane < o1) {
-                c = int(cols[p0 + lane] - base) * (FAST ? 2 * kp : 1);
+                c = int(cols[p0 + lane] - base) * kp * int(sizeof(F));
                 v = vals[p0 + lane];
             }
         };
@@ -524,118 +535,20 @@ __global__ __launch_bounds__(256) void csr_assign_kernel(
             const int first_c = next_c;
             const F first_v = next_v;
             if (q + 1 < rows) fetch(lane_value(my_o0, q + 1), lane_value(my_o1, q + 1), next_c, next_v);
-            // the row's entries in stored order, U at a time: add(columns, values, first
-            // lane, entries left, group)
-            auto entries = [&](auto&& add) {
-                for (int64_t p0 = o0; p0 < o1; p0 += 64) {
-                    const int cnt = int(min<int64_t>(64, o1 - p0));
-                    int my_c = first_c;
-                    F my_v = first_v;
-                    if (p0 != o0) fetch(p0, o1, my_c, my_v);
-                    // whole groups, then the smallest group that holds the rest: past the
-                    // last entry the column is 0, and add() leaves the value out
-                    int u = 0;
-                    for (; cnt - u > U / 2; u += U) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U>());
-                    if (cnt - u > U / 4) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U / 2>());
-                    else if (cnt > u) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U / 4>());
-                }
-            };
-            uint64_t holders = ~0ull;  // lanes whose centroids may hold the label
-            float rest = __builtin_inff();  // FAST: smallest s' of a centroid that does not
-            if (rough) {
-                float acc[JT][VEC];
-#pragma unroll
-                for (int t = 0; t < JT; ++t)
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e) acc[t][e] = 0.f;
-                int off[JT];  // a lane past k reads the last vector, for nothing
-#pragma unroll
-                for (int t = 0; t < JT; ++t) off[t] = min(VEC * (64 * t + lane), kp - VEC) * 2;
-                entries([&](int c_of, F v_of, int u0, int left, auto count) {
-                    constexpr int N = decltype(count)::value;
-                    (void)left;
-                    VH cv[N][JT];
-#pragma unroll
-                    for (int u = 0; u < N; ++u) {
-                        const int crow = lane_value(c_of, u0 + u);
-#pragma unroll
-                        for (int t = 0; t < JT; ++t) cv[u][t] = buffer_read<VH>(half_rsrc, off[t], crow);
-                    }
-#pragma unroll
-                    for (int u = 0; u < N; ++u) {
-                        const float v = float(lane_value(v_of, u0 + u));  // 0 past the last entry
-#pragma unroll
-                        for (int t = 0; t < JT; ++t)
-#pragma unroll
-                            for (int e = 0; e < VEC; ++e)
-                                acc[t][e] = __builtin_fmaf(v, float(cv[u][t][e]), acc[t][e]);
-                    }
-                });
-                float low = __builtin_inff();
-#pragma unroll
-                for (int t = 0; t < JT; ++t)
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e) {
-                        acc[t][e] = __builtin_fmaf(unscale, acc[t][e], float(csv[t][e]));
-                        low = VEC * (64 * t + lane) + e < k ? fminf(low, acc[t][e]) : low;
-                    }
-                const float top = wave_lowest(low);
-                const float lim = top + 2.0f * lane_value(my_B, q);
-                const float T = lim + fabsf(lim) * 2.4e-7f;  // not a number: every centroid stays
-                int mine = 0, at = 0;
-#pragma unroll
-                for (int t = 0; t < JT; ++t)
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e) {
-                        const int j = VEC * (64 * t + lane) + e;
-                        const bool out = acc[t][e] > T;
-                        const bool in = j < k && !out;
-                        mine += in ? 1 : 0;
-                        at = in ? j : at;
-                        rest = j < k && out ? fminf(rest, acc[t][e]) : rest;
-                    }
-                holders = __ballot(mine > 0);
-                const int src = int(__builtin_ctzll(holders | (uint64_t(1) << 63)));
-                if ((holders & (holders - 1)) == 0 && lane_value(mine, src) == 1) {
-                    const float r = rs.gap ? wave_lowest(rest) : rest;
-                    const int lab = lane_value(at, src);
-                    if (lane == q) {
-                        my_lab = lab;
-                        my_best = F(top);
-                        my_rest = r;
-                        my_rough = true;
-                    }
-                    continue;
-                }
-            }
-            ++opened;
-            const bool act = (holders >> lane) & 1u;
-            const int spare = int(__builtin_ctzll(holders | (uint64_t(1) << 63)));  // read by idle lanes
-            F bs(0), b2 = fp_traits<F>::inf;  // best and second best of this lane
-            int bj = 0;
-            bool has = false;
-            F s0(0);  // s of centroid 0 (lane 0)
             F acc[JT][VEC];
 #pragma unroll
             for (int t = 0; t < JT; ++t)
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) acc[t][e] = F(0);
-            int off[JT];
-#pragma unroll
-            for (int t = 0; t < JT; ++t) off[t] = min(VEC * (64 * t + (act ? lane : spare)), kp - VEC);
-            entries([&](int c_of, F v_of, int u0, int left, auto count) {
+            // entries u0 .. of the 64 held, the first `left` of a group
+            auto add = [&](int c_of, F v_of, int u0, int left, auto count) {
                 constexpr int N = decltype(count)::value;
                 V cv[N][JT];
 #pragma unroll
                 for (int u = 0; u < N; ++u) {
-                    const int at_c = lane_value(c_of, u0 + u);
+                    const int at = lane_value(c_of, u0 + u);
 #pragma unroll
-                    for (int t = 0; t < JT; ++t) {
-                        if constexpr (FAST)
-                            cv[u][t] = buffer_read<V>(full_rsrc, off[t] * int(sizeof(F)), at_c * int(sizeof(F) / 2));
-                        else
-                            cv[u][t] = *reinterpret_cast<const V*>(Ct + int64_t(at_c) * kp + off[t]);
-                    }
+                    for (int t = 0; t < JT; ++t) cv[u][t] = buffer_read<V>(rsrc, off[t], at);
                 }
 #pragma unroll
                 for (int u = 0; u < N; ++u) {
@@ -649,7 +562,23 @@ __global__ __launch_bounds__(256) void csr_assign_kernel(
                             acc[t][e] = acc[t][e] + pr;
                         }
                 }
-            });
+            };
+            for (int64_t p0 = o0; p0 < o1; p0 += 64) {
+                const int cnt = int(min<int64_t>(64, o1 - p0));
+                int my_c = first_c;
+                F my_v = first_v;
+                if (p0 != o0) fetch(p0, o1, my_c, my_v);
+                // whole groups, then the smallest group that holds the rest: past the
+                // last entry the column is 0, and add() leaves the value out
+                int u = 0;
+                for (; cnt - u > U / 2; u += U) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U>());
+                if (cnt - u > U / 4) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U / 2>());
+                else if (cnt > u) add(my_c, my_v, u, cnt - u, std::integral_constant<int, U / 4>());
+            }
+            F bs(0), b2 = fp_traits<F>::inf;  // best and second best of this lane
+            int bj = 0;
+            bool has = false;
+            F s0(0);  // s of centroid 0 (lane 0)
 #pragma unroll
             for (int t = 0; t < JT; ++t)
 #pragma unroll
@@ -659,67 +588,53 @@ __global__ __launch_bounds__(256) void csr_assign_kernel(
                     const F s = csv[t][e] - two_dot;
                     if (j == 0) s0 = s;
                     // ascending j in a lane: an equal value is the later one
-                    const bool in = act && j < k && s == s;
+                    const bool in = j < k && s == s;
                     const bool win = in && (!has || s < bs);
-                    if (FAST && in) b2 = win ? (has ? bs : b2) : lower(b2, s);
+                    if (BND && in) b2 = win ? (has ? bs : b2) : lower(b2, s);
                     bs = win ? s : bs;
                     bj = win ? j : bj;
                     has = has || win;
                 }
-            // the smallest s, then the lowest j that has it; every s NaN, or s_i0 (when it
-            // can matter: idle lanes' centroids are finite): label 0
+            // the smallest s, then the lowest j that has it; every s NaN, or s_i0: label 0
             const F best = wave_lowest(has ? bs : fp_traits<F>::inf);
             const int lab = wave_lowest(has && bs == best ? bj : 0x7fffffff);
             s0 = lane_value(s0, 0);
-            const bool none = lab == 0x7fffffff || ((holders & 1u) && s0 != s0);
-            F second = fp_traits<F>::inf;
-            if (FAST && rs.gap) {
-                second = wave_lowest(!has ? fp_traits<F>::inf : bj == lab ? b2 : bs);
-                rest = wave_lowest(rest);
-            }
+            const bool none = lab == 0x7fffffff || s0 != s0;
+            float second = __builtin_inff();
+            if (BND) second = wave_lowest(!has ? __builtin_inff() : float_below(double(bj == lab ? b2 : bs)));
             if (lane == q) {
                 my_lab = none ? 0 : lab;
                 my_best = none ? s0 : best;
                 my_second = second;
-                my_rest = rest;
-                my_none = none;
             }
         }
         if (lane < rows) {
             labels[my_row] = my_lab;
-            if (!FAST) closest[my_row] = my_best + my_xs;
-            if (FAST && rs.gap) {
-                float gap = -__builtin_inff();
-                if (!my_none && band < BOUND_MAX) {
-                    const double x2 = double(my_xs), rough = double(my_B) + 1.5 * band;
-                    const double up2 = double(my_best) + x2 + (my_rough ? rough : 4.5 * band);
-                    const double lo2 = fmin(double(my_second) - 4.5 * band, double(my_rest) - rough) + x2;
-                    gap = float_below(double(bound_gap(up2, lo2, rs.gam, rs.base[my_lab])) - sqrt(6.3 * band));
-                }
-                rs.gap[my_row] = gap;
-            }
+            closest[my_row] = my_best + my_xs;
+            if (BND)
+                rs.gap[my_row] = csr_gap(double(my_best), double(my_second), double(my_xs), band, 0.0, rs, my_lab);
         }
-    }
-    if (FAST && kb.open && lane == 0) {
-        if (opened) atomicAdd(kb.open, opened);
-        if (wave == 0) kb.open[1] = int32_t(nsel);
     }
 }
 
-// closest_i of every row with its label known (no pass with FAST writes it): the
-// arithmetic of csr_assign_kernel for one centroid, a lane per row
+// closest_i of rows with their label known: the arithmetic of csr_assign_kernel for one
+// centroid, a lane per row.  With gap, of the settled rows alone (bound_select_kernel's
+// test), which the next assignment leaves out: an assigned row gets its closest there.
 template <typename F>
 __global__ __launch_bounds__(256) void csr_closest_kernel(
     const F* __restrict__ vals, const int64_t* __restrict__ cols, const int64_t* __restrict__ offs, int64_t base,
     int64_t n, int d, const F* __restrict__ C, const F* __restrict__ cs, const F* __restrict__ xs,
-    const int32_t* __restrict__ labels, F* __restrict__ closest) {
+    const int32_t* __restrict__ labels, F* __restrict__ closest, const float* __restrict__ gap,
+    const double* __restrict__ bound) {
     constexpr int U = 8;  // gathers in flight
     __shared__ int32_t sc[CSR_WINDOW];
     __shared__ F sv[CSR_WINDOW];
     for (int64_t r0 = blockIdx.x * int64_t(256); r0 < n; r0 += int64_t(gridDim.x) * 256) {
         const int64_t i = r0 + threadIdx.x;
-        const int64_t o0 = i < n ? offs[i] - base : 0, o1 = i < n ? offs[i + 1] - base : 0;
         const int lab = i < n ? labels[i] : 0;
+        const bool mine = i < n && (!gap || double(gap[i]) > bound[lab] + BOUND_SLACK);
+        if (!__syncthreads_or(mine)) continue;
+        const int64_t o0 = mine ? offs[i] - base : 0, o1 = mine ? offs[i + 1] - base : 0;
         const F* c = C + int64_t(lab) * d;
         F acc(0);
         csr_walk(
@@ -745,7 +660,7 @@ __global__ __launch_bounds__(256) void csr_closest_kernel(
                     }
                 }
             });
-        if (i < n) {
+        if (mine) {
             const F two_dot = F(2) * acc;
             const F s = cs[lab] - two_dot;
             closest[i] = s + xs[i];

@@ -149,7 +149,7 @@ struct km_ctx {
     km::dbuf b_gap, b_rows, b_count, b_base, b_drift, cand_lo, coll_lo, seg_cand_lo, seg_coll_lo;
     // CSR path: values, column indices, row offsets (when uploaded), row squares,
     // transposed centroids, centroid squares, closest distances, structure flag
-    km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cth, csr_open, csr_cs, csr_closest, csr_flag;
+    km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_second, csr_cs, csr_closest, csr_flag;
     // step_ticket: zero between launches; step_max: centroid_step_kernel's workspace.
     // Both live from the context's creation on.
     km::dbuf step_ticket, step_max;
@@ -254,7 +254,6 @@ struct work {
     int32_t* open_rows = nullptr;
     int32_t* open_count = nullptr;
     unsigned long long* acc = nullptr;
-    int32_t* csr_open = nullptr;  // sparse rows: csr_bounds::open
     // workspace source: a fixed arena, or (null) the context's buffers
     arena* A = nullptr;
 };
@@ -369,7 +368,6 @@ static void step_centroids(km_ctx* ctx, work<F>& w, int path, F* C, const F* col
     s.sel_count = w.open_count;
     s.counters = w.L.counters;
     s.acc = cold ? w.acc : nullptr;
-    s.csr_open = w.csr_open;
     s.ticket = ctx->step_ticket.get<uint32_t>(1);
     s.wgmax = ctx->step_max.get<unsigned long long>(4 * STEP_MAX_GRID);
     const int grid = std::min(w.k, STEP_MAX_GRID);
@@ -815,14 +813,15 @@ struct cluster_lists {
     int32_t* perm;
 };
 
-// ls.changed must be clear before the call; the empty clusters are reported with seq
+// ls.changed must be clear before the call; the empty clusters (and *open, when given) are
+// reported with seq
 static void label_group(km_ctx* ctx, const label_sort& ls, const int32_t* labels, const cluster_lists& o,
-                        uint32_t seq) {
+                        uint32_t seq, const int32_t* open = nullptr) {
     const int k = ls.k;
     if (ls.small) {
         hipLaunchKernelGGL(small_group_kernel, dim3(1), dim3(1024), small_group_lds_bytes(k), ctx->stream, labels,
                            ls.prev, int(ls.n), k, o.counts, ls.changed, o.offsets, o.chunk_base, o.empty_list, o.meta,
-                           o.perm, ctx->report, seq);
+                           o.perm, ctx->report, open, seq);
         KM_LAUNCH_CHECK();
         return;
     }
@@ -845,7 +844,7 @@ static void label_group(km_ctx* ctx, const label_sort& ls, const int32_t* labels
     }
     hipLaunchKernelGGL(scan_clusters_kernel, dim3(1), dim3(1024), 0, ctx->stream, o.counts,
                        ls.csort ? ls.gsum : (const int32_t*)nullptr, ls.G, k, o.offsets, o.chunk_base, o.empty_list,
-                       o.meta, ls.changed, ctx->report, seq);
+                       o.meta, ls.changed, ctx->report, open, seq);
     KM_LAUNCH_CHECK();
     if (!ls.csort) {
         sort_by_label(ctx, labels, ls.n, k, o.perm);
@@ -1318,37 +1317,35 @@ static csr_view<F> csr_prepare(km_ctx* ctx, const F* vals, const int64_t* cols,
     return v;
 }
 
-// Half-precision distances first (csr_assign_kernel, FAST): rows whose columns increase strictly, and
-// at most one block of centroids.  n=1e6, 20 entries a row, k=256: 0.8-1.0 ms a pass
-// against 1.3 ms.  Columns in another order may repeat, and then the entries' norm does
-// not bound the products; past one block the rough values would have to be kept.
+// closest distances of rows to their labels' centroids: of all of them, or with sel.gap of the
+// settled ones (after csr_assign against C, or inside it)
 template <typename F>
-static bool csr_fast(int k, bool increasing) {
-    return increasing && k <= 64 * csr_vec<F>::N * 4;
+static void csr_label_closest(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, const F* xs,
+                              const int32_t* labels, F* closest, const row_select& sel) {
+    hipLaunchKernelGGL(csr_closest_kernel<F>, dim3(grid_for(ctx, x.n, 256, 8)), dim3(256), 0, ctx->stream, x.vals,
+                       x.cols, x.offs, x.base, x.n, int(x.d), C, ctx->csr_cs.get<F>(k), xs, labels, closest, sel.gap,
+                       sel.base);
+    KM_LAUNCH_CHECK();
 }
 
-static csr_bounds csr_make_bounds(const unsigned long long* xmax, const double* cmax, int d, double u) {
-    return {xmax, cmax, gamma_m(double(d + 4), u), float(gamma_m(double(d + 4), fp_traits<float>::u) * (1.0 + 1e-6)),
-            nullptr};
-}
-
-// labels of the selected rows against C (k x d), and without fast their closest distances
+// labels and closest distances of the selected rows against C (k x d); bounded: with
+// their gaps.  settled: the closest distances of the other rows first
 template <typename F>
 static void csr_assign(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, const F* xs,
-                       int32_t* labels, F* closest, bool fast, const row_select& sel, const csr_bounds& kb) {
+                       int32_t* labels, F* closest, bool bounded, const row_select& sel, const csr_bounds& kb,
+                       bool settled = false) {
     constexpr int VEC = csr_vec<F>::N;
     const int kp = (k + VEC - 1) / VEC * VEC;  // Ct row stride: whole 16-byte vectors
     F* ct = ctx->csr_ct.get<F>(int64_t(kp) * x.d);
-    _Float16* cth = fast ? ctx->csr_cth.get<_Float16>(int64_t(kp) * x.d) : nullptr;
     F* cs = ctx->csr_cs.get<F>(k);
     hipLaunchKernelGGL(csr_transpose_kernel<F>,
                        dim3(unsigned((x.d + 63) / 64), unsigned(std::min((kp + 63) / 64, 65535))),
-                       dim3(256), 0, ctx->stream, C, int64_t(k), int64_t(kp), x.d, ct, cth,
-                       kb.cmax);
+                       dim3(256), 0, ctx->stream, C, int64_t(k), int64_t(kp), x.d, ct);
     KM_LAUNCH_CHECK();
     hipLaunchKernelGGL(csr_centroid_squares_kernel<F>, dim3(unsigned(std::min(k, ctx->cu_count * 8))),
                        dim3(64), size_t(csr_sq_len(int(x.d))) * sizeof(F), ctx->stream, C, int64_t(k), int(x.d), cs);
     KM_LAUNCH_CHECK();
+    if (settled && sel.rows) csr_label_closest<F>(ctx, x, C, k, xs, labels, closest, sel);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing) {
         e0 = ctx->event();
@@ -1356,36 +1353,34 @@ static void csr_assign(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, con
         KM_HIP(hipEventRecord(e0, ctx->stream));
     }
     const int grid = grid_for(ctx, x.n * 64, 256, 8);
-#define KM_CSRA(JT_, FAST_)                                                                         \
-    hipLaunchKernelGGL((csr_assign_kernel<F, JT_, FAST_>), dim3(grid), dim3(256), 0, ctx->stream,    \
-                       x.vals, x.cols, x.offs, x.base, x.n, int(x.d), k, kp, ct, cth, cs, xs, labels, closest, \
-                       sel, kb)
-    // centroids per lane and block: VEC * JT
-    if (fast) {
-        if (k <= 64 * VEC) KM_CSRA(1, true);
-        else if (k <= 128 * VEC) KM_CSRA(2, true);
-        else KM_CSRA(4, true);
-    } else if (k <= 64 * VEC) {
-        KM_CSRA(1, false);
-    } else if (k <= 128 * VEC) {
-        KM_CSRA(2, false);
+    // centroids per lane: VEC * JT
+    const bool runs = k <= 128 * VEC && int64_t(kp) * x.d * int64_t(sizeof(F)) <= CSR_RUNS_BYTES;
+    float* second = bounded && !runs ? ctx->csr_second.get<float>(x.n) : nullptr;
+#define KM_CSRA(JT_, BND_)                                                                          \
+    hipLaunchKernelGGL((csr_assign_kernel<F, JT_, BND_>), dim3(grid), dim3(256), 0, ctx->stream,     \
+                       x.vals, x.cols, x.offs, x.base, x.n, int(x.d), k, kp, ct, cs, xs, labels, closest, sel, kb)
+#define KM_CSRB(BND_)                                                                               \
+    hipLaunchKernelGGL((csr_assign_blocks_kernel<F, BND_>), dim3(grid), dim3(256), 0, ctx->stream,   \
+                       x.vals, x.cols, x.offs, x.base, x.n, k, kp, ct, cs, xs, labels, closest, sel, second)
+    if (runs && k <= 64 * VEC) {
+        if (bounded) KM_CSRA(1, true);
+        else KM_CSRA(1, false);
+    } else if (runs) {
+        if (bounded) KM_CSRA(2, true);
+        else KM_CSRA(2, false);
+    } else if (bounded) {
+        KM_CSRB(true);
+        KM_LAUNCH_CHECK();
+        hipLaunchKernelGGL(csr_gap_kernel<F>, dim3(grid_for(ctx, x.n, 256, 8)), dim3(256), 0, ctx->stream, x.n, xs,
+                           closest, second, labels, sel, kb);
     } else {
-        hipLaunchKernelGGL(csr_assign_blocks_kernel<F>, dim3(grid), dim3(256), 0, ctx->stream, x.vals, x.cols, x.offs,
-                           x.base, x.n, k, kp, ct, cs, xs, labels, closest);
+        KM_CSRB(false);
     }
 #undef KM_CSRA
+#undef KM_CSRB
     KM_LAUNCH_CHECK();
     if (ctx->timing) KM_HIP(hipEventRecord(e1, ctx->stream));
     ctx->stats.assign_launches++;
-}
-
-// closest distances of all rows to their labels' centroids, after csr_assign against C
-template <typename F>
-static void csr_all_closest(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, const F* xs, const int32_t* labels,
-                            F* closest) {
-    hipLaunchKernelGGL(csr_closest_kernel<F>, dim3(grid_for(ctx, x.n, 256, 8)), dim3(256), 0, ctx->stream, x.vals,
-                       x.cols, x.offs, x.base, x.n, int(x.d), C, ctx->csr_cs.get<F>(k), xs, labels, closest);
-    KM_LAUNCH_CHECK();
 }
 
 // objective = sum of closest (as double) in the fixed order; d64 per row if asked
@@ -1444,6 +1439,9 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     F* xs = ctx->csr_xs.get<F>(n);
     F* closest = ctx->csr_closest.get<F>(n);
     int32_t* labels = ctx->labels.get<int32_t>(n);
+    // bounds for rows whose columns increase strictly: others may repeat a column, and then the
+    // entries' norm does not bound the products
+    bool bounded = increasing;
     unsigned long long* xmax = ctx->xmax.get<unsigned long long>(2);
     fill<unsigned long long>(ctx, xmax, 2, 0ull);
     hipLaunchKernelGGL(csr_row_squares_kernel<F>, dim3(grid_for(ctx, n, 256, 4)), dim3(256), 0,
@@ -1462,7 +1460,7 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     KM_HIP(hipFuncSetAttribute((const void*)sums, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     double* d64 = ctx->d64.get<double>(n);  // refill candidates' keys
     const label_sort lsort = label_sort_setup(ctx, n, k);
-    // the centroid step's view, and bounds where the rough distances are used
+    // the centroid step's view, and bounds
     work<F> w;
     csr_step_view(ctx, w, n, d, k);
     w.base = ctx->b_base.get<double>(k);
@@ -1472,9 +1470,8 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     w.open_count = ctx->b_count.get<int32_t>(1);
     w.sel.base = w.base;
     w.sel.gam = 1e-6;
-    csr_bounds kb = csr_make_bounds(xmax, w.maxima, d, fp_traits<F>::u);
-    const bool fast = csr_fast<F>(k, increasing);
-    if (fast) {
+    const csr_bounds kb{xmax, w.maxima, gamma_m(double(d + 4), fp_traits<F>::u)};
+    if (bounded) {
         w.open_rows = ctx->b_rows.get<int32_t>(n);
         w.sel.gap = ctx->b_gap.get<float>(n);
     }
@@ -1485,24 +1482,21 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     double prev = double(std::numeric_limits<F>::max());
     int64_t iter = 0;
     for (iter = 0; iter < max_iter; ++iter) {
-        csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest, fast, w.sel, kb);
+        csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest, bounded, w.sel, kb, need_obj);
         const uint32_t seq = next_seq(ctx);
-        label_group(ctx, lsort, labels, o, seq);
+        label_group(ctx, lsort, labels, o, seq, w.sel.count);
         const int64_t max_chunks = n / REDUCE_CHUNK + k + 1;
         hipLaunchKernelGGL(sums, dim3(grid_for(ctx, max_chunks * 64, 64, 16)),
                            dim3(64), lds, ctx->stream, x.vals, x.cols, x.offs, x.base, d, k, o.perm,
                            o.offsets, o.chunk_base, o.meta, part);
         KM_LAUNCH_CHECK();
         double* objp = nullptr;
-        if (need_obj) {
-            if (fast) csr_all_closest<F>(ctx, x, Ccur, k, xs, labels, closest);
-            objp = csr_objective<F>(ctx, closest, n, d64);
-        }
+        if (need_obj) objp = csr_objective<F>(ctx, closest, n, d64);
         step_centroids<F>(ctx, w, path, Cnext, Ccur, {part, o.counts, o.chunk_base});
         wait_report(ctx, &ctx->report->seq, seq);  // as in train()
         if (ctx->report->empties > 0) {
             if (!need_obj) {
-                if (fast) csr_all_closest<F>(ctx, x, Ccur, k, xs, labels, closest);
+                if (w.sel.rows) csr_label_closest<F>(ctx, x, Ccur, k, xs, labels, closest, row_select{});
                 csr_objective<F>(ctx, closest, n, d64);
             }
             int32_t* cand = launch_empty_clusters<F>(ctx, (const F*)nullptr, n, d, k, o, Cnext, d64, objp);
@@ -1513,6 +1507,14 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
             ctx->stats.empty_cluster_events++;
         }
         std::swap(Ccur, Cnext);
+        // Bounds that have settled hardly a row by the fifth pass are given up: rows in random
+        // columns, which they cost up to a sixth of a pass (n=3e5, d=4000, 40 entries, k=500 in
+        // double, 8 iterations: 30.0 ms, 31.8 with the bounds kept, 30.1 without any).  A pass
+        // earlier is too soon for many clusters (d=2000, 20 entries, k=1000: 16.8 ms, 13.7 so).
+        if (bounded && iter >= 4 && int64_t(ctx->report->open) > n - n / 64) {
+            bounded = false;
+            w.sel = row_select{};
+        }
         if (w.sel.gap) {
             hipLaunchKernelGGL(bound_select_kernel, dim3(grid_for(ctx, n, SELECT_ROWS, 8)), dim3(256), 0, ctx->stream,
                                labels, w.sel.gap, w.base, n, w.open_rows, w.open_count);
@@ -1532,8 +1534,7 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
             prev = obj;
         }
     }
-    csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest, fast, w.sel, kb);
-    if (fast) csr_all_closest<F>(ctx, x, Ccur, k, xs, labels, closest);
+    csr_assign<F>(ctx, x, Ccur, k, xs, labels, closest, bounded, w.sel, kb, true);
     double* objp = csr_objective<F>(ctx, closest, n, nullptr);
     if (ctx->timing) KM_HIP(hipEventRecord(loop1, ctx->stream));
     KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1561,34 +1562,20 @@ static void infer_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     const bool dev = flags & KM_FLAG_DEVICE_POINTERS;
     ctx->stats = km_stats{};
     ctx->ev_used = 0;
-    bool increasing = false;
-    const csr_view<F> x = csr_prepare<F>(ctx, vals, cols, offs, n, d, nnz, indexing, dev, &increasing);
-    // one pass: the rough one has to earn its centroid step and, with the objective, the
-    // closest distances (n=2e4, 30 entries, k=64: 108 us without, 128 with; n=3e5, 40 entries,
-    // k=500: 1585 and 1237)
-    const bool fast = csr_fast<F>(k, increasing) && double(nnz) * k >= 2e9;
-    unsigned long long* xmax = nullptr;
-    if (fast) {
-        xmax = ctx->xmax.get<unsigned long long>(2);
-        fill<unsigned long long>(ctx, xmax, 2, 0ull);
-    }
+    const csr_view<F> x = csr_prepare<F>(ctx, vals, cols, offs, n, d, nnz, indexing, dev);
     F* xs = ctx->csr_xs.get<F>(n);
     F* closest = ctx->csr_closest.get<F>(n);
     int32_t* labels = ctx->labels.get<int32_t>(n);
     hipLaunchKernelGGL(csr_row_squares_kernel<F>, dim3(grid_for(ctx, n, 256, 4)), dim3(256), 0,
-                       ctx->stream, x.vals, x.offs, x.base, n, xs, xmax);
+                       ctx->stream, x.vals, x.offs, x.base, n, xs, (unsigned long long*)nullptr);
     KM_LAUNCH_CHECK();
     F* Cd = ctx->c_cur.get<F>(int64_t(k) * d);
     KM_HIP(hipMemcpyAsync(Cd, C, sizeof(F) * k * d,
                           dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-    work<F> w;  // the centroid step's view: max ||c_j||
-    csr_step_view(ctx, w, n, d, k);
-    if (fast) step_centroids<F>(ctx, w, 1, Cd);
-    csr_assign<F>(ctx, x, Cd, k, xs, labels, closest, fast, w.sel, csr_make_bounds(xmax, w.maxima, d, fp_traits<F>::u));
+    csr_assign<F>(ctx, x, Cd, k, xs, labels, closest, false, row_select{}, csr_bounds{});
     int32_t* pin = ctx->pinned;
     const bool want_obj = flags & KM_FLAG_EXACT_OBJECTIVE;
     if (want_obj) {
-        if (fast) csr_all_closest<F>(ctx, x, Cd, k, xs, labels, closest);
         double* objp = csr_objective<F>(ctx, closest, n, nullptr);
         KM_HIP(hipMemcpyAsync(pin + 6, objp, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     }
@@ -2636,7 +2623,7 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
                         &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
                         &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->step_ticket, &ctx->step_max, &ctx->c_split, &ctx->c_pieces, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
-                        &ctx->csr_ct, &ctx->csr_cth, &ctx->csr_open, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
+                        &ctx->csr_ct, &ctx->csr_second, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();
     ctx->bws_fin.release();

@@ -105,7 +105,6 @@ struct centroid_step {
     // re-score counters: added into acc (when not null), then cleared
     int32_t* counters;
     unsigned long long* acc;
-    int32_t* csr_open;  // sparse rows (csr_bounds::open): the pass's counts become the previous ones
     // workspace of the launch: a ticket (0 between launches) and STEP_MAX_GRID x 4 maxima
     uint32_t* ticket;
     unsigned long long* wgmax;
@@ -268,12 +267,6 @@ __global__ __launch_bounds__(256) void centroid_step_kernel(centroid_step<F> s) 
         if (s.acc) s.acc[t] += (unsigned long long)s.counters[t];
         s.counters[t] = 0;
     }
-    if (t == 0 && s.csr_open && s.cold && s.csr_open[1] > 0) {  // not again after a refill
-        s.csr_open[2] = s.csr_open[0];
-        s.csr_open[3] = s.csr_open[1];
-        s.csr_open[0] = 0;
-        s.csr_open[1] = 0;
-    }
     if (t == 0) *s.ticket = 0u;
 }
 
@@ -294,7 +287,7 @@ __global__ __launch_bounds__(1024) void small_group_kernel(
     const int32_t* __restrict__ labels, int32_t* __restrict__ prev, int n, int k, int32_t* __restrict__ counts,
     int32_t* __restrict__ changed, int64_t* __restrict__ offsets, int32_t* __restrict__ chunk_base,
     int32_t* __restrict__ empty_list, int32_t* __restrict__ meta, int32_t* __restrict__ perm,
-    host_report* report, uint32_t seq) {
+    host_report* report, const int32_t* __restrict__ open, uint32_t seq) {
     extern __shared__ int32_t glds[];
     int32_t* chg = glds + 16 * k;   // [k] members changed
     int32_t* first = chg + k;       // [k] first member position
@@ -366,7 +359,7 @@ __global__ __launch_bounds__(1024) void small_group_kernel(
         chunk_base[k] = sc;
         meta[0] = se;
         meta[1] = sc;
-        report_empties(report, se, seq);
+        report_empties(report, se, open, seq);
     }
     __syncthreads();
 #pragma unroll

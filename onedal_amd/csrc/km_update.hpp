@@ -98,16 +98,19 @@ __global__ __launch_bounds__(256) void count_kernel(const int32_t* __restrict__ 
 // cluster whose members did not change (changed[j] = 0) has no chunks: its sums,
 // and so its centroid, are those of the previous iteration.  With gsum (the counting
 // sort) the counts are first taken as its column sums over G groups.  The number
-// of empty clusters also goes to host memory (report), followed by seq, so the
-// host can leave out the refill's launches without waiting for the stream.
+// of empty clusters also goes to host memory (report) with the number of rows that the
+// pass assigned (*open; null: not told), followed by seq, so the host can leave out the
+// refill's launches, or bounds that settle nothing, without waiting for the stream.
 // ---------------------------------------------------------------------------
 struct host_report {
     int32_t empties;
+    int32_t open;
     uint32_t seq;
 };
 
-__device__ __forceinline__ void report_empties(host_report* report, int32_t empties, uint32_t seq) {
+__device__ __forceinline__ void report_empties(host_report* report, int32_t empties, const int32_t* open, uint32_t seq) {
     if (!report) return;
+    if (open) __hip_atomic_store(&report->open, *open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(&report->empties, empties, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(&report->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -147,7 +150,8 @@ __global__ __launch_bounds__(1024) void scan_clusters_kernel(int32_t* __restrict
                                                              int32_t* __restrict__ empty_list,
                                                              int32_t* __restrict__ meta,
                                                              const int32_t* __restrict__ changed,
-                                                             host_report* report, uint32_t seq) {
+                                                             host_report* report,
+                                                             const int32_t* __restrict__ open, uint32_t seq) {
     __shared__ int32_t sums[3][16];
     __shared__ int32_t last[3];
     const int t = threadIdx.x;
@@ -187,7 +191,7 @@ __global__ __launch_bounds__(1024) void scan_clusters_kernel(int32_t* __restrict
         chunk_base[k] = c_chk;
         meta[0] = c_emp;
         meta[1] = c_chk;
-        report_empties(report, c_emp, seq);
+        report_empties(report, c_emp, open, seq);
     }
 }
 
