@@ -195,6 +195,9 @@ __device__ __forceinline__ bf16_params make_bf16_params(double C, double Ch, dou
     float fb = float(B);
     if (double(fb) < B) fb = __uint_as_float(__float_as_uint(fb) + 1u);
     p.B = double(fb);
+    // Where a value could pass the float range, the nearest centroid's too, nothing is settled
+    // and nothing collected: without a threshold every row goes to the full re-score.
+    if (p.B + C * C + 2.0 * (X + ex) * Ch >= 1e38) p.B = __builtin_nan("");
     return p;
 }
 
