@@ -99,9 +99,9 @@ struct dbuf {
 // per-row, per-cluster and per-chunk arrays, sort scratch
 struct batch_ws {
     dbuf inst, pre, labels, keys, perm, d64, ccur, cnext, counts, offsets, cb, empty, meta, qpre,
-        part, objc, obj, sort_tmp, asel, apre, bhist, ticket, prev, changed, gap, rows, count, base, drift;
+        part, objc, obj, sort_tmp, asel, apre, bhist, ticket, prev, changed, gap, count, base, drift;
     void release() {
-        dbuf* all[] = {&prev, &changed, &gap, &rows, &count, &base, &drift,
+        dbuf* all[] = {&prev, &changed, &gap, &count, &base, &drift,
                        &inst, &pre,  &labels, &keys, &perm,     &d64,  &ccur, &cnext, &counts, &offsets, &cb,
                        &empty, &meta, &qpre,  &part, &objc, &obj, &sort_tmp, &asel, &apre, &bhist, &ticket};
         for (dbuf* b : all) b->release();
@@ -144,12 +144,11 @@ struct km_ctx {
     km::dbuf stat_acc, ec_wcnt;  // device-side statistics; per-workgroup counts of ec_count_kernel
     km::dbuf cs_inst, cs_pre, cs_hist, cs_gsum;  // single-instance counting sort (label_sort)
     km::dbuf cs_prev, cs_changed;                // its previous labels and changed-cluster flags
-    // distance bounds of a training (row_bounds): gap and open rows, per row; base
-    // and drift, per cluster
-    km::dbuf b_gap, b_rows, b_count, b_base, b_drift, cand_lo, coll_lo, seg_cand_lo, seg_coll_lo;
+    // distance bounds of a training: gap per row; base and drift, per cluster
+    km::dbuf b_gap, b_count, b_base, b_drift, cand_lo, coll_lo, seg_cand_lo, seg_coll_lo;
     // CSR path: values, column indices, row offsets (when uploaded), row squares,
     // transposed centroids, centroid squares, closest distances, structure flag
-    km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_second, csr_cs, csr_closest, csr_flag;
+    km::dbuf csr_vals, csr_cols, csr_offs, csr_xs, csr_ct, csr_cs, csr_closest, csr_flag;
     // step_ticket: zero between launches; step_max: centroid_step_kernel's workspace.
     // Both live from the context's creation on.
     km::dbuf step_ticket, step_max;
@@ -659,6 +658,14 @@ static void launch_objective_sum(km_ctx* ctx, const double* d64, int64_t n, doub
     KM_LAUNCH_CHECK();
 }
 
+// The rows' d64 take the place of the candidate ids, which the pass has re-scored by then:
+// they last until the next assignment.
+template <typename F>
+static double* rows_d64(const work<F>& w) {
+    static_assert(MAXC * sizeof(int32_t) >= sizeof(double), "d64 fits the candidate ids");
+    return reinterpret_cast<double*>(w.L.cand_ids);
+}
+
 // objective of the current labels against C; d64 holds the rows' distances afterwards
 template <typename F>
 static double* objective(km_ctx* ctx, work<F>& w, const F* C, double* d64, uint32_t seq) {
@@ -1002,7 +1009,7 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
     const cluster_lists o = take_cluster_lists(ctx, n, k);
     double* part = ctx->part.get<double>((n / REDUCE_CHUNK + k + 1) * int64_t(d));
     const bool need_obj = thr > 0;
-    double* d64 = ctx->d64.get<double>(n);
+    double* d64 = rows_d64<F>(w);
     const label_sort lsort = label_sort_setup(ctx, n, k);
     // bounds (km_bounds.hpp): every pass after the first assigns only the rows
     // whose label could have changed
@@ -1011,7 +1018,7 @@ static void train(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C0,
         fill<double>(ctx, w.base, k, 0.0);
         w.drift = ctx->b_drift.get<double>(k);
         w.changed = lsort.changed;
-        w.open_rows = ctx->b_rows.get<int32_t>(n);
+        w.open_rows = o.perm;  // from the selection to the assignment; the grouping then takes it
         w.open_count = ctx->b_count.get<int32_t>(1);
         w.acc = ctx->stat_acc.get<unsigned long long>(3);
         fill<unsigned long long>(ctx, w.acc, 3, 0ull);
@@ -1129,7 +1136,7 @@ static void infer(km_ctx* ctx, const F* X, int64_t n, int64_t d64_, const F* C, 
     const bool want_obj = flags & KM_FLAG_EXACT_OBJECTIVE;
     const uint32_t seq = next_seq(ctx);
     if (want_obj) {
-        objective<F>(ctx, w, Cd, ctx->d64.get<double>(n), seq);
+        objective<F>(ctx, w, Cd, rows_d64<F>(w), seq);
     } else {
         hipLaunchKernelGGL(refine_report_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->obj_report, w.L.counters,
                            (const unsigned long long*)nullptr, seq);
@@ -1239,9 +1246,7 @@ static void infer_noalloc(km_ctx* ctx, const float* X, int64_t n, int64_t d64_, 
         assign<F>(ctx, w, C, path);
         const uint32_t seq = next_seq(ctx);
         if (want_obj) {
-            // the rows' d64 take the candidate ids' place (re-scored by now)
-            static_assert(MAXC * sizeof(int32_t) >= sizeof(double), "d64 fits the candidate ids");
-            double* d64 = reinterpret_cast<double*>(w.L.cand_ids);
+            double* d64 = rows_d64<F>(w);
             double* chunks = A.get<double>((rows + OBJ_CHUNK - 1) / OBJ_CHUNK);
             launch_d64<F>(ctx, w.X, w.n, w.d, C, w.labels, d64);
             launch_objective_sum(ctx, d64, w.n, chunks, acc, acc, w.L.counters, nullptr, seq);
@@ -1355,7 +1360,8 @@ static void csr_assign(km_ctx* ctx, const csr_view<F>& x, const F* C, int k, con
     const int grid = grid_for(ctx, x.n * 64, 256, 8);
     // centroids per lane: VEC * JT
     const bool runs = k <= 128 * VEC && int64_t(kp) * x.d * int64_t(sizeof(F)) <= CSR_RUNS_BYTES;
-    float* second = bounded && !runs ? ctx->csr_second.get<float>(x.n) : nullptr;
+    // (in the place of the rows' d64, which are taken after the pass)
+    float* second = bounded && !runs ? reinterpret_cast<float*>(ctx->d64.get<double>(x.n)) : nullptr;
 #define KM_CSRA(JT_, BND_)                                                                          \
     hipLaunchKernelGGL((csr_assign_kernel<F, JT_, BND_>), dim3(grid), dim3(256), 0, ctx->stream,     \
                        x.vals, x.cols, x.offs, x.base, x.n, int(x.d), k, kp, ct, cs, xs, labels, closest, sel, kb)
@@ -1472,7 +1478,7 @@ static void train_csr(km_ctx* ctx, const F* vals, const int64_t* cols, const int
     w.sel.gam = 1e-6;
     const csr_bounds kb{xmax, w.maxima, gamma_m(double(d + 4), fp_traits<F>::u)};
     if (bounded) {
-        w.open_rows = ctx->b_rows.get<int32_t>(n);
+        w.open_rows = o.perm;  // as in train()
         w.sel.gap = ctx->b_gap.get<float>(n);
     }
     const int path = 1;  // the step prepares nothing else
@@ -1838,7 +1844,6 @@ static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p, int64_t iterat
         p.base = ws.base.get<double>(p.kk);
         fill<double>(ctx, p.base, p.kk, 0.0);
         p.drift = ws.drift.get<double>(p.kk);
-        p.rows_open = ws.rows.get<int32_t>(p.rows);
         p.count_open = ws.count.get<int32_t>(B);
         p.sel = {nullptr, nullptr, ws.gap.get<float>(p.rows), p.base};
     }
@@ -1854,6 +1859,7 @@ static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p, int64_t iterat
         p.labels = ws.labels.get<int32_t>(p.rows);
         if (!p.csort) p.skeys = ws.keys.get<uint32_t>(2 * p.rows);  // keys, then their sorted copy
         p.perm = ws.perm.get<int32_t>(p.rows);
+        if (p.bounds) p.rows_open = p.perm;  // from the selection to the assignment, as in train()
         p.Cnext = ws.cnext.get<float>(p.cfl);
         p.counts = ws.counts.get<int32_t>(p.kk);
         p.offsets = ws.offsets.get<int64_t>(p.kk + B);
@@ -2621,9 +2627,9 @@ km_status km_context_destroy(km_ctx* ctx) {
                         &ctx->init_d2, &ctx->init_chunks, &ctx->init_chosen, &ctx->init_ids, &ctx->init_near, &ctx->init_cnew, &ctx->init_thr,
                         &ctx->gt_d, &ctx->stat_acc, &ctx->ec_wcnt, &ctx->cs_inst, &ctx->cs_pre,
                         &ctx->cs_hist, &ctx->cs_gsum, &ctx->cs_prev, &ctx->cs_changed, &ctx->b_gap,
-                        &ctx->b_rows, &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
+                        &ctx->b_count, &ctx->b_base, &ctx->b_drift, &ctx->cand_lo, &ctx->coll_lo,
                         &ctx->seg_cand_lo, &ctx->seg_coll_lo, &ctx->step_ticket, &ctx->step_max, &ctx->c_split, &ctx->c_pieces, &ctx->csr_vals, &ctx->csr_cols, &ctx->csr_offs, &ctx->csr_xs,
-                        &ctx->csr_ct, &ctx->csr_second, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
+                        &ctx->csr_ct, &ctx->csr_cs, &ctx->csr_closest, &ctx->csr_flag};
     for (auto* b : bufs) b->release();
     ctx->bws.release();
     ctx->bws_fin.release();
