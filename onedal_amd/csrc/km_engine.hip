@@ -14,6 +14,7 @@
 // host decides by to host memory, and the stream is not waited for.
 
 #include <hip/hip_runtime.h>
+#include <sched.h>
 
 #include <cstring>
 #include <rocprim/device/device_radix_sort.hpp>
@@ -681,6 +682,7 @@ static double* objective(km_ctx* ctx, work<F>& w, const F* C, double* d64, uint3
 // on while the stream is busy; a failed or drained stream ends the wait.
 static void wait_report(km_ctx* ctx, const uint32_t* word, uint32_t seq) {
     for (uint64_t spin = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) != seq; ++spin) {
+        if (spin % 256 == 0) sched_yield();  // a thread that waits for this core goes first
         if (spin % 4096) continue;
         const hipError_t e = hipStreamQuery(ctx->stream);
         if (e == hipErrorNotReady) continue;
