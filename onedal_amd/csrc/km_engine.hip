@@ -1618,6 +1618,7 @@ struct batch_plan {
     int64_t rows = 0, cfl = 0, kk = 0, pp = 0, oo = 0, hh = 0;
     unsigned kbits = 1, lbits = 0;
     int maxk = 0;
+    double work = 0.0;  // sum of n d k
     // rows grouped by label with the counting sort (every k <= BATCH_HIST_MAX), or
     // with one radix sort of (instance, label) keys
     bool csort = false;
@@ -1680,11 +1681,12 @@ static int tile_bucket(int64_t d, int64_t k) {
 
 static bool mfma_tile_ok(int64_t d, int64_t k) { return d <= 128 && k <= BATCH_MFMA_MAXK; }
 
-// untuned choice per (d, k) bucket: what the tuner picks on this chip (the fastest of
-// the eight variants at each bucket's largest shape).  The matrix cores win from
-// d = 17 on wherever they apply, except for k <= 8 at d <= 64, where 32 centroid
-// columns are mostly padding; narrow VALU tiles win elsewhere.
-static int default_tile(int64_t d, int64_t k) {
+// Untuned choice, the same for all of a plan.  With the table: what the tuner picks on this chip
+// per (d, k) bucket (the fastest of the eight variants at each bucket's largest shape).  The
+// matrix cores win from d = 17 on wherever they apply, except for k <= 8 at d in 33..64, where
+// 32 centroid columns are mostly padding; narrow VALU tiles win elsewhere.  Without it: the
+// narrowest VALU tile that still holds k.
+static int default_tile(int64_t d, int64_t k, bool table) {
     static const int8_t best[KM_BATCH_TILE_BUCKETS] = {
         4, 4, 4, 4, 4, 4,  // d <= 8:   (8, 8)
         4, 4, 4, 4, 7, 4,  // d <= 16:  matrix cores for k in 65..128
@@ -1694,14 +1696,21 @@ static int default_tile(int64_t d, int64_t k) {
         4, 6, 2, 0, 0, 0,  // d <= 256: (8, 8), (16, 4), (32, 8), (64, 8)
         4, 3, 2, 0, 0, 0,  // more
     };
+    if (!table) return k <= 8 ? 4 : k <= 16 ? 3 : k <= 32 ? 2 : 0;
     const int t = best[tile_bucket(d, k)];
     return t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k) ? 4 : t;
 }
 
-// tile variant of an instance (the matrix-core variant only where it applies)
-static int tile_for(const km_ctx* ctx, int64_t d, int64_t k) {
+// Whether a plan of that work (the sum of n d k) and those elements (of n d) takes the table.  Its
+// tile kinds are launched one after the other, and the table has more of them: four
+// iterations of 2 to 128 instances, the table's time by the other's: work 1e6 to 1e8 0.87 to 1.34,
+// 1.08 on average; 1.4e8 to 2.4e9 with a mean k above 16 0.54 to 0.99, below it 0.94 to 1.21.
+static bool plan_table(double work, double elements) { return work >= 1.2e8 && work >= 16.0 * elements; }
+
+// tile variant of an instance (the matrix-core variant only where it applies) of a plan
+static int tile_for(const km_ctx* ctx, int64_t d, int64_t k, bool table) {
     int t = ctx->tile_force > 0 ? ctx->tile_force - 1 : ctx->tile_table[tile_bucket(d, k)];
-    if (t < 0 || (t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k))) t = default_tile(d, k);
+    if (t < 0 || (t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k))) t = default_tile(d, k, table);
     return t;
 }
 
@@ -1793,7 +1802,13 @@ static void plan_build(batch_plan& p, const km_ctx* ctx, const km_batch_instance
     p.kbits = std::max(1u, lbits + ibits);
     // assignment launches: instances grouped by tile variant, in instance order
     std::vector<int> var(B);
-    for (int i = 0; i < B; ++i) var[i] = launch_kind(tile_for(ctx, inst[i].d, inst[i].k), inst[i].d);
+    double elements = 0.0;
+    for (int i = 0; i < B; ++i) {
+        elements += double(inst[i].n) * double(inst[i].d);
+        p.work += double(inst[i].n) * double(inst[i].d) * double(inst[i].k);
+    }
+    const bool table = plan_table(p.work, elements);
+    for (int i = 0; i < B; ++i) var[i] = launch_kind(tile_for(ctx, inst[i].d, inst[i].k, table), inst[i].d);
     p.asel.clear();
     p.apre.clear();
     p.launches.clear();
@@ -2235,7 +2250,7 @@ static void batch_autotune(km_ctx* ctx, int32_t* table_out, int64_t table_len) {
             for (int i = 0; i < NI; ++i)
                 q[i] = km_batch_instance_f32{X + i * n * d, C + int64_t(i) * k * d, nullptr, lab + i * n, n, d, k};
             float best_ms = std::numeric_limits<float>::infinity();
-            int best_v = default_tile(d, k);
+            int best_v = default_tile(d, k, true);
             for (int v = 0; v < BATCH_TILES; ++v) {
                 if (v == BATCH_TILE_MFMA && !mfma_tile_ok(d, k)) continue;
                 ctx->tile_force = v + 1;
