@@ -1846,13 +1846,18 @@ static int batch_grid(const km_ctx* ctx, int64_t items) {
     return int(std::max<int64_t>(1, std::min<int64_t>(items, cap)));
 }
 
+// least iterations times work of a plan that keeps bounds
+constexpr double BATCH_BOUND_WORK = 2e10;
+
 // Device workspace of the plan and the table upload (stream-ordered: the host
 // tables must stay alive until the stream has passed the copies).
 static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p, int64_t iterations = 0) {
     const int B = p.B;
-    // Bounds pay from the fourth iteration on, when most rows are certain; fewer
-    // iterations would only add their two launches each
-    p.bounds = p.train && p.csort && iterations >= 5;
+    // Bounds pay from the fourth iteration on, when most rows are certain, and where an
+    // iteration's work is more than their launches, about 40 us.  Work 3e10: 5 iterations 11.6 ->
+    // 9.4 ms; 2.9e9, 8 iterations even, 20 iterations 6.8 -> 6.4; 1.1e9, 20 iterations 6.0 -> 6.4 and
+    // 6.8 -> 6.3 (16 and 128 instances); 5e8 4.2 -> 4.7 and 4.5 -> 3.9; 1.5e7 1.8 -> 2.2
+    p.bounds = p.train && p.csort && iterations >= 5 && double(iterations) * p.work >= BATCH_BOUND_WORK;
     if (p.bounds) {
         p.prev = ws.prev.get<int32_t>(p.rows);
         fill<int32_t>(ctx, p.prev, p.rows, -1);
