@@ -1851,7 +1851,7 @@ constexpr double BATCH_BOUND_WORK = 2e10;
 
 // Device workspace of the plan and the table upload (stream-ordered: the host
 // tables must stay alive until the stream has passed the copies).
-static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p, int64_t iterations = 0) {
+static void plan_upload(km_ctx* ctx, batch_ws& ws, batch_plan& p, int64_t iterations) {
     const int B = p.B;
     // Bounds pay from the fourth iteration on, when most rows are certain, and where an
     // iteration's work is more than their launches, about 40 us.  Work 3e10: 5 iterations 11.6 ->
@@ -2164,17 +2164,6 @@ static void batch_train(km_ctx* ctx, const km_batch_instance_f32* inst, int64_t 
         }
         return;
     }
-    // final assignment (into the callers' label buffers), objective, centroids out
-    plan_finish(ctx, p);
-    if (ctx->timing) KM_HIP(hipEventRecord(e1, ctx->stream));
-    KM_HIP(hipMemcpyAsync(obj_out, p.objd, sizeof(double) * p.B, hipMemcpyDeviceToHost, ctx->stream));
-    KM_HIP(hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < p.B; ++i) iters_out[i] = max_iter;
-    if (ctx->timing) {
-        float ms = 0.f;
-        KM_HIP(hipEventElapsedTime(&ms, e0, e1));
-        ctx->stats.iterations_ms = ms;
-    }
 }
 
 // One step of a continuous batch (km_batch_step_f32): `iterations` Lloyd
@@ -2196,18 +2185,19 @@ static void batch_step(km_ctx* ctx, const km_batch_instance_f32* it, int64_t n_i
     if (n_fin > 0) plan_build(pf, ctx, fin, n_fin, false);
     ctx->stats = km_stats{};
     if (n_it > 0 && iterations > 0) {
-        plan_upload(ctx, ctx->bws, pi);
+        // no bounds: a serving loop's step iterates four times at most
+        plan_upload(ctx, ctx->bws, pi, 0);
         plan_copy_centroids(ctx, pi, 0);
         for (int64_t t = 0; t < iterations; ++t) plan_iteration(ctx, pi);
         plan_copy_centroids(ctx, pi, 1);
     } else if (n_it > 0) {
         // zero iterations: centroids are carried over unchanged
-        plan_upload(ctx, ctx->bws, pi);
+        plan_upload(ctx, ctx->bws, pi, 0);
         plan_copy_centroids(ctx, pi, 0);
         plan_copy_centroids(ctx, pi, 1);
     }
     if (n_fin > 0) {
-        plan_upload(ctx, ctx->bws_fin, pf);
+        plan_upload(ctx, ctx->bws_fin, pf, 0);
         plan_copy_centroids(ctx, pf, 0);
         plan_finish(ctx, pf);
         KM_HIP(hipMemcpyAsync(obj_out, pf.objd, sizeof(double) * pf.B, hipMemcpyDeviceToHost,
@@ -2261,7 +2251,7 @@ static void batch_autotune(km_ctx* ctx, int32_t* table_out, int64_t table_len) {
                 ctx->tile_force = v + 1;
                 batch_plan p;
                 plan_build(p, ctx, q.data(), NI, false);
-                plan_upload(ctx, ctx->bws_fin, p);
+                plan_upload(ctx, ctx->bws_fin, p, 0);
                 plan_copy_centroids(ctx, p, 0);
                 plan_assign(ctx, p, nullptr, nullptr, 1, p.sel);  // warm-up
                 float ms_v = std::numeric_limits<float>::infinity();
