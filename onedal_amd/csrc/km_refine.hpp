@@ -290,10 +290,12 @@ __global__ __launch_bounds__(256) void refine_full_kernel(const F* __restrict__ 
 // register chunk of 32 bytes per feature group loaded one chunk ahead of use, and
 // forms the exact-form sums of 8 rows in feature order, reading the rows as LDS
 // broadcasts.  Same scan semantics as refine_full_kernel.
-// The list is usually short, so the kernel is bound by one wave's chain of
-// centroid reads, not by their volume: WS waves of a workgroup share 8 rows and
-// take every WS-th tile (WS = 4 for k > 128, where one wave alone took the 16 tiles
-// of k = 1024, d = 128 in 0.23 ms a pass), and their results meet in LDS.
+// A short list is bound by one wave's chain of centroid reads, not by their volume: WS waves
+// of a workgroup share 8 rows and take every WS-th tile (up to 4 for k > 128, where one
+// wave alone took the 16 tiles of k = 1024, d = 128 in 0.23 ms a pass), and their results meet
+// in LDS.  A list that fills the workgroups without that is not shared: five tiles on four
+// waves take two turns (rows without clusters, n=3e5, d=200, k=300, most of them listed: 1.34
+// ms a pass shared by four, 0.77 not shared).
 template <typename F>
 __global__ __launch_bounds__(256) void refine_full_vec_kernel(const F* __restrict__ X, int d,
                                                               const F* __restrict__ C, int k,
@@ -309,10 +311,12 @@ __global__ __launch_bounds__(256) void refine_full_vec_kernel(const F* __restric
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int WS = k > 128 ? 4 : k > 64 ? 2 : 1;  // waves per row group
-    const int RB = RW * (4 / WS);                 // rows per workgroup
-    const int rg = wave / WS, cw = wave % WS;     // this wave's row group and tile phase
     const int total = L.counters[1];
+    // waves per row group: the most that leave no row to a second turn of the workgroups
+    const int64_t turn = int64_t(gridDim.x) * RW;  // rows of a turn with four
+    const int WS = total > 2 * turn ? 1 : k > 128 && total <= turn ? 4 : k > 64 ? 2 : 1;
+    const int RB = RW * (4 / WS);              // rows per workgroup
+    const int rg = wave / WS, cw = wave % WS;  // this wave's row group and tile phase
     const int nbatch = (total + RB - 1) / RB;
     const int nv = d / 4;
     const bool one_chunk = nv <= VT;
