@@ -2374,17 +2374,24 @@ static void init_centroids(km_ctx* ctx, const F* X, int64_t n, int64_t d, int64_
         const int64_t first = int64_t(rng_index(seed, RNG_STREAM_PLUS_PLUS, 0, uint64_t(n)));
         hipLaunchKernelGGL(init_first_kernel<F>, dim3(1), dim3(256), 0, ctx->stream, Xd, di, first, Cd, s.cnew, dp);
         KM_LAUNCH_CHECK();
-        const int grid = grid_for(ctx, n, INIT_PART, 4);
+        const bool few = n <= INIT_FEW_ROWS;
+        const int grid = grid_for(ctx, n, few ? 256 : 1024, 4);
         const int vectors = int((d * int64_t(sizeof(F)) + 15) / 16);  // 16-byte vectors of a row
         for (int64_t t = 1; t < k; ++t) {
             s.t = t;
             s.u = rng_uniform01(seed, RNG_STREAM_PLUS_PLUS, uint64_t(t));
-#define KM_INIT_STEP(PP_) \
-    hipLaunchKernelGGL((init_step_kernel<F, PP_>), dim3(grid), dim3(256), 0, ctx->stream, s)
-            if (vectors <= 1) KM_INIT_STEP(1);
-            else if (vectors <= 2) KM_INIT_STEP(2);
-            else if (vectors <= 4) KM_INIT_STEP(4);
-            else KM_INIT_STEP(8);
+#define KM_INIT_STEP(PP_)                                                                                     \
+    if (few) hipLaunchKernelGGL((init_step_kernel<F, PP_, 1>), dim3(grid), dim3(256), 0, ctx->stream, s);     \
+    else hipLaunchKernelGGL((init_step_kernel<F, PP_, 4>), dim3(grid), dim3(256), 0, ctx->stream, s)
+            if (vectors <= 1) {
+                KM_INIT_STEP(1);
+            } else if (vectors <= 2) {
+                KM_INIT_STEP(2);
+            } else if (vectors <= 4) {
+                KM_INIT_STEP(4);
+            } else {
+                KM_INIT_STEP(8);
+            }
 #undef KM_INIT_STEP
             KM_LAUNCH_CHECK();
             hipLaunchKernelGGL(init_pick_kernel<F>, dim3(grid_for(ctx, nchunks, 1, 2)), dim3(256), 0, ctx->stream, s,

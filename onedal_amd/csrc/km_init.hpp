@@ -245,14 +245,18 @@ __global__ __launch_bounds__(256) void init_select_kernel(const double* __restri
 // rounding, above D2 means that D2 stays, and the row is not read (12 bytes a row
 // instead of d elements).  On clustered rows about half of the reads remain.
 //
-// A workgroup takes INIT_PART rows; each wave packs its open rows into a list and
+// A workgroup takes 256 U rows (U = 4, or 1 where that would leave the chip idle); each wave packs its open rows into a list and
 // takes 64 at a time: PP lanes read one piece of PP x 16 bytes of a row, so for wide
 // rows (PP = 8) every load is a full 128-byte line; the pieces pass through LDS
 // (swizzled: 16-byte vector p of row r at p ^ (r % PP)) to the lane that owns the row,
 // and the next piece's loads are in flight while a piece is summed.  Each D2 is
 // summed in feature order; padding adds exact zeros.
 // ---------------------------------------------------------------------------
-constexpr int INIT_PART = 1024;  // rows per workgroup item
+// Rows up to which an item is 256 rows instead of 1024: a wave's four lists of 64 rows one after
+// the other are the time of a step that has no work for the chip.  60 centroids on (n, d), items of
+// 1024 and of 256 rows: (20000, 300) 4.66 and 2.12 ms, (1e5, 512) 7.32 and 3.63, (3e5, 128) 2.80 and
+// 2.71, (5e5, 64) 2.45 and 2.56, (1e6, 64) 3.07 and 3.47, as fewer rows pack less well.
+constexpr int64_t INIT_FEW_ROWS = 400000;
 
 template <typename F>
 struct init_step {
@@ -270,26 +274,26 @@ struct init_step {
     uint32_t* ticket;
 };
 
-template <typename F, int PP>
+template <typename F, int PP, int U>
 __global__ __launch_bounds__(256, 4) void init_step_kernel(init_step<F> s) {
+    constexpr int PART = 256 * U;           // rows per workgroup item
     constexpr int N = 16 / int(sizeof(F));  // elements per 16 bytes
     constexpr int FP = PP * N;              // features per piece
     constexpr int RL = 64 / PP;             // rows per load instruction
     typedef F V __attribute__((ext_vector_type(N)));
     typedef F VU __attribute__((ext_vector_type(N), aligned(sizeof(F))));  // rows of any width
-    constexpr int U = INIT_PART / 256;
     __shared__ __align__(16) V stage[4][64 * PP];
-    __shared__ uint16_t list[4][INIT_PART / 4];
+    __shared__ uint16_t list[4][PART / 4];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int d = s.d;
     const int pieces = (d + FP - 1) / FP;
     const bool first = s.t == 1;
     const double* __restrict__ c = s.cnew;
-    const int64_t nparts = (s.n + INIT_PART - 1) / INIT_PART;
+    const int64_t nparts = (s.n + PART - 1) / PART;
     const uint64_t below = (uint64_t(1) << lane) - 1u;
     for (int64_t b = blockIdx.x; b < nparts; b += gridDim.x) {
-        const int64_t r0 = b * INIT_PART;
-        const int rows = int(min<int64_t>(INIT_PART, s.n - r0));
+        const int64_t r0 = b * PART;
+        const int rows = int(min<int64_t>(PART, s.n - r0));
         int cnt = 0;
         {
             double v[U];
