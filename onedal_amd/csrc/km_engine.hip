@@ -643,8 +643,15 @@ static void assign(km_ctx* ctx, work<F>& w, const F* C, int path) {
 // d64 of every row against its label's centroid
 template <typename F>
 static void launch_d64(km_ctx* ctx, const F* X, int64_t n, int d, const F* C, const int32_t* labels, double* d64) {
-    hipLaunchKernelGGL(row_d64_kernel<F>, dim3(grid_for(ctx, n, D64_ROWS, 8)), dim3(256), 0, ctx->stream, X, n, d, C,
-                       labels, d64);
+#define KM_D64(PP_)                                                                                                 \
+    hipLaunchKernelGGL((row_d64_kernel<F, PP_>), dim3(grid_for(ctx, n, D64_ROWS, 8)), dim3(256), 0, ctx->stream, X, \
+                       n, d, C, labels, d64)
+    const int vectors = int((d * int64_t(sizeof(F)) + 15) / 16);  // 16-byte vectors of a row
+    if (vectors <= 1) KM_D64(1);
+    else if (vectors <= 2) KM_D64(2);
+    else if (vectors <= 4) KM_D64(4);
+    else KM_D64(8);
+#undef KM_D64
     KM_LAUNCH_CHECK();
 }
 

@@ -394,8 +394,10 @@ __global__ __launch_bounds__(256) void reduce_chunks_vec_kernel(
 // t+512, ... in order; the 256 partials are combined by the tree p[t] += p[t+s],
 // s = 128..1; chunk sums are added in chunk order.
 // ---------------------------------------------------------------------------
-// d64 of every row: a wave takes 64 rows, a piece of eight 16-byte vectors at a time.
-// Eight lanes read a row's piece and their label's centroid's (so every load is whole
+// d64 of every row: a wave takes 64 rows, a piece of PP 16-byte vectors at a time (PP = 8,
+// less for rows of fewer vectors: at d = 2 seven of eight lanes would idle, n=1e6 28 us,
+// 6.6 with PP = 1).
+// PP lanes read a row's piece and their label's centroid's (so every load is whole
 // lines: a lane reading its own row asks for a line per lane and load), form the squares
 // and pass them through LDS (16-byte chunk q of row r at q ^ (r % chunks)) to the lane
 // that owns the row, which adds them in feature order while the next piece's loads are in
@@ -403,36 +405,37 @@ __global__ __launch_bounds__(256) void reduce_chunks_vec_kernel(
 // Bound by HBM: n=2e7, d=128 3.25 -> 2.12 ms (4.8 TB/s), n=1e6, d=33 109 -> 44 us, n=3e5,
 // d=50 in double 34 -> 29 us.
 constexpr int D64_ROWS = 256;
-template <typename F>
+template <typename F, int PP>
 __global__ __launch_bounds__(256, 2) void row_d64_kernel(const F* __restrict__ X, int64_t n, int d,
                                                          const F* __restrict__ C,
                                                          const int32_t* __restrict__ labels,
                                                          double* __restrict__ d64) {
     constexpr int N = 16 / int(sizeof(F));  // elements per 16 bytes
-    constexpr int PP = 8, FP = PP * N;      // vectors and features of a piece
+    constexpr int FP = PP * N;              // features of a piece
+    constexpr int RL = 64 / PP;             // rows per load instruction
     constexpr int CH = FP / 2;              // 16-byte chunks of a row's squares
     typedef F V __attribute__((ext_vector_type(N)));
     typedef F VU __attribute__((ext_vector_type(N), aligned(sizeof(F))));  // rows of any width
     typedef double D2 __attribute__((ext_vector_type(2)));
     __shared__ __align__(16) D2 sq[4][64 * CH];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p = lane & 7;
+    const int p = lane % PP;
     const int pieces = (d + FP - 1) / FP;
     for (int64_t w0 = int64_t(blockIdx.x) * D64_ROWS + 64 * wave; w0 < n; w0 += int64_t(gridDim.x) * D64_ROWS) {
         const int rows = int(min<int64_t>(64, n - w0));
         const int lab = labels[w0 + min(lane, rows - 1)];
-        const F *xs[8], *cs[8];  // this lane's vector of rows lane / 8 + 8 i
+        const F *xs[PP], *cs[PP];  // this lane's vector of rows lane / PP + RL i
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = min(rows - 1, 8 * i + (lane >> 3));
+        for (int i = 0; i < PP; ++i) {
+            const int e = min(rows - 1, RL * i + lane / PP);
             xs[i] = X + (w0 + e) * d + p * N;
             cs[i] = C + int64_t(__shfl(lab, e)) * d + p * N;
         }
-        V xv[8], cv[8];
+        V xv[PP], cv[PP];
         auto load = [&](int f0) {
             const int left = d - f0 - p * N;  // elements from this lane's vector to the row's end
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < PP; ++i) {
                 V x{}, c{};
                 if (left >= N) {
                     x = *reinterpret_cast<const VU*>(xs[i] + f0);
@@ -453,8 +456,8 @@ __global__ __launch_bounds__(256, 2) void row_d64_kernel(const F* __restrict__ X
         double acc = 0.0;
         for (int pc = 0; pc < pieces; ++pc) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int r = 8 * i + (lane >> 3);
+            for (int i = 0; i < PP; ++i) {
+                const int r = RL * i + lane / PP;
 #pragma unroll
                 for (int u = 0; u < N / 2; ++u) {
                     const double da = double(xv[i][2 * u]) - double(cv[i][2 * u]);
