@@ -1708,11 +1708,14 @@ static int default_tile(int64_t d, int64_t k, bool table) {
     return t == BATCH_TILE_MFMA && !mfma_tile_ok(d, k) ? 4 : t;
 }
 
-// Whether a plan of that work (the sum of n d k) and those elements (of n d) takes the table.  Its
-// tile kinds are launched one after the other, and the table has more of them: four
-// iterations of 2 to 128 instances, the table's time by the other's: work 1e6 to 1e8 0.87 to 1.34,
-// 1.08 on average; 1.4e8 to 2.4e9 with a mean k above 16 0.54 to 0.99, below it 0.94 to 1.21.
-static bool plan_table(double work, double elements) { return work >= 1.2e8 && work >= 16.0 * elements; }
+// Whether a plan of that work (the sum of n d k) and those elements (of n d) takes the table, which
+// would give it `kinds` tile kinds against `narrow`.  The kinds are launched one after the
+// other: four iterations of 2 to 128 instances, the table's time by the other's: work 1e6 to
+// 1e8 0.87 to 1.34, 1.08 on average; 1.4e8 to 2.4e9 with a mean k above 16 0.54 to 0.99, below it
+// 0.94 to 1.21 with more kinds, 0.75 with as many (128 instances of d = 16, k = 10).
+static bool plan_table(double work, double elements, int kinds, int narrow) {
+    return work >= 1.2e8 && (work >= 16.0 * elements || kinds <= narrow);
+}
 
 // tile variant of an instance (the matrix-core variant only where it applies) of a plan
 static int tile_for(const km_ctx* ctx, int64_t d, int64_t k, bool table) {
@@ -1814,7 +1817,13 @@ static void plan_build(batch_plan& p, const km_ctx* ctx, const km_batch_instance
         elements += double(inst[i].n) * double(inst[i].d);
         p.work += double(inst[i].n) * double(inst[i].d) * double(inst[i].k);
     }
-    const bool table = plan_table(p.work, elements);
+    int kinds[2] = {0, 0};  // without the table and with it
+    for (int t = 0; t < 2; ++t) {
+        bool used[BATCH_LAUNCH_KINDS] = {};
+        for (int i = 0; i < B; ++i) used[launch_kind(tile_for(ctx, inst[i].d, inst[i].k, t == 1), inst[i].d)] = true;
+        for (bool u : used) kinds[t] += u ? 1 : 0;
+    }
+    const bool table = plan_table(p.work, elements, kinds[1], kinds[0]);
     for (int i = 0; i < B; ++i) var[i] = launch_kind(tile_for(ctx, inst[i].d, inst[i].k, table), inst[i].d);
     p.asel.clear();
     p.apre.clear();

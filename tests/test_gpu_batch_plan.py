@@ -20,15 +20,16 @@ def run(engine, shapes, iters, graph=True):
     return xs, c0s, [c.cpu().numpy() for c in cs], [l.cpu().numpy() for l in ls], objs
 
 
-# work 2e6, 5e8 and 1.7e9 (narrow tiles, the table twice), and 2e8 with a mean k of 9 (narrow tiles);
+# work 2e6, 5e8 and 1.7e9 (narrow tiles, the table twice), 2e8 with a mean k of 9
+# (narrow tiles), and with one kind either way (the table);
 # iterations times work below and above 2e10; k on both sides of 8 and 16
 PLANS = [([(1000, 8, 4), (1500, 32, 8), (900, 64, 16), (700, 16, 17)], 6),
          ([(20000, 64, 128), (30000, 128, 80), (5000, 32, 8), (9000, 32, 16)], 6),
          ([(70000, 128, 128), (40000, 64, 100), (8000, 32, 8), (9000, 128, 16), (3000, 33, 30)], 16),
-         ([(300000, 64, 9), (60000, 128, 8), (2000, 32, 40)], 5)]
+         ([(300000, 64, 9), (60000, 128, 8), (2000, 32, 40)], 5), ([(900000, 16, 10)], 5)]
 
 
-@pytest.mark.parametrize("plan", PLANS, ids=["small", "middle", "large", "few_clusters"])
+@pytest.mark.parametrize("plan", PLANS, ids=["small", "middle", "large", "few_clusters", "one_kind"])
 def test_plans_equal_the_oracle(engine, oracle, plan):
     shapes, iters = plan
     xs, c0s, cs, ls, objs = run(engine, shapes, iters)
