@@ -29,7 +29,7 @@ PEAK = {"fp32_mfma_tflops": 157.3, "bf16_mfma_tflops": 2500.0, "hbm_gbs": 8000.0
 # passes (FETCH_SIZE, WRITE_SIZE) scaled by a 1 GiB copy of the same run
 # (profiles/traffic_precision_n20M_d128_k1024.md); hardware counters cannot be read
 # from inside this process.
-MEASURED_TRAFFIC = {"precision_c3": {"bytes": 5.538e9, "read": 5.300e9, "write": 0.238e9,
+MEASURED_TRAFFIC = {"precision_c3": {"bytes": 5.646e9, "read": 5.302e9, "write": 0.344e9,
                                      "source": "profiles/traffic_precision_n20M_d128_k1024.md"}}
 
 WORKLOADS = {
@@ -749,8 +749,8 @@ def run_dense(torch, args, name, steps, warmup, compare=True, cpu_on=True, label
 
     # roofline of the dominant kernel (assignment) over a pass that takes every row (the
     # timed steps' later passes take only the rows whose bounds are open): a call of no
-    # iterations is one such pass.  2*k*d flops per row, three BF16 products each on the
-    # FP32 path.
+    # iterations is one such pass.  2*k*d flops per row, six BF16 products each on the
+    # FP32 path (values in three pieces).
     launches = sum(s["assign_launches"] for s in stats)
     kern_ms = sum(s["assign_kernel_ms"] for s in stats)
     full = []
@@ -758,14 +758,14 @@ def run_dense(torch, args, name, steps, warmup, compare=True, cpu_on=True, label
         eng.train_device(x, c_out, 0, 0.0, bf16=wl["bf16"], out=(torch.empty_like(c_out), torch.empty_like(l_out)))
         full.append(eng.stats()["assign_kernel_ms"])
     avg_ms = sorted(full)[1]
-    flops_per_launch = 2.0 * k * d * n * (1 if wl["bf16"] else 3)
+    flops_per_launch = 2.0 * k * d * n * (1 if wl["bf16"] else 6)
     achieved = flops_per_launch / (avg_ms * 1e-3) / 1e12
     peak = PEAK["bf16_mfma_tflops"]
     mt = MEASURED_TRAFFIC.get(name)
     roof = {"bound": "mfma", "achieved": round(achieved, 2), "peak": peak, "unit": "TFLOP/s",
             "frac": round(achieved / peak, 4), "traffic": mt["bytes"] if mt else None,
             "kernel": "assign (fused distance GEMM + argmin), one pass over every row" +
-                      ("" if wl["bf16"] else "; three BF16 products per FP32 product"),
+                      ("" if wl["bf16"] else "; six BF16 products per FP32 product"),
             "full_launch_ms": round(avg_ms, 4),
             "avg_launch_ms_over_steps": round(kern_ms / max(1, launches), 4)}
     if mt:
@@ -784,7 +784,8 @@ def run_dense(torch, args, name, steps, warmup, compare=True, cpu_on=True, label
 
     comparison = None
     if wl["bf16"] and compare:
-        # same data and init on the plain FP32 path: throughput ratio and label identity
+        # same data and init on the FP32 path (whose products are split BF16, so the ratio is
+        # not the one to FP32 matrix cores): throughput ratio and label identity
         log("fp32 path on the same workload ...")
         c32 = torch.empty_like(c_out)
         l32 = torch.empty_like(l_out)
@@ -794,7 +795,8 @@ def run_dense(torch, args, name, steps, warmup, compare=True, cpu_on=True, label
         t32 = time.perf_counter() - t0
         st32 = eng.stats()
         same = bool(torch.equal(l32, l_out)) and bool(torch.equal(c32, c_out))
-        comparison = {"fp32_path_value": n * iters / t32, "fp32_path_ms_per_step": 1e3 * t32,
+        comparison = {"fp32_path": "split BF16: three pieces a value, six products",
+                      "fp32_path_value": n * iters / t32, "fp32_path_ms_per_step": 1e3 * t32,
                       "speedup_vs_fp32": (n * iters / t32 and pit / (n * iters / t32)),
                       "labels_and_centroids_identical_to_fp32": same,
                       "fp32_assign_avg_launch_ms": st32["assign_kernel_ms"] / max(1, st32["assign_launches"]),
